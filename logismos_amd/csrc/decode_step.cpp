@@ -4,6 +4,7 @@
 // the launchers of this library only.  Nothing is allocated, nothing
 // synchronises; a caller may capture the whole step into a HIP graph.
 #include "launch_common.hpp"
+#include "q4_rows.hpp"
 
 #include <math.h>
 
@@ -185,6 +186,98 @@ bool config_ok(const logismos_decode_config_t* c, int num_seqs, int t, int max_s
     return true;
 }
 
+// Whether every projection of the step can run on the fused few-row kernels.
+bool few_rows(const logismos_decode_config_t& c, const logismos_decode_layer_t* layers, int t) {
+    const int qd = c.num_q_heads * c.head_dim;
+    const int widest = qd > c.intermediate ? qd : c.intermediate;
+    for (int l = 0; l < c.num_layers; ++l)
+        for (const logismos_q4_weight_t* W : {&layers[l].qkv, &layers[l].o, &layers[l].gate_up, &layers[l].down})
+            if (!lg::qgemm_q4_rows_applies(t, c.hidden, widest,
+                                           qd + 2 * c.num_kv_heads * c.head_dim, W->scale, W->zero))
+                return false;
+    return true;
+}
+
+#define LG_TRY(call)                                  \
+    do {                                              \
+        logismos_status_t st__ = (call);              \
+        if (st__ != 0) return st__;                   \
+    } while (0)
+
+// The layers of a step of up to 16 rows on the fused few-row projections (qgemm_q4_rows.hip):
+// every projection is one launch with the norm in front of it and what follows it folded in.
+logismos_status_t few_rows_layers(const logismos_decode_config_t& c,
+                                  const logismos_decode_layer_t* layers,
+                                  const logismos_decode_batch_t* batch, const Workspace& w, int t,
+                                  int max_q, bool direct, logismos_stream_t stream) {
+    hipStream_t st = static_cast<hipStream_t>(stream);
+    const int qd = c.num_q_heads * c.head_dim;
+    const int width = qd + 2 * c.num_kv_heads * c.head_dim;
+    const float scale = 1.0f / sqrtf((float)c.head_dim);
+    lg::RowsArgs base{};
+    base.b = t;
+    base.eps = c.rms_eps;
+    base.h = static_cast<float*>(batch->hidden_f32);
+    auto with = [&](const logismos_q4_weight_t& W, int n, int k) {
+        lg::RowsArgs a = base;
+        a.qw = static_cast<const uint8_t*>(W.qw);
+        a.scale = static_cast<const __half*>(W.scale);
+        a.zero = static_cast<const __half*>(W.zero);
+        a.tiles = n / 16;
+        a.k = k;
+        return a;
+    };
+    for (int l = 0; l < c.num_layers; ++l) {
+        const logismos_decode_layer_t& L = layers[l];
+        lg::RowsArgs a = with(L.qkv, width, c.hidden);
+        a.gain = static_cast<const float*>(L.norm1_w_f32);
+        if (c.kv_turbo3) {
+            // the encoder wants whole head rows: the product as it is, then the operator
+            a.e.out_f32 = reinterpret_cast<float*>(w.qkv);
+            LG_TRY(lg::qgemm_q4_rows_launch(true, lg::kRowsF32, a, st));
+            LG_TRY(logismos_launch_rope_kv_write_f32p_turbo3_bias(
+                w.qkv, 1, L.qkv_bias_f32, batch->positions, batch->rope_cos_f32,
+                batch->rope_sin_f32, batch->slot_mapping, w.q, L.k_pool_f16, L.v_pool_f16, t,
+                c.num_q_heads, c.num_kv_heads, c.head_dim, c.max_pos, stream));
+        } else {
+            a.e.bias = static_cast<const float*>(L.qkv_bias_f32);
+            a.e.positions = batch->positions;
+            a.e.cos_t = static_cast<const float*>(batch->rope_cos_f32);
+            a.e.sin_t = static_cast<const float*>(batch->rope_sin_f32);
+            a.e.slots = batch->slot_mapping;
+            a.e.q_out = reinterpret_cast<__half*>(w.q);
+            a.e.k_pool = static_cast<__half*>(L.k_pool_f16);
+            a.e.v_pool = static_cast<__half*>(L.v_pool_f16);
+            a.e.hq = c.num_q_heads;
+            a.e.hkv = c.num_kv_heads;
+            a.e.head_dim = c.head_dim;
+            a.e.max_pos = c.max_pos;
+            a.e.tiles_per_head_inv = (unsigned)(((1 << 20) + c.head_dim / 16 - 1) / (c.head_dim / 16));
+            LG_TRY(lg::qgemm_q4_rows_launch(true, lg::kRowsQkv, a, st));
+        }
+        LG_TRY(lg::paged_attn_launch(
+            w.q, L.k_pool_f16, L.v_pool_f16, batch->block_tables, batch->cu_seqlens,
+            batch->context_lens, direct ? w.attn_b : w.attn_out, w.attn_ws, batch->num_seqs, t, max_q,
+            c.num_q_heads, c.num_kv_heads, c.head_dim, c.block_size, c.max_blocks_per_seq,
+            batch->num_splits, scale, 1, LOGISMOS_ATTN_PHASE_ALL, direct ? 2 : 1,
+            c.kv_turbo3 ? 1 : 0, stream));
+        if (!direct)
+            LG_TRY(logismos_launch_q4_prepare_x_bf16(w.attn_out, w.attn_b, t, qd, stream));
+        a = with(L.o, c.hidden, qd);
+        a.xprep = reinterpret_cast<const lg::uint4_t*>(w.attn_b);
+        LG_TRY(lg::qgemm_q4_rows_launch(false, lg::kRowsRes, a, st));
+        a = with(L.gate_up, 2 * c.intermediate, c.hidden);
+        a.gain = static_cast<const float*>(L.norm2_w_f32);
+        a.e.inter = c.intermediate;
+        a.e.act = reinterpret_cast<lg::uint4_t*>(w.act);
+        LG_TRY(lg::qgemm_q4_rows_launch(true, lg::kRowsSilu, a, st));
+        a = with(L.down, c.hidden, c.intermediate);
+        a.xprep = reinterpret_cast<const lg::uint4_t*>(w.act);
+        LG_TRY(lg::qgemm_q4_rows_launch(false, lg::kRowsRes, a, st));
+    }
+    return 0;
+}
+
 // total_tokens / max_seqlen_q of a batch: 0 means "one new token per sequence"
 int batch_tokens(const logismos_decode_batch_t* b) {
     return b->total_tokens > 0 ? b->total_tokens : b->num_seqs;
@@ -206,12 +299,6 @@ extern "C" size_t logismos_decode_step_workspace_bytes_tokens(const logismos_dec
     if (!config_ok(cfg, num_seqs, total_tokens, 1) || num_splits <= 0) return 0;
     return carve(*cfg, num_seqs, total_tokens, num_splits, nullptr).total;
 }
-
-#define LG_TRY(call)                                  \
-    do {                                              \
-        logismos_status_t st__ = (call);              \
-        if (st__ != 0) return st__;                   \
-    } while (0)
 
 extern "C" logismos_status_t logismos_launch_decode_step(const logismos_decode_config_t* cfg,
                                                          const logismos_decode_layer_t* layers,
@@ -386,77 +473,81 @@ extern "C" logismos_status_t logismos_launch_decode_step(const logismos_decode_c
                                                  c.rms_eps, stream));
         return last_only ? project_last_rows() : 0;
     }
-    // The normed input of a layer's first half is produced where the residual stream is
-    // completed: before layer 0 here, afterwards by the add + norm that folds a chunk's down
-    // projection into h (with the NEXT layer's gains).
-    for (int ch = 0; ch < w.chunks; ++ch)
-        LG_TRY(logismos_launch_add_rms_norm_f32p_xprep(
-            h + (int64_t)ch * kChunkRows * c.hidden, nullptr, 0, layers[0].norm1_w_f32,
-            w.xn + ch * w.xn_stride, rows_of(ch), c.hidden, c.rms_eps, stream));
     int res_parts = 0;  // split-K parts of the last down projection not yet folded into h
-    for (int l = 0; l < c.num_layers; ++l) {
-        const logismos_decode_layer_t& L = layers[l];
-        const bool last_layer = l + 1 == c.num_layers;
-        // ---- first half, chunk by chunk: q/k/v projection, RoPE, K/V rows into the pools
-        for (int ch = 0; ch < w.chunks; ++ch) {
-            const int r0 = ch * kChunkRows, rows = rows_of(ch);
-            LG_TRY(logismos_launch_qgemm_q4g128_f32_splitk_xprep(
-                w.xn + ch * w.xn_stride, L.qkv.qw, L.qkv.scale, L.qkv.zero, w.qkv, rows, width,
-                c.hidden, stream));
-            const int j = logismos_qgemm_q4g128_splitk_xprep_parts(rows, width, c.hidden);
-            const auto rope_kv_write = c.kv_turbo3 ? logismos_launch_rope_kv_write_f32p_turbo3_bias
-                                                   : logismos_launch_rope_kv_write_f32p_bias;
-            LG_TRY(rope_kv_write(w.qkv, j, L.qkv_bias_f32, batch->positions + r0,
-                                 batch->rope_cos_f32, batch->rope_sin_f32,
-                                 batch->slot_mapping + r0, w.q + (size_t)r0 * qd * 2, L.k_pool_f16,
-                                 L.v_pool_f16, rows, c.num_q_heads, c.num_kv_heads, c.head_dim,
-                                 c.max_pos, stream));
-        }
-        // ---- attention over the whole ragged batch.  One chunk of decode rows: the result
-        // goes straight into the prepared layout of the o projection; otherwise bf16 rows that
-        // each chunk prepares for itself.
-        LG_TRY(lg::paged_attn_launch(
-            w.q, L.k_pool_f16, L.v_pool_f16, batch->block_tables, batch->cu_seqlens,
-            batch->context_lens, direct ? w.attn_b : w.attn_out,
-            w.attn_ws, num_seqs, t, max_q, c.num_q_heads, c.num_kv_heads, c.head_dim, c.block_size,
-            c.max_blocks_per_seq, batch->num_splits, scale, 1, LOGISMOS_ATTN_PHASE_ALL,
-            direct ? 2 : 1, c.kv_turbo3 ? 1 : 0, stream));
-        // ---- second half, chunk by chunk
-        for (int ch = 0; ch < w.chunks; ++ch) {
-            const int r0 = ch * kChunkRows, rows = rows_of(ch);
-            float* hc = h + (int64_t)r0 * c.hidden;
-            if (!direct)
-                LG_TRY(logismos_launch_q4_prepare_x_bf16(w.attn_out + (size_t)r0 * qd * 2, w.attn_b,
-                                                         rows, qd, stream));
-            LG_TRY(logismos_launch_qgemm_q4g128_f32_splitk_xprep(
-                w.attn_b, L.o.qw, L.o.scale, L.o.zero, w.proj, rows, c.hidden, qd, stream));
+    if (few_rows(c, layers, t)) {
+        LG_TRY(few_rows_layers(c, layers, batch, w, t, max_q, direct, stream));
+    } else {
+        // The normed input of a layer's first half is produced where the residual stream is
+        // completed: before layer 0 here, afterwards by the add + norm that folds a chunk's down
+        // projection into h (with the NEXT layer's gains).
+        for (int ch = 0; ch < w.chunks; ++ch)
             LG_TRY(logismos_launch_add_rms_norm_f32p_xprep(
-                hc, w.proj, logismos_qgemm_q4g128_splitk_xprep_parts(rows, c.hidden, qd),
-                L.norm2_w_f32, w.xn + ch * w.xn_stride, rows, c.hidden, c.rms_eps, stream));
-            LG_TRY(logismos_launch_qgemm_q4g128_f32_splitk_xprep(
-                w.xn + ch * w.xn_stride, L.gate_up.qw, L.gate_up.scale, L.gate_up.zero, w.gate_up,
-                rows, 2 * c.intermediate, c.hidden, stream));
-            LG_TRY(logismos_launch_silu_mul_f32p_xprep(
-                w.gate_up,
-                logismos_qgemm_q4g128_splitk_xprep_parts(rows, 2 * c.intermediate, c.hidden), w.act,
-                rows, c.intermediate, stream));
-            LG_TRY(logismos_launch_qgemm_q4g128_f32_splitk_xprep(
-                w.act, L.down.qw, L.down.scale, L.down.zero, w.proj, rows, c.hidden, c.intermediate,
-                stream));
-            const int j_down =
-                logismos_qgemm_q4g128_splitk_xprep_parts(rows, c.hidden, c.intermediate);
-            if (!last_layer) {
-                // fold the down projection into h and norm for the next layer's first half
+                h + (int64_t)ch * kChunkRows * c.hidden, nullptr, 0, layers[0].norm1_w_f32,
+                w.xn + ch * w.xn_stride, rows_of(ch), c.hidden, c.rms_eps, stream));
+        for (int l = 0; l < c.num_layers; ++l) {
+            const logismos_decode_layer_t& L = layers[l];
+            const bool last_layer = l + 1 == c.num_layers;
+            // ---- first half, chunk by chunk: q/k/v projection, RoPE, K/V rows into the pools
+            for (int ch = 0; ch < w.chunks; ++ch) {
+                const int r0 = ch * kChunkRows, rows = rows_of(ch);
+                LG_TRY(logismos_launch_qgemm_q4g128_f32_splitk_xprep(
+                    w.xn + ch * w.xn_stride, L.qkv.qw, L.qkv.scale, L.qkv.zero, w.qkv, rows, width,
+                    c.hidden, stream));
+                const int j = logismos_qgemm_q4g128_splitk_xprep_parts(rows, width, c.hidden);
+                const auto rope_kv_write = c.kv_turbo3 ? logismos_launch_rope_kv_write_f32p_turbo3_bias
+                                                       : logismos_launch_rope_kv_write_f32p_bias;
+                LG_TRY(rope_kv_write(w.qkv, j, L.qkv_bias_f32, batch->positions + r0,
+                                     batch->rope_cos_f32, batch->rope_sin_f32,
+                                     batch->slot_mapping + r0, w.q + (size_t)r0 * qd * 2, L.k_pool_f16,
+                                     L.v_pool_f16, rows, c.num_q_heads, c.num_kv_heads, c.head_dim,
+                                     c.max_pos, stream));
+            }
+            // ---- attention over the whole ragged batch.  One chunk of decode rows: the result
+            // goes straight into the prepared layout of the o projection; otherwise bf16 rows that
+            // each chunk prepares for itself.
+            LG_TRY(lg::paged_attn_launch(
+                w.q, L.k_pool_f16, L.v_pool_f16, batch->block_tables, batch->cu_seqlens,
+                batch->context_lens, direct ? w.attn_b : w.attn_out,
+                w.attn_ws, num_seqs, t, max_q, c.num_q_heads, c.num_kv_heads, c.head_dim, c.block_size,
+                c.max_blocks_per_seq, batch->num_splits, scale, 1, LOGISMOS_ATTN_PHASE_ALL,
+                direct ? 2 : 1, c.kv_turbo3 ? 1 : 0, stream));
+            // ---- second half, chunk by chunk
+            for (int ch = 0; ch < w.chunks; ++ch) {
+                const int r0 = ch * kChunkRows, rows = rows_of(ch);
+                float* hc = h + (int64_t)r0 * c.hidden;
+                if (!direct)
+                    LG_TRY(logismos_launch_q4_prepare_x_bf16(w.attn_out + (size_t)r0 * qd * 2, w.attn_b,
+                                                             rows, qd, stream));
+                LG_TRY(logismos_launch_qgemm_q4g128_f32_splitk_xprep(
+                    w.attn_b, L.o.qw, L.o.scale, L.o.zero, w.proj, rows, c.hidden, qd, stream));
                 LG_TRY(logismos_launch_add_rms_norm_f32p_xprep(
-                    hc, w.proj, j_down, layers[l + 1].norm1_w_f32, w.xn + ch * w.xn_stride, rows,
-                    c.hidden, c.rms_eps, stream));
-            } else if (!one_chunk) {
-                // last layer of a multi-chunk step: the final norm of this chunk's rows
-                LG_TRY(logismos_launch_add_rms_norm_f32p(
-                    hc, w.proj, j_down, batch->final_norm_w_f32,
-                    norm_dst + (size_t)r0 * c.hidden * 2, rows, c.hidden, c.rms_eps, stream));
-            } else {
-                res_parts = j_down;
+                    hc, w.proj, logismos_qgemm_q4g128_splitk_xprep_parts(rows, c.hidden, qd),
+                    L.norm2_w_f32, w.xn + ch * w.xn_stride, rows, c.hidden, c.rms_eps, stream));
+                LG_TRY(logismos_launch_qgemm_q4g128_f32_splitk_xprep(
+                    w.xn + ch * w.xn_stride, L.gate_up.qw, L.gate_up.scale, L.gate_up.zero, w.gate_up,
+                    rows, 2 * c.intermediate, c.hidden, stream));
+                LG_TRY(logismos_launch_silu_mul_f32p_xprep(
+                    w.gate_up,
+                    logismos_qgemm_q4g128_splitk_xprep_parts(rows, 2 * c.intermediate, c.hidden), w.act,
+                    rows, c.intermediate, stream));
+                LG_TRY(logismos_launch_qgemm_q4g128_f32_splitk_xprep(
+                    w.act, L.down.qw, L.down.scale, L.down.zero, w.proj, rows, c.hidden, c.intermediate,
+                    stream));
+                const int j_down =
+                    logismos_qgemm_q4g128_splitk_xprep_parts(rows, c.hidden, c.intermediate);
+                if (!last_layer) {
+                    // fold the down projection into h and norm for the next layer's first half
+                    LG_TRY(logismos_launch_add_rms_norm_f32p_xprep(
+                        hc, w.proj, j_down, layers[l + 1].norm1_w_f32, w.xn + ch * w.xn_stride, rows,
+                        c.hidden, c.rms_eps, stream));
+                } else if (!one_chunk) {
+                    // last layer of a multi-chunk step: the final norm of this chunk's rows
+                    LG_TRY(logismos_launch_add_rms_norm_f32p(
+                        hc, w.proj, j_down, batch->final_norm_w_f32,
+                        norm_dst + (size_t)r0 * c.hidden * 2, rows, c.hidden, c.rms_eps, stream));
+                } else {
+                    res_parts = j_down;
+                }
             }
         }
     }
