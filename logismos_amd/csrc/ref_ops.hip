@@ -15,6 +15,7 @@
 // takes any M, N, K.
 #include "device_utils.hpp"
 #include "launch_common.hpp"
+#include "q4_common.hpp"
 
 #include <hip/hip_fp16.h>
 #include <math.h>
@@ -63,6 +64,45 @@ __global__ __launch_bounds__(kRowThreads) void rms_norm_fp16_kernel(
         yr[j] = __float2half_rn(__half2float(xr[j]) * inv_rms * __half2float(w[j]));
 }
 
+// The same for rows of whole 16-byte pieces that fit a wave's registers (n a multiple of 8, at
+// most 512 * NP): one wave per row, read once, four rows per workgroup, instead of two passes of
+// 2-byte accesses by a workgroup per row.  For 2036 x 1536 this and the rotation below together
+// went from 11.8 to 5.7 us (12 MB each way through memory).
+template <int NP>
+__global__ __launch_bounds__(256) void rms_norm_fp16_wave_kernel(const uint4_t* __restrict__ x,
+                                                                 const uint4_t* __restrict__ w,
+                                                                 uint4_t* __restrict__ y, int m,
+                                                                 int pieces, float inv_n, float eps) {
+    const int row = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+    if (row >= m) return;
+    uint4_t xv[NP], wv[NP];
+#pragma unroll
+    for (int p = 0; p < NP; ++p) {
+        xv[p] = wv[p] = uint4_t{0u, 0u, 0u, 0u};
+        if (p * 64 + lane < pieces) {
+            xv[p] = x[(int64_t)row * pieces + p * 64 + lane];
+            wv[p] = w[p * 64 + lane];
+        }
+    }
+    float part = 0.0f;
+#pragma unroll
+    for (int p = 0; p < NP; ++p) {
+        const half8_t v = __builtin_bit_cast(half8_t, xv[p]);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) part = fmaf((float)v[e], (float)v[e], part);
+    }
+    const float inv_rms = 1.0f / sqrtf(wave_sum(part) * inv_n + eps);
+#pragma unroll
+    for (int p = 0; p < NP; ++p) {
+        if (p * 64 + lane >= pieces) continue;
+        const half8_t v = __builtin_bit_cast(half8_t, xv[p]), g = __builtin_bit_cast(half8_t, wv[p]);
+        half8_t o;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) o[e] = (_Float16)((float)v[e] * inv_rms * (float)g[e]);
+        y[(int64_t)row * pieces + p * 64 + lane] = __builtin_bit_cast(uint4_t, o);
+    }
+}
+
 // Row softmax, fp32 inside: max-subtracted exponentials times the reciprocal of their sum; a
 // row whose maximum is -inf (every entry -inf) becomes uniform 1/n
 // (`softmax_fp16_ref`, crates/kernels/src/softmax/cpu.rs:14-74)
@@ -108,6 +148,32 @@ __global__ __launch_bounds__(256) void rope_fp16_kernel(unsigned* __restrict__ q
     const float y1 = x0 * cs.y + x1 * cs.x;
     qk_pairs[idx] = (unsigned)__half_as_ushort(__float2half_rn(y0)) |
                     ((unsigned)__half_as_ushort(__float2half_rn(y1)) << 16);
+}
+
+// The same for head rows of whole 16-byte pieces (head_dim a multiple of 8): one thread per four
+// pairs, grid (pieces of a token, seq, batch), no 64-bit division.
+__global__ __launch_bounds__(256) void rope_fp16_pieces_kernel(uint4_t* __restrict__ qk,
+                                                               const float4_t* __restrict__ cos_sin,
+                                                               int token_pieces, int head_pieces) {
+    const int t = blockIdx.x * 256 + threadIdx.x;
+    if (t >= token_pieces) return;
+    const int s = blockIdx.y;
+    const unsigned i = (unsigned)t % (unsigned)head_pieces;
+    uint4_t* const at = qk + ((int64_t)blockIdx.z * gridDim.y + s) * token_pieces + t;
+    const float4_t* const cs = cos_sin + ((int64_t)s * head_pieces + i) * 2;
+    const half8_t v = __builtin_bit_cast(half8_t, *at);
+    half8_t o;
+#pragma unroll
+    for (int q = 0; q < 2; ++q) {
+        const float4_t c = cs[q];
+#pragma unroll
+        for (int p = 0; p < 2; ++p) {
+            const float x0 = (float)v[4 * q + 2 * p], x1 = (float)v[4 * q + 2 * p + 1];
+            o[4 * q + 2 * p] = (_Float16)(x0 * c[2 * p] - x1 * c[2 * p + 1]);
+            o[4 * q + 2 * p + 1] = (_Float16)(x0 * c[2 * p + 1] + x1 * c[2 * p]);
+        }
+    }
+    *at = __builtin_bit_cast(uint4_t, o);
 }
 
 // D = A[M,K] . B[K,N], one thread per output element, fp32 accumulation in ascending k with
@@ -271,6 +337,153 @@ __global__ __launch_bounds__(256) void matmul_mfma_fp16_kernel(const _Float16* _
         }
 }
 
+// The same product for rows that are whole 16-byte pieces (n and k multiples of 8): a workgroup
+// of four waves owns a TM x TN tile, each wave a quarter.  A [TM x KS] and B [KS x TN] slabs go to
+// LDS as they lie in memory; the B operand -- eight consecutive k of one column -- comes out of
+// the row-major slab through the transposing LDS read (two ds_read_b64_tr_b16: inside 16 lanes,
+// lane L receives element L % 4 of the 8-byte pieces that the lanes L / 4 + 4 i point at, so
+// lanes pointing at 4 k x 16 columns come back with 4 k of one column each).  A slab is asked
+// for one slab ahead of its LDS store, two ahead of its products; LDS is double buffered, one
+// barrier per slab.
+//
+// What bounds it at an encoder's sizes: a slab is a chain store -> barrier -> operand read ->
+// products of about 0.5 us whatever its size, so small matrices take small tiles (more
+// workgroups share a compute unit and fill each other's waits) and long slabs.  The kernel
+// above, one 128 x 128 tile per compute unit and 32 columns per slab, takes 0.9 us per slab.
+// us, this kernel / the one above:  2036 x 1536 x 1536 22.9 / 44.0 (419 TFLOP/s),
+// 16 x 1536 x 1536 10.4 / 33.1, 128 x 4096 x 4096 26.7 / 102.8, 4096^3 211 / 259,
+// 8192 x 8192 x 4096 735 / 816 (748 TFLOP/s).
+template <int TM, int TN, int KS>
+__global__ __launch_bounds__(256) void matmul_tiled_fp16_kernel(const _Float16* __restrict__ a,
+                                                                const _Float16* __restrict__ b,
+                                                                _Float16* __restrict__ d, int m,
+                                                                int n, int k) {
+    typedef short short4_t __attribute__((ext_vector_type(4)));
+    typedef __attribute__((address_space(3))) short4_t lds_short4_t;
+    constexpr int AS = KS + 8;                     // halfs per LDS row of A: operand reads conflict-free
+    constexpr int BS = TN + 16;                    // ... and of B
+    constexpr int AP = TM * KS / 8 / 256;        // pieces per thread
+    constexpr int BP = TN * KS / 8 / 256;
+    constexpr int MB = TM / 64, NB = TN / 64;      // 32 x 32 blocks per wave and direction
+    __shared__ __attribute__((aligned(16))) _Float16 as[2][TM * AS];
+    __shared__ __attribute__((aligned(16))) _Float16 bs[2][KS * BS];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int row0 = blockIdx.y * TM, col0 = blockIdx.x * TN;
+    const int wr = (wave >> 1) * (TM / 2), wc = (wave & 1) * (TN / 2);
+    const int r = lane & 31, h = lane >> 5;
+
+    // pieces of this thread: eight k of rows of A, eight columns of k rows of B
+    const int a_row = tid / (KS / 8), a_k = (tid % (KS / 8)) * 8;
+    const int b_col = (tid % (TN / 8)) * 8, b_k = tid / (TN / 8);
+    constexpr int AR = 256 / (KS / 8), BK = 256 / (TN / 8);  // rows between a thread's pieces
+    unsigned a_off[AP];
+#pragma unroll
+    for (int u = 0; u < AP; ++u) a_off[u] = (unsigned)min(row0 + a_row + AR * u, m - 1) * (unsigned)k;
+    const bool col_in = col0 + b_col < n;
+    half8_t ra[AP], rb[BP];
+    const half8_t zero = {0, 0, 0, 0, 0, 0, 0, 0};
+    auto gload = [&](int k0) {
+        const int gk = k0 + a_k;
+#pragma unroll
+        for (int u = 0; u < AP; ++u)
+            ra[u] = gk < k ? *reinterpret_cast<const half8_t*>(a + (a_off[u] + (unsigned)gk)) : zero;
+#pragma unroll
+        for (int u = 0; u < BP; ++u) {
+            const int gr = k0 + b_k + BK * u;
+            rb[u] = gr < k && col_in
+                             ? *reinterpret_cast<const half8_t*>(b + ((unsigned)gr * (unsigned)n + (unsigned)(col0 + b_col)))
+                             : zero;
+        }
+    };
+    auto lstore = [&](int buf) {
+#pragma unroll
+        for (int u = 0; u < AP; ++u)
+            *reinterpret_cast<half8_t*>(&as[buf][(a_row + AR * u) * AS + a_k]) = ra[u];
+#pragma unroll
+        for (int u = 0; u < BP; ++u)
+            *reinterpret_cast<half8_t*>(&bs[buf][(b_k + BK * u) * BS + b_col]) = rb[u];
+    };
+    float16_t acc[MB][NB];
+#pragma unroll
+    for (int i = 0; i < MB; ++i)
+#pragma unroll
+        for (int j = 0; j < NB; ++j)
+#pragma unroll
+            for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.0f;
+    const int s16 = lane & 15;
+    const int b_lane = (8 * h + (s16 >> 2)) * BS + wc + 16 * ((lane >> 4) & 1) + 4 * (s16 & 3);
+    auto multiply = [&](int buf) {
+#pragma unroll
+        for (int kk = 0; kk < KS; kk += 16) {
+            half8_t av[MB], bv[NB];
+#pragma unroll
+            for (int i = 0; i < MB; ++i)
+                av[i] = *reinterpret_cast<const half8_t*>(&as[buf][(wr + 32 * i + r) * AS + kk + 8 * h]);
+#pragma unroll
+            for (int j = 0; j < NB; ++j) {
+                const _Float16* src = &bs[buf][b_lane + kk * BS + 32 * j];
+                short4_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_short4_t*)src);
+                short4_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_short4_t*)(src + 4 * BS));
+                typedef short short8_t __attribute__((ext_vector_type(8)));
+                bv[j] = __builtin_bit_cast(half8_t, (short8_t)__builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+            }
+#pragma unroll
+            for (int i = 0; i < MB; ++i)
+#pragma unroll
+                for (int j = 0; j < NB; ++j)
+                    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(av[i], bv[j], acc[i][j], 0, 0, 0);
+        }
+    };
+    // slab s is multiplied out of buffer s % 2; slab s + 1 goes from its registers to the other
+    // buffer, whose last reader was slab s - 1, before the last barrier
+    const int slabs = (k + KS - 1) / KS;
+    gload(0);
+    lstore(0);
+    if (slabs > 1) gload(KS);
+    __syncthreads();
+    for (int s = 0; s < slabs; ++s) {
+        multiply(s & 1);
+        if (s + 1 < slabs) lstore((s + 1) & 1);
+        if (s + 2 < slabs) gload((s + 2) * KS);
+        __syncthreads();
+    }
+    // lane (h, r) holds column r, rows 8 * (e / 4) + 4h + e % 4 of each 32 x 32 block
+#pragma unroll
+    for (int i = 0; i < MB; ++i)
+#pragma unroll
+        for (int j = 0; j < NB; ++j) {
+            const int gc = col0 + wc + 32 * j + r;
+            if (gc >= n) continue;
+#pragma unroll
+            for (int e = 0; e < 16; ++e) {
+                const int gr = row0 + wr + 32 * i + 8 * (e >> 2) + 4 * h + (e & 3);
+                if (gr < m) d[(int64_t)gr * n + gc] = (_Float16)acc[i][j][e];
+            }
+        }
+}
+
+template <int TM, int TN, int KS>
+static hipError_t matmul_tiled_launch(const void* a, const void* b, void* d, int m, int n, int k,
+                                      hipStream_t st) {
+    matmul_tiled_fp16_kernel<TM, TN, KS><<<dim3((n + TN - 1) / TN, (m + TM - 1) / TM), dim3(256), 0, st>>>(
+        static_cast<const _Float16*>(a), static_cast<const _Float16*>(b), static_cast<_Float16*>(d), m, n, k);
+    return hipGetLastError();
+}
+
+// 128 x 128 tiles once two of them fall on every compute unit (4096 x 2048 x 4096: 110 us, 154 on
+// 64 x 64); below that 64 x 64, with slabs of 128 while there are at most two such tiles per
+// compute unit (500 x 1024 x 1200: 9.6 us, 10.0 with 64) and of 64 where more of them share its
+// LDS (2036 x 1536 x 1536, three per unit: 22.9 us, 26.7 with 128).
+static hipError_t matmul_tiled(const void* a, const void* b, void* d, int m, int n, int k, void* stream) {
+    hipStream_t st = static_cast<hipStream_t>(stream);
+    const int64_t cus = device_cu_count();
+    const int64_t big = (int64_t)((m + 127) / 128) * ((n + 127) / 128);
+    const int64_t small = (int64_t)((m + 63) / 64) * ((n + 63) / 64);
+    if (big >= 2 * cus) return matmul_tiled_launch<128, 128, 64>(a, b, d, m, n, k, st);
+    if (small <= 2 * cus) return matmul_tiled_launch<64, 64, 128>(a, b, d, m, n, k, st);
+    return matmul_tiled_launch<64, 64, 64>(a, b, d, m, n, k, st);
+}
+
 // `check_matmul_shape` (crates/kernels/src/matmul/mod.rs:89-117)
 static bool matmul_shape_ok(int m, int n, int k) {
     if (m <= 0 || n <= 0 || k <= 0) return false;
@@ -361,6 +574,17 @@ extern "C" logismos_status_t logismos_launch_rms_norm_fp16(const void* x_fp16, c
                                                            logismos_stream_t stream) {
     if (m <= 0 || n <= 0 || (int64_t)m * n > (int64_t)INT32_MAX) return hipErrorInvalidValue;
     if (!x_fp16 || !w_fp16 || !y_fp16) return hipErrorInvalidValue;
+    if (n % 8 == 0 && n <= 4096 &&
+        ((reinterpret_cast<uintptr_t>(x_fp16) | reinterpret_cast<uintptr_t>(w_fp16) |
+          reinterpret_cast<uintptr_t>(y_fp16)) & 15u) == 0) {
+        const auto kernel = n <= 1024   ? lg::rms_norm_fp16_wave_kernel<2>
+                            : n <= 2048 ? lg::rms_norm_fp16_wave_kernel<4>
+                                        : lg::rms_norm_fp16_wave_kernel<8>;
+        kernel<<<dim3((m + 3) / 4), dim3(256), 0, static_cast<hipStream_t>(stream)>>>(
+            static_cast<const lg::uint4_t*>(x_fp16), static_cast<const lg::uint4_t*>(w_fp16),
+            static_cast<lg::uint4_t*>(y_fp16), m, n / 8, 1.0f / (float)n, eps);
+        return hipGetLastError();
+    }
     lg::rms_norm_fp16_kernel<<<dim3(m), dim3(lg::kRowThreads), 0,
                                static_cast<hipStream_t>(stream)>>>(
         static_cast<const __half*>(x_fp16), static_cast<const __half*>(w_fp16),
@@ -394,6 +618,15 @@ extern "C" logismos_status_t logismos_launch_rope_fp16(void* qk_fp16, const void
     if (!qk_fp16 || !cos_sin_f32) return hipErrorInvalidValue;
     if ((reinterpret_cast<uintptr_t>(qk_fp16) & 3u) || (reinterpret_cast<uintptr_t>(cos_sin_f32) & 7u))
         return hipErrorInvalidValue;
+    if (head_dim % 8 == 0 && seq <= 65535 && batch <= 65535 &&
+        ((reinterpret_cast<uintptr_t>(qk_fp16) | reinterpret_cast<uintptr_t>(cos_sin_f32)) & 15u) == 0) {
+        const int token_pieces = heads * (head_dim / 8);
+        lg::rope_fp16_pieces_kernel<<<dim3((token_pieces + 255) / 256, seq, batch), dim3(256), 0,
+                                      static_cast<hipStream_t>(stream)>>>(
+            static_cast<lg::uint4_t*>(qk_fp16), static_cast<const lg::float4_t*>(cos_sin_f32),
+            token_pieces, head_dim / 8);
+        return hipGetLastError();
+    }
     const int64_t total_pairs = total / 2;
     lg::rope_fp16_kernel<<<dim3((unsigned)((total_pairs + 255) / 256)), dim3(256), 0,
                            static_cast<hipStream_t>(stream)>>>(
@@ -421,6 +654,7 @@ extern "C" logismos_status_t logismos_launch_matmul_wmma_fp16(const void* a_fp16
     if (!lg::matmul_shape_ok(m, n, k) || !a_fp16 || !b_fp16 || !d_fp16) return hipErrorInvalidValue;
     if ((reinterpret_cast<uintptr_t>(a_fp16) | reinterpret_cast<uintptr_t>(b_fp16)) & 15u)
         return hipErrorInvalidValue;
+    if (n % 8 == 0 && k % 8 == 0) return lg::matmul_tiled(a_fp16, b_fp16, d_fp16, m, n, k, stream);
     lg::matmul_mfma_fp16_kernel<<<dim3((n + lg::kMmTile - 1) / lg::kMmTile,
                                        (m + lg::kMmTile - 1) / lg::kMmTile),
                                   dim3(256), 0, static_cast<hipStream_t>(stream)>>>(
