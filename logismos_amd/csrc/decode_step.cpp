@@ -374,13 +374,23 @@ extern "C" logismos_status_t logismos_launch_decode_step(const logismos_decode_c
         // (fp32 products, consumed un-rounded by the next operator as in the chunked path), the
         // small operators run over all rows at once
         hipStream_t st = static_cast<hipStream_t>(stream);
+        // The tiled GEMM over a workspace.  An odd number of groups of K only where its 16-byte
+        // loads are aligned (the kernel that stages x itself takes any address; a layer of width
+        // 896 at 1030 rows takes 215 us on that one, 201 here).
+        auto tiled = [&](const logismos_q4_weight_t& W, const void* gains, int n, int k) {
+            if (!lg::qgemm_q4_tallp_applies(t, n, k)) return false;
+            const uintptr_t at = reinterpret_cast<uintptr_t>(W.qw) |
+                                 reinterpret_cast<uintptr_t>(gains) |
+                                 reinterpret_cast<uintptr_t>(batch->hidden_f32);
+            return k % 256 == 0 || (at & 15u) == 0;
+        };
         auto gemm = [&](const void* x_bf16, const logismos_q4_weight_t& W, const void* bias,
                         void* y_f32, int n, int k) -> logismos_status_t {
-            // K in pairs of groups: the kernel that takes x through a first pass into the
-            // workspace; otherwise the one that stages x itself
-            if (logismos_check_qgemm_q4g128_tall_shape(t, n, k, nullptr, 0) == 0)
-                return logismos_launch_qgemm_q4g128_tall(x_bf16, W.qw, W.scale, W.zero, bias, y_f32,
-                                                         1, w.t_gemm, t, n, k, stream);
+            // the kernel that takes x through a first pass into the workspace; past its sizes the
+            // one that stages x itself
+            if (tiled(W, nullptr, n, k))
+                return lg::qgemm_q4_tallp(x_bf16, W.qw, W.scale, W.zero, bias, y_f32, 1, w.t_gemm, t,
+                                          n, k, st);
             return lg::qgemm_q4_tall_f32_launch(x_bf16, W.qw, W.scale, W.zero,
                                                 static_cast<const float*>(bias), y_f32, t, n, k, st);
         };
@@ -389,14 +399,12 @@ extern "C" logismos_status_t logismos_launch_decode_step(const logismos_decode_c
         // kernel's operand order (no first pass over them)
         auto norm_then_gemm = [&](int parts, const void* gains, const logismos_q4_weight_t& W,
                                   void* y_f32, int n) -> logismos_status_t {
-            if (logismos_check_qgemm_q4g128_tall_shape(t, n, c.hidden, nullptr, 0) == 0 &&
-                c.hidden <= 16384) {
-                LG_TRY(logismos_launch_add_rms_norm_f32p_tall(
+            if (tiled(W, gains, n, c.hidden) && c.hidden <= 16384) {
+                LG_TRY(lg::add_rms_norm_tall(
                     batch->hidden_f32, w.t_proj, parts, gains, w.t_gemm, t, c.hidden, c.rms_eps,
-                    logismos_qgemm_q4g128_tall_pairs_per_load(c.hidden, W.scale, W.zero), stream));
-                return logismos_launch_qgemm_q4g128_tall_prepared(W.qw, W.scale, W.zero, nullptr,
-                                                                  y_f32, 1, w.t_gemm, t, n,
-                                                                  c.hidden, stream);
+                    logismos_qgemm_q4g128_tall_pairs_per_load(c.hidden, W.scale, W.zero), st));
+                return lg::qgemm_q4_tallp_prepared(W.qw, W.scale, W.zero, nullptr, y_f32, 1, w.t_gemm,
+                                                   t, n, c.hidden, st);
             }
             LG_TRY(logismos_launch_add_rms_norm_f32p(batch->hidden_f32, w.t_proj, parts, gains,
                                                      w.t_xn, t, c.hidden, c.rms_eps, stream));
@@ -418,33 +426,31 @@ extern "C" logismos_status_t logismos_launch_decode_step(const logismos_decode_c
                 c.num_kv_heads, c.head_dim, c.block_size, c.max_blocks_per_seq, batch->num_splits,
                 scale, 1, LOGISMOS_ATTN_PHASE_ALL, 1, c.kv_turbo3 ? 1 : 0, stream));
             LG_TRY(gemm(w.attn_out, L.o, nullptr, w.t_proj, c.hidden, qd));
-            if (logismos_check_qgemm_q4g128_tall_shape(t, 2 * c.intermediate, c.hidden, nullptr, 0) ==
-                    0 &&
-                c.hidden <= 16384) {
+            if (tiled(L.gate_up, L.norm2_w_f32, 2 * c.intermediate, c.hidden) && c.hidden <= 16384) {
                 // the gate/up projection with the SwiGLU where its products are summed: the
                 // fp32 gate and up products never go to memory
-                LG_TRY(logismos_launch_add_rms_norm_f32p_tall(
+                LG_TRY(lg::add_rms_norm_tall(
                     batch->hidden_f32, w.t_proj, 1, L.norm2_w_f32, w.t_gemm, t, c.hidden, c.rms_eps,
                     logismos_qgemm_q4g128_tall_pairs_per_load(c.hidden, L.gate_up.scale,
                                                               L.gate_up.zero),
-                    stream));
+                    st));
                 if (w.t_act_is_workspace &&
                     logismos_check_qgemm_q4g128_tall_shape(t, c.hidden, c.intermediate, nullptr,
                                                            0) == 0) {
                     // ... and the activations written as the down projection's operand, in its
                     // own workspace: no bf16 rows in between, no first pass over them
-                    LG_TRY(logismos_launch_qgemm_q4g128_tall_swiglu_operand(
+                    LG_TRY(lg::qgemm_q4_tallp_swiglu_operand(
                         L.gate_up.qw, L.gate_up.scale, L.gate_up.zero, w.t_act,
                         logismos_qgemm_q4g128_tall_pairs_per_load(c.intermediate, L.down.scale,
                                                                   L.down.zero),
-                        w.t_gemm, t, c.intermediate, c.hidden, stream));
-                    LG_TRY(logismos_launch_qgemm_q4g128_tall_prepared(
+                        w.t_gemm, t, c.intermediate, c.hidden, st));
+                    LG_TRY(lg::qgemm_q4_tallp_prepared(
                         L.down.qw, L.down.scale, L.down.zero, nullptr, w.t_proj, 1, w.t_act, t,
-                        c.hidden, c.intermediate, stream));
+                        c.hidden, c.intermediate, st));
                 } else {
-                    LG_TRY(logismos_launch_qgemm_q4g128_tall_swiglu_prepared(
-                        L.gate_up.qw, L.gate_up.scale, L.gate_up.zero, w.t_act, w.t_gemm, t,
-                        c.intermediate, c.hidden, stream));
+                    LG_TRY(lg::qgemm_q4_tallp_swiglu(L.gate_up.qw, L.gate_up.scale, L.gate_up.zero,
+                                                     w.t_act, w.t_gemm, t, c.intermediate, c.hidden,
+                                                     st));
                     LG_TRY(gemm(w.t_act, L.down, nullptr, w.t_proj, c.hidden, c.intermediate));
                 }
                 res_parts = 1;

@@ -70,6 +70,27 @@ hipError_t qgemm_q4_tall_f32_launch(const void* x_bf16, const void* qw, const vo
                                     const void* zero, const float* bias, void* y_f32, int b,
                                     int n, int k, hipStream_t stream);
 
+// The tiled GEMM over a workspace (qgemm_q4_tallp.hip) for any whole number of groups of K (the
+// exported entry points of the same names take pairs of groups).
+bool qgemm_q4_tallp_applies(int m, int n, int k);
+hipError_t qgemm_q4_tallp(const void* x_bf16, const void* qw, const void* scale, const void* zero,
+                          const void* bias, void* y, int y_is_f32, void* workspace, int m, int n,
+                          int k, hipStream_t stream);
+hipError_t qgemm_q4_tallp_prepared(const void* qw, const void* scale, const void* zero,
+                                   const void* bias, void* y, int y_is_f32, void* workspace, int m,
+                                   int n, int k, hipStream_t stream);
+hipError_t qgemm_q4_tallp_swiglu(const void* gate_up_qw, const void* scale, const void* zero,
+                                 void* act_bf16, void* workspace, int m, int inter, int k,
+                                 hipStream_t stream);
+hipError_t qgemm_q4_tallp_swiglu_operand(const void* gate_up_qw, const void* scale, const void* zero,
+                                         void* next_workspace, int next_pairs_per_load,
+                                         void* workspace, int m, int inter, int k,
+                                         hipStream_t stream);
+// h += parts; RMSNorm of h as that kernel's operand (step_ops.hip), likewise
+hipError_t add_rms_norm_tall(void* h_f32, const void* parts_f32, int num_parts, const void* w_f32,
+                             void* workspace, int rows, int n, float eps, int pairs_per_load,
+                             hipStream_t stream);
+
 // dst[s][:] = src[cu_seqlens[s + 1] - 1][:], bf16 rows of `hidden` elements (step_ops.hip): the
 // last packed row of every sequence of a ragged batch.
 hipError_t gather_last_rows_bf16_launch(const void* src_bf16, const int32_t* cu_seqlens,

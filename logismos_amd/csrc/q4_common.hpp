@@ -71,7 +71,7 @@ __host__ __device__ inline size_t tall_sums_offset(int m, int k) {
 }
 __host__ __device__ inline int64_t tall_sum_index(int64_t row, int g, int k, int w) {
     const int bl = 2 * w;
-    const int64_t block = (row / kTallTileRows) * ((k >> 7) / bl) + g / bl;
+    const int64_t block = (row / kTallTileRows) * (((k >> 7) + bl - 1) / bl) + g / bl;
     const int in_block = g % bl;
     return ((block * 2 + (in_block & 1)) * kTallTileRows + row % kTallTileRows) * w + (in_block >> 1);
 }

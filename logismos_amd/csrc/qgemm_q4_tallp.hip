@@ -69,7 +69,9 @@ static_assert(kTpTileM == kTallTileRows, "the layout helpers of q4_common.hpp ar
 __host__ __device__ inline int tp_padded_rows(int m) { return tall_padded_rows(m); }
 __host__ __device__ inline size_t tp_sums_offset(int m, int k) { return tall_sums_offset(m, k); }
 __host__ __device__ inline size_t tp_partials_offset(int m, int k) {
-    return (tp_sums_offset(m, k) + (size_t)tp_padded_rows(m) * (k / 128) * 4 + 255) & ~(size_t)255;
+    // (whole pairs of groups: the sums of a missing last group have a place, which nothing uses)
+    return (tp_sums_offset(m, k) + (size_t)tp_padded_rows(m) * ((k / 128 + 1) & ~1) * 4 + 255) &
+           ~(size_t)255;
 }
 
 // How a launch of `tiles` workgroup tiles is laid over `cus` CUs: the first `full` tiles whole,
@@ -163,7 +165,12 @@ __device__ __forceinline__ float tp_group_sum(const float (&cs)[4][4]) {
 
 // W: pairs of groups whose scales, zeros and group sums a lane loads at once (1, 2 or 4: a
 // dword, two or four per load; K a multiple of 256 W).
-template <int OUT, int W>
+// ODD (W = 1): an odd number of groups.  Rows of scales are then only 2-byte aligned and come
+// as halves; the last pair has one group, whose missing partner adds 0 * 0 to the zero-point
+// product.  1030 rows x 896 (seven groups): 9728 gate/up rows with the activation 45.5 us, 52.6
+// + 11.0 on the kernel of qgemm_q4_tall.hip with the activation behind it; 1152 rows of q/k/v
+// 23.4 (24.5).
+template <int OUT, int W, bool ODD>
 __global__ __launch_bounds__(512) void qgemm_q4g128_tallp_kernel(
     const uint16_t* __restrict__ xp, const float* __restrict__ xs, const uint8_t* __restrict__ qw,
     const __half* __restrict__ scale, const __half* __restrict__ zero,
@@ -178,15 +185,16 @@ __global__ __launch_bounds__(512) void qgemm_q4g128_tallp_kernel(
     const int h = lane >> 5;
     // workgroup -> tile (columns fastest) and, past the whole tiles, part of a tile: groups
     // [g_begin, groups) of K, both multiples of BL
+    static_assert(!ODD || W == 1, "an odd number of groups is taken pair by pair");
     int tile = blockIdx.x, part = -1;
     int g_begin = 0, groups = k >> 7;
     if (tile >= full_tiles) {
         const int p = tile - full_tiles;
         tile = full_tiles + p / split;
         part = p;
-        const int blocks = groups / BL, q = p % split;
+        const int blocks = (groups + BL - 1) / BL, q = p % split;
         g_begin = BL * (int)((int64_t)blocks * q / split);
-        groups = BL * (int)((int64_t)blocks * (q + 1) / split);
+        groups = min(groups, BL * (int)((int64_t)blocks * (q + 1) / split));
     }
     const int row_tile = tile / tiles_n;
     const int row0 = row_tile * kTpTileM;
@@ -278,6 +286,8 @@ __global__ __launch_bounds__(512) void qgemm_q4g128_tallp_kernel(
     struct Small {
         TpRegs<unsigned, W> s[2], z[2];
         TpRegs<float, W> xs[2];
+        unsigned s_hi[2];  // ODD: s and s_hi the scales of the pair's two groups, z the zero of
+                           // this lane's group of the pair
     };
     unsigned soff[2], xsoff[2];
 #pragma unroll
@@ -288,10 +298,17 @@ __global__ __launch_bounds__(512) void qgemm_q4g128_tallp_kernel(
     auto gload_small = [&](int g, Small& v) {
         const __half* sb = scale + g;
         const __half* zb = zero + g;
-        const float* xb = xs + ((size_t)row_tile * (groups_row / BL) + g / BL) * (2 * kTpTileM * W);
+        const float* xb = xs + ((size_t)row_tile * ((groups_row + BL - 1) / BL) + g / BL) * (2 * kTpTileM * W);
 #pragma unroll
         for (int j = 0; j < 2; ++j) {
-            if constexpr (W == 1) {
+            if constexpr (ODD) {
+                // (a missing second group re-reads the first)
+                const unsigned second = soff[j] + (g + 1 < groups_row ? 2u : 0u);
+                const unsigned own = h ? second : soff[j];
+                asm volatile("global_load_ushort %0, %1, %2" : "=&v"(v.s[j].raw) : "v"(soff[j]), "s"(sb) : "memory");
+                asm volatile("global_load_ushort %0, %1, %2" : "=&v"(v.s_hi[j]) : "v"(second), "s"(sb) : "memory");
+                asm volatile("global_load_ushort %0, %1, %2" : "=&v"(v.z[j].raw) : "v"(own), "s"(zb) : "memory");
+            } else if constexpr (W == 1) {
                 asm volatile("global_load_dword %0, %1, %2" : "=&v"(v.s[j].raw) : "v"(soff[j]), "s"(sb) : "memory");
                 asm volatile("global_load_dword %0, %1, %2" : "=&v"(v.z[j].raw) : "v"(soff[j]), "s"(zb) : "memory");
             } else if constexpr (W == 2) {
@@ -317,11 +334,18 @@ __global__ __launch_bounds__(512) void qgemm_q4g128_tallp_kernel(
     // into LDS complete in order with each other is not relied on.  The requests of the group
     // after next, issued most of a group ago, are waited for with them -- once per block.)
     auto small_loads_landed = [&](Small& v) {
-        asm volatile("s_waitcnt vmcnt(0)"
-                     : "+v"(v.s[0].raw), "+v"(v.s[1].raw), "+v"(v.z[0].raw), "+v"(v.z[1].raw),
-                       "+v"(v.xs[0].raw), "+v"(v.xs[1].raw)
-                     :
-                     : "memory");
+        if constexpr (ODD)
+            asm volatile("s_waitcnt vmcnt(0)"
+                         : "+v"(v.s[0].raw), "+v"(v.s[1].raw), "+v"(v.z[0].raw), "+v"(v.z[1].raw),
+                           "+v"(v.xs[0].raw), "+v"(v.xs[1].raw), "+v"(v.s_hi[0]), "+v"(v.s_hi[1])
+                         :
+                         : "memory");
+        else
+            asm volatile("s_waitcnt vmcnt(0)"
+                         : "+v"(v.s[0].raw), "+v"(v.s[1].raw), "+v"(v.z[0].raw), "+v"(v.z[1].raw),
+                           "+v"(v.xs[0].raw), "+v"(v.xs[1].raw)
+                         :
+                         : "memory");
     };
     // One block's values are in use while the next one's are on their way (W = 1), or the
     // next block's are loaded over them behind their last use (W > 1: a block lasts four or
@@ -340,7 +364,7 @@ __global__ __launch_bounds__(512) void qgemm_q4g128_tallp_kernel(
 
     gload_small(g_begin, cur);
     request_group(g_begin, 0);
-    request_group(g_begin + 1, kTpBufBytes);  // (a range holds at least one pair)
+    if (!ODD || g_begin + 1 < groups) request_group(g_begin + 1, kTpBufBytes);  // (else whole pairs)
     small_loads_landed(cur);
 
     // The requests of the group after next go into the buffer everybody stopped reading before
@@ -353,6 +377,29 @@ __global__ __launch_bounds__(512) void qgemm_q4g128_tallp_kernel(
             if (dst >= kTpBufs * kTpBufBytes) dst -= kTpBufs * kTpBufBytes;
             request_group(g + 2, dst);
         }
+    };
+
+    // zero-point term of a pair of groups (lanes h = 0 the first, h = 1 the second):
+    // y[m][n] += sum_x[m][g'] * (-scale[n][g'] * (128 + zero[n][g'])).  lone: the second is missing
+    auto zero_term = [&](auto pair_c, bool lone) {
+        constexpr int P = decltype(pair_c)::value;
+        float cv[2], sum[2];
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+            const unsigned sd = cur.s[j][P], zd = cur.z[j][P];
+            const unsigned short sb =
+                (unsigned short)(ODD ? (h ? cur.s_hi[j] : sd) : (h ? (sd >> 16) : sd));
+            const unsigned short zb = (unsigned short)(ODD ? zd : (h ? (zd >> 16) : zd));
+            cv[j] = -__half2float(__builtin_bit_cast(__half, sb)) *
+                    (128.0f + __half2float(__builtin_bit_cast(__half, zb)));
+            sum[j] = cur.xs[j][P];
+            if (ODD && lone && h) cv[j] = sum[j] = 0.0f;
+        }
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+            for (int j = 0; j < 2; ++j)
+                yacc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(sum[i], cv[j], yacc[i][j], 0, 0, 0);
     };
 
     // One group of 128 columns out of the buffer at byte `buf_off` of the ring; U: the group's
@@ -370,7 +417,9 @@ __global__ __launch_bounds__(512) void qgemm_q4g128_tallp_kernel(
         // after the barrier everybody's requests for this group have landed, and everybody is
         // done reading the buffer of the group before it, which the group after next reuses
         __builtin_amdgcn_s_barrier();
-        if constexpr (W == 1) {
+        if constexpr (ODD && U == 1) {
+            gload_small(g + 1 < groups ? g + 1 : g - 1, nxt);
+        } else if constexpr (W == 1) {
             if (U == 1 && g + 1 < groups) gload_small(g + 1, nxt);
         }
         issue_requests(g, buf_off);
@@ -461,7 +510,8 @@ __global__ __launch_bounds__(512) void qgemm_q4g128_tallp_kernel(
 #pragma unroll
         for (int j = 0; j < 2; ++j) {
             const unsigned sd = cur.s[j][U >> 1];
-            const unsigned short sb = (unsigned short)(PAR ? (sd >> 16) : sd);
+            const unsigned short sb =
+                (unsigned short)(ODD ? (PAR ? cur.s_hi[j] : sd) : (PAR ? (sd >> 16) : sd));
             const float sf = __half2float(__builtin_bit_cast(__half, sb));
 #pragma unroll
             for (int i = 0; i < 2; ++i)
@@ -469,24 +519,11 @@ __global__ __launch_bounds__(512) void qgemm_q4g128_tallp_kernel(
                 for (int e = 0; e < 16; ++e) yacc[i][j][e] = fmaf(sf, acc[i][j][e], yacc[i][j][e]);
         }
         if constexpr (PAR == 1) {
-            // zero-point term of the groups g - 1 (lanes h = 0) and g (h = 1):
-            // y[m][n] += sum_x[m][g'] * (-scale[n][g'] * (128 + zero[n][g']))
-            float cv[2];
-#pragma unroll
-            for (int j = 0; j < 2; ++j) {
-                const unsigned sd = cur.s[j][U >> 1], zd = cur.z[j][U >> 1];
-                const unsigned short sb = (unsigned short)(h ? (sd >> 16) : sd);
-                const unsigned short zb = (unsigned short)(h ? (zd >> 16) : zd);
-                cv[j] = -__half2float(__builtin_bit_cast(__half, sb)) *
-                        (128.0f + __half2float(__builtin_bit_cast(__half, zb)));
-            }
-#pragma unroll
-            for (int i = 0; i < 2; ++i)
-#pragma unroll
-                for (int j = 0; j < 2; ++j)
-                    yacc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(cur.xs[i][U >> 1], cv[j],
-                                                                      yacc[i][j], 0, 0, 0);
-            if constexpr (W == 1) {
+            zero_term(ic<(U >> 1)>{}, false);
+            if constexpr (ODD) {
+                small_loads_landed(nxt);
+                cur = nxt;
+            } else if constexpr (W == 1) {
                 if (g + 1 < groups) {
                     small_loads_landed(nxt);
                     cur = nxt;
@@ -498,11 +535,27 @@ __global__ __launch_bounds__(512) void qgemm_q4g128_tallp_kernel(
     };
     // ranges are whole blocks (K is a multiple of 256 W); buffers go round in threes
     int buf_off = 0;
-    for (int g0 = g_begin; g0 < groups; g0 += BL) {
-        static_for<BL>([&](auto uc) {
-            group(uc, g0 + decltype(uc)::value, buf_off);
-            buf_off = buf_off + kTpBufBytes == kTpBufs * kTpBufBytes ? 0 : buf_off + kTpBufBytes;
-        });
+    auto next_buf = [&]() {
+        buf_off = buf_off + kTpBufBytes == kTpBufs * kTpBufBytes ? 0 : buf_off + kTpBufBytes;
+    };
+    if constexpr (ODD) {
+        int g0 = g_begin;
+        for (; g0 + 1 < groups; g0 += 2) {
+            group(ic<0>{}, g0, buf_off);
+            next_buf();
+            group(ic<1>{}, g0 + 1, buf_off);
+            next_buf();
+        }
+        if (g0 < groups) {
+            group(ic<0>{}, g0, buf_off);
+            zero_term(ic<0>{}, true);
+        }
+    } else {
+        for (int g0 = g_begin; g0 < groups; g0 += BL)
+            static_for<BL>([&](auto uc) {
+                group(uc, g0 + decltype(uc)::value, buf_off);
+                next_buf();
+            });
     }
 
     if (part >= 0) {
@@ -677,14 +730,24 @@ inline int tp_pairs_per_load(int k, const void* scale, const void* zero) {
     return tall_pairs_per_load(k, scale, zero);
 }
 
-template <int OUT, int W>
+// 32-bit offsets of the kernels
+static bool tp_sizes_ok(int m, int n, int k) {
+    const int64_t lim = INT32_MAX;
+    return (int64_t)n * k <= lim && (int64_t)tp_padded_rows(m) * k * 2 <= lim && (int64_t)m * n <= lim;
+}
+
+bool qgemm_q4_tallp_applies(int m, int n, int k) {
+    return m > 0 && n > 0 && k > 0 && k % 128 == 0 && tp_sizes_ok(m, n, k);
+}
+
+template <int OUT, int W, bool ODD = false>
 static hipError_t tallp_launch(const uint16_t* xp, const float* xs, float* partials,
                                const uint8_t* qw, const __half* scale, const __half* zero,
                                const float* bias, void* y, int m, int n, int k, hipStream_t st,
                                int out_pairs = 0) {
     constexpr size_t lds = (size_t)kTpBufs * kTpBufBytes;
     static const hipError_t opt = hipFuncSetAttribute(
-        reinterpret_cast<const void*>(qgemm_q4g128_tallp_kernel<OUT, W>),
+        reinterpret_cast<const void*>(qgemm_q4g128_tallp_kernel<OUT, W, ODD>),
         hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     if (opt != hipSuccess) return opt;
     constexpr int tile_outputs = tp_is_swiglu(OUT) ? kTpTileN / 2 : kTpTileN;
@@ -694,7 +757,7 @@ static hipError_t tallp_launch(const uint16_t* xp, const float* xs, float* parti
     if (cus <= 0) return hipErrorInvalidDevice;
     const TpPlan plan = tp_plan(tiles, k >> 7, 2 * W, cus);
     const int parts = (tiles - plan.full) * plan.split;
-    qgemm_q4g128_tallp_kernel<OUT, W>
+    qgemm_q4g128_tallp_kernel<OUT, W, ODD>
         <<<dim3(plan.full + (plan.split > 1 ? parts : 0)), dim3(512), lds, st>>>(
             xp, xs, qw, scale, zero, bias, y, partials, m, n, k, tiles_n, plan.full, plan.split,
             out_pairs);
@@ -717,6 +780,9 @@ static hipError_t tallp_launch_w(int w, const uint16_t* xp, const float* xs, flo
                                  const uint8_t* qw, const __half* scale, const __half* zero,
                                  const float* bias, void* y, int m, int n, int k, hipStream_t st,
                                  int out_pairs = 0) {
+    if ((k >> 7) & 1)
+        return tallp_launch<OUT, 1, true>(xp, xs, partials, qw, scale, zero, bias, y, m, n, k, st,
+                                          out_pairs);
     switch (w) {
         case 4:
             return tallp_launch<OUT, 4>(xp, xs, partials, qw, scale, zero, bias, y, m, n, k, st,
@@ -755,114 +821,150 @@ extern "C" size_t logismos_qgemm_q4g128_tall_workspace_bytes(int m, int k) {
     return lg::tp_partials_offset(m, k) + (size_t)lg::kTpMaxParts * lg::kTpTileElems * 4;
 }
 
-static logismos_status_t tall_args_ok(const void* qw_u8, const void* scale_f16,
-                                      const void* zero_f16, const void* y, const void* workspace,
-                                      int m, int n, int k) {
-    if (logismos_check_qgemm_q4g128_tall_shape(m, n, k, nullptr, 0) != 0)
-        return hipErrorInvalidValue;
-    if (!qw_u8 || !scale_f16 || !zero_f16 || !y || !workspace) return hipErrorInvalidValue;
-    if ((reinterpret_cast<uintptr_t>(qw_u8) | reinterpret_cast<uintptr_t>(workspace)) & 15u)
-        return hipErrorInvalidValue;
-    if ((reinterpret_cast<uintptr_t>(scale_f16) | reinterpret_cast<uintptr_t>(zero_f16)) & 3u)
-        return hipErrorInvalidValue;
-    return hipSuccess;
-}
-
 extern "C" int logismos_qgemm_q4g128_tall_pairs_per_load(int k, const void* scale_f16,
                                                          const void* zero_f16) {
     return lg::tall_pairs_per_load(k, scale_f16, zero_f16);
 }
 
-extern "C" logismos_status_t logismos_launch_qgemm_q4g128_tall_prepared(
+namespace lg {
+
+// (an odd number of groups: the rows of scales and zeros are halves, loaded as halves)
+static hipError_t tall_args_ok(const void* qw_u8, const void* scale_f16,
+                                      const void* zero_f16, const void* y, const void* workspace,
+                                      int m, int n, int k) {
+    if (!qgemm_q4_tallp_applies(m, n, k)) return hipErrorInvalidValue;
+    if (!qw_u8 || !scale_f16 || !zero_f16 || !y || !workspace) return hipErrorInvalidValue;
+    if ((reinterpret_cast<uintptr_t>(qw_u8) | reinterpret_cast<uintptr_t>(workspace)) & 15u)
+        return hipErrorInvalidValue;
+    const uintptr_t align = k % 256 == 0 ? 3u : 1u;
+    if ((reinterpret_cast<uintptr_t>(scale_f16) | reinterpret_cast<uintptr_t>(zero_f16)) & align)
+        return hipErrorInvalidValue;
+    return hipSuccess;
+}
+
+hipError_t qgemm_q4_tallp_prepared(
     const void* qw_u8, const void* scale_f16, const void* zero_f16, const void* bias_f32, void* y,
-    int y_is_f32, void* workspace, int m, int n, int k, logismos_stream_t stream) {
-    if (const logismos_status_t e = tall_args_ok(qw_u8, scale_f16, zero_f16, y, workspace, m, n, k))
+    int y_is_f32, void* workspace, int m, int n, int k, hipStream_t st) {
+    if (const hipError_t e = tall_args_ok(qw_u8, scale_f16, zero_f16, y, workspace, m, n, k))
         return e;
-    hipStream_t st = static_cast<hipStream_t>(stream);
     const uint16_t* xp = static_cast<const uint16_t*>(workspace);
     const float* xs =
-        reinterpret_cast<const float*>(static_cast<char*>(workspace) + lg::tp_sums_offset(m, k));
+        reinterpret_cast<const float*>(static_cast<char*>(workspace) + tp_sums_offset(m, k));
     float* partials = reinterpret_cast<float*>(static_cast<char*>(workspace) +
-                                               lg::tp_partials_offset(m, k));
-    const int w = lg::tp_pairs_per_load(k, scale_f16, zero_f16);
+                                               tp_partials_offset(m, k));
+    const int w = tp_pairs_per_load(k, scale_f16, zero_f16);
     if (y_is_f32)
-        return lg::tallp_launch_w<lg::kTpOutF32>(w, xp, xs, partials, static_cast<const uint8_t*>(qw_u8),
+        return tallp_launch_w<kTpOutF32>(w, xp, xs, partials, static_cast<const uint8_t*>(qw_u8),
                                         static_cast<const __half*>(scale_f16),
                                         static_cast<const __half*>(zero_f16),
                                         static_cast<const float*>(bias_f32), y, m, n, k, st);
-    return lg::tallp_launch_w<lg::kTpOutBf16>(w, xp, xs, partials, static_cast<const uint8_t*>(qw_u8),
+    return tallp_launch_w<kTpOutBf16>(w, xp, xs, partials, static_cast<const uint8_t*>(qw_u8),
                                      static_cast<const __half*>(scale_f16),
                                      static_cast<const __half*>(zero_f16),
                                      static_cast<const float*>(bias_f32), y, m, n, k, st);
 }
 
-extern "C" logismos_status_t logismos_launch_qgemm_q4g128_tall_swiglu_prepared(
+hipError_t qgemm_q4_tallp_swiglu(
     const void* gate_up_qw_u8, const void* scale_f16, const void* zero_f16, void* act_bf16,
-    void* workspace, int m, int inter, int k, logismos_stream_t stream) {
+    void* workspace, int m, int inter, int k, hipStream_t st) {
     // the weights are 2 * inter rows (gate, then up); the output is m x inter
     if (inter <= 0 || inter > INT32_MAX / 2) return hipErrorInvalidValue;
-    if (const logismos_status_t e = tall_args_ok(gate_up_qw_u8, scale_f16, zero_f16, act_bf16,
+    if (const hipError_t e = tall_args_ok(gate_up_qw_u8, scale_f16, zero_f16, act_bf16,
                                                  workspace, m, 2 * inter, k))
         return e;
-    hipStream_t st = static_cast<hipStream_t>(stream);
     const uint16_t* xp = static_cast<const uint16_t*>(workspace);
     const float* xs =
-        reinterpret_cast<const float*>(static_cast<char*>(workspace) + lg::tp_sums_offset(m, k));
+        reinterpret_cast<const float*>(static_cast<char*>(workspace) + tp_sums_offset(m, k));
     float* partials = reinterpret_cast<float*>(static_cast<char*>(workspace) +
-                                               lg::tp_partials_offset(m, k));
-    const int w = lg::tp_pairs_per_load(k, scale_f16, zero_f16);
-    return lg::tallp_launch_w<lg::kTpOutSwiglu>(
+                                               tp_partials_offset(m, k));
+    const int w = tp_pairs_per_load(k, scale_f16, zero_f16);
+    return tallp_launch_w<kTpOutSwiglu>(
         w, xp, xs, partials, static_cast<const uint8_t*>(gate_up_qw_u8),
         static_cast<const __half*>(scale_f16), static_cast<const __half*>(zero_f16), nullptr,
         act_bf16, m, inter, k, st);
 }
 
-extern "C" logismos_status_t logismos_launch_qgemm_q4g128_tall_swiglu_operand(
+hipError_t qgemm_q4_tallp_swiglu_operand(
     const void* gate_up_qw_u8, const void* scale_f16, const void* zero_f16, void* next_workspace,
-    int next_pairs_per_load, void* workspace, int m, int inter, int k, logismos_stream_t stream) {
+    int next_pairs_per_load, void* workspace, int m, int inter, int k, hipStream_t st) {
     // the output is the operand of a product over K = inter: whole pairs of groups, and as many
     // pairs per load as the caller's next launch will ask for (whole blocks of them)
     if (inter <= 0 || inter > INT32_MAX / 2 || inter % 256 != 0) return hipErrorInvalidValue;
     if (next_pairs_per_load != 1 && next_pairs_per_load != 2 && next_pairs_per_load != 4)
         return hipErrorInvalidValue;
     if (inter % (256 * next_pairs_per_load) != 0) return hipErrorInvalidValue;
-    if (const logismos_status_t e = tall_args_ok(gate_up_qw_u8, scale_f16, zero_f16,
+    if (const hipError_t e = tall_args_ok(gate_up_qw_u8, scale_f16, zero_f16,
                                                  next_workspace, workspace, m, 2 * inter, k))
         return e;
     // (the next launch's own shape: rows * inter * 2 within 32 bits)
-    if (logismos_check_qgemm_q4g128_tall_shape(m, 1, inter, nullptr, 0) != 0)
+    if (!qgemm_q4_tallp_applies(m, 1, inter))
         return hipErrorInvalidValue;
     if ((reinterpret_cast<uintptr_t>(next_workspace) & 15u) || next_workspace == workspace)
         return hipErrorInvalidValue;
-    hipStream_t st = static_cast<hipStream_t>(stream);
     const uint16_t* xp = static_cast<const uint16_t*>(workspace);
     const float* xs =
-        reinterpret_cast<const float*>(static_cast<char*>(workspace) + lg::tp_sums_offset(m, k));
+        reinterpret_cast<const float*>(static_cast<char*>(workspace) + tp_sums_offset(m, k));
     float* partials = reinterpret_cast<float*>(static_cast<char*>(workspace) +
-                                               lg::tp_partials_offset(m, k));
-    const int w = lg::tp_pairs_per_load(k, scale_f16, zero_f16);
-    return lg::tallp_launch_w<lg::kTpOutSwigluOperand>(
+                                               tp_partials_offset(m, k));
+    const int w = tp_pairs_per_load(k, scale_f16, zero_f16);
+    return tallp_launch_w<kTpOutSwigluOperand>(
         w, xp, xs, partials, static_cast<const uint8_t*>(gate_up_qw_u8),
         static_cast<const __half*>(scale_f16), static_cast<const __half*>(zero_f16), nullptr,
         next_workspace, m, inter, k, st, next_pairs_per_load);
+}
+
+hipError_t qgemm_q4_tallp(
+    const void* x_bf16, const void* qw_u8, const void* scale_f16, const void* zero_f16,
+    const void* bias_f32, void* y, int y_is_f32, void* workspace, int m, int n, int k,
+    hipStream_t st) {
+    if (const hipError_t e = tall_args_ok(qw_u8, scale_f16, zero_f16, y, workspace, m, n, k))
+        return e;
+    if (!x_bf16 || (reinterpret_cast<uintptr_t>(x_bf16) & 15u)) return hipErrorInvalidValue;
+    const int m_pad = tp_padded_rows(m);
+    uint16_t* xp = static_cast<uint16_t*>(workspace);
+    float* xs = reinterpret_cast<float*>(static_cast<char*>(workspace) + tp_sums_offset(m, k));
+    const int64_t chunks = (int64_t)m_pad * (k / 8);
+    const int w = tp_pairs_per_load(k, scale_f16, zero_f16);
+    q4_tall_prepare_kernel<<<dim3((unsigned)((chunks + 255) / 256)), dim3(256), 0, st>>>(
+        static_cast<const uint16_t*>(x_bf16), xp, xs, m, m_pad, k, w);
+    if (const hipError_t e = hipGetLastError()) return e;
+    return qgemm_q4_tallp_prepared(qw_u8, scale_f16, zero_f16, bias_f32, y,
+                                                      y_is_f32, workspace, m, n, k, st);
+}
+
+}  // namespace lg
+
+// The exported entry points take whole pairs of groups.
+extern "C" logismos_status_t logismos_launch_qgemm_q4g128_tall_prepared(
+    const void* qw_u8, const void* scale_f16, const void* zero_f16, const void* bias_f32, void* y,
+    int y_is_f32, void* workspace, int m, int n, int k, logismos_stream_t stream) {
+    if (k % 256 != 0) return hipErrorInvalidValue;
+    return lg::qgemm_q4_tallp_prepared(qw_u8, scale_f16, zero_f16, bias_f32, y, y_is_f32, workspace,
+                                       m, n, k, static_cast<hipStream_t>(stream));
+}
+
+extern "C" logismos_status_t logismos_launch_qgemm_q4g128_tall_swiglu_prepared(
+    const void* gate_up_qw_u8, const void* scale_f16, const void* zero_f16, void* act_bf16,
+    void* workspace, int m, int inter, int k, logismos_stream_t stream) {
+    if (k % 256 != 0) return hipErrorInvalidValue;
+    return lg::qgemm_q4_tallp_swiglu(gate_up_qw_u8, scale_f16, zero_f16, act_bf16, workspace, m,
+                                     inter, k, static_cast<hipStream_t>(stream));
+}
+
+extern "C" logismos_status_t logismos_launch_qgemm_q4g128_tall_swiglu_operand(
+    const void* gate_up_qw_u8, const void* scale_f16, const void* zero_f16, void* next_workspace,
+    int next_pairs_per_load, void* workspace, int m, int inter, int k, logismos_stream_t stream) {
+    if (k % 256 != 0) return hipErrorInvalidValue;
+    return lg::qgemm_q4_tallp_swiglu_operand(gate_up_qw_u8, scale_f16, zero_f16, next_workspace,
+                                             next_pairs_per_load, workspace, m, inter, k,
+                                             static_cast<hipStream_t>(stream));
 }
 
 extern "C" logismos_status_t logismos_launch_qgemm_q4g128_tall(
     const void* x_bf16, const void* qw_u8, const void* scale_f16, const void* zero_f16,
     const void* bias_f32, void* y, int y_is_f32, void* workspace, int m, int n, int k,
     logismos_stream_t stream) {
-    if (const logismos_status_t e = tall_args_ok(qw_u8, scale_f16, zero_f16, y, workspace, m, n, k))
-        return e;
-    if (!x_bf16 || (reinterpret_cast<uintptr_t>(x_bf16) & 15u)) return hipErrorInvalidValue;
-    hipStream_t st = static_cast<hipStream_t>(stream);
-    const int m_pad = lg::tp_padded_rows(m);
-    uint16_t* xp = static_cast<uint16_t*>(workspace);
-    float* xs = reinterpret_cast<float*>(static_cast<char*>(workspace) + lg::tp_sums_offset(m, k));
-    const int64_t chunks = (int64_t)m_pad * (k / 8);
-    const int w = lg::tp_pairs_per_load(k, scale_f16, zero_f16);
-    lg::q4_tall_prepare_kernel<<<dim3((unsigned)((chunks + 255) / 256)), dim3(256), 0, st>>>(
-        static_cast<const uint16_t*>(x_bf16), xp, xs, m, m_pad, k, w);
-    if (const hipError_t e = hipGetLastError()) return e;
-    return logismos_launch_qgemm_q4g128_tall_prepared(qw_u8, scale_f16, zero_f16, bias_f32, y,
-                                                      y_is_f32, workspace, m, n, k, stream);
+    if (k % 256 != 0) return hipErrorInvalidValue;
+    return lg::qgemm_q4_tallp(x_bf16, qw_u8, scale_f16, zero_f16, bias_f32, y, y_is_f32, workspace, m,
+                              n, k, static_cast<hipStream_t>(stream));
 }

@@ -926,12 +926,13 @@ extern "C" logismos_status_t logismos_launch_add_rms_norm_f32p_xprep(
     return hipGetLastError();
 }
 
-extern "C" logismos_status_t logismos_launch_add_rms_norm_f32p_tall(
-    void* h_f32, const void* parts_f32, int num_parts, const void* w_f32, void* workspace,
-    int rows, int n, float eps, int pairs_per_load, logismos_stream_t stream) {
+hipError_t lg::add_rms_norm_tall(void* h_f32, const void* parts_f32, int num_parts,
+                                 const void* w_f32, void* workspace, int rows, int n, float eps,
+                                 int pairs_per_load, hipStream_t stream) {
     if (rows <= 0 || n <= 0 || num_parts < 0 ||
         (pairs_per_load != 1 && pairs_per_load != 2 && pairs_per_load != 4) ||
-        n % (256 * pairs_per_load) != 0 || n > 8 * lg::kPrepThreads * lg::kPrepMaxPasses)
+        n % (pairs_per_load == 1 ? 128 : 256 * pairs_per_load) != 0 ||
+        n > 8 * lg::kPrepThreads * lg::kPrepMaxPasses)
         return hipErrorInvalidValue;
     const int rows_pad = lg::tall_padded_rows(rows);
     if ((int64_t)rows_pad * n * 2 > (int64_t)INT32_MAX) return hipErrorInvalidValue;
@@ -940,12 +941,19 @@ extern "C" logismos_status_t logismos_launch_add_rms_norm_f32p_tall(
     if ((reinterpret_cast<uintptr_t>(h_f32) | reinterpret_cast<uintptr_t>(parts_f32) |
          reinterpret_cast<uintptr_t>(w_f32) | reinterpret_cast<uintptr_t>(workspace)) & 15u)
         return hipErrorInvalidValue;
-    lg::add_rms_norm_xprep_kernel<true><<<dim3(rows_pad), dim3(lg::kPrepThreads), 0,
-                                          static_cast<hipStream_t>(stream)>>>(
+    lg::add_rms_norm_xprep_kernel<true><<<dim3(rows_pad), dim3(lg::kPrepThreads), 0, stream>>>(
         static_cast<float*>(h_f32), static_cast<const float*>(parts_f32), num_parts,
         (int64_t)rows * n, static_cast<const float*>(w_f32), workspace, rows, n, eps,
         pairs_per_load);
     return hipGetLastError();
+}
+
+extern "C" logismos_status_t logismos_launch_add_rms_norm_f32p_tall(
+    void* h_f32, const void* parts_f32, int num_parts, const void* w_f32, void* workspace,
+    int rows, int n, float eps, int pairs_per_load, logismos_stream_t stream) {
+    if (n % 256 != 0) return hipErrorInvalidValue;
+    return lg::add_rms_norm_tall(h_f32, parts_f32, num_parts, w_f32, workspace, rows, n, eps,
+                                 pairs_per_load, static_cast<hipStream_t>(stream));
 }
 
 extern "C" logismos_status_t logismos_launch_silu_mul_f32p_xprep(const void* parts_f32,
