@@ -48,17 +48,29 @@
 #include "q4_common.hpp"
 
 #include <hip/hip_fp16.h>
+#include <type_traits>
 
 namespace lg {
 
 typedef __attribute__((address_space(3))) void* tp_lds_ptr_t;
 typedef const __attribute__((address_space(1))) void* tp_glb_ptr_t;
 
-constexpr int kTpTileM = 128;             // rows of x per workgroup
-constexpr int kTpTileN = 256;             // weight rows per workgroup
-constexpr int kTpSlabBytes = 128 * 256;   // one group's slab of x: 128 rows x 128 bf16
-constexpr int kTpWBytes = 256 * 64;       // one group's tile of weights: 256 rows x 128 nibbles
-constexpr int kTpBufBytes = kTpSlabBytes + kTpWBytes;
+// A workgroup's tile: two rows of ACROSS waves, a wave takes 32 * BLOCKS rows of x by 64 weight rows.
+template <int BLOCKS, int ACROSS>
+struct TpTile {
+    static constexpr int kBlocks = BLOCKS, kAcross = ACROSS, kWaves = 2 * ACROSS;
+    static constexpr int kM = 64 * BLOCKS, kN = 64 * ACROSS;
+    static constexpr int kSlabBytes = kM * 256;  // one group's slab of x: kM rows x 128 bf16
+    static constexpr int kBufBytes = kSlabBytes + kN * 64;  // ... and its tile of nibbles
+    static constexpr int kXRequests = kM / 4 / kWaves;      // 1 KiB requests of x per wave
+    static constexpr bool kBig = BLOCKS == 2 && ACROSS == 4;
+    static_assert(kXRequests == 2 || kXRequests == 4, "what request_group spells out");
+};
+using TpBig = TpTile<2, 4>;
+using TpHalf = TpTile<1, 4>;
+using TpSmall = TpTile<1, 2>;
+constexpr int kTpTileM = TpBig::kM;  // 128 rows of x per workgroup
+constexpr int kTpTileN = TpBig::kN;  // 256 weight rows per workgroup
 constexpr int kTpBufs = 3;                // groups in LDS: one in use, two on their way
 
 constexpr int kTpTileElems = kTpTileM * kTpTileN;
@@ -170,14 +182,16 @@ __device__ __forceinline__ float tp_group_sum(const float (&cs)[4][4]) {
 // product.  1030 rows x 896 (seven groups): 9728 gate/up rows with the activation 45.5 us, 52.6
 // + 11.0 on the kernel of qgemm_q4_tall.hip with the activation behind it; 1152 rows of q/k/v
 // 23.4 (24.5).
-template <int OUT, int W, bool ODD>
-__global__ __launch_bounds__(512) void qgemm_q4g128_tallp_kernel(
+template <int OUT, int W, bool ODD, class T>
+__global__ __launch_bounds__(64 * T::kWaves) void qgemm_q4g128_tallp_kernel(
     const uint16_t* __restrict__ xp, const float* __restrict__ xs, const uint8_t* __restrict__ qw,
     const __half* __restrict__ scale, const __half* __restrict__ zero,
     const float* __restrict__ bias, void* __restrict__ y_out, float* __restrict__ partials, int m,
     int n, int k, int tiles_n, int full_tiles, int split, int out_pairs) {
     extern __shared__ uint4_t tp_lds[];  // kTpBufs x {slab of x, tile of weights}
     constexpr int BL = 2 * W;            // groups per block of small loads
+    constexpr int MI = T::kBlocks, WN = T::kAcross;
+    constexpr int kSlab = T::kSlabBytes, kBuf = T::kBufBytes;
     const int tid = threadIdx.x;
     const int lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -197,9 +211,9 @@ __global__ __launch_bounds__(512) void qgemm_q4g128_tallp_kernel(
         groups = min(groups, BL * (int)((int64_t)blocks * (q + 1) / split));
     }
     const int row_tile = tile / tiles_n;
-    const int row0 = row_tile * kTpTileM;
-    // (SwiGLU: a tile is 128 outputs wide -- 128 gate and 128 up rows of the weights)
-    constexpr int kTileOutputs = tp_is_swiglu(OUT) ? kTpTileN / 2 : kTpTileN;
+    const int row0 = row_tile * T::kM;
+    // (SwiGLU: a tile is half as many outputs wide, as many gate as up rows of the weights)
+    constexpr int kTileOutputs = tp_is_swiglu(OUT) ? T::kN / 2 : T::kN;
     const int col0 = (tile % tiles_n) * kTileOutputs;
     // weight row behind row L of the tile in LDS (a wave's B operand rows are L = wc + 32 j + r)
     auto weight_row = [&](int L) {
@@ -210,23 +224,24 @@ __global__ __launch_bounds__(512) void qgemm_q4g128_tallp_kernel(
             return min(col0 + L, n - 1);  // a row past n re-reads the last row
         }
     };
-    const int wr = (wave >> 2) * 64;  // this wave's 64 x 64 part of the 128 x 256 tile
-    const int wc = (wave & 3) * 64;
+    const int wr = (wave / WN) * 32 * MI;  // this wave's part of the tile
+    const int wc = (wave % WN) * 64;
     const int groups_row = k >> 7;    // scales and zeros: groups per weight row
     unsigned magic;
     asm volatile("v_mov_b32 %0, 0x43004300" : "=v"(magic));
     const unsigned lds_base = (unsigned)(uintptr_t)(tp_lds_ptr_t)tp_lds;
 
     // ---- requests of a group, straight into LDS (a request writes 1 KiB of consecutive LDS).
-    // x: request q of this wave covers rows 16 wave + 4 q .. + 3, lane -> row + lane / 16, LDS
+    // x: request q of this wave covers rows 4 kXReq wave + 4 q .. + 3, lane -> row + lane / 16, LDS
     // position lane % 16 of that row, which holds the row's chunk (position ^ row % 16).
     // weights: request q covers rows 32 wave + 16 q .. + 15 of the tile, lane -> row + lane / 4,
     // position lane % 4 of the row's 64 bytes, which holds piece (position ^ (row / 4) % 4).
     // Byte offsets fit 32 bits (m_pad * K * 2 and N * K < 2^31 are checked on the host).
-    unsigned xoff[4], woff[2];
+    constexpr int kXReq = T::kXRequests;
+    unsigned xoff[kXReq], woff[2];
 #pragma unroll
-    for (int q = 0; q < 4; ++q) {
-        const int row = 16 * wave + 4 * q + (lane >> 4);
+    for (int q = 0; q < kXReq; ++q) {
+        const int row = 4 * kXReq * wave + 4 * q + (lane >> 4);
         const int c = (lane & 15) ^ (row & 15);
         xoff[q] = ((unsigned)(row0 + row) * (unsigned)k + (unsigned)c * 8u) * 2u;
     }
@@ -245,24 +260,36 @@ __global__ __launch_bounds__(512) void qgemm_q4g128_tallp_kernel(
         // (scalar registers for sure: a value the compiler takes for lane-dependent would be
         // handed to the statement in vector registers)
         const unsigned xdst = __builtin_amdgcn_readfirstlane(lds_base + (unsigned)buf_off +
-                                                             (unsigned)wave * 4096u);
-        const unsigned wdst = xdst + kTpSlabBytes - (unsigned)wave * 2048u;
-        asm volatile(
-            "s_mov_b32 m0, %8\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %6\n\t"
-            "s_add_u32 m0, %8, 0x400\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %6\n\t"
-            "s_add_u32 m0, %8, 0x800\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %2, %6\n\t"
-            "s_add_u32 m0, %8, 0xc00\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %3, %6\n\t"
-            "s_mov_b32 m0, %9\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %4, %7\n\t"
-            "s_add_u32 m0, %9, 0x400\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %5, %7"
-            :
-            : "v"(xoff[0]), "v"(xoff[1]), "v"(xoff[2]), "v"(xoff[3]), "v"(woff[0]), "v"(woff[1]),
-              "s"(xsrc), "s"(wsrc), "s"(xdst), "s"(wdst)
-            : "memory", "scc");
+                                                             (unsigned)wave * (1024u * kXReq));
+        const unsigned wdst = xdst + kSlab - (unsigned)wave * (1024u * kXReq - 2048u);
+        if constexpr (kXReq == 4) {
+            asm volatile(
+                "s_mov_b32 m0, %8\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %6\n\t"
+                "s_add_u32 m0, %8, 0x400\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %6\n\t"
+                "s_add_u32 m0, %8, 0x800\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %2, %6\n\t"
+                "s_add_u32 m0, %8, 0xc00\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %3, %6\n\t"
+                "s_mov_b32 m0, %9\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %4, %7\n\t"
+                "s_add_u32 m0, %9, 0x400\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %5, %7"
+                :
+                : "v"(xoff[0]), "v"(xoff[1]), "v"(xoff[kXReq - 2]), "v"(xoff[kXReq - 1]), "v"(woff[0]), "v"(woff[1]),
+                  "s"(xsrc), "s"(wsrc), "s"(xdst), "s"(wdst)
+                : "memory", "scc");
+        } else {
+            asm volatile(
+                "s_mov_b32 m0, %6\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %4\n\t"
+                "s_add_u32 m0, %6, 0x400\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %4\n\t"
+                "s_mov_b32 m0, %7\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %2, %5\n\t"
+                "s_add_u32 m0, %7, 0x400\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %3, %5"
+                :
+                : "v"(xoff[0]), "v"(xoff[1]), "v"(woff[0]), "v"(woff[1]), "s"(xsrc), "s"(wsrc),
+                  "s"(xdst), "s"(wdst)
+                : "memory", "scc");
+        }
     };
-    constexpr int kReq = 6;  // requests per group and wave
+    constexpr int kReq = kXReq + 2;  // requests per group and wave
     // ---- A operand reads: lane (r, h) at step s8 wants chunk 8 h + s8 of row wr + 32 i + r,
     // stored at position (8 h + s8) ^ (r % 16): a0 ^ (s8 << 4), the i-tile as an immediate
-    // (a buffer's offset in the ring is a multiple of 16 KiB: adding it commutes with the XOR)
+    // (a buffer's offset in the ring is a multiple of 8 KiB: adding it commutes with the XOR)
     const unsigned a0 = lds_base + (unsigned)(wr + r) * 256u +
                         (unsigned)(((8 * h) ^ (r & 8)) | (r & 7)) * 16u;
     // ---- B operand reads: lane (r, h) of n-tile j wants the pieces 2 h, 2 h + 1 of row
@@ -270,7 +297,7 @@ __global__ __launch_bounds__(512) void qgemm_q4g128_tallp_kernel(
     unsigned b_addr[2];
 #pragma unroll
     for (int t = 0; t < 2; ++t)
-        b_addr[t] = lds_base + kTpSlabBytes + (unsigned)(wc + r) * 64u +
+        b_addr[t] = lds_base + kSlab + (unsigned)(wc + r) * 64u +
                     (unsigned)((2 * h + t) ^ ((r >> 2) & 3)) * 16u;
 
     // ---- The small loads of a block of W pairs of groups, from global memory into registers:
@@ -285,20 +312,22 @@ __global__ __launch_bounds__(512) void qgemm_q4g128_tallp_kernel(
     // here must not be touched before `small_loads_landed` has named it.
     struct Small {
         TpRegs<unsigned, W> s[2], z[2];
-        TpRegs<float, W> xs[2];
+        TpRegs<float, W> xs[2];  // (one of them with one block of rows per wave)
         unsigned s_hi[2];  // ODD: s and s_hi the scales of the pair's two groups, z the zero of
                            // this lane's group of the pair
     };
-    unsigned soff[2], xsoff[2];
+    unsigned soff[2], xsoff[MI];
 #pragma unroll
     for (int j = 0; j < 2; ++j)
         soff[j] = (unsigned)weight_row(wc + 32 * j + r) * (unsigned)groups_row * 2u;
 #pragma unroll
-    for (int i = 0; i < 2; ++i) xsoff[i] = (unsigned)((h * kTpTileM + wr + 32 * i + r) * W) * 4u;
+    for (int i = 0; i < MI; ++i)
+        xsoff[i] = (unsigned)((h * kTallTileRows + (row0 % kTallTileRows) + wr + 32 * i + r) * W) * 4u;
     auto gload_small = [&](int g, Small& v) {
         const __half* sb = scale + g;
         const __half* zb = zero + g;
-        const float* xb = xs + ((size_t)row_tile * ((groups_row + BL - 1) / BL) + g / BL) * (2 * kTpTileM * W);
+        const float* xb = xs + ((size_t)(row0 / kTallTileRows) * ((groups_row + BL - 1) / BL) + g / BL) *
+                                   (2 * kTallTileRows * W);
 #pragma unroll
         for (int j = 0; j < 2; ++j) {
             if constexpr (ODD) {
@@ -320,7 +349,7 @@ __global__ __launch_bounds__(512) void qgemm_q4g128_tallp_kernel(
             }
         }
 #pragma unroll
-        for (int i = 0; i < 2; ++i) {
+        for (int i = 0; i < MI; ++i) {
             if constexpr (W == 1)
                 asm volatile("global_load_dword %0, %1, %2" : "=&v"(v.xs[i].raw) : "v"(xsoff[i]), "s"(xb) : "memory");
             else if constexpr (W == 2)
@@ -334,18 +363,13 @@ __global__ __launch_bounds__(512) void qgemm_q4g128_tallp_kernel(
     // into LDS complete in order with each other is not relied on.  The requests of the group
     // after next, issued most of a group ago, are waited for with them -- once per block.)
     auto small_loads_landed = [&](Small& v) {
-        if constexpr (ODD)
-            asm volatile("s_waitcnt vmcnt(0)"
-                         : "+v"(v.s[0].raw), "+v"(v.s[1].raw), "+v"(v.z[0].raw), "+v"(v.z[1].raw),
-                           "+v"(v.xs[0].raw), "+v"(v.xs[1].raw), "+v"(v.s_hi[0]), "+v"(v.s_hi[1])
-                         :
-                         : "memory");
-        else
-            asm volatile("s_waitcnt vmcnt(0)"
-                         : "+v"(v.s[0].raw), "+v"(v.s[1].raw), "+v"(v.z[0].raw), "+v"(v.z[1].raw),
-                           "+v"(v.xs[0].raw), "+v"(v.xs[1].raw)
-                         :
-                         : "memory");
+        asm volatile("s_waitcnt vmcnt(0)"
+                     : "+v"(v.s[0].raw), "+v"(v.s[1].raw), "+v"(v.z[0].raw), "+v"(v.z[1].raw),
+                       "+v"(v.xs[0].raw)
+                     :
+                     : "memory");
+        if constexpr (MI == 2) asm volatile("" : "+v"(v.xs[1].raw)::"memory");
+        if constexpr (ODD) asm volatile("" : "+v"(v.s_hi[0]), "+v"(v.s_hi[1])::"memory");
     };
     // One block's values are in use while the next one's are on their way (W = 1), or the
     // next block's are loaded over them behind their last use (W > 1: a block lasts four or
@@ -354,9 +378,9 @@ __global__ __launch_bounds__(512) void qgemm_q4g128_tallp_kernel(
     Small cur;
     Small nxt;  // W == 1 only
 
-    float16_t yacc[2][2];
+    float16_t yacc[MI][2];
 #pragma unroll
-    for (int i = 0; i < 2; ++i)
+    for (int i = 0; i < MI; ++i)
 #pragma unroll
         for (int j = 0; j < 2; ++j)
 #pragma unroll
@@ -364,7 +388,7 @@ __global__ __launch_bounds__(512) void qgemm_q4g128_tallp_kernel(
 
     gload_small(g_begin, cur);
     request_group(g_begin, 0);
-    if (!ODD || g_begin + 1 < groups) request_group(g_begin + 1, kTpBufBytes);  // (else whole pairs)
+    if (!ODD || g_begin + 1 < groups) request_group(g_begin + 1, kBuf);  // (else whole pairs)
     small_loads_landed(cur);
 
     // The requests of the group after next go into the buffer everybody stopped reading before
@@ -373,8 +397,8 @@ __global__ __launch_bounds__(512) void qgemm_q4g128_tallp_kernel(
     // feeds the matrix pipe while the other is held up by its burst of requests; no change.)
     auto issue_requests = [&](int g, int buf_off) {
         if (g + 2 < groups) {
-            int dst = buf_off + 2 * kTpBufBytes;
-            if (dst >= kTpBufs * kTpBufBytes) dst -= kTpBufs * kTpBufBytes;
+            int dst = buf_off + 2 * kBuf;
+            if (dst >= kTpBufs * kBuf) dst -= kTpBufs * kBuf;
             request_group(g + 2, dst);
         }
     };
@@ -383,7 +407,7 @@ __global__ __launch_bounds__(512) void qgemm_q4g128_tallp_kernel(
     // y[m][n] += sum_x[m][g'] * (-scale[n][g'] * (128 + zero[n][g'])).  lone: the second is missing
     auto zero_term = [&](auto pair_c, bool lone) {
         constexpr int P = decltype(pair_c)::value;
-        float cv[2], sum[2];
+        float cv[2], sum[MI];
 #pragma unroll
         for (int j = 0; j < 2; ++j) {
             const unsigned sd = cur.s[j][P], zd = cur.z[j][P];
@@ -392,11 +416,12 @@ __global__ __launch_bounds__(512) void qgemm_q4g128_tallp_kernel(
             const unsigned short zb = (unsigned short)(ODD ? zd : (h ? (zd >> 16) : zd));
             cv[j] = -__half2float(__builtin_bit_cast(__half, sb)) *
                     (128.0f + __half2float(__builtin_bit_cast(__half, zb)));
-            sum[j] = cur.xs[j][P];
-            if (ODD && lone && h) cv[j] = sum[j] = 0.0f;
+            if (ODD && lone && h) cv[j] = 0.0f;
         }
 #pragma unroll
-        for (int i = 0; i < 2; ++i)
+        for (int i = 0; i < MI; ++i) sum[i] = ODD && lone && h ? 0.0f : cur.xs[i][P];
+#pragma unroll
+        for (int i = 0; i < MI; ++i)
 #pragma unroll
             for (int j = 0; j < 2; ++j)
                 yacc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(sum[i], cv[j], yacc[i][j], 0, 0, 0);
@@ -423,8 +448,8 @@ __global__ __launch_bounds__(512) void qgemm_q4g128_tallp_kernel(
             if (U == 1 && g + 1 < groups) gload_small(g + 1, nxt);
         }
         issue_requests(g, buf_off);
-        float16_t acc[2][2];
-        bf16x8_t av[2][2];  // [step parity][i]
+        float16_t acc[MI][2];
+        bf16x8_t av[2][MI];  // [step parity][i]
         bf16x8_t bv[2][2];  // [step parity][j]
         uint4_t wq[2][2];   // [j][half of the group]: the group's nibbles of this lane's rows
         // (the buffer's offset is added here: LDS offsets of up to 144 KiB do not fit the
@@ -438,14 +463,18 @@ __global__ __launch_bounds__(512) void qgemm_q4g128_tallp_kernel(
                      : "v"(b_addr[0]), "v"(b_addr[1]), "s"(buf_off)
                      : "memory");
         const unsigned a_buf = a0 + (unsigned)buf_off;
-        asm volatile("ds_read_b128 %0, %2\n\tds_read_b128 %1, %2 offset:8192"
-                     : "=&v"(av[0][0]), "=&v"(av[0][1])
-                     : "v"(a_buf)
-                     : "memory");
+        if constexpr (MI == 2)
+            asm volatile("ds_read_b128 %0, %2\n\tds_read_b128 %1, %2 offset:8192"
+                         : "=&v"(av[0][0]), "=&v"(av[0][MI - 1])
+                         : "v"(a_buf)
+                         : "memory");
+        else
+            asm volatile("ds_read_b128 %0, %1" : "=&v"(av[0][0]) : "v"(a_buf) : "memory");
         __builtin_amdgcn_sched_barrier(0);
         asm volatile("s_waitcnt lgkmcnt(0)"
                      : "+v"(wq[0][0]), "+v"(wq[0][1]), "+v"(wq[1][0]), "+v"(wq[1][1]),
-                       "+v"(av[0][0]), "+v"(av[0][1])::"memory");
+                       "+v"(av[0][0])::"memory");
+        if constexpr (MI == 2) asm volatile("" : "+v"(av[0][MI - 1])::"memory");
         auto unpack = [&](auto s8c, bf16x8_t (&b)[2]) {
             constexpr int s8 = decltype(s8c)::value;
 #pragma unroll
@@ -468,16 +497,22 @@ __global__ __launch_bounds__(512) void qgemm_q4g128_tallp_kernel(
             constexpr int cur_p = s8 & 1;
             if constexpr (s8 < 7) {
                 unsigned ta;
-                asm volatile("v_xor_b32 %2, %c4, %3\n\t"
-                             "ds_read_b128 %0, %2\n\tds_read_b128 %1, %2 offset:8192"
-                             : "=&v"(av[cur_p ^ 1][0]), "=&v"(av[cur_p ^ 1][1]), "=&v"(ta)
-                             : "v"(a_buf), "n"((s8 + 1) << 4)
-                             : "memory");
+                if constexpr (MI == 2)
+                    asm volatile("v_xor_b32 %2, %c4, %3\n\t"
+                                 "ds_read_b128 %0, %2\n\tds_read_b128 %1, %2 offset:8192"
+                                 : "=&v"(av[cur_p ^ 1][0]), "=&v"(av[cur_p ^ 1][MI - 1]), "=&v"(ta)
+                                 : "v"(a_buf), "n"((s8 + 1) << 4)
+                                 : "memory");
+                else
+                    asm volatile("v_xor_b32 %1, %c3, %2\n\tds_read_b128 %0, %1"
+                                 : "=&v"(av[cur_p ^ 1][0]), "=&v"(ta)
+                                 : "v"(a_buf), "n"((s8 + 1) << 4)
+                                 : "memory");
             }
             __builtin_amdgcn_sched_barrier(0);
             if constexpr (s8 < 7) unpack(ic<(s8 < 7 ? s8 + 1 : 7)>{}, bv[cur_p ^ 1]);
 #pragma unroll
-            for (int i = 0; i < 2; ++i)
+            for (int i = 0; i < MI; ++i)
 #pragma unroll
                 for (int j = 0; j < 2; ++j) {
                     if constexpr (s8 == 0) {
@@ -492,14 +527,15 @@ __global__ __launch_bounds__(512) void qgemm_q4g128_tallp_kernel(
                     }
                 }
 #pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // one MFMA
-                __builtin_amdgcn_sched_group_barrier(0x002, 4, 0);  // four vector instructions
+            for (int q = 0; q < 2 * MI; ++q) {
+                __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);       // one MFMA
+                __builtin_amdgcn_sched_group_barrier(0x002, 8 / MI, 0);  // vector instructions
             }
             __builtin_amdgcn_sched_barrier(0);
-            if constexpr (s8 < 7)
-                asm volatile("s_waitcnt lgkmcnt(0)"
-                             : "+v"(av[cur_p ^ 1][0]), "+v"(av[cur_p ^ 1][1])::"memory");
+            if constexpr (s8 < 7) {
+                asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(av[cur_p ^ 1][0])::"memory");
+                if constexpr (MI == 2) asm volatile("" : "+v"(av[cur_p ^ 1][MI - 1])::"memory");
+            }
         });
         if constexpr (W > 1 && U == 0) {
             // the block's values, requested at the end of the group before this one
@@ -514,7 +550,7 @@ __global__ __launch_bounds__(512) void qgemm_q4g128_tallp_kernel(
                 (unsigned short)(ODD ? (PAR ? cur.s_hi[j] : sd) : (PAR ? (sd >> 16) : sd));
             const float sf = __half2float(__builtin_bit_cast(__half, sb));
 #pragma unroll
-            for (int i = 0; i < 2; ++i)
+            for (int i = 0; i < MI; ++i)
 #pragma unroll
                 for (int e = 0; e < 16; ++e) yacc[i][j][e] = fmaf(sf, acc[i][j][e], yacc[i][j][e]);
         }
@@ -536,7 +572,7 @@ __global__ __launch_bounds__(512) void qgemm_q4g128_tallp_kernel(
     // ranges are whole blocks (K is a multiple of 256 W); buffers go round in threes
     int buf_off = 0;
     auto next_buf = [&]() {
-        buf_off = buf_off + kTpBufBytes == kTpBufs * kTpBufBytes ? 0 : buf_off + kTpBufBytes;
+        buf_off = buf_off + kBuf == kTpBufs * kBuf ? 0 : buf_off + kBuf;
     };
     if constexpr (ODD) {
         int g0 = g_begin;
@@ -558,11 +594,11 @@ __global__ __launch_bounds__(512) void qgemm_q4g128_tallp_kernel(
             });
     }
 
-    if (part >= 0) {
+    if (T::kBig && part >= 0) {
         // a part of a tile: the wave's 64 x 64 results as they lie in registers, lane fastest
         float* dst = partials + (size_t)part * kTpTileElems + (size_t)wave * 4096 + lane;
 #pragma unroll
-        for (int i = 0; i < 2; ++i)
+        for (int i = 0; i < MI; ++i)
 #pragma unroll
             for (int j = 0; j < 2; ++j)
 #pragma unroll
@@ -577,9 +613,10 @@ __global__ __launch_bounds__(512) void qgemm_q4g128_tallp_kernel(
         // the ring is done with once every wave has read its last operands
         __syncthreads();
         float* const red = reinterpret_cast<float*>(tp_lds);  // [wave column][chunk of it][row]
-        const int wq = wave & 3, cq = r >> 3;
+        static_assert(WN == 4, "a tile's outputs are one group of the next K");
+        const int wq = wave % WN, cq = r >> 3;
 #pragma unroll
-        for (int i = 0; i < 2; ++i)
+        for (int i = 0; i < MI; ++i)
 #pragma unroll
             for (int e = 0; e < 16; ++e) {
                 const int row = wr + 32 * i + 8 * (e >> 2) + 4 * h + (e & 3);
@@ -587,15 +624,15 @@ __global__ __launch_bounds__(512) void qgemm_q4g128_tallp_kernel(
                 const uint16_t b = f32_to_bf16_rne(g / (1.0f + expf(-g)) * u);
                 xo[(int64_t)(row0 + row) * n + (gn & ~7) + tp_pair_slot(gn & 7)] = b;
                 const float cs = tp_chunk_sum_across_lanes(__uint_as_float((unsigned)b << 16));
-                if ((r & 7) == 0) red[(wq * 4 + cq) * kTpTileM + row] = cs;
+                if ((r & 7) == 0) red[(wq * 4 + cq) * T::kM + row] = cs;
             }
         __syncthreads();
-        if (tid < kTpTileM) {
+        if (tid < T::kM) {
             float cs[4][4];
 #pragma unroll
             for (int a = 0; a < 4; ++a)
 #pragma unroll
-                for (int c = 0; c < 4; ++c) cs[a][c] = red[(a * 4 + c) * kTpTileM + tid];
+                for (int c = 0; c < 4; ++c) cs[a][c] = red[(a * 4 + c) * T::kM + tid];
             so[tall_sum_index(row0 + tid, col0 >> 7, n, out_pairs)] = tp_group_sum(cs);
         }
         return;
@@ -604,7 +641,7 @@ __global__ __launch_bounds__(512) void qgemm_q4g128_tallp_kernel(
         const int gn = col0 + (wc >> 1) + r;
         if (gn >= n) return;
 #pragma unroll
-        for (int i = 0; i < 2; ++i)
+        for (int i = 0; i < MI; ++i)
 #pragma unroll
             for (int e = 0; e < 16; ++e) {
                 const int gr = row0 + wr + 32 * i + 8 * (e >> 2) + 4 * h + (e & 3);
@@ -622,7 +659,7 @@ __global__ __launch_bounds__(512) void qgemm_q4g128_tallp_kernel(
         if (gn >= n) continue;
         const float bv = bias ? bias[gn] : 0.0f;
 #pragma unroll
-        for (int i = 0; i < 2; ++i)
+        for (int i = 0; i < MI; ++i)
 #pragma unroll
             for (int e = 0; e < 16; ++e) {
                 const int gr = row0 + wr + 32 * i + 8 * (e >> 2) + 4 * h + (e & 3);
@@ -740,25 +777,58 @@ bool qgemm_q4_tallp_applies(int m, int n, int k) {
     return m > 0 && n > 0 && k > 0 && k % 128 == 0 && tp_sizes_ok(m, n, k);
 }
 
-template <int OUT, int W, bool ODD = false>
-static hipError_t tallp_launch(const uint16_t* xp, const float* xs, float* partials,
+// Whether a launch takes the smaller tiles.  A 128 x 256 tile costs about 7 us + 2 us per group
+// whatever else runs, a 64 x 128 one 4 us + 1 us (a chain of requests, barriers and operand reads,
+// not arithmetic), so with few groups of K and few tiles the smaller ones win by filling the chip.
+// us, 128 x 256 / 64 x 128 (the first with the sum of its K parts):
+//   K  768, 1152 columns:  100 rows 19.1 / 11.0, 1030 20.2 / 11.6, 2060 20.7 / 15.5, 4120 22.2 / 24.7
+//   K 1536, 1536 columns:  100 rows 13.0 / 15.5,  520 18.7 / 15.9, 2060 28.9 / 22.7, 4120 31.3 / 40.2
+//   K 4096, 4096 columns:  300 rows 29.8 / 31.4, 1030 58.8 / 63.7
+// hence: at most 16 groups, all tiles resident at once (two per compute unit), and where the big
+// tiles could be split over K at least 20 of them.  A next product's operand is written by
+// 64 x 256 tiles, one per compute unit, whose round takes five eighths of a big one's:
+//   K  768, 4864 outputs:  200 rows 18.9 / 12.7,  520 19.9 / 24.4, 1030 38.2 / 36.2, 2060 56.7 / 69.7
+//   K 1536, 8960 outputs:  100 rows 24.5 / 18.7,  200 28.4 / 37.3, 1030 82.9 / 91.0
+template <int OUT>
+static bool tp_less(int m, int n, int k, int block_groups, int cus) {
+    const int groups = k >> 7;
+    if (groups > 16) return false;
+    auto tiles = [&](int rows, int tm, int tn) {
+        return (int64_t)((rows + tm - 1) / tm) * ((n + tn - 1) / tn);
+    };
+    if (OUT == kTpOutSwigluOperand) {
+        const int rows = tp_padded_rows(m);
+        const int64_t big = (tiles(rows, TpBig::kM, TpBig::kN / 2) + cus - 1) / cus;
+        const int64_t half = (tiles(rows, TpHalf::kM, TpHalf::kN / 2) + cus - 1) / cus;
+        return 5 * half < 8 * big;
+    }
+    const int div = tp_is_swiglu(OUT) ? 2 : 1;
+    if (tiles(m, TpSmall::kM, TpSmall::kN / div) > 2 * cus) return false;
+    const int big = (int)tiles(m, TpBig::kM, TpBig::kN / div);
+    return big >= 20 || tp_plan(big, groups, block_groups, cus).split == 1;
+}
+
+template <int OUT, int W, bool ODD, class T>
+static hipError_t tallp_launch_tile(const uint16_t* xp, const float* xs, float* partials,
                                const uint8_t* qw, const __half* scale, const __half* zero,
-                               const float* bias, void* y, int m, int n, int k, hipStream_t st,
-                               int out_pairs = 0) {
-    constexpr size_t lds = (size_t)kTpBufs * kTpBufBytes;
+                                    const float* bias, void* y, int m, int n, int k, hipStream_t st,
+                                    int out_pairs) {
+    constexpr size_t lds = (size_t)kTpBufs * T::kBufBytes;
     static const hipError_t opt = hipFuncSetAttribute(
-        reinterpret_cast<const void*>(qgemm_q4g128_tallp_kernel<OUT, W, ODD>),
+        reinterpret_cast<const void*>(qgemm_q4g128_tallp_kernel<OUT, W, ODD, T>),
         hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     if (opt != hipSuccess) return opt;
-    constexpr int tile_outputs = tp_is_swiglu(OUT) ? kTpTileN / 2 : kTpTileN;
+    constexpr int tile_outputs = tp_is_swiglu(OUT) ? T::kN / 2 : T::kN;
     const int tiles_n = (n + tile_outputs - 1) / tile_outputs;
-    const int tiles = tiles_n * (tp_padded_rows(m) / kTpTileM);
+    // (an operand's padding rows are written too)
+    const int rows = OUT == kTpOutSwigluOperand ? tp_padded_rows(m) : m;
+    const int tiles = tiles_n * ((rows + T::kM - 1) / T::kM);
     const int cus = device_cu_count();
     if (cus <= 0) return hipErrorInvalidDevice;
-    const TpPlan plan = tp_plan(tiles, k >> 7, 2 * W, cus);
+    const TpPlan plan = T::kBig ? tp_plan(tiles, k >> 7, 2 * W, cus) : TpPlan{tiles, 1};
     const int parts = (tiles - plan.full) * plan.split;
-    qgemm_q4g128_tallp_kernel<OUT, W, ODD>
-        <<<dim3(plan.full + (plan.split > 1 ? parts : 0)), dim3(512), lds, st>>>(
+    qgemm_q4g128_tallp_kernel<OUT, W, ODD, T>
+        <<<dim3(plan.full + (plan.split > 1 ? parts : 0)), dim3(64 * T::kWaves), lds, st>>>(
             xp, xs, qw, scale, zero, bias, y, partials, m, n, k, tiles_n, plan.full, plan.split,
             out_pairs);
     if (plan.split > 1) {
@@ -773,6 +843,21 @@ static hipError_t tallp_launch(const uint16_t* xp, const float* xs, float* parti
         }
     }
     return hipGetLastError();
+}
+
+template <int OUT, int W, bool ODD = false>
+static hipError_t tallp_launch(const uint16_t* xp, const float* xs, float* partials,
+                               const uint8_t* qw, const __half* scale, const __half* zero,
+                               const float* bias, void* y, int m, int n, int k, hipStream_t st,
+                               int out_pairs = 0) {
+    using Less = std::conditional_t<OUT == kTpOutSwigluOperand, TpHalf, TpSmall>;
+    const int cus = device_cu_count();
+    if (cus <= 0) return hipErrorInvalidDevice;
+    if (tp_less<OUT>(m, n, k, 2 * W, cus))
+        return tallp_launch_tile<OUT, W, ODD, Less>(xp, xs, partials, qw, scale, zero, bias, y, m, n,
+                                                    k, st, out_pairs);
+    return tallp_launch_tile<OUT, W, ODD, TpBig>(xp, xs, partials, qw, scale, zero, bias, y, m, n, k,
+                                                 st, out_pairs);
 }
 
 template <int OUT>

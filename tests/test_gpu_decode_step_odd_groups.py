@@ -4,6 +4,7 @@ kernel's tiles of 128 rows, MLP widths of an odd and an even number of groups.""
 import numpy as np
 import pytest
 
+from logismos_amd import kernels
 from tests import workloads
 from tests.test_gpu_decode_step import _rel_l2, _run_both
 
@@ -28,3 +29,39 @@ def test_rows_and_widths(rows, hidden, hq, hkv, d, inter):
     assert _rel_l2(got, want) < 4e-3
     assert np.all(np.abs(got - want) <= 1.2e-2 + 1.6e-2 * np.abs(want))
     assert _rel_l2(r.h.to_numpy(np.float32, bat["h"].shape), bat["h"]) < 4e-3
+
+
+@pytest.mark.parametrize("m,n,k", [
+    (1, 128, 256), (64, 5120, 512), (65, 5121, 512), (33, 4999, 2048),  # one, two row tiles of 64
+    (191, 2500, 768),    # three row tiles, a ragged column tile
+    (700, 5888, 512),    # 11 x 46 tiles of 64 x 128: two per compute unit
+    (705, 5888, 512),    # 12 x 46: past it, tiles of 128 x 256
+    (300, 640, 2304),    # 18 groups: tiles of 128 x 256
+])
+@pytest.mark.parametrize("f32", [0, 1])
+def test_tile_choice_of_the_product(m, n, k, f32):
+    import ctypes as C
+    torch = pytest.importorskip("torch")
+    gen = torch.Generator(device="cuda").manual_seed(m + n + k)
+    x = torch.randn(m, k, device="cuda", generator=gen).bfloat16()
+    q = torch.randint(0, 16, (n, k), device="cuda", generator=gen, dtype=torch.uint8)
+    qw = (q[:, 0::2] | (q[:, 1::2] << 4)).contiguous()
+    scale = (0.01 + 0.01 * torch.rand(n, k // 128, device="cuda", generator=gen)).half()
+    zero = (7.5 + 0.4 * torch.randn(n, k // 128, device="cuda", generator=gen)).half()
+    bias = torch.randn(n, device="cuda", generator=gen)
+    y = torch.full((m + 1, n), 7.0, device="cuda", dtype=torch.float32 if f32 else torch.bfloat16)
+    ws = torch.empty(kernels.qgemm_q4g128_tall_workspace_bytes(m, k), device="cuda", dtype=torch.uint8)
+    p = lambda t: C.c_void_p(t.data_ptr())
+    torch.cuda.synchronize()
+    assert kernels.library().logismos_launch_qgemm_q4g128_tall(
+        p(x), p(qw), p(scale), p(zero), p(bias), p(y), f32, p(ws), m, n, k, None) == 0
+    torch.cuda.synchronize()
+    s = scale.double().repeat_interleave(128, 1)
+    w = (q.double() - zero.double().repeat_interleave(128, 1)) * s
+    want = x.double() @ w.T + bias.double()
+    # fp32 sums of k products with terms up to (128 + 15) instead of |q - zero|: 16 * eps of them
+    bound = 16 * 2.0 ** -24 * (x.double().abs() @ (143 * s).T + bias.double().abs())
+    if not f32:
+        bound = bound + want.abs() * 2.0 ** -8
+    assert bool(((y[:m].double() - want).abs() <= bound).all())
+    assert bool((y[m] == 7.0).all())  # nothing past the last row
