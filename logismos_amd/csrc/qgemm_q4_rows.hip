@@ -291,7 +291,9 @@ __host__ __device__ __forceinline__ int rows_waves_per_row(int nw, int b) {
 // of a square root, for a tenth of its instructions; every wave of every workgroup takes it).
 __device__ __forceinline__ float rows_rsqrt(float x) {
     const float y = __builtin_amdgcn_rsqf(x);
-    return fmaf(0.5f * y, fmaf(-x * y, y, 1.0f), y);
+    // (0 and infinity, of sums of squares that overflow or vanish, are exact: the step would
+    // make them 0 * inf)
+    return __builtin_amdgcn_classf(y, 0x264) ? y : fmaf(0.5f * y, fmaf(-x * y, y, 1.0f), y);
 }
 
 // The sums of W waves' partial products (16 x 16 floats in the MFMA layout, 1 KiB apart by

@@ -56,3 +56,17 @@ def test_three_bit_pools_and_a_chunk():
         new_tokens=[1, 13, 1])
     _, got, want, _, _ = _run_both(cfg, layers, batch)
     assert _rel_l2(got, want) < 6e-3
+
+
+def test_sum_of_squares_past_fp32():
+    # a row whose sum of squares overflows: its norm is 0 (1 / sqrt(inf)), not a NaN, so that the
+    # layer adds nothing to that row; the other row is untouched by it
+    rng = np.random.default_rng(79)
+    cfg, layers, batch = workloads.decode_step_problem(
+        rng, num_layers=1, hidden=512, hq=4, hkv=2, inter=1024, ctx=[1, 9])
+    batch["h"][0] = np.float32(1e20)
+    with np.errstate(over="ignore"):
+        r, got, want, _, bat = _run_both(cfg, layers, batch)
+    h = r.h.to_numpy(np.float32, bat["h"].shape)
+    assert np.all(got[0] == 0) and np.all(h[0] == np.float32(1e20))
+    assert _rel_l2(got[1], want[1]) < 6e-3
