@@ -384,40 +384,56 @@ extern "C" logismos_status_t logismos_launch_decode_step(const logismos_decode_c
                                  reinterpret_cast<uintptr_t>(batch->hidden_f32);
             return k % 256 == 0 || (at & 15u) == 0;
         };
-        auto gemm = [&](const void* x_bf16, const logismos_q4_weight_t& W, const void* bias,
-                        void* y_f32, int n, int k) -> logismos_status_t {
+        // A launch of fewer tiles than compute units is split over K; its fp32 parts are added up
+        // by the operator that follows (in part order) instead of by a launch of their own, which
+        // took 7.5 us three times per layer (200 rows of the 4096-wide layers).  The parts lie in
+        // the launch's workspace behind its operand, K wide; the norm that adds them up writes an
+        // operand hidden wide to the front of t_gemm, hence `keep`.
+        auto product = [&](const logismos_q4_weight_t& W, char* y_f32, char* workspace, int n, int k,
+                           bool keep, lg::TallParts* out) -> logismos_status_t {
+            if (keep)
+                return lg::qgemm_q4_tallp_prepared_parts(W.qw, W.scale, W.zero, y_f32, workspace, t, n,
+                                                         k, out, st);
+            *out = {y_f32, 1};
+            return lg::qgemm_q4_tallp_prepared(W.qw, W.scale, W.zero, nullptr, y_f32, 1, workspace, t,
+                                               n, k, st);
+        };
+        auto gemm = [&](const void* x_bf16, const logismos_q4_weight_t& W, char* y_f32, int n, int k,
+                        bool keep, lg::TallParts* out) -> logismos_status_t {
             // the kernel that takes x through a first pass into the workspace; past its sizes the
             // one that stages x itself
-            if (tiled(W, nullptr, n, k))
-                return lg::qgemm_q4_tallp(x_bf16, W.qw, W.scale, W.zero, bias, y_f32, 1, w.t_gemm, t,
-                                          n, k, st);
-            return lg::qgemm_q4_tall_f32_launch(x_bf16, W.qw, W.scale, W.zero,
-                                                static_cast<const float*>(bias), y_f32, t, n, k, st);
+            if (tiled(W, nullptr, n, k)) {
+                LG_TRY(lg::qgemm_q4_tallp_prepare(x_bf16, W.scale, W.zero, w.t_gemm, t, k, st));
+                return product(W, y_f32, w.t_gemm, n, k, keep, out);
+            }
+            *out = {y_f32, 1};
+            return lg::qgemm_q4_tall_f32_launch(x_bf16, W.qw, W.scale, W.zero, nullptr, y_f32, t, n, k,
+                                                st);
         };
+        lg::TallParts res{w.t_proj, 0};  // what is to be added to the residual stream
         // add + norm followed by a projection of the normed rows: where the tiled GEMM with a
         // workspace takes the shape, the normed rows go straight into its workspace in the
         // kernel's operand order (no first pass over them)
-        auto norm_then_gemm = [&](int parts, const void* gains, const logismos_q4_weight_t& W,
-                                  void* y_f32, int n) -> logismos_status_t {
+        auto norm_then_gemm = [&](const void* gains, const logismos_q4_weight_t& W, char* y_f32, int n,
+                                  bool keep, lg::TallParts* out) -> logismos_status_t {
             if (tiled(W, gains, n, c.hidden) && c.hidden <= 16384) {
                 LG_TRY(lg::add_rms_norm_tall(
-                    batch->hidden_f32, w.t_proj, parts, gains, w.t_gemm, t, c.hidden, c.rms_eps,
+                    batch->hidden_f32, res.src, res.count, gains, w.t_gemm, t, c.hidden, c.rms_eps,
                     logismos_qgemm_q4g128_tall_pairs_per_load(c.hidden, W.scale, W.zero), st));
-                return lg::qgemm_q4_tallp_prepared(W.qw, W.scale, W.zero, nullptr, y_f32, 1, w.t_gemm,
-                                                   t, n, c.hidden, st);
+                return product(W, y_f32, w.t_gemm, n, c.hidden, keep, out);
             }
-            LG_TRY(logismos_launch_add_rms_norm_f32p(batch->hidden_f32, w.t_proj, parts, gains,
+            LG_TRY(logismos_launch_add_rms_norm_f32p(batch->hidden_f32, res.src, res.count, gains,
                                                      w.t_xn, t, c.hidden, c.rms_eps, stream));
-            return gemm(w.t_xn, W, nullptr, y_f32, n, c.hidden);
+            return gemm(w.t_xn, W, y_f32, n, c.hidden, keep, out);
         };
-        int res_parts = 0;
         for (int l = 0; l < c.num_layers; ++l) {
             const logismos_decode_layer_t& L = layers[l];
-            LG_TRY(norm_then_gemm(res_parts, L.norm1_w_f32, L.qkv, w.t_qkv, width));
+            lg::TallParts qkv;
+            LG_TRY(norm_then_gemm(L.norm1_w_f32, L.qkv, w.t_qkv, width, true, &qkv));
             const auto rope_kv_write = c.kv_turbo3 ? logismos_launch_rope_kv_write_f32p_turbo3_bias
                                                    : logismos_launch_rope_kv_write_f32p_bias;
-            LG_TRY(rope_kv_write(w.t_qkv, 1, L.qkv_bias_f32, batch->positions, batch->rope_cos_f32,
-                                 batch->rope_sin_f32, batch->slot_mapping, w.q, L.k_pool_f16,
+            LG_TRY(rope_kv_write(qkv.src, qkv.count, L.qkv_bias_f32, batch->positions,
+                                 batch->rope_cos_f32, batch->rope_sin_f32, batch->slot_mapping, w.q, L.k_pool_f16,
                                  L.v_pool_f16, t, c.num_q_heads, c.num_kv_heads, c.head_dim,
                                  c.max_pos, stream));
             LG_TRY(lg::paged_attn_launch(
@@ -425,12 +441,12 @@ extern "C" logismos_status_t logismos_launch_decode_step(const logismos_decode_c
                 batch->context_lens, w.attn_out, w.attn_ws, num_seqs, t, max_q, c.num_q_heads,
                 c.num_kv_heads, c.head_dim, c.block_size, c.max_blocks_per_seq, batch->num_splits,
                 scale, 1, LOGISMOS_ATTN_PHASE_ALL, 1, c.kv_turbo3 ? 1 : 0, stream));
-            LG_TRY(gemm(w.attn_out, L.o, nullptr, w.t_proj, c.hidden, qd));
+            LG_TRY(gemm(w.attn_out, L.o, w.t_proj, c.hidden, qd, qd >= c.hidden, &res));
             if (tiled(L.gate_up, L.norm2_w_f32, 2 * c.intermediate, c.hidden) && c.hidden <= 16384) {
                 // the gate/up projection with the SwiGLU where its products are summed: the
                 // fp32 gate and up products never go to memory
                 LG_TRY(lg::add_rms_norm_tall(
-                    batch->hidden_f32, w.t_proj, 1, L.norm2_w_f32, w.t_gemm, t, c.hidden, c.rms_eps,
+                    batch->hidden_f32, res.src, res.count, L.norm2_w_f32, w.t_gemm, t, c.hidden, c.rms_eps,
                     logismos_qgemm_q4g128_tall_pairs_per_load(c.hidden, L.gate_up.scale,
                                                               L.gate_up.zero),
                     st));
@@ -444,37 +460,37 @@ extern "C" logismos_status_t logismos_launch_decode_step(const logismos_decode_c
                         logismos_qgemm_q4g128_tall_pairs_per_load(c.intermediate, L.down.scale,
                                                                   L.down.zero),
                         w.t_gemm, t, c.intermediate, c.hidden, st));
-                    LG_TRY(lg::qgemm_q4_tallp_prepared(
-                        L.down.qw, L.down.scale, L.down.zero, nullptr, w.t_proj, 1, w.t_act, t,
-                        c.hidden, c.intermediate, st));
+                    LG_TRY(product(L.down, w.t_proj, w.t_act, c.hidden, c.intermediate, true, &res));
                 } else {
                     LG_TRY(lg::qgemm_q4_tallp_swiglu(L.gate_up.qw, L.gate_up.scale, L.gate_up.zero,
                                                      w.t_act, w.t_gemm, t, c.intermediate, c.hidden,
                                                      st));
-                    LG_TRY(gemm(w.t_act, L.down, nullptr, w.t_proj, c.hidden, c.intermediate));
+                    LG_TRY(gemm(w.t_act, L.down, w.t_proj, c.hidden, c.intermediate,
+                                c.intermediate >= c.hidden, &res));
                 }
-                res_parts = 1;
                 continue;
             }
-            LG_TRY(norm_then_gemm(1, L.norm2_w_f32, L.gate_up, w.t_gu, 2 * c.intermediate));
+            lg::TallParts gu;
+            LG_TRY(norm_then_gemm(L.norm2_w_f32, L.gate_up, w.t_gu, 2 * c.intermediate, false, &gu));
             if (logismos_check_qgemm_q4g128_tall_shape(t, c.hidden, c.intermediate, nullptr, 0) == 0) {
                 // the activation goes straight into the down projection's workspace, in the
                 // kernel's operand order: no first pass over it
                 LG_TRY(logismos_launch_silu_mul_f32p_tall(
-                    w.t_gu, 1, w.t_gemm, t, c.intermediate,
+                    gu.src, gu.count, w.t_gemm, t, c.intermediate,
                     logismos_qgemm_q4g128_tall_pairs_per_load(c.intermediate, L.down.scale,
                                                               L.down.zero),
                     stream));
                 LG_TRY(logismos_launch_qgemm_q4g128_tall_prepared(L.down.qw, L.down.scale, L.down.zero,
                                                                   nullptr, w.t_proj, 1, w.t_gemm, t,
                                                                   c.hidden, c.intermediate, stream));
+                res = {w.t_proj, 1};
             } else {
-                LG_TRY(logismos_launch_silu_mul_f32p(w.t_gu, 1, w.t_act, t, c.intermediate, stream));
-                LG_TRY(gemm(w.t_act, L.down, nullptr, w.t_proj, c.hidden, c.intermediate));
+                LG_TRY(logismos_launch_silu_mul_f32p(gu.src, gu.count, w.t_act, t, c.intermediate, stream));
+                LG_TRY(gemm(w.t_act, L.down, w.t_proj, c.hidden, c.intermediate,
+                            c.intermediate >= c.hidden, &res));
             }
-            res_parts = 1;
         }
-        LG_TRY(logismos_launch_add_rms_norm_f32p(batch->hidden_f32, w.t_proj, res_parts,
+        LG_TRY(logismos_launch_add_rms_norm_f32p(batch->hidden_f32, res.src, res.count,
                                                  batch->final_norm_w_f32, norm_dst, t, c.hidden,
                                                  c.rms_eps, stream));
         return last_only ? project_last_rows() : 0;

@@ -79,6 +79,18 @@ hipError_t qgemm_q4_tallp(const void* x_bf16, const void* qw, const void* scale,
 hipError_t qgemm_q4_tallp_prepared(const void* qw, const void* scale, const void* zero,
                                    const void* bias, void* y, int y_is_f32, void* workspace, int m,
                                    int n, int k, hipStream_t stream);
+// The first pass over x alone, and the fp32 product with its K parts left to the consumer: `count`
+// matrices [m][n] one behind the other at `src`, in the workspace behind the operand (count > 1)
+// or the finished product in y (1).
+struct TallParts {
+    char* src;
+    int count;
+};
+hipError_t qgemm_q4_tallp_prepare(const void* x_bf16, const void* scale, const void* zero,
+                                  void* workspace, int m, int k, hipStream_t stream);
+hipError_t qgemm_q4_tallp_prepared_parts(const void* qw, const void* scale, const void* zero,
+                                         void* y_f32, void* workspace, int m, int n, int k,
+                                         TallParts* out, hipStream_t stream);
 hipError_t qgemm_q4_tallp_swiglu(const void* gate_up_qw, const void* scale, const void* zero,
                                  void* act_bf16, void* workspace, int m, int inter, int k,
                                  hipStream_t stream);

@@ -175,6 +175,8 @@ __device__ __forceinline__ float tp_group_sum(const float (&cs)[4][4]) {
     return (quad[0] + quad[2]) + (quad[1] + quad[3]);
 }
 
+// out_pairs (kTpOutSwigluOperand): the following launch's W.  (kTpOutF32): 1 where the K parts are
+// left to the consumer (a launch that has nothing but parts), 0 otherwise.
 // W: pairs of groups whose scales, zeros and group sums a lane loads at once (1, 2 or 4: a
 // dword, two or four per load; K a multiple of 256 W).
 // ODD (W = 1): an odd number of groups.  Rows of scales are then only 2-byte aligned and come
@@ -594,6 +596,23 @@ __global__ __launch_bounds__(64 * T::kWaves) void qgemm_q4g128_tallp_kernel(
             });
     }
 
+    if (OUT == kTpOutF32 && T::kBig && part >= 0 && out_pairs != 0) {
+        // a part of a launch whose consumer adds up the parts: rows of an [m][n] matrix each
+        float* dst = partials + (size_t)(part % split) * ((size_t)m * n);
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+            const int gn = col0 + wc + 32 * j + r;
+            if (gn >= n) continue;
+#pragma unroll
+            for (int i = 0; i < MI; ++i)
+#pragma unroll
+                for (int e = 0; e < 16; ++e) {
+                    const int gr = row0 + wr + 32 * i + 8 * (e >> 2) + 4 * h + (e & 3);
+                    if (gr < m) dst[(int64_t)gr * n + gn] = yacc[i][j][e];
+                }
+        }
+        return;
+    }
     if (T::kBig && part >= 0) {
         // a part of a tile: the wave's 64 x 64 results as they lie in registers, lane fastest
         float* dst = partials + (size_t)part * kTpTileElems + (size_t)wave * 4096 + lane;
@@ -831,7 +850,7 @@ static hipError_t tallp_launch_tile(const uint16_t* xp, const float* xs, float* 
         <<<dim3(plan.full + (plan.split > 1 ? parts : 0)), dim3(64 * T::kWaves), lds, st>>>(
             xp, xs, qw, scale, zero, bias, y, partials, m, n, k, tiles_n, plan.full, plan.split,
             out_pairs);
-    if (plan.split > 1) {
+    if (plan.split > 1 && !(OUT == kTpOutF32 && out_pairs != 0)) {
         if constexpr (OUT == kTpOutSwigluOperand) {
             q4_tall_reduce_operand_kernel<<<dim3((tiles - plan.full) * 16), dim3(256), 0, st>>>(
                 partials, y, m, n, tiles_n, plan.full, plan.split, out_pairs);
@@ -927,6 +946,47 @@ static hipError_t tall_args_ok(const void* qw_u8, const void* scale_f16,
     return hipSuccess;
 }
 
+// How many K parts the launch leaves to a consumer that asks for them; 1: the finished product.
+static int tallp_parts(const void* scale_f16, const void* zero_f16, int m, int n, int k) {
+    const int cus = device_cu_count();
+    if (cus <= 0) return 1;
+    const int block_groups = ((k >> 7) & 1) ? 2 : 2 * tp_pairs_per_load(k, scale_f16, zero_f16);
+    if (tp_less<kTpOutF32>(m, n, k, block_groups, cus)) return 1;
+    const int tiles = ((m + kTpTileM - 1) / kTpTileM) * ((n + kTpTileN - 1) / kTpTileN);
+    const TpPlan plan = tp_plan(tiles, k >> 7, block_groups, cus);
+    return plan.full == 0 ? plan.split : 1;
+}
+
+hipError_t qgemm_q4_tallp_prepared_parts(const void* qw_u8, const void* scale_f16,
+                                         const void* zero_f16, void* y_f32, void* workspace, int m,
+                                         int n, int k, TallParts* out, hipStream_t st) {
+    if (const hipError_t e = tall_args_ok(qw_u8, scale_f16, zero_f16, y_f32, workspace, m, n, k))
+        return e;
+    out->count = tallp_parts(scale_f16, zero_f16, m, n, k);
+    out->src = out->count > 1 ? static_cast<char*>(workspace) + tp_partials_offset(m, k)
+                              : static_cast<char*>(y_f32);
+    const int w = tp_pairs_per_load(k, scale_f16, zero_f16);
+    return tallp_launch_w<kTpOutF32>(
+        w, static_cast<const uint16_t*>(workspace),
+        reinterpret_cast<const float*>(static_cast<char*>(workspace) + tp_sums_offset(m, k)),
+        reinterpret_cast<float*>(static_cast<char*>(workspace) + tp_partials_offset(m, k)),
+        static_cast<const uint8_t*>(qw_u8), static_cast<const __half*>(scale_f16),
+        static_cast<const __half*>(zero_f16), nullptr, y_f32, m, n, k, st, out->count > 1 ? 1 : 0);
+}
+
+hipError_t qgemm_q4_tallp_prepare(const void* x_bf16, const void* scale_f16, const void* zero_f16,
+                                  void* workspace, int m, int k, hipStream_t st) {
+    if (!x_bf16 || ((reinterpret_cast<uintptr_t>(x_bf16) | reinterpret_cast<uintptr_t>(workspace)) & 15u))
+        return hipErrorInvalidValue;
+    const int m_pad = tp_padded_rows(m);
+    const int64_t chunks = (int64_t)m_pad * (k / 8);
+    q4_tall_prepare_kernel<<<dim3((unsigned)((chunks + 255) / 256)), dim3(256), 0, st>>>(
+        static_cast<const uint16_t*>(x_bf16), static_cast<uint16_t*>(workspace),
+        reinterpret_cast<float*>(static_cast<char*>(workspace) + tp_sums_offset(m, k)), m, m_pad, k,
+        tp_pairs_per_load(k, scale_f16, zero_f16));
+    return hipGetLastError();
+}
+
 hipError_t qgemm_q4_tallp_prepared(
     const void* qw_u8, const void* scale_f16, const void* zero_f16, const void* bias_f32, void* y,
     int y_is_f32, void* workspace, int m, int n, int k, hipStream_t st) {
@@ -1005,14 +1065,8 @@ hipError_t qgemm_q4_tallp(
     if (const hipError_t e = tall_args_ok(qw_u8, scale_f16, zero_f16, y, workspace, m, n, k))
         return e;
     if (!x_bf16 || (reinterpret_cast<uintptr_t>(x_bf16) & 15u)) return hipErrorInvalidValue;
-    const int m_pad = tp_padded_rows(m);
-    uint16_t* xp = static_cast<uint16_t*>(workspace);
-    float* xs = reinterpret_cast<float*>(static_cast<char*>(workspace) + tp_sums_offset(m, k));
-    const int64_t chunks = (int64_t)m_pad * (k / 8);
-    const int w = tp_pairs_per_load(k, scale_f16, zero_f16);
-    q4_tall_prepare_kernel<<<dim3((unsigned)((chunks + 255) / 256)), dim3(256), 0, st>>>(
-        static_cast<const uint16_t*>(x_bf16), xp, xs, m, m_pad, k, w);
-    if (const hipError_t e = hipGetLastError()) return e;
+    if (const hipError_t e = qgemm_q4_tallp_prepare(x_bf16, scale_f16, zero_f16, workspace, m, k, st))
+        return e;
     return qgemm_q4_tallp_prepared(qw_u8, scale_f16, zero_f16, bias_f32, y,
                                                       y_is_f32, workspace, m, n, k, st);
 }

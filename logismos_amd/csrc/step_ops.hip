@@ -408,16 +408,23 @@ __global__ __launch_bounds__(256) void rope_kv_write_rows_kernel(
     const int head = (int)(th - t * heads);
     const int64_t off = th * 128;
     float4_t x0 = {0.0f, 0.0f, 0.0f, 0.0f}, x1 = x0;
-    for (int q = 0; q < num_parts; ++q) {
-        const float* src = qkv_parts + (int64_t)q * part_stride + off + i;
-        const float4_t a = *reinterpret_cast<const float4_t*>(src);
-        const float4_t b = *reinterpret_cast<const float4_t*>(src + 64);
+    for_part_rounds<4>(num_parts, [&](auto nc, int q0) {
+        constexpr int N = decltype(nc)::value;
+        float4_t a[N], b[N];
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            x0[e] += a[e];
-            x1[e] += b[e];
+        for (int u = 0; u < N; ++u) {
+            const float* src = qkv_parts + (int64_t)(q0 + u) * part_stride + off + i;
+            a[u] = *reinterpret_cast<const float4_t*>(src);
+            b[u] = *reinterpret_cast<const float4_t*>(src + 64);
         }
-    }
+#pragma unroll
+        for (int u = 0; u < N; ++u)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                x0[e] += a[u][e];
+                x1[e] += b[u][e];
+            }
+    });
     if (bias) {
         const float4_t b0 = *reinterpret_cast<const float4_t*>(bias + head * 128 + i);
         const float4_t b1 = *reinterpret_cast<const float4_t*>(bias + head * 128 + i + 64);

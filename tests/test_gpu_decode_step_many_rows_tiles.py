@@ -1,6 +1,7 @@
-"""Steps of 97 packed rows and more whose projections have an odd number of groups of K, against
-the oracle: one group, three, seven and nine (which are split over K), row counts around the
-kernel's tiles of 128 rows, MLP widths of an odd and an even number of groups."""
+"""Steps of 97 packed rows and more on the tiled projections, at the edges of their dispatch,
+against the oracle: an odd number of groups of K (one, three, seven, and nine, which are split over
+K), row counts around the tiles of 128 rows, tiles of 64 rows, K parts added up by the operator
+behind a projection."""
 import numpy as np
 import pytest
 
@@ -65,3 +66,21 @@ def test_tile_choice_of_the_product(m, n, k, f32):
         bound = bound + want.abs() * 2.0 ** -8
     assert bool(((y[:m].double() - want).abs() <= bound).all())
     assert bool((y[m] == 7.0).all())  # nothing past the last row
+
+
+@pytest.mark.parametrize("hidden,hq,hkv,d,inter,turbo3", [
+    (2304, 24, 8, 96, 2304, False),  # 18 groups everywhere: the consumers add up the K parts
+    (2560, 20, 4, 128, 3072, True),  # ... and the 3-bit writer
+    (2560, 18, 2, 128, 2304, False),  # o and down narrower than the norm behind them
+    (2304, 18, 2, 128, 2432, False),  # an odd number of groups behind the activation
+])
+def test_parts_left_to_the_consumer(hidden, hq, hkv, d, inter, turbo3):
+    rng = np.random.default_rng(hidden + inter)
+    cfg, layers, batch = workloads.decode_step_problem(
+        rng, num_layers=2, hidden=hidden, hq=hq, hkv=hkv, d=d, inter=inter, ctx=[40, 150, 3],
+        new_tokens=[1, 99, 1], kv_turbo3=turbo3)
+    r, got, want, lay, bat = _run_both(cfg, layers, batch)
+    # two layers over many rows; 3-bit pools: the bound of the steps over them
+    bound = 1e-2 if turbo3 else 6e-3
+    assert _rel_l2(got, want) < bound
+    assert _rel_l2(r.h.to_numpy(np.float32, bat["h"].shape), bat["h"]) < bound
