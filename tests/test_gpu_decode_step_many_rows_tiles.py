@@ -71,8 +71,8 @@ def test_tile_choice_of_the_product(m, n, k, f32):
 @pytest.mark.parametrize("hidden,hq,hkv,d,inter,turbo3", [
     (2304, 24, 8, 96, 2304, False),  # 18 groups everywhere: the consumers add up the K parts
     (2560, 20, 4, 128, 3072, True),  # ... and the 3-bit writer
-    (2560, 18, 2, 128, 2304, False),  # o and down narrower than the norm behind them
-    (2304, 18, 2, 128, 2432, False),  # an odd number of groups behind the activation
+    (2560, 18, 3, 128, 2304, False),  # o and down narrower than the norm behind them
+    (2304, 18, 3, 128, 2432, False),  # an odd number of groups behind the activation
 ])
 def test_parts_left_to_the_consumer(hidden, hq, hkv, d, inter, turbo3):
     rng = np.random.default_rng(hidden + inter)
