@@ -376,7 +376,7 @@ extern "C" logismos_status_t logismos_launch_decode_step(const logismos_decode_c
         hipStream_t st = static_cast<hipStream_t>(stream);
         // The tiled GEMM over a workspace.  An odd number of groups of K only where its 16-byte
         // loads are aligned (the kernel that stages x itself takes any address; a layer of width
-        // 896 at 1030 rows takes 215 us on that one, 201 here).
+        // 896 at 1030 rows takes 215 us on that one, 177 here).
         auto tiled = [&](const logismos_q4_weight_t& W, const void* gains, int n, int k) {
             if (!lg::qgemm_q4_tallp_applies(t, n, k)) return false;
             const uintptr_t at = reinterpret_cast<uintptr_t>(W.qw) |

@@ -181,9 +181,9 @@ __device__ __forceinline__ float tp_group_sum(const float (&cs)[4][4]) {
 // dword, two or four per load; K a multiple of 256 W).
 // ODD (W = 1): an odd number of groups.  Rows of scales are then only 2-byte aligned and come
 // as halves; the last pair has one group, whose missing partner adds 0 * 0 to the zero-point
-// product.  1030 rows x 896 (seven groups): 9728 gate/up rows with the activation 45.5 us, 52.6
+// product.  1030 rows x 896 (seven groups): 9728 gate/up rows with the activation 44.2 us, 52.6
 // + 11.0 on the kernel of qgemm_q4_tall.hip with the activation behind it; 1152 rows of q/k/v
-// 23.4 (24.5).
+// 14.1 (24.5), both on the smaller tiles of `tp_less`.
 template <int OUT, int W, bool ODD, class T>
 __global__ __launch_bounds__(64 * T::kWaves) void qgemm_q4g128_tallp_kernel(
     const uint16_t* __restrict__ xp, const float* __restrict__ xs, const uint8_t* __restrict__ qw,
