@@ -385,8 +385,9 @@ extern "C" logismos_status_t logismos_launch_decode_step(const logismos_decode_c
             return k % 256 == 0 || (at & 15u) == 0;
         };
         // A launch of fewer tiles than compute units is split over K; its fp32 parts are added up
-        // by the operator that follows (in part order) instead of by a launch of their own, which
-        // took 7.5 us three times per layer (200 rows of the 4096-wide layers).  The parts lie in
+        // by the operator that follows instead of by a launch of their own, which took 7.5 us three
+        // times per layer (200 rows of the 4096-wide layers): in part order from zero, the same
+        // sum, which is then added to the residual stream or rotated.  The parts lie in
         // the launch's workspace behind its operand, K wide; the norm that adds them up writes an
         // operand hidden wide to the front of t_gemm, hence `keep`.
         auto product = [&](const logismos_q4_weight_t& W, char* y_f32, char* workspace, int n, int k,
@@ -418,12 +419,12 @@ extern "C" logismos_status_t logismos_launch_decode_step(const logismos_decode_c
                                   bool keep, lg::TallParts* out) -> logismos_status_t {
             if (tiled(W, gains, n, c.hidden) && c.hidden <= 16384) {
                 LG_TRY(lg::add_rms_norm_tall(
-                    batch->hidden_f32, res.src, res.count, gains, w.t_gemm, t, c.hidden, c.rms_eps,
+                    batch->hidden_f32, res.src, res.count, true, gains, w.t_gemm, t, c.hidden, c.rms_eps,
                     logismos_qgemm_q4g128_tall_pairs_per_load(c.hidden, W.scale, W.zero), st));
                 return product(W, y_f32, w.t_gemm, n, c.hidden, keep, out);
             }
-            LG_TRY(logismos_launch_add_rms_norm_f32p(batch->hidden_f32, res.src, res.count, gains,
-                                                     w.t_xn, t, c.hidden, c.rms_eps, stream));
+            LG_TRY(lg::add_rms_norm_f32p(batch->hidden_f32, res.src, res.count, true, gains, w.t_xn, t,
+                                         c.hidden, c.rms_eps, st));
             return gemm(w.t_xn, W, y_f32, n, c.hidden, keep, out);
         };
         for (int l = 0; l < c.num_layers; ++l) {
@@ -446,7 +447,8 @@ extern "C" logismos_status_t logismos_launch_decode_step(const logismos_decode_c
                 // the gate/up projection with the SwiGLU where its products are summed: the
                 // fp32 gate and up products never go to memory
                 LG_TRY(lg::add_rms_norm_tall(
-                    batch->hidden_f32, res.src, res.count, L.norm2_w_f32, w.t_gemm, t, c.hidden, c.rms_eps,
+                    batch->hidden_f32, res.src, res.count, true, L.norm2_w_f32, w.t_gemm, t, c.hidden,
+                    c.rms_eps,
                     logismos_qgemm_q4g128_tall_pairs_per_load(c.hidden, L.gate_up.scale,
                                                               L.gate_up.zero),
                     st));
@@ -490,9 +492,8 @@ extern "C" logismos_status_t logismos_launch_decode_step(const logismos_decode_c
                             c.intermediate >= c.hidden, &res));
             }
         }
-        LG_TRY(logismos_launch_add_rms_norm_f32p(batch->hidden_f32, res.src, res.count,
-                                                 batch->final_norm_w_f32, norm_dst, t, c.hidden,
-                                                 c.rms_eps, stream));
+        LG_TRY(lg::add_rms_norm_f32p(batch->hidden_f32, res.src, res.count, true,
+                                     batch->final_norm_w_f32, norm_dst, t, c.hidden, c.rms_eps, st));
         return last_only ? project_last_rows() : 0;
     }
     int res_parts = 0;  // split-K parts of the last down projection not yet folded into h

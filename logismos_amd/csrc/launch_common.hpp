@@ -98,9 +98,14 @@ hipError_t qgemm_q4_tallp_swiglu_operand(const void* gate_up_qw, const void* sca
                                          void* next_workspace, int next_pairs_per_load,
                                          void* workspace, int m, int inter, int k,
                                          hipStream_t stream);
-// h += parts; RMSNorm of h as that kernel's operand (step_ops.hip), likewise
-hipError_t add_rms_norm_tall(void* h_f32, const void* parts_f32, int num_parts, const void* w_f32,
-                             void* workspace, int rows, int n, float eps, int pairs_per_load,
+// h += parts; RMSNorm of h as that kernel's operand (step_ops.hip), likewise; and as bf16 rows.
+// sum_first: the parts are added up from zero and that sum is added to h (the exported entry points
+// add them to h one by one).
+hipError_t add_rms_norm_tall(void* h_f32, const void* parts_f32, int num_parts, bool sum_first,
+                             const void* w_f32, void* workspace, int rows, int n, float eps,
+                             int pairs_per_load, hipStream_t stream);
+hipError_t add_rms_norm_f32p(void* h_f32, const void* parts_f32, int num_parts, bool sum_first,
+                             const void* w_f32, void* out_bf16, int rows, int n, float eps,
                              hipStream_t stream);
 
 // dst[s][:] = src[cu_seqlens[s + 1] - 1][:], bf16 rows of `hidden` elements (step_ops.hip): the

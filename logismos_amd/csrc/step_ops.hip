@@ -30,6 +30,13 @@ __device__ __forceinline__ unsigned short f32_to_bf16(float f) {
 constexpr int kNormThreads = 1024;
 constexpr int kNormMaxPasses = 4;  // rows up to 16384 wide stay in registers
 
+// What the fp32 parts of a product are added to.  false: the residual itself, one part after the
+// other (h + p0) + p1 ..; true: each other, from zero, and that sum to the residual once,
+// h + ((0 + p0) + p1 ..), which is the finished product added: every part is rounded at the size
+// of the product and not at that of the residual, and the bits do not depend on whether a
+// product's launch or the operator behind it adds its parts up (a last bit in front of a 3-bit
+// K/V row flips a whole code).  Steps of many rows take the second form.
+template <bool SUM_FIRST>
 __global__ __launch_bounds__(kNormThreads) void add_rms_norm_kernel(
     float* __restrict__ h, const uint16_t* __restrict__ y, const float* __restrict__ yp,
     int num_parts, int64_t part_stride, const float* __restrict__ w, uint16_t* __restrict__ out,
@@ -55,6 +62,8 @@ __global__ __launch_bounds__(kNormThreads) void add_rms_norm_kernel(
                     *reinterpret_cast<float4_t*>(hr + j) = v[p];
                 } else if (yp) {
                     // fp32 partial sums of a split-K projection, added in part order
+                    float4_t s = {0.0f, 0.0f, 0.0f, 0.0f};
+                    if constexpr (!SUM_FIRST) s = v[p];
                     for_part_rounds<4>(num_parts, [&](auto nc, int q0) {
                         constexpr int N = decltype(nc)::value;
                         float4_t t4[N];
@@ -65,8 +74,10 @@ __global__ __launch_bounds__(kNormThreads) void add_rms_norm_kernel(
 #pragma unroll
                         for (int u = 0; u < N; ++u)
 #pragma unroll
-                            for (int e = 0; e < 4; ++e) v[p][e] += t4[u][e];
+                            for (int e = 0; e < 4; ++e) s[e] += t4[u][e];
                     });
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) v[p][e] = SUM_FIRST ? v[p][e] + s[e] : s[e];
                     *reinterpret_cast<float4_t*>(hr + j) = v[p];
                 }
 #pragma unroll
@@ -80,7 +91,9 @@ __global__ __launch_bounds__(kNormThreads) void add_rms_norm_kernel(
                 t += bf16_to_f32(y[row * n + j]);
                 hr[j] = t;
             } else if (yp) {
-                for (int q = 0; q < num_parts; ++q) t += yp[(int64_t)q * part_stride + row * n + j];
+                float s = SUM_FIRST ? 0.0f : t;
+                for (int q = 0; q < num_parts; ++q) s += yp[(int64_t)q * part_stride + row * n + j];
+                t = SUM_FIRST ? t + s : s;
                 hr[j] = t;
             }
             sum_sq = fmaf(t, t, sum_sq);
@@ -123,7 +136,7 @@ constexpr int kPrepMaxPasses = 4;  // rows up to 16384 wide
 // TALL: the normed rows leave as the operand of the tiled GEMM for many rows instead
 // (q4_common.hpp: row-major in pair order, `pairs` pairs of groups per block of sums; the grid
 // covers the rows padded to the GEMM's 128-row tiles, and a padding row is written as zeros).
-template <bool TALL>
+template <bool TALL, bool SUM_FIRST>
 __global__ __launch_bounds__(kPrepThreads) void add_rms_norm_xprep_kernel(
     float* __restrict__ h, const float* __restrict__ yp, int num_parts, int64_t part_stride,
     const float* __restrict__ w, void* __restrict__ xprep, int rows, int n, float eps,
@@ -154,8 +167,9 @@ __global__ __launch_bounds__(kPrepThreads) void add_rms_norm_xprep_kernel(
             const float4_t a = *reinterpret_cast<const float4_t*>(hr + j);
             const float4_t b = *reinterpret_cast<const float4_t*>(hr + j + 4);
             float4_t s0 = a, s1 = b;
-            // h + part 0 + part 1 + ... in this order; the loads of up to six parts in flight
-            // per round (a round is one trip to memory: 4 parts take one, 12 take two)
+            if constexpr (SUM_FIRST) s0 = s1 = float4_t{0.0f, 0.0f, 0.0f, 0.0f};
+            // parts in order; the loads of up to six in flight per round (a round is one trip to
+            // memory: 4 parts take one, 12 take two)
             for_part_rounds<6>(num_parts, [&](auto nc, int q0) {
                 constexpr int N = decltype(nc)::value;
                 float4_t t0[N], t1[N];
@@ -175,8 +189,8 @@ __global__ __launch_bounds__(kPrepThreads) void add_rms_norm_xprep_kernel(
             });
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
-                v[p][e] = s0[e];
-                v[p][4 + e] = s1[e];
+                v[p][e] = SUM_FIRST ? a[e] + s0[e] : s0[e];
+                v[p][4 + e] = SUM_FIRST ? b[e] + s1[e] : s1[e];
             }
             if (num_parts > 0) {
                 *reinterpret_cast<float4_t*>(hr + j) = float4_t{v[p][0], v[p][1], v[p][2], v[p][3]};
@@ -688,10 +702,26 @@ extern "C" logismos_status_t logismos_launch_add_rms_norm_bf16(void* h_f32, cons
                                                                logismos_stream_t stream) {
     if (rows <= 0 || n <= 0 || (int64_t)rows * n > (int64_t)INT32_MAX) return hipErrorInvalidValue;
     if (!h_f32 || !w_f32 || !out_bf16) return hipErrorInvalidValue;
-    lg::add_rms_norm_kernel<<<dim3(rows), dim3(lg::kNormThreads), 0,
+    lg::add_rms_norm_kernel<false><<<dim3(rows), dim3(lg::kNormThreads), 0,
                               static_cast<hipStream_t>(stream)>>>(
         static_cast<float*>(h_f32), static_cast<const uint16_t*>(y_bf16), nullptr, 0, 0,
         static_cast<const float*>(w_f32), static_cast<uint16_t*>(out_bf16), n, eps);
+    return hipGetLastError();
+}
+
+hipError_t lg::add_rms_norm_f32p(void* h_f32, const void* parts_f32, int num_parts,
+                                 bool sum_first, const void* w_f32, void* out_bf16, int rows, int n,
+                                 float eps, hipStream_t stream) {
+    if (rows <= 0 || n <= 0 || (int64_t)rows * n > (int64_t)INT32_MAX) return hipErrorInvalidValue;
+    if (!h_f32 || !w_f32 || !out_bf16 || num_parts < 0 || (num_parts > 0 && !parts_f32))
+        return hipErrorInvalidValue;
+    const auto kernel = sum_first && num_parts > 1 ? lg::add_rms_norm_kernel<true>
+                                                   : lg::add_rms_norm_kernel<false>;
+    kernel<<<dim3(rows), dim3(lg::kNormThreads), 0, stream>>>(
+        static_cast<float*>(h_f32), nullptr,
+        num_parts > 0 ? static_cast<const float*>(parts_f32) : nullptr, num_parts,
+        (int64_t)rows * n, static_cast<const float*>(w_f32), static_cast<uint16_t*>(out_bf16), n,
+        eps);
     return hipGetLastError();
 }
 
@@ -700,16 +730,8 @@ extern "C" logismos_status_t logismos_launch_add_rms_norm_f32p(void* h_f32, cons
                                                                void* out_bf16, int rows, int n,
                                                                float eps,
                                                                logismos_stream_t stream) {
-    if (rows <= 0 || n <= 0 || (int64_t)rows * n > (int64_t)INT32_MAX) return hipErrorInvalidValue;
-    if (!h_f32 || !w_f32 || !out_bf16 || num_parts < 0 || (num_parts > 0 && !parts_f32))
-        return hipErrorInvalidValue;
-    lg::add_rms_norm_kernel<<<dim3(rows), dim3(lg::kNormThreads), 0,
-                              static_cast<hipStream_t>(stream)>>>(
-        static_cast<float*>(h_f32), nullptr,
-        num_parts > 0 ? static_cast<const float*>(parts_f32) : nullptr, num_parts,
-        (int64_t)rows * n, static_cast<const float*>(w_f32), static_cast<uint16_t*>(out_bf16), n,
-        eps);
-    return hipGetLastError();
+    return lg::add_rms_norm_f32p(h_f32, parts_f32, num_parts, false, w_f32, out_bf16, rows, n, eps,
+                                 static_cast<hipStream_t>(stream));
 }
 
 extern "C" logismos_status_t logismos_launch_rope_kv_write_fp16(
@@ -926,7 +948,7 @@ extern "C" logismos_status_t logismos_launch_add_rms_norm_f32p_xprep(
         return hipErrorInvalidValue;
     if (!h_f32 || !w_f32 || !x_prepared || num_parts < 0 || (num_parts > 0 && !parts_f32))
         return hipErrorInvalidValue;
-    lg::add_rms_norm_xprep_kernel<false><<<dim3(rows), dim3(lg::kPrepThreads), 0,
+    lg::add_rms_norm_xprep_kernel<false, false><<<dim3(rows), dim3(lg::kPrepThreads), 0,
                                            static_cast<hipStream_t>(stream)>>>(
         static_cast<float*>(h_f32), static_cast<const float*>(parts_f32), num_parts,
         (int64_t)rows * n, static_cast<const float*>(w_f32), x_prepared, rows, n, eps, 0);
@@ -934,8 +956,8 @@ extern "C" logismos_status_t logismos_launch_add_rms_norm_f32p_xprep(
 }
 
 hipError_t lg::add_rms_norm_tall(void* h_f32, const void* parts_f32, int num_parts,
-                                 const void* w_f32, void* workspace, int rows, int n, float eps,
-                                 int pairs_per_load, hipStream_t stream) {
+                                 bool sum_first, const void* w_f32, void* workspace, int rows, int n,
+                                 float eps, int pairs_per_load, hipStream_t stream) {
     if (rows <= 0 || n <= 0 || num_parts < 0 ||
         (pairs_per_load != 1 && pairs_per_load != 2 && pairs_per_load != 4) ||
         n % (pairs_per_load == 1 ? 128 : 256 * pairs_per_load) != 0 ||
@@ -948,7 +970,9 @@ hipError_t lg::add_rms_norm_tall(void* h_f32, const void* parts_f32, int num_par
     if ((reinterpret_cast<uintptr_t>(h_f32) | reinterpret_cast<uintptr_t>(parts_f32) |
          reinterpret_cast<uintptr_t>(w_f32) | reinterpret_cast<uintptr_t>(workspace)) & 15u)
         return hipErrorInvalidValue;
-    lg::add_rms_norm_xprep_kernel<true><<<dim3(rows_pad), dim3(lg::kPrepThreads), 0, stream>>>(
+    const auto kernel = sum_first && num_parts > 1 ? lg::add_rms_norm_xprep_kernel<true, true>
+                                                   : lg::add_rms_norm_xprep_kernel<true, false>;
+    kernel<<<dim3(rows_pad), dim3(lg::kPrepThreads), 0, stream>>>(
         static_cast<float*>(h_f32), static_cast<const float*>(parts_f32), num_parts,
         (int64_t)rows * n, static_cast<const float*>(w_f32), workspace, rows, n, eps,
         pairs_per_load);
@@ -959,7 +983,7 @@ extern "C" logismos_status_t logismos_launch_add_rms_norm_f32p_tall(
     void* h_f32, const void* parts_f32, int num_parts, const void* w_f32, void* workspace,
     int rows, int n, float eps, int pairs_per_load, logismos_stream_t stream) {
     if (n % 256 != 0) return hipErrorInvalidValue;
-    return lg::add_rms_norm_tall(h_f32, parts_f32, num_parts, w_f32, workspace, rows, n, eps,
+    return lg::add_rms_norm_tall(h_f32, parts_f32, num_parts, false, w_f32, workspace, rows, n, eps,
                                  pairs_per_load, static_cast<hipStream_t>(stream));
 }
 

@@ -5,8 +5,9 @@ behind a projection."""
 import numpy as np
 import pytest
 
-from logismos_amd import kernels
+from logismos_amd import hip, kernels
 from tests import workloads
+from tests.gpu_harness import DecodeStepRunner
 from tests.test_gpu_decode_step import _rel_l2, _run_both
 
 pytestmark = pytest.mark.gpu
@@ -84,3 +85,42 @@ def test_parts_left_to_the_consumer(hidden, hq, hkv, d, inter, turbo3):
     bound = 1e-2 if turbo3 else 6e-3
     assert _rel_l2(got, want) < bound
     assert _rel_l2(r.h.to_numpy(np.float32, bat["h"].shape), bat["h"]) < bound
+
+
+@pytest.mark.parametrize("num_layers", [1, 2])
+@pytest.mark.parametrize("hidden,hq,hkv,d,inter,turbo3", [
+    (2304, 18, 3, 128, 2304, False),
+    (2304, 18, 3, 128, 2816, True),
+])
+def test_parts_are_added_to_the_residual_as_one_sum(num_layers, hidden, hq, hkv, d, inter, turbo3):
+    # the residual stream takes a projection whose K parts were left to the norm behind it as the
+    # projection itself gives it: the parts added up from zero, then that sum added once.  Bit for
+    # bit the finished product of the projection's own launch.  (o and every later layer add
+    # nothing: their scales are 0.  One layer: the final norm adds the parts up; two: the norm in
+    # front of the next projection.)
+    rng = np.random.default_rng(hidden + inter + num_layers)
+    cfg, layers, batch = workloads.decode_step_problem(
+        rng, num_layers=num_layers, hidden=hidden, hq=hq, hkv=hkv, d=d, inter=inter,
+        ctx=[40, 150, 3], new_tokens=[1, 99, 1], kv_turbo3=turbo3)
+    for i, L in enumerate(layers):
+        L["o"] = (L["o"][0], np.zeros_like(L["o"][1]), L["o"][2])
+        if i:
+            L["down"] = (L["down"][0], np.zeros_like(L["down"][1]), L["down"][2])
+    r = DecodeStepRunner(cfg, layers, batch)
+    r.launch()
+    r.result_bits()
+    t = batch["h"].shape[0]
+    got = r.h.to_numpy(np.float32, (t, hidden))
+
+    up = hip.DeviceBuffer.from_numpy
+    dev = {n: [up(np.ascontiguousarray(a).view(np.uint16 if a.dtype == np.float16 else a.dtype))
+               for a in layers[0][n]] for n in ("gate_up", "down")}
+    ws = hip.DeviceBuffer(kernels.qgemm_q4g128_tall_workspace_bytes(t, max(hidden, inter)))
+    h, act, y = up(batch["h"]), hip.DeviceBuffer(t * inter * 2), hip.DeviceBuffer(t * hidden * 4)
+    pairs = kernels.qgemm_q4g128_tall_pairs_per_load(hidden, *dev["gate_up"][1:])
+    kernels.launch_add_rms_norm_f32p_tall(h, None, 0, up(layers[0]["norm2"]), ws, t, hidden,
+                                          cfg["eps"], pairs)
+    kernels.launch_qgemm_q4g128_tall_swiglu_prepared(*dev["gate_up"], act, ws, t, inter, hidden)
+    kernels.launch_qgemm_q4g128_tall(act, *dev["down"], y, ws, t, hidden, inter, f32_out=True)
+    hip.synchronize()
+    assert np.array_equal(got, batch["h"] + y.to_numpy(np.float32, (t, hidden)))
