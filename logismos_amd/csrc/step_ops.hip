@@ -169,8 +169,10 @@ __global__ __launch_bounds__(kPrepThreads) void add_rms_norm_xprep_kernel(
             float4_t s0 = a, s1 = b;
             if constexpr (SUM_FIRST) s0 = s1 = float4_t{0.0f, 0.0f, 0.0f, 0.0f};
             // parts in order; the loads of up to six in flight per round (a round is one trip to
-            // memory: 4 parts take one, 12 take two)
-            for_part_rounds<6>(num_parts, [&](auto nc, int q0) {
+            // memory: 4 parts take one, 12 take two), of five beside a residual that waits: the
+            // sixth takes 130 registers, and with them half of the workgroups off a compute unit
+            // (24 layers of width 896 at 1030 rows: 1.9 % of the step, 80 us)
+            for_part_rounds<SUM_FIRST ? 5 : 6>(num_parts, [&](auto nc, int q0) {
                 constexpr int N = decltype(nc)::value;
                 float4_t t0[N], t1[N];
 #pragma unroll
