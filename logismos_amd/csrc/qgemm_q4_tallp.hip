@@ -56,7 +56,9 @@ typedef __attribute__((address_space(3))) void* tp_lds_ptr_t;
 typedef const __attribute__((address_space(1))) void* tp_glb_ptr_t;
 
 // A workgroup's tile: two rows of ACROSS waves, a wave takes 32 * BLOCKS rows of x by 64 weight rows.
-template <int BLOCKS, int ACROSS>
+// CUTS: adds up in the parts a 128 x 256 tile would be split into (32 more registers; the code for it
+// costs 0.3-0.9 us of a launch, about 0.2 us of one that has no parts).
+template <int BLOCKS, int ACROSS, bool CUTS = false>
 struct TpTile {
     static constexpr int kBlocks = BLOCKS, kAcross = ACROSS, kWaves = 2 * ACROSS;
     static constexpr int kM = 64 * BLOCKS, kN = 64 * ACROSS;
@@ -64,11 +66,14 @@ struct TpTile {
     static constexpr int kBufBytes = kSlabBytes + kN * 64;  // ... and its tile of nibbles
     static constexpr int kXRequests = kM / 4 / kWaves;      // 1 KiB requests of x per wave
     static constexpr bool kBig = BLOCKS == 2 && ACROSS == 4;
+    static constexpr bool kCuts = CUTS;
     static_assert(kXRequests == 2 || kXRequests == 4, "what request_group spells out");
 };
 using TpBig = TpTile<2, 4>;
-using TpHalf = TpTile<1, 4>;
-using TpSmall = TpTile<1, 2>;
+template <bool CUTS>
+using TpHalf = TpTile<1, 4, CUTS>;
+template <bool CUTS>
+using TpSmall = TpTile<1, 2, CUTS>;
 constexpr int kTpTileM = TpBig::kM;  // 128 rows of x per workgroup
 constexpr int kTpTileN = TpBig::kN;  // 256 weight rows per workgroup
 constexpr int kTpBufs = 3;                // groups in LDS: one in use, two on their way
@@ -199,12 +204,12 @@ __global__ __launch_bounds__(64 * T::kWaves) void qgemm_q4g128_tallp_kernel(
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int r = lane & 31;
     const int h = lane >> 5;
-    // workgroup -> tile (columns fastest) and, past the whole tiles, part of a tile: groups
-    // [g_begin, groups) of K, both multiples of BL
+    // workgroup -> tile (columns fastest) and, for 128 x 256 tiles past the whole ones, part of a
+    // tile: groups [g_begin, groups) of K, both multiples of BL
     static_assert(!ODD || W == 1, "an odd number of groups is taken pair by pair");
     int tile = blockIdx.x, part = -1;
     int g_begin = 0, groups = k >> 7;
-    if (tile >= full_tiles) {
+    if (T::kBig && tile >= full_tiles) {
         const int p = tile - full_tiles;
         tile = full_tiles + p / split;
         part = p;
@@ -228,6 +233,16 @@ __global__ __launch_bounds__(64 * T::kWaves) void qgemm_q4g128_tallp_kernel(
     };
     const int wr = (wave / WN) * 32 * MI;  // this wave's part of the tile
     const int wc = (wave % WN) * 64;
+    // A smaller tile takes all of K, and adds up what it has at the places where the 128 x 256 tile
+    // it lies in would be split over K (full_tiles and split are the plan for those): a product's
+    // bits do not depend on the tile a launch takes (in front of a 3-bit K/V row a last bit flips
+    // whole codes).  next_cut: the first group behind the part.
+    int cuts = 1, next_cut = 0;
+    if constexpr (T::kCuts) {
+        constexpr int kBigOutputs = tp_is_swiglu(OUT) ? kTpTileN / 2 : kTpTileN;
+        const int big = (row0 / kTpTileM) * ((n + kBigOutputs - 1) / kBigOutputs) + col0 / kBigOutputs;
+        if (big >= full_tiles) cuts = split;
+    }
     const int groups_row = k >> 7;    // scales and zeros: groups per weight row
     unsigned magic;
     asm volatile("v_mov_b32 %0, 0x43004300" : "=v"(magic));
@@ -387,6 +402,31 @@ __global__ __launch_bounds__(64 * T::kWaves) void qgemm_q4g128_tallp_kernel(
         for (int j = 0; j < 2; ++j)
 #pragma unroll
             for (int e = 0; e < 16; ++e) yacc[i][j][e] = 0.0f;
+    float16_t parts_sum[MI][2];  // smaller tiles: the parts before this one
+    const int part_blocks = (groups + BL - 1) / BL;
+    int cut = 0;
+    auto next_part = [&]() {
+#pragma unroll
+        for (int i = 0; i < MI; ++i)
+#pragma unroll
+            for (int j = 0; j < 2; ++j)
+#pragma unroll
+                for (int e = 0; e < 16; ++e) {
+                    parts_sum[i][j][e] += yacc[i][j][e];
+                    yacc[i][j][e] = 0.0f;
+                }
+        ++cut;
+        next_cut = BL * (part_blocks * (cut + 1) / cuts);
+    };
+    if constexpr (T::kCuts) {
+#pragma unroll
+        for (int i = 0; i < MI; ++i)
+#pragma unroll
+            for (int j = 0; j < 2; ++j)
+#pragma unroll
+                for (int e = 0; e < 16; ++e) parts_sum[i][j][e] = 0.0f;
+        next_cut = BL * (part_blocks / cuts);
+    }
 
     gload_small(g_begin, cur);
     request_group(g_begin, 0);
@@ -579,21 +619,38 @@ __global__ __launch_bounds__(64 * T::kWaves) void qgemm_q4g128_tallp_kernel(
     if constexpr (ODD) {
         int g0 = g_begin;
         for (; g0 + 1 < groups; g0 += 2) {
+            if constexpr (T::kCuts)
+                if (g0 == next_cut) next_part();
             group(ic<0>{}, g0, buf_off);
             next_buf();
             group(ic<1>{}, g0 + 1, buf_off);
             next_buf();
         }
         if (g0 < groups) {
+            if constexpr (T::kCuts)
+                if (g0 == next_cut) next_part();
             group(ic<0>{}, g0, buf_off);
             zero_term(ic<0>{}, true);
         }
     } else {
-        for (int g0 = g_begin; g0 < groups; g0 += BL)
+        for (int g0 = g_begin; g0 < groups; g0 += BL) {
+            if constexpr (T::kCuts)
+                if (g0 == next_cut) next_part();
             static_for<BL>([&](auto uc) {
                 group(uc, g0 + decltype(uc)::value, buf_off);
                 next_buf();
             });
+        }
+    }
+    if constexpr (T::kCuts) {
+        if (cuts > 1) {
+#pragma unroll
+            for (int i = 0; i < MI; ++i)
+#pragma unroll
+                for (int j = 0; j < 2; ++j)
+#pragma unroll
+                    for (int e = 0; e < 16; ++e) yacc[i][j][e] = parts_sum[i][j][e] + yacc[i][j][e];
+        }
     }
 
     if (OUT == kTpOutF32 && T::kBig && part >= 0 && out_pairs != 0) {
@@ -801,13 +858,13 @@ bool qgemm_q4_tallp_applies(int m, int n, int k) {
 // not arithmetic), so with few groups of K and few tiles the smaller ones win by filling the chip.
 // us, 128 x 256 / 64 x 128 (the first with the sum of its K parts):
 //   K  768, 1152 columns:  100 rows 19.1 / 11.0, 1030 20.2 / 11.6, 2060 20.7 / 15.5, 4120 22.2 / 24.7
-//   K 1536, 1536 columns:  100 rows 13.0 / 15.5,  520 18.7 / 15.9, 2060 28.9 / 22.7, 4120 31.3 / 40.2
+//   K 1536, 1536 columns:  100 rows 13.0 / 15.5,  520 19.3 / 16.9, 2060 29.5 / 23.7, 4120 31.3 / 40.2
 //   K 4096, 4096 columns:  300 rows 29.8 / 31.4, 1030 58.8 / 63.7
 // hence: at most 16 groups, all tiles resident at once (two per compute unit), and where the big
 // tiles could be split over K at least 20 of them.  A next product's operand is written by
 // 64 x 256 tiles, one per compute unit, whose round takes five eighths of a big one's:
 //   K  768, 4864 outputs:  200 rows 18.9 / 12.7,  520 19.9 / 24.4, 1030 38.2 / 36.2, 2060 56.7 / 69.7
-//   K 1536, 8960 outputs:  100 rows 24.5 / 18.7,  200 28.4 / 37.3, 1030 82.9 / 91.0
+//   K 1536, 8960 outputs:  100 rows 24.9 / 19.2,  200 28.4 / 37.3, 1030 82.9 / 91.0
 template <int OUT>
 static bool tp_less(int m, int n, int k, int block_groups, int cus) {
     const int groups = k >> 7;
@@ -818,13 +875,22 @@ static bool tp_less(int m, int n, int k, int block_groups, int cus) {
     if (OUT == kTpOutSwigluOperand) {
         const int rows = tp_padded_rows(m);
         const int64_t big = (tiles(rows, TpBig::kM, TpBig::kN / 2) + cus - 1) / cus;
-        const int64_t half = (tiles(rows, TpHalf::kM, TpHalf::kN / 2) + cus - 1) / cus;
+        const int64_t half = (tiles(rows, TpHalf<false>::kM, TpHalf<false>::kN / 2) + cus - 1) / cus;
         return 5 * half < 8 * big;
     }
     const int div = tp_is_swiglu(OUT) ? 2 : 1;
-    if (tiles(m, TpSmall::kM, TpSmall::kN / div) > 2 * cus) return false;
+    if (tiles(m, TpSmall<false>::kM, TpSmall<false>::kN / div) > 2 * cus) return false;
     const int big = (int)tiles(m, TpBig::kM, TpBig::kN / div);
     return big >= 20 || tp_plan(big, groups, block_groups, cus).split == 1;
+}
+
+// The plan of a launch's 128 x 256 tiles (which the smaller tiles add up by).
+template <int OUT>
+static TpPlan tp_big_plan(int m, int n, int k, int block_groups, int cus) {
+    constexpr int outputs = tp_is_swiglu(OUT) ? kTpTileN / 2 : kTpTileN;
+    // (an operand's padding rows are written too: whole tiles as well)
+    return tp_plan(((n + outputs - 1) / outputs) * ((m + kTpTileM - 1) / kTpTileM), k >> 7, block_groups,
+                   cus);
 }
 
 template <int OUT, int W, bool ODD, class T>
@@ -844,13 +910,13 @@ static hipError_t tallp_launch_tile(const uint16_t* xp, const float* xs, float* 
     const int tiles = tiles_n * ((rows + T::kM - 1) / T::kM);
     const int cus = device_cu_count();
     if (cus <= 0) return hipErrorInvalidDevice;
-    const TpPlan plan = T::kBig ? tp_plan(tiles, k >> 7, 2 * W, cus) : TpPlan{tiles, 1};
-    const int parts = (tiles - plan.full) * plan.split;
+    const TpPlan plan = tp_big_plan<OUT>(m, n, k, 2 * W, cus);
+    const int parts = T::kBig && plan.split > 1 ? (tiles - plan.full) * plan.split : 0;
     qgemm_q4g128_tallp_kernel<OUT, W, ODD, T>
-        <<<dim3(plan.full + (plan.split > 1 ? parts : 0)), dim3(64 * T::kWaves), lds, st>>>(
+        <<<dim3(parts ? plan.full + parts : tiles), dim3(64 * T::kWaves), lds, st>>>(
             xp, xs, qw, scale, zero, bias, y, partials, m, n, k, tiles_n, plan.full, plan.split,
             out_pairs);
-    if (plan.split > 1 && !(OUT == kTpOutF32 && out_pairs != 0)) {
+    if (parts && !(OUT == kTpOutF32 && out_pairs != 0)) {
         if constexpr (OUT == kTpOutSwigluOperand) {
             q4_tall_reduce_operand_kernel<<<dim3((tiles - plan.full) * 16), dim3(256), 0, st>>>(
                 partials, y, m, n, tiles_n, plan.full, plan.split, out_pairs);
@@ -869,12 +935,18 @@ static hipError_t tallp_launch(const uint16_t* xp, const float* xs, float* parti
                                const uint8_t* qw, const __half* scale, const __half* zero,
                                const float* bias, void* y, int m, int n, int k, hipStream_t st,
                                int out_pairs = 0) {
-    using Less = std::conditional_t<OUT == kTpOutSwigluOperand, TpHalf, TpSmall>;
+    constexpr bool operand = OUT == kTpOutSwigluOperand;
+    using Less = std::conditional_t<operand, TpHalf<false>, TpSmall<false>>;
+    using LessCuts = std::conditional_t<operand, TpHalf<true>, TpSmall<true>>;
     const int cus = device_cu_count();
     if (cus <= 0) return hipErrorInvalidDevice;
-    if (tp_less<OUT>(m, n, k, 2 * W, cus))
+    if (tp_less<OUT>(m, n, k, 2 * W, cus)) {
+        if (tp_big_plan<OUT>(m, n, k, 2 * W, cus).split > 1)
+            return tallp_launch_tile<OUT, W, ODD, LessCuts>(xp, xs, partials, qw, scale, zero, bias, y,
+                                                            m, n, k, st, out_pairs);
         return tallp_launch_tile<OUT, W, ODD, Less>(xp, xs, partials, qw, scale, zero, bias, y, m, n,
                                                     k, st, out_pairs);
+    }
     return tallp_launch_tile<OUT, W, ODD, TpBig>(xp, xs, partials, qw, scale, zero, bias, y, m, n, k,
                                                  st, out_pairs);
 }

@@ -124,3 +124,90 @@ def test_parts_are_added_to_the_residual_as_one_sum(num_layers, hidden, hq, hkv,
     kernels.launch_qgemm_q4g128_tall(act, *dev["down"], y, ws, t, hidden, inter, f32_out=True)
     hip.synchronize()
     assert np.array_equal(got, batch["h"] + y.to_numpy(np.float32, (t, hidden)))
+
+
+def _problem(m, n, k):
+    torch = pytest.importorskip("torch")
+    gen = torch.Generator(device="cuda").manual_seed(m + n + k)
+    x = torch.randn(m, k, device="cuda", generator=gen).bfloat16()
+    qw = torch.randint(0, 256, (n, k // 2), device="cuda", generator=gen, dtype=torch.uint8)
+    scale = (0.01 + 0.01 * torch.rand(n, k // 128, device="cuda", generator=gen)).half()
+    zero = (7.5 + 0.4 * torch.randn(n, k // 128, device="cuda", generator=gen)).half()
+    return torch, x, qw, scale, zero
+
+
+def _p(t):
+    import ctypes as C
+    return C.c_void_p(t.data_ptr())
+
+
+def _product(torch, x, qw, scale, zero, g0, g1):
+    """fp32 x @ w.T over the groups [g0, g1) of K, as a product of its own."""
+    x, qw = x[:, g0 * 128:g1 * 128].contiguous(), qw[:, g0 * 64:g1 * 64].contiguous()
+    scale, zero = scale[:, g0:g1].contiguous(), zero[:, g0:g1].contiguous()
+    m, n, k = x.shape[0], qw.shape[0], x.shape[1]
+    y = torch.empty(m, n, device="cuda")
+    ws = torch.empty(kernels.qgemm_q4g128_tall_workspace_bytes(m, k), device="cuda", dtype=torch.uint8)
+    kernels.launch_qgemm_q4g128_tall(_p(x), _p(qw), _p(scale), _p(zero), _p(y), _p(ws), m, n, k,
+                                     f32_out=True)
+    torch.cuda.synchronize()
+    return y
+
+
+def _parts(torch, k, tiles):
+    """How a launch of `tiles` 128 x 256 tiles is split over K: whole tiles, bounds of the parts."""
+    cus, groups = torch.cuda.get_device_properties(0).multi_processor_count, k // 128
+    block = 8 if k % 1024 == 0 else (4 if k % 512 == 0 else 2)
+    rest = tiles % cus
+    split = min(cus // rest, groups // max(block, 4)) if rest else 1
+    full = tiles - rest if split > 1 else tiles
+    return full, [block * (groups // block * q // max(split, 1)) for q in range(max(split, 1) + 1)]
+
+
+@pytest.mark.parametrize("m,n,k", [(520, 1536, 1536), (513, 1501, 1536), (300, 2048, 2048),
+                                   (260, 2000, 1792)])
+def test_smaller_tiles_add_up_the_parts_of_the_large(m, n, k):
+    # products on 64 x 128 tiles whose 128 x 256 tiles would be split over K: bit for bit the sum,
+    # from zero and in order, of the parts as products of their own
+    torch, *args = _problem(m, n, k)
+    full, bounds = _parts(torch, k, -(-m // 128) * -(-n // 256))
+    assert full == 0 and len(bounds) > 2
+    want = torch.zeros(m, n, device="cuda")
+    for g0, g1 in zip(bounds, bounds[1:]):
+        assert g1 - g0 < 8 or k % 1024 == 0  # a part is not split again
+        want += _product(torch, *args, g0, g1)
+    assert torch.equal(_product(torch, *args, 0, k // 128), want)
+
+
+@pytest.mark.parametrize("m,inter,k", [
+    (100, 8960, 1536),   # every tile split
+    (1030, 4352, 1536),  # 306 tiles: the last 50 split
+])
+def test_smaller_tiles_of_the_activation_add_up_the_parts(m, inter, k):
+    # the same for the gate/up projection that writes the next operand, on 64 x 256 tiles
+    torch, x, qw, scale, zero = _problem(m, 2 * inter, k)
+    tiles_n = inter // 128
+    full, bounds = _parts(torch, k, -(-m // 128) * tiles_n)
+    assert len(bounds) > 2
+    parts = sum(_product(torch, x, qw, scale, zero, a, b) for a, b in zip(bounds, bounds[1:]))
+    if full:
+        # the whole tiles' sums: from launches of half the columns, which are not split
+        whole = torch.empty_like(parts)
+        for c in (slice(0, inter), slice(inter, 2 * inter)):
+            f, b = _parts(torch, k, -(-m // 128) * -(-inter // 256))
+            assert len(b) == 2
+            whole[:, c] = _product(torch, x, qw[c], scale[c], zero[c], 0, k // 128)
+        r, c = torch.arange(m, device="cuda") // 128, torch.arange(2 * inter, device="cuda") % inter // 128
+        parts = torch.where(r[:, None] * tiles_n + c[None, :] < full, whole, parts)
+    nxt = kernels.qgemm_q4g128_tall_workspace_bytes(m, inter)
+    got, want = (torch.zeros(nxt, device="cuda", dtype=torch.uint8) for _ in range(2))
+    kernels.launch_silu_mul_f32p_tall(_p(parts), 1, _p(want), m, inter, 1)
+    ws = torch.empty(kernels.qgemm_q4g128_tall_workspace_bytes(m, k), device="cuda", dtype=torch.uint8)
+    # (a product of 128 columns, for the operand it leaves in the workspace)
+    y = torch.empty(m, 128, device="cuda")
+    kernels.launch_qgemm_q4g128_tall(_p(x), _p(qw), _p(scale), _p(zero), _p(y), _p(ws), m, 128, k,
+                                     f32_out=True)
+    kernels.launch_qgemm_q4g128_tall_swiglu_operand(_p(qw), _p(scale), _p(zero), _p(got), 1, _p(ws), m,
+                                                    inter, k)
+    torch.cuda.synchronize()
+    assert torch.equal(got, want)
