@@ -233,16 +233,6 @@ __global__ __launch_bounds__(64 * T::kWaves) void qgemm_q4g128_tallp_kernel(
     };
     const int wr = (wave / WN) * 32 * MI;  // this wave's part of the tile
     const int wc = (wave % WN) * 64;
-    // A smaller tile takes all of K, and adds up what it has at the places where the 128 x 256 tile
-    // it lies in would be split over K (full_tiles and split are the plan for those): a product's
-    // bits do not depend on the tile a launch takes (in front of a 3-bit K/V row a last bit flips
-    // whole codes).  next_cut: the first group behind the part.
-    int cuts = 1, next_cut = 0;
-    if constexpr (T::kCuts) {
-        constexpr int kBigOutputs = tp_is_swiglu(OUT) ? kTpTileN / 2 : kTpTileN;
-        const int big = (row0 / kTpTileM) * ((n + kBigOutputs - 1) / kBigOutputs) + col0 / kBigOutputs;
-        if (big >= full_tiles) cuts = split;
-    }
     const int groups_row = k >> 7;    // scales and zeros: groups per weight row
     unsigned magic;
     asm volatile("v_mov_b32 %0, 0x43004300" : "=v"(magic));
@@ -402,9 +392,12 @@ __global__ __launch_bounds__(64 * T::kWaves) void qgemm_q4g128_tallp_kernel(
         for (int j = 0; j < 2; ++j)
 #pragma unroll
             for (int e = 0; e < 16; ++e) yacc[i][j][e] = 0.0f;
-    float16_t parts_sum[MI][2];  // smaller tiles: the parts before this one
+    // (kCuts) A smaller tile takes all of K, and adds up what it has at the places where the 128 x 256
+    // tile it lies in would be split over K (`split` parts): a product's bits do not depend on the tile
+    // a launch takes (in front of a 3-bit K/V row a last bit flips whole codes).
+    float16_t parts_sum[MI][2];  // the parts before this one
     const int part_blocks = (groups + BL - 1) / BL;
-    int cut = 0;
+    int cut = 0, next_cut = 0;   // next_cut: the first group behind this part
     auto next_part = [&]() {
 #pragma unroll
         for (int i = 0; i < MI; ++i)
@@ -416,7 +409,7 @@ __global__ __launch_bounds__(64 * T::kWaves) void qgemm_q4g128_tallp_kernel(
                     yacc[i][j][e] = 0.0f;
                 }
         ++cut;
-        next_cut = BL * (part_blocks * (cut + 1) / cuts);
+        next_cut = BL * (part_blocks * (cut + 1) / split);
     };
     if constexpr (T::kCuts) {
 #pragma unroll
@@ -425,7 +418,7 @@ __global__ __launch_bounds__(64 * T::kWaves) void qgemm_q4g128_tallp_kernel(
             for (int j = 0; j < 2; ++j)
 #pragma unroll
                 for (int e = 0; e < 16; ++e) parts_sum[i][j][e] = 0.0f;
-        next_cut = BL * (part_blocks / cuts);
+        next_cut = BL * (part_blocks / split);
     }
 
     gload_small(g_begin, cur);
@@ -643,14 +636,12 @@ __global__ __launch_bounds__(64 * T::kWaves) void qgemm_q4g128_tallp_kernel(
         }
     }
     if constexpr (T::kCuts) {
-        if (cuts > 1) {
 #pragma unroll
-            for (int i = 0; i < MI; ++i)
+        for (int i = 0; i < MI; ++i)
 #pragma unroll
-                for (int j = 0; j < 2; ++j)
+            for (int j = 0; j < 2; ++j)
 #pragma unroll
-                    for (int e = 0; e < 16; ++e) yacc[i][j][e] = parts_sum[i][j][e] + yacc[i][j][e];
-        }
+                for (int e = 0; e < 16; ++e) yacc[i][j][e] = parts_sum[i][j][e] + yacc[i][j][e];
     }
 
     if (OUT == kTpOutF32 && T::kBig && part >= 0 && out_pairs != 0) {
@@ -853,6 +844,15 @@ bool qgemm_q4_tallp_applies(int m, int n, int k) {
     return m > 0 && n > 0 && k > 0 && k % 128 == 0 && tp_sizes_ok(m, n, k);
 }
 
+// The plan of a launch's 128 x 256 tiles (which the smaller tiles add up by).
+template <int OUT>
+static TpPlan tp_big_plan(int m, int n, int k, int block_groups, int cus) {
+    constexpr int outputs = tp_is_swiglu(OUT) ? kTpTileN / 2 : kTpTileN;
+    // (an operand's padding rows are written too: whole tiles as well)
+    return tp_plan(((n + outputs - 1) / outputs) * ((m + kTpTileM - 1) / kTpTileM), k >> 7, block_groups,
+                   cus);
+}
+
 // Whether a launch takes the smaller tiles.  A 128 x 256 tile costs about 7 us + 2 us per group
 // whatever else runs, a 64 x 128 one 4 us + 1 us (a chain of requests, barriers and operand reads,
 // not arithmetic), so with few groups of K and few tiles the smaller ones win by filling the chip.
@@ -862,9 +862,13 @@ bool qgemm_q4_tallp_applies(int m, int n, int k) {
 //   K 4096, 4096 columns:  300 rows 29.8 / 31.4, 1030 58.8 / 63.7
 // hence: at most 16 groups, all tiles resident at once (two per compute unit), and where the big
 // tiles could be split over K at least 20 of them.  A next product's operand is written by
-// 64 x 256 tiles, one per compute unit, whose round takes five eighths of a big one's:
+// 64 x 256 tiles, one per compute unit, whose round takes five eighths of a big one's (a last round
+// that is split over K about six of them):
 //   K  768, 4864 outputs:  200 rows 18.9 / 12.7,  520 19.9 / 24.4, 1030 38.2 / 36.2, 2060 56.7 / 69.7
-//   K 1536, 8960 outputs:  100 rows 24.9 / 19.2,  200 28.4 / 37.3, 1030 82.9 / 91.0
+//   K 1536, 8960 outputs:  100 rows 24.9 / 19.2,  200 28.4 / 37.3,  500 50.2 / 58.6, 1030 82.9 / 91.0
+//   K 2048, 6144 outputs:  700 rows 59.3 / 66.3 (288 tiles: one round and 32 split ones)
+// Whole large tiles in front of split ones keep the large tiles (none of the above is lost by it), so
+// that a launch on the smaller ones adds up all of its tiles alike.
 template <int OUT>
 static bool tp_less(int m, int n, int k, int block_groups, int cus) {
     const int groups = k >> 7;
@@ -872,25 +876,17 @@ static bool tp_less(int m, int n, int k, int block_groups, int cus) {
     auto tiles = [&](int rows, int tm, int tn) {
         return (int64_t)((rows + tm - 1) / tm) * ((n + tn - 1) / tn);
     };
+    const TpPlan plan = tp_big_plan<OUT>(m, n, k, block_groups, cus);
+    if (plan.split > 1 && plan.full > 0) return false;
     if (OUT == kTpOutSwigluOperand) {
         const int rows = tp_padded_rows(m);
-        const int64_t big = (tiles(rows, TpBig::kM, TpBig::kN / 2) + cus - 1) / cus;
+        const int64_t big = plan.split > 1 ? 6 : 8 * ((plan.full + cus - 1) / cus);
         const int64_t half = (tiles(rows, TpHalf<false>::kM, TpHalf<false>::kN / 2) + cus - 1) / cus;
-        return 5 * half < 8 * big;
+        return 5 * half < big;
     }
     const int div = tp_is_swiglu(OUT) ? 2 : 1;
     if (tiles(m, TpSmall<false>::kM, TpSmall<false>::kN / div) > 2 * cus) return false;
-    const int big = (int)tiles(m, TpBig::kM, TpBig::kN / div);
-    return big >= 20 || tp_plan(big, groups, block_groups, cus).split == 1;
-}
-
-// The plan of a launch's 128 x 256 tiles (which the smaller tiles add up by).
-template <int OUT>
-static TpPlan tp_big_plan(int m, int n, int k, int block_groups, int cus) {
-    constexpr int outputs = tp_is_swiglu(OUT) ? kTpTileN / 2 : kTpTileN;
-    // (an operand's padding rows are written too: whole tiles as well)
-    return tp_plan(((n + outputs - 1) / outputs) * ((m + kTpTileM - 1) / kTpTileM), k >> 7, block_groups,
-                   cus);
+    return tiles(m, TpBig::kM, TpBig::kN / div) >= 20 || plan.split == 1;
 }
 
 template <int OUT, int W, bool ODD, class T>

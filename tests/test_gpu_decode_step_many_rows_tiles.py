@@ -181,10 +181,12 @@ def test_smaller_tiles_add_up_the_parts_of_the_large(m, n, k):
 
 @pytest.mark.parametrize("m,inter,k", [
     (100, 8960, 1536),   # every tile split
-    (1030, 4352, 1536),  # 306 tiles: the last 50 split
+    (300, 4352, 1536),   # three row tiles, the last one half empty
+    (1030, 4352, 1536),  # 306 tiles, the last 50 split: a launch that stays on 128 x 256
 ])
 def test_smaller_tiles_of_the_activation_add_up_the_parts(m, inter, k):
-    # the same for the gate/up projection that writes the next operand, on 64 x 256 tiles
+    # the same for the gate/up projection that writes the next operand, on 64 x 256 tiles and on
+    # the large ones
     torch, x, qw, scale, zero = _problem(m, 2 * inter, k)
     tiles_n = inter // 128
     full, bounds = _parts(torch, k, -(-m // 128) * tiles_n)
