@@ -186,6 +186,24 @@ bool config_ok(const logismos_decode_config_t* c, int num_seqs, int t, int max_s
     return true;
 }
 
+// The operands that every step on the 32-row or the few-row projections reads: all there, and the
+// nibbles of every projection on 16 bytes (their loads).  Looked at for all layers before the first
+// launch: the fused kernels check no pointer themselves, and no step is launched in part.
+bool operands_ok(const logismos_decode_config_t& c, const logismos_decode_layer_t* layers,
+                 const logismos_decode_batch_t& b) {
+    if (!b.hidden_f32 || !b.final_norm_w_f32 || !b.block_tables || !b.cu_seqlens ||
+        !b.context_lens || !b.positions || !b.slot_mapping || !b.rope_cos_f32 || !b.rope_sin_f32)
+        return false;
+    for (int l = 0; l < c.num_layers; ++l) {
+        const logismos_decode_layer_t& L = layers[l];
+        if (!L.norm1_w_f32 || !L.norm2_w_f32 || !L.k_pool_f16 || !L.v_pool_f16) return false;
+        for (const logismos_q4_weight_t* W : {&L.qkv, &L.o, &L.gate_up, &L.down})
+            if (!W->qw || !W->scale || !W->zero || (reinterpret_cast<uintptr_t>(W->qw) & 15u))
+                return false;
+    }
+    return true;
+}
+
 // Whether every projection of the step can run on the fused few-row kernels.
 bool few_rows(const logismos_decode_config_t& c, const logismos_decode_layer_t* layers, int t) {
     const int qd = c.num_q_heads * c.head_dim;
@@ -331,6 +349,7 @@ extern "C" logismos_status_t logismos_launch_decode_step(const logismos_decode_c
     // row of a step of up to 32, or (tokens_for_last_rows) the last row of every sequence
     if (tokens_out && !last_only && t > kChunkRows) return hipErrorInvalidValue;
     const Workspace w = carve(c, num_seqs, t, batch->num_splits, static_cast<char*>(workspace));
+    if (!w.tall && !operands_ok(c, layers, *batch)) return hipErrorInvalidValue;
     const int qd = c.num_q_heads * c.head_dim;
     const int kvd = c.num_kv_heads * c.head_dim;
     const int width = qd + 2 * kvd;
