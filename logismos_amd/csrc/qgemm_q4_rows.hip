@@ -287,15 +287,6 @@ __host__ __device__ __forceinline__ int rows_waves_per_row(int nw, int b) {
     return nw / (b > 8 ? 16 : (b > 4 ? 8 : (b > 2 ? 4 : b)));
 }
 
-// 1 / sqrt(x): the hardware's estimate and one Newton step (half an ulp more than the division
-// of a square root, for a tenth of its instructions; every wave of every workgroup takes it).
-__device__ __forceinline__ float rows_rsqrt(float x) {
-    const float y = __builtin_amdgcn_rsqf(x);
-    // (0 and infinity, of sums of squares that overflow or vanish, are exact: the step would
-    // make them 0 * inf)
-    return __builtin_amdgcn_classf(y, 0x264) ? y : fmaf(0.5f * y, fmaf(-x * y, y, 1.0f), y);
-}
-
 // The sums of W waves' partial products (16 x 16 floats in the MFMA layout, 1 KiB apart by
 // `step`) of batch row r and weight row n.
 template <int W>
@@ -335,7 +326,7 @@ template <int EPI, int NW, int W, int GPW, int TN, int CR>
 __global__ __launch_bounds__(64 * NW) void qgemm_q4g128_rows_norm_kernel(
     const float* __restrict__ h, const float* __restrict__ gain, const uint8_t* __restrict__ qw,
     const __half* __restrict__ scale, const __half* __restrict__ zero, int b, int k, int tiles,
-    float eps, float inv_k, int lds_ssq, int lds_x, int lds_stage, const RowsEpilogueArgs e) {
+    float eps, int lds_ssq, int lds_x, int lds_stage, const RowsEpilogueArgs e) {
     using Stage = RowsStage<GPW>;
     constexpr int TEAMS = NW / W;
     constexpr int TILES = TN * TEAMS;
@@ -411,7 +402,7 @@ __global__ __launch_bounds__(64 * NW) void qgemm_q4g128_rows_norm_kernel(
         if (4 * (i * THREADS + tid) < k) gains[i * THREADS + tid] = gv[i];
     __syncthreads();
     const float total = row16_sum((lane & 15) < wpr ? ssq[row * 16 + (lane & 15)] : 0.0f);
-    const float inv = rows_rsqrt(total * inv_k + eps);
+    const float inv = 1.0f / sqrtf(total / (float)k + eps);
 #pragma unroll
     for (int i = 0; i < CR; ++i) {
         const int c = (i * wpr + part) * 64 + lane;
@@ -548,7 +539,7 @@ hipError_t rows_norm_launch(const RowsArgs& a, hipStream_t st) {
     constexpr int tiles = TN * NW / W;
     const RowsNormLds l(tiles, NW * RowsStage<GPW>::BYTES, TN * NW * 1024, a.b, a.k);
     kernel<<<dim3((unsigned)((a.tiles + tiles - 1) / tiles)), dim3(64 * NW), (size_t)l.bytes, st>>>(
-        a.h, a.gain, a.qw, a.scale, a.zero, a.b, a.k, a.tiles, a.eps, 1.0f / (float)a.k, l.ssq, l.x, l.stage, a.e);
+        a.h, a.gain, a.qw, a.scale, a.zero, a.b, a.k, a.tiles, a.eps, l.ssq, l.x, l.stage, a.e);
     return hipGetLastError();
 }
 
