@@ -72,7 +72,7 @@ template <int NP>
 __global__ __launch_bounds__(256) void rms_norm_fp16_wave_kernel(const uint4_t* __restrict__ x,
                                                                  const uint4_t* __restrict__ w,
                                                                  uint4_t* __restrict__ y, int m,
-                                                                 int pieces, float inv_n, float eps) {
+                                                                 int pieces, float eps) {
     const int row = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
     if (row >= m) return;
     uint4_t xv[NP], wv[NP];
@@ -84,14 +84,22 @@ __global__ __launch_bounds__(256) void rms_norm_fp16_wave_kernel(const uint4_t* 
             wv[p] = w[p * 64 + lane];
         }
     }
-    float part = 0.0f;
+    // squares in pairs, pieces in pairs: no longer chains than a workgroup's 256 partial sums have
+    float part[NP];
 #pragma unroll
     for (int p = 0; p < NP; ++p) {
         const half8_t v = __builtin_bit_cast(half8_t, xv[p]);
+        float pair[4];
 #pragma unroll
-        for (int e = 0; e < 8; ++e) part = fmaf((float)v[e], (float)v[e], part);
+        for (int e = 0; e < 4; ++e)
+            pair[e] = fmaf((float)v[2 * e + 1], (float)v[2 * e + 1], (float)v[2 * e] * (float)v[2 * e]);
+        part[p] = (pair[0] + pair[1]) + (pair[2] + pair[3]);
     }
-    const float inv_rms = 1.0f / sqrtf(wave_sum(part) * inv_n + eps);
+#pragma unroll
+    for (int d = 1; d < NP; d *= 2)
+#pragma unroll
+        for (int p = 0; p < NP; p += 2 * d) part[p] += part[p + d];
+    const float inv_rms = 1.0f / sqrtf(wave_sum(part[0]) / (float)(8 * pieces) + eps);
 #pragma unroll
     for (int p = 0; p < NP; ++p) {
         if (p * 64 + lane >= pieces) continue;
@@ -582,7 +590,7 @@ extern "C" logismos_status_t logismos_launch_rms_norm_fp16(const void* x_fp16, c
                                         : lg::rms_norm_fp16_wave_kernel<8>;
         kernel<<<dim3((m + 3) / 4), dim3(256), 0, static_cast<hipStream_t>(stream)>>>(
             static_cast<const lg::uint4_t*>(x_fp16), static_cast<const lg::uint4_t*>(w_fp16),
-            static_cast<lg::uint4_t*>(y_fp16), m, n / 8, 1.0f / (float)n, eps);
+            static_cast<lg::uint4_t*>(y_fp16), m, n / 8, eps);
         return hipGetLastError();
     }
     lg::rms_norm_fp16_kernel<<<dim3(m), dim3(lg::kRowThreads), 0,

@@ -5,6 +5,7 @@ import numpy as np
 import pytest
 
 import oracle as O
+from logismos_amd import hip, kernels
 from tests.test_gpu_reference_ops import _dev, _f16, _matmul, _parity
 
 pytestmark = pytest.mark.gpu
@@ -21,7 +22,6 @@ def test_matmul_of_whole_pieces(m, n, k):
 
 def test_matmul_leaves_out_what_lies_behind_k():
     # the piece behind a row's last column belongs to the next row: infinities there do not count
-    from logismos_amd import hip, kernels
     m, n, k = 3, 8, 72
     rng = np.random.default_rng(6)
     a, b = _f16(rng, m, k), _f16(rng, k, n)
@@ -36,7 +36,6 @@ def test_matmul_leaves_out_what_lies_behind_k():
 
 @pytest.mark.parametrize("m,n", [(1, 8), (5, 1024), (6, 1032), (3, 2048), (7, 2056), (4, 4096), (2, 4104)])
 def test_rms_norm_of_whole_pieces(m, n):
-    from logismos_amd import hip, kernels
     rng = np.random.default_rng(n)
     x, w = _f16(rng, m, n), _f16(rng, n)
     y = hip.DeviceBuffer(m * n * 2)
@@ -48,7 +47,6 @@ def test_rms_norm_of_whole_pieces(m, n):
 
 @pytest.mark.parametrize("batch,seq,heads,d", [(1, 1, 1, 8), (2, 3, 5, 24), (3, 33, 12, 64), (1, 7, 33, 72)])
 def test_rope_of_whole_pieces(batch, seq, heads, d):
-    from logismos_amd import hip, kernels
     rng = np.random.default_rng(seq)
     qk = _f16(rng, batch, seq, heads, d)
     table = O.build_cos_sin_table(seq, d, 10_000.0)
@@ -56,3 +54,26 @@ def test_rope_of_whole_pieces(batch, seq, heads, d):
     kernels.launch_rope_fp16_in_place(dev, _dev(table), batch, seq, heads, d)
     hip.synchronize()
     _parity(dev.to_numpy(np.float16, (qk.size,)), O.rope_apply_fp16_ref(qk, table, batch, seq, heads, d))
+
+
+@pytest.mark.parametrize("n", [328, 656, 1000, 1536, 2504, 4040])
+def test_rms_norm_to_the_last_bit(n):
+    # 1 / sqrt(mean + eps) with every operation rounded once, over whole numbers whose sum of
+    # squares is exact in any order.  The inputs tell it from a mean that is a product with 1 / n.
+    rng = np.random.default_rng(n)
+    m, eps, one = 400, np.float32(1e-5), np.float32(1)
+    x = rng.integers(-9, 10, size=(m, n)).astype(np.float32)
+    w = rng.normal(1, 0.1, n).astype(np.float16)
+    total = (x.astype(np.float64) ** 2).sum(1, keepdims=True).astype(np.float32)
+    mean = total / np.float32(n)
+
+    def norm(mean):
+        return (x * (one / np.sqrt(mean + eps)) * w.astype(np.float32)).astype(np.float16)
+
+    want = norm(mean)
+    assert (want != norm(total * (one / np.float32(n)))).any()
+    up = hip.DeviceBuffer.from_numpy
+    d_y = hip.DeviceBuffer(m * n * 2)
+    kernels.launch_rms_norm_fp16(up(x.astype(np.float16)), up(w), d_y, m, n, float(eps))
+    hip.synchronize()
+    assert np.array_equal(d_y.to_numpy(np.float16, (m, n)), want)
