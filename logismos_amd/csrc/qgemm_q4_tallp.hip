@@ -28,7 +28,8 @@
 //   want ([row tile][block of pairs][group's place in its pair][row][pair]);
 // * the zero-point term -scale * (128 + zero) * sum_x is a rank-(K/128) product of its own:
 //   one v_mfma_f32_32x32x2_f32 per output tile and PAIR of groups, accumulating into the same
-//   registers, in place of a multiply-add per result and group;
+//   registers, in place of a multiply-add per result and group (an odd number of groups: one per
+//   group, into the group's own sum);
 // * what is left per group and wave: the unpack (a lane of the v_mfma_f32_32x32x16_bf16 B
 //   operand is one weight row and one dword of nibbles, made bf16 `128 + q` with an and-or per
 //   pair, exact), one multiply-add per result for the group's scale, 32 MFMAs.
@@ -185,8 +186,9 @@ __device__ __forceinline__ float tp_group_sum(const float (&cs)[4][4]) {
 // W: pairs of groups whose scales, zeros and group sums a lane loads at once (1, 2 or 4: a
 // dword, two or four per load; K a multiple of 256 W).
 // ODD (W = 1): an odd number of groups.  Rows of scales are then only 2-byte aligned and come
-// as halves; the last pair has one group, whose missing partner adds 0 * 0 to the zero-point
-// product.  1030 rows x 896 (seven groups): 9728 gate/up rows with the activation 44.2 us, 52.6
+// as halves; the last pair has one group.  The zero-point term is taken off group by group, halfway
+// through a group's columns: error against 64 bits at 896 columns 5.3e-7, 9.7e-7 with a term per pair
+// as below, 6.5e-7 on the kernel of qgemm_q4_tall.hip.  1030 rows x 896 (seven groups): 9728 gate/up rows with the activation 44.2 us, 52.6
 // + 11.0 on the kernel of qgemm_q4_tall.hip with the activation behind it; 1152 rows of q/k/v
 // 14.1 (24.5), both on the smaller tiles of `tp_less`.
 template <int OUT, int W, bool ODD, class T>
@@ -439,27 +441,40 @@ __global__ __launch_bounds__(64 * T::kWaves) void qgemm_q4g128_tallp_kernel(
     };
 
     // zero-point term of a pair of groups (lanes h = 0 the first, h = 1 the second):
-    // y[m][n] += sum_x[m][g'] * (-scale[n][g'] * (128 + zero[n][g'])).  lone: the second is missing
-    auto zero_term = [&](auto pair_c, bool lone) {
+    // y[m][n] += sum_x[m][g'] * (-scale[n][g'] * (128 + zero[n][g']))
+    auto zero_term = [&](auto pair_c) {
         constexpr int P = decltype(pair_c)::value;
-        float cv[2], sum[MI];
+        float cv[2];
 #pragma unroll
         for (int j = 0; j < 2; ++j) {
             const unsigned sd = cur.s[j][P], zd = cur.z[j][P];
-            const unsigned short sb =
-                (unsigned short)(ODD ? (h ? cur.s_hi[j] : sd) : (h ? (sd >> 16) : sd));
-            const unsigned short zb = (unsigned short)(ODD ? zd : (h ? (zd >> 16) : zd));
+            const unsigned short sb = (unsigned short)(h ? (sd >> 16) : sd);
+            const unsigned short zb = (unsigned short)(h ? (zd >> 16) : zd);
             cv[j] = -__half2float(__builtin_bit_cast(__half, sb)) *
                     (128.0f + __half2float(__builtin_bit_cast(__half, zb)));
-            if (ODD && lone && h) cv[j] = 0.0f;
         }
-#pragma unroll
-        for (int i = 0; i < MI; ++i) sum[i] = ODD && lone && h ? 0.0f : cur.xs[i][P];
 #pragma unroll
         for (int i = 0; i < MI; ++i)
 #pragma unroll
             for (int j = 0; j < 2; ++j)
-                yacc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(sum[i], cv[j], yacc[i][j], 0, 0, 0);
+                yacc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(cur.xs[i][P], cv[j], yacc[i][j], 0, 0, 0);
+    };
+    // ODD: the same term of one group, -sum_x[m][g] * (128 + zero[n][g]) (the lanes of the pair's other
+    // group give 0), added to the group's sum halfway through its columns: the sum then runs from 0 to
+    // half of the large term, to minus half of it and back, is small when it is scaled, and the large
+    // term is never rounded at its full size nor into y.
+    auto zero_halfway = [&](auto par_c, float16_t (&acc)[MI][2]) {
+        const bool own = h == decltype(par_c)::value;
+#pragma unroll
+        for (int i = 0; i < MI; ++i)
+#pragma unroll
+            for (int j = 0; j < 2; ++j) {
+                const unsigned short zb = (unsigned short)cur.z[j][0];
+                acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(
+                    own ? cur.xs[i][0] : 0.0f,
+                    own ? -(128.0f + __half2float(__builtin_bit_cast(__half, zb))) : 0.0f, acc[i][j],
+                    0, 0, 0);
+            }
     };
 
     // One group of 128 columns out of the buffer at byte `buf_off` of the ring; U: the group's
@@ -545,6 +560,10 @@ __global__ __launch_bounds__(64 * T::kWaves) void qgemm_q4g128_tallp_kernel(
                                  : "memory");
             }
             __builtin_amdgcn_sched_barrier(0);
+            if constexpr (ODD && s8 == 4) {
+                zero_halfway(ic<PAR>{}, acc);
+                __builtin_amdgcn_sched_barrier(0);
+            }
             if constexpr (s8 < 7) unpack(ic<(s8 < 7 ? s8 + 1 : 7)>{}, bv[cur_p ^ 1]);
 #pragma unroll
             for (int i = 0; i < MI; ++i)
@@ -590,7 +609,7 @@ __global__ __launch_bounds__(64 * T::kWaves) void qgemm_q4g128_tallp_kernel(
                 for (int e = 0; e < 16; ++e) yacc[i][j][e] = fmaf(sf, acc[i][j][e], yacc[i][j][e]);
         }
         if constexpr (PAR == 1) {
-            zero_term(ic<(U >> 1)>{}, false);
+            if constexpr (!ODD) zero_term(ic<(U >> 1)>{});
             if constexpr (ODD) {
                 small_loads_landed(nxt);
                 cur = nxt;
@@ -623,7 +642,6 @@ __global__ __launch_bounds__(64 * T::kWaves) void qgemm_q4g128_tallp_kernel(
             if constexpr (T::kCuts)
                 if (g0 == next_cut) next_part();
             group(ic<0>{}, g0, buf_off);
-            zero_term(ic<0>{}, true);
         }
     } else {
         for (int g0 = g_begin; g0 < groups; g0 += BL) {
