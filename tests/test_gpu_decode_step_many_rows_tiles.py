@@ -2,10 +2,13 @@
 against the oracle: an odd number of groups of K (one, three, seven, and nine, which are split over
 K), row counts around the tiles of 128 rows, tiles of 64 rows, K parts added up by the operator
 behind a projection."""
+import copy
+
 import numpy as np
 import pytest
 
 import oracle as O
+from oracle import decode_step as OS
 from logismos_amd import hip, kernels
 from tests import workloads
 from tests.gpu_harness import DecodeStepRunner
@@ -256,3 +259,39 @@ def test_error_of_an_odd_number_of_groups(hidden, hq):
         return float(np.linalg.norm(a - want) / np.linalg.norm(want))
 
     assert err(got) <= err(plain), (err(got), err(plain))
+
+
+def _moved(r, array, by):
+    """Address of a device copy of `array`, `by` bytes behind the start of its allocation."""
+    raw = np.ascontiguousarray(array).view(np.uint8).ravel()
+    buf = hip.DeviceBuffer.from_numpy(np.concatenate([np.zeros(by, np.uint8), raw]))
+    r.keep.append(buf)
+    return buf.ptr.value + by
+
+
+@pytest.mark.parametrize("moved", ["gains", "gains and nibbles"])
+@pytest.mark.parametrize("hidden,hq,hkv,d,inter", [
+    (384, 3, 3, 128, 1024),   # the activation goes into the down projection's operand
+    (896, 14, 2, 64, 1152),   # ... into bf16 rows
+])
+def test_operands_off_sixteen_bytes(hidden, hq, hkv, d, inter, moved):
+    # an odd number of groups with operands that are only 4-byte aligned: gate/up products as fp32
+    # and the activation behind them, and (nibbles) the projections that stage x themselves
+    rng = np.random.default_rng(hidden + inter)
+    cfg, layers, batch = workloads.decode_step_problem(
+        rng, num_layers=2, hidden=hidden, hq=hq, hkv=hkv, d=d, inter=inter, ctx=[40, 150, 3],
+        new_tokens=[1, 99, 1], qkv_bias=True)
+    lay, bat = copy.deepcopy(layers), dict(batch, h=batch["h"].copy())
+    want = O.bf16_bits_to_f32(OS.decode_step(cfg, lay, bat))
+    r = DecodeStepRunner(cfg, layers, batch)
+    for dev, L in zip(r.layers, layers):
+        dev.norm1_w_f32, dev.norm2_w_f32 = _moved(r, L["norm1"], 4), _moved(r, L["norm2"], 4)
+        if moved != "gains":
+            for name, k in (("qkv", hidden), ("o", hq * d), ("gate_up", hidden), ("down", inter)):
+                if k // 128 % 2:
+                    getattr(dev, name).qw = _moved(r, L[name][0], 4)
+    r.launch()
+    got = O.bf16_bits_to_f32(r.result_bits())
+    # two layers over many rows: the bound of the steps whose operands are aligned
+    assert _rel_l2(got, want) < 6e-3
+    assert _rel_l2(r.h.to_numpy(np.float32, bat["h"].shape), bat["h"]) < 6e-3
