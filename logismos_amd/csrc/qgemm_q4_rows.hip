@@ -557,14 +557,17 @@ hipError_t rows_norm_by_n(const RowsArgs& a, hipStream_t st) {
     return hipErrorInvalidValue;
 }
 
-// chunks of 8 columns a lane holds: waves_per_row waves share a row
+// chunks of 8 columns a lane holds: waves_per_row waves share a row.  (More than four only with
+// more than 2048 columns, one only where fewer than nine rows share the waves or K is short.)
 template <int EPI, int NW, int W, int GPW>
 hipError_t rows_norm_by_b(const RowsArgs& a, hipStream_t st) {
     const int wpr = rows_waves_per_row(NW, a.b);
     const int cr = ((a.k >> 3) + 64 * wpr - 1) / (64 * wpr);
-    if (cr <= 1) return rows_norm_by_n<EPI, NW, W, GPW, 1>(a, st);
-    if (cr <= 4) return rows_norm_by_n<EPI, NW, W, GPW, 4>(a, st);
-    return rows_norm_by_n<EPI, NW, W, GPW, 8>(a, st);
+    if constexpr (W * GPW > 16)
+        if (cr > 4) return rows_norm_by_n<EPI, NW, W, GPW, 8>(a, st);
+    if constexpr (NW == W || GPW == 1)
+        if (cr <= 1) return rows_norm_by_n<EPI, NW, W, GPW, 1>(a, st);
+    return rows_norm_by_n<EPI, NW, W, GPW, 4>(a, st);
 }
 
 template <int EPI>
