@@ -970,9 +970,14 @@ static hipError_t tallp_launch_w(int w, const uint16_t* xp, const float* xs, flo
                                  const uint8_t* qw, const __half* scale, const __half* zero,
                                  const float* bias, void* y, int m, int n, int k, hipStream_t st,
                                  int out_pairs = 0) {
-    if ((k >> 7) & 1)
-        return tallp_launch<OUT, 1, true>(xp, xs, partials, qw, scale, zero, bias, y, m, n, k, st,
-                                          out_pairs);
+    if ((k >> 7) & 1) {
+        // (bf16 products are the exported entry points', which take pairs of groups)
+        if constexpr (OUT == kTpOutBf16)
+            return hipErrorInvalidValue;
+        else
+            return tallp_launch<OUT, 1, true>(xp, xs, partials, qw, scale, zero, bias, y, m, n, k, st,
+                                              out_pairs);
+    }
     switch (w) {
         case 4:
             return tallp_launch<OUT, 4>(xp, xs, partials, qw, scale, zero, bias, y, m, n, k, st,
