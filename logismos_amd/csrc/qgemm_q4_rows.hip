@@ -5,7 +5,9 @@
 //   activations and the weights of one projection; each launch costs its boundary, one trip to
 //   memory and its drain whatever it computes, so the chain's length is the step's time.  With
 //   fp32 K parts between the operators a layer is ten launches; here it is six (five with one
-//   attention partition):
+//   attention partition; one more for heads of other widths than 128 or a chunk in the batch, whose
+//   attention rows are prepared for the o projection by a launch of their own, and one more over
+//   3-bit pools, where rotation and encoding follow the projection):
 //     rows_norm<QKV>   RMSNorm of the residual rows, q/k/v projection, bias, rotation, q out,
 //                      K/V rows into the pools
 //     attention, merge
@@ -32,19 +34,20 @@
 // What bounds it, from clock stamps: 0.4-0.8 us until the workgroup's waves are there, about
 // 0.5 us of address arithmetic, one trip to memory, then instructions: with four waves per SIMD
 // every instruction of the prologue costs 16 clocks, so it is written for their number (one tile
-// in flight, eight waves up to 8 rows of at most 2048 columns, reciprocals from the host).  More
+// in flight, eight waves up to 8 rows of at most 2048 columns, a tile's head by a reciprocal from
+// the host).  The root, the mean and its reciprocal are divisions and a root all the same, 0.1-0.2
+// us of a launch, as in every other norm.  More
 // tiles in flight are slower (six: 16.8 us instead of 12.9 for the 24576 x 4096 product): a
 // wave whose requests fill the compute unit's queue stands still, and the others wait for its
 // rows at the next barrier.
 //
-// The four projections of a layer with their norms, rotation and activation, us per layer, in a
-// captured chain over weights that exceed the caches, one row / 16 rows (before: the ten
-// launches' own times, traced):
-//   hidden  896, 14 / 2 heads of 64, MLP 4864     14.9 / 17.8   (40 / -)
-//   hidden 1536, 12 / 2 heads of 128, MLP 8960    19.5 / 24.9   (- / 52)
-//   hidden 4096, 32 / 8 heads of 128, MLP 12288   32.4 / 42.7   (62 / -)
-// Whole steps: 24 layers of the first with one sequence 1322 -> 782 us, 28 of the second with
-// 16 sequences 1796 -> 1164, 36 of the third with one 2775 -> 1882.
+// The four projections of a layer with their norms, rotation and activation, us per layer, traced
+// (the ten launches they replace):
+//   hidden  896, 14 / 2 heads of 64, MLP 4864, one row       16.5 (40)
+//   hidden 1536, 12 / 2 heads of 128, MLP 8960, 16 rows      29.8 (52)
+//   hidden 4096, 32 / 8 heads of 128, MLP 12288, one row     36.7 (62)
+// Whole steps: 24 layers of the first 1323 -> 784 us, 28 of the second 1796 -> 1172, 36 of the third
+// 2769 -> 1882.
 #include "device_utils.hpp"
 #include "launch_common.hpp"
 #include "q4_common.hpp"

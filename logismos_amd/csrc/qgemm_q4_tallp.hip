@@ -13,8 +13,9 @@
 //   in the order the nibble unpack produces ("pair order": (x0,x4)(x1,x5)(x2,x6)(x3,x7) per
 //   16-byte chunk), rows padded with zeros to a multiple of 128, and every row's sum over each
 //   group of 128 columns;
-// * the product kernel (128 x 256 tiles, eight waves of 64 x 64, one workgroup per CU) moves
-//   a group's 128 x 128 slab of that copy and its 256 x 128 tile of nibbles from global
+// * the product kernel (128 x 256 tiles, eight waves of 64 x 64, one workgroup per CU; where K is
+//   short also 64 x 256, one per CU, and 64 x 128 of four waves of 32 x 64, two per CU) moves a
+//   group's slab of that copy (128 columns) and its tile of nibbles from global
 //   memory STRAIGHT into LDS (global_load_lds, 16 bytes per lane, no registers, no vector
 //   instructions) into a ring of three buffers, requested two groups ahead, one barrier per
 //   group.  A request writes 1 KiB of consecutive LDS, so instead of padding rows the
@@ -188,9 +189,9 @@ __device__ __forceinline__ float tp_group_sum(const float (&cs)[4][4]) {
 // ODD (W = 1): an odd number of groups.  Rows of scales are then only 2-byte aligned and come
 // as halves; the last pair has one group.  The zero-point term is taken off group by group, halfway
 // through a group's columns: error against 64 bits at 896 columns 5.3e-7, 9.7e-7 with a term per pair
-// as below, 6.5e-7 on the kernel of qgemm_q4_tall.hip.  1030 rows x 896 (seven groups): 9728 gate/up rows with the activation 44.2 us, 52.6
+// as below, 6.5e-7 on the kernel of qgemm_q4_tall.hip.  1030 rows x 896 (seven groups): 9728 gate/up rows with the activation 43.6 us, 52.6
 // + 11.0 on the kernel of qgemm_q4_tall.hip with the activation behind it; 1152 rows of q/k/v
-// 14.1 (24.5), both on the smaller tiles of `tp_less`.
+// 13.3 (24.5), both on the smaller tiles of `tp_less`.
 template <int OUT, int W, bool ODD, class T>
 __global__ __launch_bounds__(64 * T::kWaves) void qgemm_q4g128_tallp_kernel(
     const uint16_t* __restrict__ xp, const float* __restrict__ xs, const uint8_t* __restrict__ qw,
@@ -314,11 +315,12 @@ __global__ __launch_bounds__(64 * T::kWaves) void qgemm_q4g128_tallp_kernel(
     // one weight row; pair p in dword p: group 2 p in the low half), and the group sums of x
     // for the zero-point product (lane (r, h) holds row wr + 32 i + r, group 2 p + h of pair
     // p; the first pass wrote them as [row tile][block][h][row][p], so a wave reads 512
-    // consecutive bytes x W).  Six loads per block and wave, written as assembly with the
-    // wait for them spelled out below, once per block: for loads it can see the compiler
-    // waits with vmcnt(0) wherever a value is used, in every group, which also waits for
-    // every request of the groups ahead and takes the ring's depth away.  A register loaded
-    // here must not be touched before `small_loads_landed` has named it.
+    // consecutive bytes x W).  Per block and wave two loads of scales and two of zeros (ODD: a
+    // third pair, the scales of the second group) and MI of group sums, written as assembly
+    // with the wait for them spelled out below, once per block: for loads it can see the
+    // compiler waits with vmcnt(0) wherever a value is used, in every group, which also waits
+    // for every request of the groups ahead and takes the ring's depth away.  A register
+    // loaded here must not be touched before `small_loads_landed` has named it.
     struct Small {
         TpRegs<unsigned, W> s[2], z[2];
         TpRegs<float, W> xs[2];  // (one of them with one block of rows per wave)
@@ -478,8 +480,9 @@ __global__ __launch_bounds__(64 * T::kWaves) void qgemm_q4g128_tallp_kernel(
     };
 
     // One group of 128 columns out of the buffer at byte `buf_off` of the ring; U: the group's
-    // place in its block.  A wave's requests complete in the order they were issued, so "at
-    // most the six youngest outstanding" names what has landed.
+    // place in its block.  A wave's requests complete in the order they were issued, so "at most
+    // the kReq youngest outstanding" (6; 4 where eight waves share 64 rows of x) names what has
+    // landed.
     auto group = [&](auto u_c, int g, int buf_off) {
         constexpr int U = decltype(u_c)::value;
         constexpr int PAR = U & 1;
