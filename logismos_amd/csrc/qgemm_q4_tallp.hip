@@ -13,14 +13,26 @@
 //   in the order the nibble unpack produces ("pair order": (x0,x4)(x1,x5)(x2,x6)(x3,x7) per
 //   16-byte chunk), rows padded with zeros to a multiple of 128, and every row's sum over each
 //   group of 128 columns;
-// * the product kernel (128 x 256 tiles, eight waves of 64 x 64, one workgroup per CU; where K is
-//   short also 64 x 256, one per CU, and 64 x 128 of four waves of 32 x 64, two per CU) moves a
+// * the product kernel (128 x 256 tiles of eight waves, one workgroup per CU; where K is
+//   short also 64 x 256, one per CU, and 64 x 128 of four waves, two per CU) moves a
 //   group's slab of that copy (128 columns) and its tile of nibbles from global
 //   memory STRAIGHT into LDS (global_load_lds, 16 bytes per lane, no registers, no vector
 //   instructions) into a ring of three buffers, requested two groups ahead, one barrier per
 //   group.  A request writes 1 KiB of consecutive LDS, so instead of padding rows the
 //   16-byte chunks of a row are stored XOR-swizzled by the row index and the ds_read_b128 of
 //   the MFMA operands stay conflict-free;
+// * a wave takes ALL rows of the tile by 32 weight rows, so that no two waves unpack the same nibbles:
+//   56 vector instructions of unpack per 32 MFMAs instead of the 112 of 64 x 64 parts, for an LDS
+//   operand read per MFMA instead of one per two (16-byte reads come at 256 bytes per clock: 1100 of
+//   the 3600 cycles a group takes);
+// * the requests go out one per step of 16 columns.  Issued together behind the barrier, all eight
+//   waves waited in front of the texture addresser (48 requests x 16 cycles) with the matrix pipe
+//   idle: a build without any requests was 15 % faster, and this one gets most of that back.
+//   The wait and the barrier stand in the middle of a group and the first operands of the next are
+//   read in its last step, so that nothing is waited for between two groups.  Bit for bit the
+//   same products.  4000 rows, us before / now: 6144 x 4096 206 / 180, 4096 x 12288 380 / 347,
+//   24576 x 4096 with the activation 778 / 737, 1536 x 8960 144 / 113; 195 rows: 30.0 / 27.9,
+//   44.0 / 40.7, 59.7 / 55.2, 26.8 / 24.4;
 // * scales, zeros and the group sums of x reach a lane's registers for four (or two) pairs
 //   of groups per load where K allows: a lane's row of scales is 64 bytes apart from the
 //   next lane's, so each such load costs the address path a cache line per lane -- one per
@@ -33,7 +45,8 @@
 //   group, into the group's own sum);
 // * what is left per group and wave: the unpack (a lane of the v_mfma_f32_32x32x16_bf16 B
 //   operand is one weight row and one dword of nibbles, made bf16 `128 + q` with an and-or per
-//   pair, exact), one multiply-add per result for the group's scale, 32 MFMAs.
+//   pair, exact), one multiply-add per result for the group's scale, 32 MFMAs.  At 4000 rows a group
+//   takes 1.75 us, of which the matrix pipe needs 1.12 at the clock the board's power leaves.
 //
 // * workgroups all take the same time and a CU holds one, so a launch whose tile count is not
 //   a multiple of the CU count ends on a round that leaves most CUs idle (config 4's o and
@@ -54,28 +67,32 @@
 
 namespace lg {
 
+// (a lambda with two call sites is a function of its own otherwise, its captures in scratch)
+#define LG_INLINE __attribute__((always_inline))
+
 typedef __attribute__((address_space(3))) void* tp_lds_ptr_t;
 typedef const __attribute__((address_space(1))) void* tp_glb_ptr_t;
 
-// A workgroup's tile: two rows of ACROSS waves, a wave takes 32 * BLOCKS rows of x by 64 weight rows.
+// A workgroup's tile: 32 * BLOCKS rows of x by 32 weight rows for each of its WAVES waves.
 // CUTS: adds up in the parts a 128 x 256 tile would be split into (32 more registers; the code for it
 // costs 0.3-0.9 us of a launch, about 0.2 us of one that has no parts).
-template <int BLOCKS, int ACROSS, bool CUTS = false>
+template <int BLOCKS, int WAVES, bool CUTS = false>
 struct TpTile {
-    static constexpr int kBlocks = BLOCKS, kAcross = ACROSS, kWaves = 2 * ACROSS;
-    static constexpr int kM = 64 * BLOCKS, kN = 64 * ACROSS;
+    static constexpr int kBlocks = BLOCKS, kWaves = WAVES;
+    static constexpr int kM = 32 * BLOCKS, kN = 32 * WAVES;
     static constexpr int kSlabBytes = kM * 256;  // one group's slab of x: kM rows x 128 bf16
     static constexpr int kBufBytes = kSlabBytes + kN * 64;  // ... and its tile of nibbles
     static constexpr int kXRequests = kM / 4 / kWaves;      // 1 KiB requests of x per wave
-    static constexpr bool kBig = BLOCKS == 2 && ACROSS == 4;
+    static constexpr bool kBig = BLOCKS == 4 && WAVES == 8;
     static constexpr bool kCuts = CUTS;
-    static_assert(kXRequests == 2 || kXRequests == 4, "what request_group spells out");
+    static_assert(BLOCKS == 2 || BLOCKS == 4, "what the operand reads spell out");
+    static_assert(kXRequests == 2 || kXRequests == 4, "what request_x spells out");
 };
-using TpBig = TpTile<2, 4>;
+using TpBig = TpTile<4, 8>;
 template <bool CUTS>
-using TpHalf = TpTile<1, 4, CUTS>;
+using TpHalf = TpTile<2, 8, CUTS>;
 template <bool CUTS>
-using TpSmall = TpTile<1, 2, CUTS>;
+using TpSmall = TpTile<2, 4, CUTS>;
 constexpr int kTpTileM = TpBig::kM;  // 128 rows of x per workgroup
 constexpr int kTpTileN = TpBig::kN;  // 256 weight rows per workgroup
 constexpr int kTpBufs = 3;                // groups in LDS: one in use, two on their way
@@ -200,7 +217,7 @@ __global__ __launch_bounds__(64 * T::kWaves) void qgemm_q4g128_tallp_kernel(
     int n, int k, int tiles_n, int full_tiles, int split, int out_pairs) {
     extern __shared__ uint4_t tp_lds[];  // kTpBufs x {slab of x, tile of weights}
     constexpr int BL = 2 * W;            // groups per block of small loads
-    constexpr int MI = T::kBlocks, WN = T::kAcross;
+    constexpr int MI = T::kBlocks;
     constexpr int kSlab = T::kSlabBytes, kBuf = T::kBufBytes;
     const int tid = threadIdx.x;
     const int lane = tid & 63;
@@ -225,17 +242,16 @@ __global__ __launch_bounds__(64 * T::kWaves) void qgemm_q4g128_tallp_kernel(
     // (SwiGLU: a tile is half as many outputs wide, as many gate as up rows of the weights)
     constexpr int kTileOutputs = tp_is_swiglu(OUT) ? T::kN / 2 : T::kN;
     const int col0 = (tile % tiles_n) * kTileOutputs;
-    // weight row behind row L of the tile in LDS (a wave's B operand rows are L = wc + 32 j + r)
+    // weight row behind row L of the tile in LDS (a wave's B operand rows are L = 32 wave + r)
     auto weight_row = [&](int L) {
         if constexpr (tp_is_swiglu(OUT)) {
-            const int out_col = min(col0 + (L >> 6) * 32 + (L & 31), n - 1);
-            return ((L >> 5) & 1) ? n + out_col : out_col;
+            const int out_col = min(col0 + (L >> 5) * 16 + (L & 15), n - 1);
+            return ((L >> 4) & 1) ? n + out_col : out_col;
         } else {
             return min(col0 + L, n - 1);  // a row past n re-reads the last row
         }
     };
-    const int wr = (wave / WN) * 32 * MI;  // this wave's part of the tile
-    const int wc = (wave % WN) * 64;
+    const int wc = wave * 32;  // this wave's weight rows of the tile
     const int groups_row = k >> 7;    // scales and zeros: groups per weight row
     unsigned magic;
     asm volatile("v_mov_b32 %0, 0x43004300" : "=v"(magic));
@@ -248,13 +264,12 @@ __global__ __launch_bounds__(64 * T::kWaves) void qgemm_q4g128_tallp_kernel(
     // position lane % 4 of the row's 64 bytes, which holds piece (position ^ (row / 4) % 4).
     // Byte offsets fit 32 bits (m_pad * K * 2 and N * K < 2^31 are checked on the host).
     constexpr int kXReq = T::kXRequests;
-    unsigned xoff[kXReq], woff[2];
-#pragma unroll
-    for (int q = 0; q < kXReq; ++q) {
-        const int row = 4 * kXReq * wave + 4 * q + (lane >> 4);
-        const int c = (lane & 15) ^ (row & 15);
-        xoff[q] = ((unsigned)(row0 + row) * (unsigned)k + (unsigned)c * 8u) * 2u;
-    }
+    // (Request q of x is four rows on, whose chunks are swizzled by another 4 q: rows are multiples of
+    // 256 bytes apart, so its offsets are the first one's ^ 64 q from a base 4 q rows on.)
+    const int xrow = 4 * kXReq * wave + (lane >> 4);
+    const unsigned xoff = ((unsigned)(row0 + xrow) * (unsigned)k +
+                           (unsigned)((lane & 15) ^ (xrow & 15)) * 8u) * 2u;
+    unsigned woff[2];
 #pragma unroll
     for (int q = 0; q < 2; ++q) {
         const int row = 32 * wave + 16 * q + (lane >> 2);
@@ -264,154 +279,137 @@ __global__ __launch_bounds__(64 * T::kWaves) void qgemm_q4g128_tallp_kernel(
     // As assembly: the 32-bit offsets above with a scalar base (the builtin widens each to a
     // 64-bit address in two more registers); M0 holds the LDS address of lane 0's 16 bytes and
     // nothing else in this kernel uses M0.
-    auto request_group = [&](int g, int buf_off) {
-        const char* xsrc = reinterpret_cast<const char*>(xp) + (size_t)g * 256;
-        const char* wsrc = reinterpret_cast<const char*>(qw) + (size_t)g * 64;
+    auto request = [&](const char* src, unsigned off, unsigned dst) LG_INLINE {
+        asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
+                     :
+                     : "v"(off), "s"(src), "s"(dst)
+                     : "memory");
+    };
+    // request q of group g's x and weights, into the buffer at byte `buf_off` of the ring
+    auto request_x = [&](auto q_c, int g, int buf_off) LG_INLINE {
+        constexpr int Q = decltype(q_c)::value;
         // (scalar registers for sure: a value the compiler takes for lane-dependent would be
         // handed to the statement in vector registers)
-        const unsigned xdst = __builtin_amdgcn_readfirstlane(lds_base + (unsigned)buf_off +
-                                                             (unsigned)wave * (1024u * kXReq));
-        const unsigned wdst = xdst + kSlab - (unsigned)wave * (1024u * kXReq - 2048u);
-        if constexpr (kXReq == 4) {
-            asm volatile(
-                "s_mov_b32 m0, %8\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %6\n\t"
-                "s_add_u32 m0, %8, 0x400\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %6\n\t"
-                "s_add_u32 m0, %8, 0x800\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %2, %6\n\t"
-                "s_add_u32 m0, %8, 0xc00\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %3, %6\n\t"
-                "s_mov_b32 m0, %9\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %4, %7\n\t"
-                "s_add_u32 m0, %9, 0x400\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %5, %7"
-                :
-                : "v"(xoff[0]), "v"(xoff[1]), "v"(xoff[kXReq - 2]), "v"(xoff[kXReq - 1]), "v"(woff[0]), "v"(woff[1]),
-                  "s"(xsrc), "s"(wsrc), "s"(xdst), "s"(wdst)
-                : "memory", "scc");
-        } else {
-            asm volatile(
-                "s_mov_b32 m0, %6\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %4\n\t"
-                "s_add_u32 m0, %6, 0x400\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %4\n\t"
-                "s_mov_b32 m0, %7\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %2, %5\n\t"
-                "s_add_u32 m0, %7, 0x400\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %3, %5"
-                :
-                : "v"(xoff[0]), "v"(xoff[1]), "v"(woff[0]), "v"(woff[1]), "s"(xsrc), "s"(wsrc),
-                  "s"(xdst), "s"(wdst)
-                : "memory", "scc");
-        }
+        request(reinterpret_cast<const char*>(xp) + ((size_t)g * 256 + (size_t)Q * 8 * (unsigned)k),
+                xoff ^ (64u * Q),
+                __builtin_amdgcn_readfirstlane(lds_base + (unsigned)buf_off +
+                                               (unsigned)(wave * kXReq + Q) * 1024u));
     };
-    constexpr int kReq = kXReq + 2;  // requests per group and wave
-    // ---- A operand reads: lane (r, h) at step s8 wants chunk 8 h + s8 of row wr + 32 i + r,
+    auto request_w = [&](auto q_c, int g, int buf_off) LG_INLINE {
+        constexpr int Q = decltype(q_c)::value;
+        request(reinterpret_cast<const char*>(qw) + (size_t)g * 64, woff[Q],
+                __builtin_amdgcn_readfirstlane(lds_base + (unsigned)buf_off + kSlab +
+                                               (unsigned)(wave * 2 + Q) * 1024u));
+    };
+    auto request_group = [&](int g, int buf_off) LG_INLINE {
+        static_for<kXReq>([&](auto q) LG_INLINE { request_x(q, g, buf_off); });
+        static_for<2>([&](auto q) LG_INLINE { request_w(q, g, buf_off); });
+    };
+    // ---- A operand reads: lane (r, h) at step s8 wants chunk 8 h + s8 of row 32 i + r,
     // stored at position (8 h + s8) ^ (r % 16): a0 ^ (s8 << 4), the i-tile as an immediate
     // (a buffer's offset in the ring is a multiple of 8 KiB: adding it commutes with the XOR)
-    const unsigned a0 = lds_base + (unsigned)(wr + r) * 256u +
+    const unsigned a0 = lds_base + (unsigned)r * 256u +
                         (unsigned)(((8 * h) ^ (r & 8)) | (r & 7)) * 16u;
-    // ---- B operand reads: lane (r, h) of n-tile j wants the pieces 2 h, 2 h + 1 of row
-    // wc + 32 j + r (dword s8 % 4 of piece 2 h + s8 / 4 feeds step s8); j as an immediate
-    unsigned b_addr[2];
-#pragma unroll
-    for (int t = 0; t < 2; ++t)
-        b_addr[t] = lds_base + kSlab + (unsigned)(wc + r) * 64u +
-                    (unsigned)((2 * h + t) ^ ((r >> 2) & 3)) * 16u;
+    // ---- B operand reads: lane (r, h) wants the pieces 2 h, 2 h + 1 of row wc + r (dword s8 % 4 of
+    // piece 2 h + s8 / 4 feeds step s8)
+    // (piece 2 h + 1 sits at the address ^ 16)
+    const unsigned b_addr = lds_base + kSlab + (unsigned)(wc + r) * 64u +
+                            (unsigned)((2 * h) ^ ((r >> 2) & 3)) * 16u;
 
     // ---- The small loads of a block of W pairs of groups, from global memory into registers:
-    // scales and zeros of this lane's two weight rows (a lane's 16 results of a tile belong to
-    // one weight row; pair p in dword p: group 2 p in the low half), and the group sums of x
-    // for the zero-point product (lane (r, h) holds row wr + 32 i + r, group 2 p + h of pair
+    // scales and zeros of this lane's weight row (a lane's results all belong to one weight row;
+    // pair p in dword p: group 2 p in the low half), and the group sums of x
+    // for the zero-point product (lane (r, h) holds row 32 i + r, group 2 p + h of pair
     // p; the first pass wrote them as [row tile][block][h][row][p], so a wave reads 512
-    // consecutive bytes x W).  Per block and wave two loads of scales and two of zeros (ODD: a
-    // third pair, the scales of the second group) and MI of group sums, written as assembly
+    // consecutive bytes x W).  Per block and wave one load of scales and one of zeros (ODD: a
+    // second one of scales, of the second group) and MI of group sums, written as assembly
     // with the wait for them spelled out below, once per block: for loads it can see the
     // compiler waits with vmcnt(0) wherever a value is used, in every group, which also waits
     // for every request of the groups ahead and takes the ring's depth away.  A register
     // loaded here must not be touched before `small_loads_landed` has named it.
+    // (The group sums of four pairs come as two loads of two, the second behind the first half of the
+    // block: 8 registers less.)
+    constexpr int WX = W == 4 ? 2 : W;
     struct Small {
-        TpRegs<unsigned, W> s[2], z[2];
-        TpRegs<float, W> xs[2];  // (one of them with one block of rows per wave)
-        unsigned s_hi[2];  // ODD: s and s_hi the scales of the pair's two groups, z the zero of
-                           // this lane's group of the pair
+        TpRegs<unsigned, W> s, z;
+        TpRegs<float, WX> xs[MI];
+        unsigned s_hi;  // ODD: s and s_hi the scales of the pair's two groups, z the zero of
+                        // this lane's group of the pair
     };
-    unsigned soff[2], xsoff[MI];
-#pragma unroll
-    for (int j = 0; j < 2; ++j)
-        soff[j] = (unsigned)weight_row(wc + 32 * j + r) * (unsigned)groups_row * 2u;
-#pragma unroll
-    for (int i = 0; i < MI; ++i)
-        xsoff[i] = (unsigned)((h * kTallTileRows + (row0 % kTallTileRows) + wr + 32 * i + r) * W) * 4u;
-    auto gload_small = [&](int g, Small& v) {
+    const unsigned soff = (unsigned)weight_row(wc + r) * (unsigned)groups_row * 2u;
+    const unsigned xsoff = (unsigned)((h * kTallTileRows + (row0 % kTallTileRows) + r) * W) * 4u;
+    // the sums of the WX pairs from group g on
+    auto gload_sums = [&](int g, Small& v) LG_INLINE {
+        const float* xb = xs + ((size_t)(row0 / kTallTileRows) * ((groups_row + BL - 1) / BL) + g / BL) *
+                                   (2 * kTallTileRows * W) + (g % BL) / 2;
+        // (the row tiles 32 W floats apart, as immediates)
+        static_for<MI>([&](auto i_c) LG_INLINE {
+            constexpr int at = decltype(i_c)::value * 32 * W * 4;
+            typename TpRegs<float, WX>::raw_t& dst = v.xs[decltype(i_c)::value].raw;
+            const unsigned off = xsoff;
+            const float* const base = xb;
+            if constexpr (WX == 1)
+                asm volatile("global_load_dword %0, %1, %2 offset:%c3" : "=&v"(dst) : "v"(off), "s"(base), "n"(at) : "memory");
+            else
+                asm volatile("global_load_dwordx2 %0, %1, %2 offset:%c3" : "=&v"(dst) : "v"(off), "s"(base), "n"(at) : "memory");
+        });
+    };
+    auto gload_small = [&](int g, Small& v) LG_INLINE {
         const __half* sb = scale + g;
         const __half* zb = zero + g;
-        const float* xb = xs + ((size_t)(row0 / kTallTileRows) * ((groups_row + BL - 1) / BL) + g / BL) *
-                                   (2 * kTallTileRows * W);
-#pragma unroll
-        for (int j = 0; j < 2; ++j) {
-            if constexpr (ODD) {
-                // (a missing second group re-reads the first)
-                const unsigned second = soff[j] + (g + 1 < groups_row ? 2u : 0u);
-                const unsigned own = h ? second : soff[j];
-                asm volatile("global_load_ushort %0, %1, %2" : "=&v"(v.s[j].raw) : "v"(soff[j]), "s"(sb) : "memory");
-                asm volatile("global_load_ushort %0, %1, %2" : "=&v"(v.s_hi[j]) : "v"(second), "s"(sb) : "memory");
-                asm volatile("global_load_ushort %0, %1, %2" : "=&v"(v.z[j].raw) : "v"(own), "s"(zb) : "memory");
-            } else if constexpr (W == 1) {
-                asm volatile("global_load_dword %0, %1, %2" : "=&v"(v.s[j].raw) : "v"(soff[j]), "s"(sb) : "memory");
-                asm volatile("global_load_dword %0, %1, %2" : "=&v"(v.z[j].raw) : "v"(soff[j]), "s"(zb) : "memory");
-            } else if constexpr (W == 2) {
-                asm volatile("global_load_dwordx2 %0, %1, %2" : "=&v"(v.s[j].raw) : "v"(soff[j]), "s"(sb) : "memory");
-                asm volatile("global_load_dwordx2 %0, %1, %2" : "=&v"(v.z[j].raw) : "v"(soff[j]), "s"(zb) : "memory");
-            } else {
-                asm volatile("global_load_dwordx4 %0, %1, %2" : "=&v"(v.s[j].raw) : "v"(soff[j]), "s"(sb) : "memory");
-                asm volatile("global_load_dwordx4 %0, %1, %2" : "=&v"(v.z[j].raw) : "v"(soff[j]), "s"(zb) : "memory");
-            }
+        if constexpr (ODD) {
+            // (a missing second group re-reads the first)
+            const unsigned second = soff + (g + 1 < groups_row ? 2u : 0u);
+            const unsigned own = h ? second : soff;
+            asm volatile("global_load_ushort %0, %1, %2" : "=&v"(v.s.raw) : "v"(soff), "s"(sb) : "memory");
+            asm volatile("global_load_ushort %0, %1, %2" : "=&v"(v.s_hi) : "v"(second), "s"(sb) : "memory");
+            asm volatile("global_load_ushort %0, %1, %2" : "=&v"(v.z.raw) : "v"(own), "s"(zb) : "memory");
+        } else if constexpr (W == 1) {
+            asm volatile("global_load_dword %0, %1, %2" : "=&v"(v.s.raw) : "v"(soff), "s"(sb) : "memory");
+            asm volatile("global_load_dword %0, %1, %2" : "=&v"(v.z.raw) : "v"(soff), "s"(zb) : "memory");
+        } else if constexpr (W == 2) {
+            asm volatile("global_load_dwordx2 %0, %1, %2" : "=&v"(v.s.raw) : "v"(soff), "s"(sb) : "memory");
+            asm volatile("global_load_dwordx2 %0, %1, %2" : "=&v"(v.z.raw) : "v"(soff), "s"(zb) : "memory");
+        } else {
+            asm volatile("global_load_dwordx4 %0, %1, %2" : "=&v"(v.s.raw) : "v"(soff), "s"(sb) : "memory");
+            asm volatile("global_load_dwordx4 %0, %1, %2" : "=&v"(v.z.raw) : "v"(soff), "s"(zb) : "memory");
         }
-#pragma unroll
-        for (int i = 0; i < MI; ++i) {
-            if constexpr (W == 1)
-                asm volatile("global_load_dword %0, %1, %2" : "=&v"(v.xs[i].raw) : "v"(xsoff[i]), "s"(xb) : "memory");
-            else if constexpr (W == 2)
-                asm volatile("global_load_dwordx2 %0, %1, %2" : "=&v"(v.xs[i].raw) : "v"(xsoff[i]), "s"(xb) : "memory");
-            else
-                asm volatile("global_load_dwordx4 %0, %1, %2" : "=&v"(v.xs[i].raw) : "v"(xsoff[i]), "s"(xb) : "memory");
-        }
+        gload_sums(g, v);
     };
     // Waits for everything this wave has outstanding and hands the registers over.  (Not
     // "at most the requests issued behind them": whether loads into registers and requests
-    // into LDS complete in order with each other is not relied on.  The requests of the group
-    // after next, issued most of a group ago, are waited for with them -- once per block.)
-    auto small_loads_landed = [&](Small& v) {
+    // into LDS complete in order with each other is not relied on.)
+    auto small_loads_landed = [&](Small& v) LG_INLINE {
         asm volatile("s_waitcnt vmcnt(0)"
-                     : "+v"(v.s[0].raw), "+v"(v.s[1].raw), "+v"(v.z[0].raw), "+v"(v.z[1].raw),
-                       "+v"(v.xs[0].raw)
+                     : "+v"(v.s.raw), "+v"(v.z.raw), "+v"(v.xs[0].raw), "+v"(v.xs[1].raw)
                      :
                      : "memory");
-        if constexpr (MI == 2) asm volatile("" : "+v"(v.xs[1].raw)::"memory");
-        if constexpr (ODD) asm volatile("" : "+v"(v.s_hi[0]), "+v"(v.s_hi[1])::"memory");
+        if constexpr (MI == 4) asm volatile("" : "+v"(v.xs[MI - 2].raw), "+v"(v.xs[MI - 1].raw)::"memory");
+        if constexpr (ODD) asm volatile("" : "+v"(v.s_hi)::"memory");
     };
-    // One block's values are in use while the next one's are on their way (W = 1), or the
-    // next block's are loaded over them behind their last use (W > 1: a block lasts four or
-    // eight groups, and a load issued at the end of one group has landed by the end of the
-    // next).
+    // The next block's values are loaded over a block's behind their last use; they are waited for
+    // in the middle of the next group, and first used behind that.
     Small cur;
-    Small nxt;  // W == 1 only
 
-    float16_t yacc[MI][2];
+    float16_t yacc[MI];
 #pragma unroll
     for (int i = 0; i < MI; ++i)
 #pragma unroll
-        for (int j = 0; j < 2; ++j)
-#pragma unroll
-            for (int e = 0; e < 16; ++e) yacc[i][j][e] = 0.0f;
+        for (int e = 0; e < 16; ++e) yacc[i][e] = 0.0f;
     // (kCuts) A smaller tile takes all of K, and adds up what it has at the places where the 128 x 256
     // tile it lies in would be split over K (`split` parts): a product's bits do not depend on the tile
     // a launch takes (in front of a 3-bit K/V row a last bit flips whole codes).
-    float16_t parts_sum[MI][2];  // the parts before this one
+    float16_t parts_sum[MI];  // the parts before this one
     const int part_blocks = (groups + BL - 1) / BL;
     int cut = 0, next_cut = 0;   // next_cut: the first group behind this part
-    auto next_part = [&]() {
+    auto next_part = [&]() LG_INLINE {
 #pragma unroll
         for (int i = 0; i < MI; ++i)
 #pragma unroll
-            for (int j = 0; j < 2; ++j)
-#pragma unroll
-                for (int e = 0; e < 16; ++e) {
-                    parts_sum[i][j][e] += yacc[i][j][e];
-                    yacc[i][j][e] = 0.0f;
-                }
+            for (int e = 0; e < 16; ++e) {
+                parts_sum[i][e] += yacc[i][e];
+                yacc[i][e] = 0.0f;
+            }
         ++cut;
         next_cut = BL * (part_blocks * (cut + 1) / split);
     };
@@ -419,347 +417,336 @@ __global__ __launch_bounds__(64 * T::kWaves) void qgemm_q4g128_tallp_kernel(
 #pragma unroll
         for (int i = 0; i < MI; ++i)
 #pragma unroll
-            for (int j = 0; j < 2; ++j)
-#pragma unroll
-                for (int e = 0; e < 16; ++e) parts_sum[i][j][e] = 0.0f;
+            for (int e = 0; e < 16; ++e) parts_sum[i][e] = 0.0f;
         next_cut = BL * (part_blocks / split);
     }
 
+    // The buffer `ahead` groups on in the ring.
+    auto ring = [&](int off, int ahead) LG_INLINE {
+        off += ahead * kBuf;
+        return off >= kTpBufs * kBuf ? off - kTpBufs * kBuf : off;
+    };
     gload_small(g_begin, cur);
     request_group(g_begin, 0);
-    if (!ODD || g_begin + 1 < groups) request_group(g_begin + 1, kBuf);  // (else whole pairs)
+    if (g_begin + 1 < groups) request_group(g_begin + 1, kBuf);
     small_loads_landed(cur);
-
-    // The requests of the group after next go into the buffer everybody stopped reading before
-    // this group's barrier.  (Measured and not kept: the two waves of a SIMD issuing theirs at
-    // different times -- behind the barrier and in the middle of the group -- so that one
-    // feeds the matrix pipe while the other is held up by its burst of requests; no change.)
-    auto issue_requests = [&](int g, int buf_off) {
-        if (g + 2 < groups) {
-            int dst = buf_off + 2 * kBuf;
-            if (dst >= kTpBufs * kBuf) dst -= kTpBufs * kBuf;
-            request_group(g + 2, dst);
-        }
-    };
+    __builtin_amdgcn_s_barrier();
 
     // zero-point term of a pair of groups (lanes h = 0 the first, h = 1 the second):
     // y[m][n] += sum_x[m][g'] * (-scale[n][g'] * (128 + zero[n][g']))
-    auto zero_term = [&](auto pair_c) {
+    auto zero_term = [&](auto pair_c) LG_INLINE {
         constexpr int P = decltype(pair_c)::value;
-        float cv[2];
-#pragma unroll
-        for (int j = 0; j < 2; ++j) {
-            const unsigned sd = cur.s[j][P], zd = cur.z[j][P];
-            const unsigned short sb = (unsigned short)(h ? (sd >> 16) : sd);
-            const unsigned short zb = (unsigned short)(h ? (zd >> 16) : zd);
-            cv[j] = -__half2float(__builtin_bit_cast(__half, sb)) *
-                    (128.0f + __half2float(__builtin_bit_cast(__half, zb)));
-        }
+        const unsigned sd = cur.s[P], zd = cur.z[P];
+        const unsigned short sb = (unsigned short)(h ? (sd >> 16) : sd);
+        const unsigned short zb = (unsigned short)(h ? (zd >> 16) : zd);
+        const float cv = -__half2float(__builtin_bit_cast(__half, sb)) *
+                         (128.0f + __half2float(__builtin_bit_cast(__half, zb)));
 #pragma unroll
         for (int i = 0; i < MI; ++i)
-#pragma unroll
-            for (int j = 0; j < 2; ++j)
-                yacc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(cur.xs[i][P], cv[j], yacc[i][j], 0, 0, 0);
+            yacc[i] = __builtin_amdgcn_mfma_f32_32x32x2f32(cur.xs[i][P % WX], cv, yacc[i], 0, 0, 0);
     };
     // ODD: the same term of one group, -sum_x[m][g] * (128 + zero[n][g]) (the lanes of the pair's other
     // group give 0), added to the group's sum halfway through its columns: the sum then runs from 0 to
     // half of the large term, to minus half of it and back, is small when it is scaled, and the large
     // term is never rounded at its full size nor into y.
-    auto zero_halfway = [&](auto par_c, float16_t (&acc)[MI][2]) {
-        const bool own = h == decltype(par_c)::value;
+    auto zero_halfway = [&](int par, float16_t(&acc)[MI]) LG_INLINE {
+        const bool own = h == par;
+        const unsigned short zb = (unsigned short)cur.z[0];
+        const float off = own ? -(128.0f + __half2float(__builtin_bit_cast(__half, zb))) : 0.0f;
 #pragma unroll
         for (int i = 0; i < MI; ++i)
+            acc[i] = __builtin_amdgcn_mfma_f32_32x32x2f32(own ? cur.xs[i][0] : 0.0f, off, acc[i], 0, 0, 0);
+    };
+
+    float16_t acc[MI];
+    bf16x8_t av[2][MI];  // [step parity][i]
+    bf16x8_t bv[2];      // [step parity]
+    uint4_t wq[2];       // [half of the group]: the group's nibbles of this lane's row
+    // the x operands of a step, at byte address `a` of row r
+    auto read_x = [&](bf16x8_t(&v)[MI], unsigned a) LG_INLINE {
+        if constexpr (MI == 4)
+            asm volatile("ds_read_b128 %0, %4\n\tds_read_b128 %1, %4 offset:8192\n\t"
+                         "ds_read_b128 %2, %4 offset:16384\n\tds_read_b128 %3, %4 offset:24576"
+                         : "=&v"(v[0]), "=&v"(v[1]), "=&v"(v[MI - 2]), "=&v"(v[MI - 1])
+                         : "v"(a)
+                         : "memory");
+        else
+            asm volatile("ds_read_b128 %0, %2\n\tds_read_b128 %1, %2 offset:8192"
+                         : "=&v"(v[0]), "=&v"(v[1])
+                         : "v"(a)
+                         : "memory");
+    };
+    auto x_landed = [&](bf16x8_t(&v)[MI]) LG_INLINE {
+        asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(v[0]), "+v"(v[1])::"memory");
+        if constexpr (MI == 4) asm volatile("" : "+v"(v[MI - 2]), "+v"(v[MI - 1])::"memory");
+    };
+    // a group's nibbles and its first x operands, from the buffer at byte `buf_off` of the ring (the
+    // offset is added here: LDS offsets of up to 144 KiB do not fit the 16-bit immediate of a read)
+    auto read_first = [&](int buf_off) LG_INLINE {
+        unsigned t0, t1;
+        asm volatile("v_add_u32 %2, %5, %4\n\tv_xor_b32 %3, 16, %2\n\t"
+                     "ds_read_b128 %0, %2\n\tds_read_b128 %1, %3"
+                     : "=&v"(wq[0]), "=&v"(wq[1]), "=&v"(t0), "=&v"(t1)
+                     : "v"(b_addr), "s"(buf_off)
+                     : "memory");
+        read_x(av[0], a0 + (unsigned)buf_off);
+    };
+    auto first_landed = [&]() LG_INLINE {
+        asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(wq[0]), "+v"(wq[1])::"memory");
+        x_landed(av[0]);
+    };
+    // the x operands of step S (1 .. 7) of the group at a_buf
+    auto read_step = [&](auto s_c, unsigned a_buf) LG_INLINE {
+        constexpr int S = decltype(s_c)::value;
+        read_x(av[S & 1], a_buf ^ (unsigned)(S << 4));
+    };
+    auto step_landed = [&](auto s_c) LG_INLINE { x_landed(av[decltype(s_c)::value & 1]); };
+    auto unpack = [&](auto s_c) LG_INLINE {
+        constexpr int S = decltype(s_c)::value;
+        const unsigned wd = wq[S >> 2][S & 3];
+        uint4_t e4;
 #pragma unroll
-            for (int j = 0; j < 2; ++j) {
-                const unsigned short zb = (unsigned short)cur.z[j][0];
-                acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(
-                    own ? cur.xs[i][0] : 0.0f,
-                    own ? -(128.0f + __half2float(__builtin_bit_cast(__half, zb))) : 0.0f, acc[i][j],
-                    0, 0, 0);
-            }
+        for (int sft = 0; sft < 4; ++sft) e4[sft] = ((wd >> (4 * sft)) & kNibMask) | magic;
+        bv[S & 1] = __builtin_bit_cast(bf16x8_t, e4);
+    };
+    // the MFMA of step 0 of one tile of the wave
+    auto first_product = [&](int i) LG_INLINE {
+        float16_t z16;
+#pragma unroll
+        for (int e = 0; e < 16; ++e) z16[e] = 0.0f;
+        acc[i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(av[0][i], bv[0], z16, 0, 0, 0);
     };
 
     // One group of 128 columns out of the buffer at byte `buf_off` of the ring; U: the group's
-    // place in its block.  A wave's requests complete in the order they were issued, so "at most
-    // the kReq youngest outstanding" (6; 4 where eight waves share 64 rows of x) names what has
-    // landed.
-    auto group = [&](auto u_c, int g, int buf_off) {
+    // place in its block.  Its step 0 has been issued by the group before it, so that nothing is
+    // waited for between two groups:
+    // * the wait for the next group's requests and the workgroup's barrier stand in the middle of a
+    //   group, the reads of the next group's nibbles and first x operands in its step 7;
+    // * the tile by tile `y += scale * acc` is followed by that tile's first MFMA of the next group.
+    // LEFT: at least so many groups follow this one; LAST: exactly so many.  par: U % 2, but for the
+    // last group of an odd number of groups, which may be either of its pair.
+    auto group = [&](auto u_c, auto left_c, auto last_c, int g, int buf_off, int par) LG_INLINE {
         constexpr int U = decltype(u_c)::value;
-        constexpr int PAR = U & 1;
-        // this wave's requests of the group, issued two groups ago, have landed; those of
-        // the next group may be on their way.  (Requests complete in the order they were
-        // issued.  Behind a block's small loads the count is not raised by their number:
-        // whether they complete in order with the requests is not relied on.)
-        if (g + 1 >= groups) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-        else asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kReq) : "memory");
-        // after the barrier everybody's requests for this group have landed, and everybody is
-        // done reading the buffer of the group before it, which the group after next reuses
-        __builtin_amdgcn_s_barrier();
-        if constexpr (ODD && U == 1) {
-            gload_small(g + 1 < groups ? g + 1 : g - 1, nxt);
-        } else if constexpr (W == 1) {
-            if (U == 1 && g + 1 < groups) gload_small(g + 1, nxt);
-        }
-        issue_requests(g, buf_off);
-        float16_t acc[MI][2];
-        bf16x8_t av[2][MI];  // [step parity][i]
-        bf16x8_t bv[2][2];  // [step parity][j]
-        uint4_t wq[2][2];   // [j][half of the group]: the group's nibbles of this lane's rows
-        // (the buffer's offset is added here: LDS offsets of up to 144 KiB do not fit the
-        // 16-bit immediate of a read)
-        unsigned t0, t1;
-        asm volatile("v_add_u32 %4, %8, %6\n\tv_add_u32 %5, %8, %7\n\t"
-                     "ds_read_b128 %0, %4\n\tds_read_b128 %1, %5\n\t"
-                     "ds_read_b128 %2, %4 offset:2048\n\tds_read_b128 %3, %5 offset:2048"
-                     : "=&v"(wq[0][0]), "=&v"(wq[0][1]), "=&v"(wq[1][0]), "=&v"(wq[1][1]),
-                       "=&v"(t0), "=&v"(t1)
-                     : "v"(b_addr[0]), "v"(b_addr[1]), "s"(buf_off)
-                     : "memory");
+        constexpr int LEFT = decltype(left_c)::value;
+        constexpr bool LAST = decltype(last_c)::value;
+        constexpr bool more = LEFT > 0;
+        auto follows = [&](int d) LG_INLINE { return LEFT >= d || (!LAST && g + d < groups); };
         const unsigned a_buf = a0 + (unsigned)buf_off;
-        if constexpr (MI == 2)
-            asm volatile("ds_read_b128 %0, %2\n\tds_read_b128 %1, %2 offset:8192"
-                         : "=&v"(av[0][0]), "=&v"(av[0][MI - 1])
-                         : "v"(a_buf)
-                         : "memory");
-        else
-            asm volatile("ds_read_b128 %0, %1" : "=&v"(av[0][0]) : "v"(a_buf) : "memory");
-        __builtin_amdgcn_sched_barrier(0);
-        asm volatile("s_waitcnt lgkmcnt(0)"
-                     : "+v"(wq[0][0]), "+v"(wq[0][1]), "+v"(wq[1][0]), "+v"(wq[1][1]),
-                       "+v"(av[0][0])::"memory");
-        if constexpr (MI == 2) asm volatile("" : "+v"(av[0][MI - 1])::"memory");
-        auto unpack = [&](auto s8c, bf16x8_t (&b)[2]) {
-            constexpr int s8 = decltype(s8c)::value;
-#pragma unroll
-            for (int j = 0; j < 2; ++j) {
-                const unsigned wd = wq[j][s8 >> 2][s8 & 3];
-                uint4_t e4;
-#pragma unroll
-                for (int sft = 0; sft < 4; ++sft) e4[sft] = ((wd >> (4 * sft)) & kNibMask) | magic;
-                b[j] = __builtin_bit_cast(bf16x8_t, e4);
-            }
-        };
-        unpack(ic<0>{}, bv[0]);
         // Step s8 issues the reads of step s8 + 1, then its four MFMAs with the unpack of step
         // s8 + 1 between them (the matrix pipe takes 32 cycles per MFMA, eight issue slots of
         // the vector pipe), and only then waits for the reads.  The order is pinned: left
         // alone the scheduler sinks the MFMAs below the wait, which then sits right behind the
         // reads it waits for.
-        static_for<8>([&](auto s8c) {
-            constexpr int s8 = decltype(s8c)::value;
-            constexpr int cur_p = s8 & 1;
-            if constexpr (s8 < 7) {
-                unsigned ta;
-                if constexpr (MI == 2)
-                    asm volatile("v_xor_b32 %2, %c4, %3\n\t"
-                                 "ds_read_b128 %0, %2\n\tds_read_b128 %1, %2 offset:8192"
-                                 : "=&v"(av[cur_p ^ 1][0]), "=&v"(av[cur_p ^ 1][MI - 1]), "=&v"(ta)
-                                 : "v"(a_buf), "n"((s8 + 1) << 4)
-                                 : "memory");
-                else
-                    asm volatile("v_xor_b32 %1, %c3, %2\n\tds_read_b128 %0, %1"
-                                 : "=&v"(av[cur_p ^ 1][0]), "=&v"(ta)
-                                 : "v"(a_buf), "n"((s8 + 1) << 4)
-                                 : "memory");
+        static_for<7>([&](auto sc) LG_INLINE {
+            constexpr int s8 = decltype(sc)::value + 1;
+            if constexpr (s8 == 4) {
+                // The requests of the next group's x and weights (issued one and two groups ago)
+                // have landed; those of the weights behind it, the youngest two, may be on their
+                // way.  (Requests complete in the order they were issued.  Behind a block's
+                // small loads everything is waited for: whether loads into registers complete in
+                // order with the requests is not relied on.)
+                if (U == 0 || (W == 4 && U == 4)) small_loads_landed(cur);
+                else if (!follows(2)) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+                else asm volatile("s_waitcnt vmcnt(2)" ::: "memory");
+                // Behind the barrier everybody's have; everybody has left the group before this
+                // one, whose x slab the group after next takes, and has read this group's nibbles.
+                if constexpr (more) {
+                    __builtin_amdgcn_s_barrier();
+                }
             }
+            // One request per step: issued together they keep every wave from its next operands until
+            // the texture addresser has taken all of them.
+            if (follows(2)) {
+                if constexpr (s8 >= 4 && s8 - 4 < kXReq)
+                    request_x(ic<(s8 >= 4 && s8 - 4 < kXReq ? s8 - 4 : 0)>{}, g + 2, ring(buf_off, 2));
+                constexpr int kFirstW = U == 0 || (W == 4 && U == 4) ? 5 : 1;
+                if constexpr (s8 == kFirstW || s8 == kFirstW + 1)
+                    request_w(ic<(s8 == kFirstW ? 0 : 1)>{}, g + 2, ring(buf_off, 2));
+            }
+            if constexpr (s8 < 7) read_step(ic<(s8 < 7 ? s8 + 1 : 7)>{}, a_buf);
+            else if constexpr (more) read_first(ring(buf_off, 1));
             __builtin_amdgcn_sched_barrier(0);
             if constexpr (ODD && s8 == 4) {
-                zero_halfway(ic<PAR>{}, acc);
+                zero_halfway(par, acc);
                 __builtin_amdgcn_sched_barrier(0);
             }
-            if constexpr (s8 < 7) unpack(ic<(s8 < 7 ? s8 + 1 : 7)>{}, bv[cur_p ^ 1]);
+            if constexpr (s8 < 7) unpack(ic<(s8 < 7 ? s8 + 1 : 7)>{});
 #pragma unroll
             for (int i = 0; i < MI; ++i)
+                acc[i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(av[s8 & 1][i], bv[s8 & 1], acc[i], 0,
+                                                                 0, 0);
 #pragma unroll
-                for (int j = 0; j < 2; ++j) {
-                    if constexpr (s8 == 0) {
-                        float16_t z16;
-#pragma unroll
-                        for (int e = 0; e < 16; ++e) z16[e] = 0.0f;
-                        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
-                            av[cur_p][i], bv[cur_p][j], z16, 0, 0, 0);
-                    } else {
-                        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
-                            av[cur_p][i], bv[cur_p][j], acc[i][j], 0, 0, 0);
-                    }
-                }
-#pragma unroll
-            for (int q = 0; q < 2 * MI; ++q) {
+            for (int q = 0; q < MI; ++q) {
                 __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);       // one MFMA
                 __builtin_amdgcn_sched_group_barrier(0x002, 8 / MI, 0);  // vector instructions
             }
             __builtin_amdgcn_sched_barrier(0);
-            if constexpr (s8 < 7) {
-                asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(av[cur_p ^ 1][0])::"memory");
-                if constexpr (MI == 2) asm volatile("" : "+v"(av[cur_p ^ 1][MI - 1])::"memory");
-            }
+            if constexpr (s8 < 7) step_landed(ic<(s8 < 7 ? s8 + 1 : 7)>{});
         });
-        if constexpr (W > 1 && U == 0) {
-            // the block's values, requested at the end of the group before this one
-            if (g > g_begin) small_loads_landed(cur);
+        if constexpr (more) {
+            first_landed();
+            unpack(ic<0>{});
+            read_step(ic<1>{}, a0 + (unsigned)ring(buf_off, 1));
         }
-        // y += scale * acc  (measured and not kept: the last two steps tile by tile with a
-        // tile's multiply-adds between the MFMAs of the tiles after it; no change)
+        __builtin_amdgcn_sched_barrier(0);
+        const unsigned sd = cur.s[U >> 1];
+        const unsigned short sb =
+            (unsigned short)(ODD ? (par ? cur.s_hi : sd) : (par ? (sd >> 16) : sd));
+        const float sf = __half2float(__builtin_bit_cast(__half, sb));
 #pragma unroll
-        for (int j = 0; j < 2; ++j) {
-            const unsigned sd = cur.s[j][U >> 1];
-            const unsigned short sb =
-                (unsigned short)(ODD ? (PAR ? cur.s_hi[j] : sd) : (PAR ? (sd >> 16) : sd));
-            const float sf = __half2float(__builtin_bit_cast(__half, sb));
+        for (int i = 0; i < MI; ++i) {
 #pragma unroll
-            for (int i = 0; i < MI; ++i)
-#pragma unroll
-                for (int e = 0; e < 16; ++e) yacc[i][j][e] = fmaf(sf, acc[i][j][e], yacc[i][j][e]);
+            for (int e = 0; e < 16; ++e) yacc[i][e] = fmaf(sf, acc[i][e], yacc[i][e]);
+            if constexpr (more) first_product(i);
+            __builtin_amdgcn_sched_barrier(0);
         }
-        if constexpr (PAR == 1) {
-            if constexpr (!ODD) zero_term(ic<(U >> 1)>{});
-            if constexpr (ODD) {
-                small_loads_landed(nxt);
-                cur = nxt;
-            } else if constexpr (W == 1) {
-                if (g + 1 < groups) {
-                    small_loads_landed(nxt);
-                    cur = nxt;
-                }
-            } else if constexpr (U == BL - 1) {
-                if (g + 1 < groups) gload_small(g + 1, cur);
-            }
+        if constexpr (more) {
+            unpack(ic<1>{});
+            step_landed(ic<1>{});
         }
+        if constexpr (U % 2 == 1 && !ODD) zero_term(ic<(U >> 1)>{});
+        if constexpr (U == BL - 1 && more) gload_small(g + 1, cur);
+        if constexpr (W == 4 && U == 3) gload_sums(g + 1, cur);
     };
+    // the first group's step 0
+    read_first(0);
+    first_landed();
+    unpack(ic<0>{});
+    read_step(ic<1>{}, a0);
+#pragma unroll
+    for (int i = 0; i < MI; ++i) first_product(i);
+    unpack(ic<1>{});
+    step_landed(ic<1>{});
     // ranges are whole blocks (K is a multiple of 256 W); buffers go round in threes
     int buf_off = 0;
-    auto next_buf = [&]() {
-        buf_off = buf_off + kBuf == kTpBufs * kBuf ? 0 : buf_off + kBuf;
+    auto one_group = [&](auto u_c, auto left_c, auto last_c, int g) LG_INLINE {
+        group(u_c, left_c, last_c, g, buf_off, decltype(u_c)::value & 1);
+        buf_off = ring(buf_off, 1);
     };
+    // whole blocks with more behind them, then the last one (an odd number of groups: of one or two)
+    int g0 = g_begin;
+    for (; g0 + BL < groups; g0 += BL) {
+        if constexpr (T::kCuts)
+            if (g0 == next_cut) next_part();
+        static_for<BL>([&](auto uc) LG_INLINE {
+            constexpr int U = decltype(uc)::value;
+            one_group(uc, ic<BL - 1 - U + (ODD ? 1 : BL)>{}, ic<0>{}, g0 + U);
+        });
+    }
+    if constexpr (T::kCuts)
+        if (g0 == next_cut) next_part();
     if constexpr (ODD) {
-        int g0 = g_begin;
-        for (; g0 + 1 < groups; g0 += 2) {
-            if constexpr (T::kCuts)
-                if (g0 == next_cut) next_part();
-            group(ic<0>{}, g0, buf_off);
-            next_buf();
-            group(ic<1>{}, g0 + 1, buf_off);
-            next_buf();
-        }
-        if (g0 < groups) {
-            if constexpr (T::kCuts)
-                if (g0 == next_cut) next_part();
-            group(ic<0>{}, g0, buf_off);
-        }
+        const int par = groups - 1 - g0;
+        if (par != 0) one_group(ic<0>{}, ic<1>{}, ic<1>{}, g0);
+        group(ic<0>{}, ic<0>{}, ic<1>{}, groups - 1, buf_off, par);
     } else {
-        for (int g0 = g_begin; g0 < groups; g0 += BL) {
-            if constexpr (T::kCuts)
-                if (g0 == next_cut) next_part();
-            static_for<BL>([&](auto uc) {
-                group(uc, g0 + decltype(uc)::value, buf_off);
-                next_buf();
-            });
-        }
+        static_for<BL>([&](auto uc) LG_INLINE {
+            constexpr int U = decltype(uc)::value;
+            one_group(uc, ic<BL - 1 - U>{}, ic<1>{}, g0 + U);
+        });
     }
     if constexpr (T::kCuts) {
 #pragma unroll
         for (int i = 0; i < MI; ++i)
 #pragma unroll
-            for (int j = 0; j < 2; ++j)
-#pragma unroll
-                for (int e = 0; e < 16; ++e) yacc[i][j][e] = parts_sum[i][j][e] + yacc[i][j][e];
+            for (int e = 0; e < 16; ++e) yacc[i][e] = parts_sum[i][e] + yacc[i][e];
     }
 
     if (OUT == kTpOutF32 && T::kBig && part >= 0 && out_pairs != 0) {
         // a part of a launch whose consumer adds up the parts: rows of an [m][n] matrix each
         float* dst = partials + (size_t)(part % split) * ((size_t)m * n);
-#pragma unroll
-        for (int j = 0; j < 2; ++j) {
-            const int gn = col0 + wc + 32 * j + r;
-            if (gn >= n) continue;
-#pragma unroll
-            for (int i = 0; i < MI; ++i)
-#pragma unroll
-                for (int e = 0; e < 16; ++e) {
-                    const int gr = row0 + wr + 32 * i + 8 * (e >> 2) + 4 * h + (e & 3);
-                    if (gr < m) dst[(int64_t)gr * n + gn] = yacc[i][j][e];
-                }
-        }
-        return;
-    }
-    if (T::kBig && part >= 0) {
-        // a part of a tile: the wave's 64 x 64 results as they lie in registers, lane fastest
-        float* dst = partials + (size_t)part * kTpTileElems + (size_t)wave * 4096 + lane;
-#pragma unroll
-        for (int i = 0; i < MI; ++i)
-#pragma unroll
-            for (int j = 0; j < 2; ++j)
-#pragma unroll
-                for (int e = 0; e < 16; ++e) dst[((i * 2 + j) * 16 + e) * 64] = yacc[i][j][e];
-        return;
-    }
-    if constexpr (OUT == kTpOutSwigluOperand) {
-        // (n is a multiple of 128 here: every column of the tile is a result)
-        const int gn = col0 + (wc >> 1) + r;
-        uint16_t* const xo = static_cast<uint16_t*>(y_out);
-        float* const so = reinterpret_cast<float*>(static_cast<char*>(y_out) + tall_sums_offset(m, n));
-        // the ring is done with once every wave has read its last operands
-        __syncthreads();
-        float* const red = reinterpret_cast<float*>(tp_lds);  // [wave column][chunk of it][row]
-        static_assert(WN == 4, "a tile's outputs are one group of the next K");
-        const int wq = wave % WN, cq = r >> 3;
-#pragma unroll
-        for (int i = 0; i < MI; ++i)
-#pragma unroll
-            for (int e = 0; e < 16; ++e) {
-                const int row = wr + 32 * i + 8 * (e >> 2) + 4 * h + (e & 3);
-                const float g = yacc[i][0][e], u = yacc[i][1][e];
-                const uint16_t b = f32_to_bf16_rne(g / (1.0f + expf(-g)) * u);
-                xo[(int64_t)(row0 + row) * n + (gn & ~7) + tp_pair_slot(gn & 7)] = b;
-                const float cs = tp_chunk_sum_across_lanes(__uint_as_float((unsigned)b << 16));
-                if ((r & 7) == 0) red[(wq * 4 + cq) * T::kM + row] = cs;
-            }
-        __syncthreads();
-        if (tid < T::kM) {
-            float cs[4][4];
-#pragma unroll
-            for (int a = 0; a < 4; ++a)
-#pragma unroll
-                for (int c = 0; c < 4; ++c) cs[a][c] = red[(a * 4 + c) * T::kM + tid];
-            so[tall_sum_index(row0 + tid, col0 >> 7, n, out_pairs)] = tp_group_sum(cs);
-        }
-        return;
-    }
-    if constexpr (OUT == kTpOutSwiglu) {
-        const int gn = col0 + (wc >> 1) + r;
+        const int gn = col0 + wc + r;
         if (gn >= n) return;
 #pragma unroll
         for (int i = 0; i < MI; ++i)
 #pragma unroll
             for (int e = 0; e < 16; ++e) {
-                const int gr = row0 + wr + 32 * i + 8 * (e >> 2) + 4 * h + (e & 3);
-                if (gr < m) {
-                    const float g = yacc[i][0][e], u = yacc[i][1][e];
-                    static_cast<uint16_t*>(y_out)[(int64_t)gr * n + gn] =
-                        f32_to_bf16_rne(g / (1.0f + expf(-g)) * u);
-                }
+                const int gr = row0 + 32 * i + 8 * (e >> 2) + 4 * h + (e & 3);
+                if (gr < m) dst[(int64_t)gr * n + gn] = yacc[i][e];
             }
         return;
     }
-#pragma unroll
-    for (int j = 0; j < 2; ++j) {
-        const int gn = col0 + wc + 32 * j + r;
-        if (gn >= n) continue;
-        const float bv = bias ? bias[gn] : 0.0f;
+    if (T::kBig && part >= 0) {
+        // a part of a tile: the wave's 128 x 32 results as they lie in registers, lane fastest
+        float* dst = partials + (size_t)part * kTpTileElems + (size_t)wave * 4096 + lane;
 #pragma unroll
         for (int i = 0; i < MI; ++i)
 #pragma unroll
-            for (int e = 0; e < 16; ++e) {
-                const int gr = row0 + wr + 32 * i + 8 * (e >> 2) + 4 * h + (e & 3);
-                if (gr < m) {
-                    if constexpr (OUT == kTpOutF32)
-                        static_cast<float*>(y_out)[(int64_t)gr * n + gn] = yacc[i][j][e] + bv;
-                    else
-                        static_cast<uint16_t*>(y_out)[(int64_t)gr * n + gn] =
-                            f32_to_bf16_rne(yacc[i][j][e] + bv);
-                }
-            }
+            for (int e = 0; e < 16; ++e) dst[(i * 16 + e) * 64] = yacc[i][e];
+        return;
     }
+    if constexpr (tp_is_swiglu(OUT)) {
+        // Lanes r < 16 hold the gate, r >= 16 the up products of outputs 16 wave + r % 16.  Result e of
+        // the upper lanes and result e + 8 of the lower ones change places, and every lane has both
+        // products of eight rows per block: e of the lower, e + 8 of the upper lanes.
+#pragma unroll
+        for (int i = 0; i < MI; ++i)
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                const auto sw = __builtin_amdgcn_permlane16_swap(
+                    __float_as_uint(yacc[i][e]), __float_as_uint(yacc[i][e + 8]), false, false);
+                yacc[i][e] = __uint_as_float(sw[0]);      // gate
+                yacc[i][e + 8] = __uint_as_float(sw[1]);  // up
+            }
+        // the row of result e (0 .. 7) of block i
+        auto row_of = [&](int i, int e) { return 32 * i + 8 * (e >> 2) + (r & 16) + 4 * h + (e & 3); };
+        auto activation = [&](int i, int e) {
+            const float g = yacc[i][e], u = yacc[i][e + 8];
+            return f32_to_bf16_rne(g / (1.0f + expf(-g)) * u);
+        };
+        if constexpr (OUT == kTpOutSwigluOperand) {
+            // (n is a multiple of 128 here: every column of the tile is a result)
+            uint16_t* const xo = static_cast<uint16_t*>(y_out);
+            float* const so = reinterpret_cast<float*>(static_cast<char*>(y_out) + tall_sums_offset(m, n));
+            // The bf16 tile goes through LDS, rows 16 bytes apart from a multiple of their 256, and
+            // comes back as the first pass of a product takes it: a thread a chunk of eight, the 16
+            // lanes of a row of lanes a row's group.
+            __syncthreads();  // the ring is done with once every wave has read its last operands
+            constexpr int kPitch = 128 + 8;
+            uint16_t* const tile_b = reinterpret_cast<uint16_t*>(tp_lds);
+            static_assert(T::kWaves == 8, "a tile's outputs are one group of the next K");
+#pragma unroll
+            for (int i = 0; i < MI; ++i)
+#pragma unroll
+                for (int e = 0; e < 8; ++e)
+                    tile_b[row_of(i, e) * kPitch + 16 * wave + (r & 15)] = activation(i, e);
+            __syncthreads();
+#pragma unroll
+            for (int u = 0; u < T::kM / 32; ++u) {
+                const int row = 32 * u + (tid >> 4), c = tid & 15;
+                const uint4_t v = *reinterpret_cast<const uint4_t*>(tile_b + row * kPitch + 8 * c);
+                const float gs = row16_sum(sum8_bf16(v));
+                *reinterpret_cast<uint4_t*>(xo + (int64_t)(row0 + row) * n + col0 + 8 * c) = pair_order(v);
+                if (c == 0) so[tall_sum_index(row0 + row, col0 >> 7, n, out_pairs)] = gs;
+            }
+        } else {
+            const int gn = col0 + (wc >> 1) + (r & 15);
+            if (gn >= n) return;
+#pragma unroll
+            for (int i = 0; i < MI; ++i)
+#pragma unroll
+                for (int e = 0; e < 8; ++e) {
+                    const int gr = row0 + row_of(i, e);
+                    if (gr < m) static_cast<uint16_t*>(y_out)[(int64_t)gr * n + gn] = activation(i, e);
+                }
+        }
+        return;
+    }
+    const int gn = col0 + wc + r;
+    if (gn >= n) return;
+    const float bv_n = bias ? bias[gn] : 0.0f;
+#pragma unroll
+    for (int i = 0; i < MI; ++i)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) {
+            const int gr = row0 + 32 * i + 8 * (e >> 2) + 4 * h + (e & 3);
+            if (gr < m) {
+                if constexpr (OUT == kTpOutF32)
+                    static_cast<float*>(y_out)[(int64_t)gr * n + gn] = yacc[i][e] + bv_n;
+                else
+                    static_cast<uint16_t*>(y_out)[(int64_t)gr * n + gn] = f32_to_bf16_rne(yacc[i][e] + bv_n);
+            }
+        }
 }
 
 // Sums the `split` fp32 parts of each tile of the last round, in part order, adds the bias and
@@ -776,25 +763,23 @@ __global__ __launch_bounds__(256) void q4_tall_reduce_kernel(const float* __rest
     constexpr int kPerTile = OUT == kTpOutSwiglu ? kTpTileElems / 2 : kTpTileElems;
     const int t = blockIdx.x / (kPerTile / 256);
     int idx = (blockIdx.x % (kPerTile / 256)) * 256 + threadIdx.x;
-    if constexpr (OUT == kTpOutSwiglu) idx = ((idx >> 10) << 11) | (idx & 1023);  // j = 0
-    const int lane = idx & 63, e = (idx >> 6) & 15, j = (idx >> 10) & 1, i = (idx >> 11) & 1;
-    const int wave = idx >> 12;
+    if constexpr (OUT == kTpOutSwiglu) idx = ((idx >> 4) << 5) | (idx & 15);  // the gate's lanes
+    const int lane = idx & 63, e = (idx >> 6) & 15, i = (idx >> 10) & 3, wave = idx >> 12;
     const int tile = full_tiles + t;
-    const int gr = (tile / tiles_n) * kTpTileM + (wave >> 2) * 64 + 32 * i + 8 * (e >> 2) +
-                   4 * (lane >> 5) + (e & 3);
+    const int gr = (tile / tiles_n) * kTpTileM + 32 * i + 8 * (e >> 2) + 4 * (lane >> 5) + (e & 3);
     const float* src = partials + (size_t)t * split * kTpTileElems + idx;
     if constexpr (OUT == kTpOutSwiglu) {
-        const int gn = (tile % tiles_n) * (kTpTileN / 2) + (wave & 3) * 32 + (lane & 31);
+        const int gn = (tile % tiles_n) * (kTpTileN / 2) + wave * 16 + (lane & 15);
         if (gr >= m || gn >= n) return;
         float g = 0.0f, u = 0.0f;
         for (int q = 0; q < split; ++q) {
             g += src[(size_t)q * kTpTileElems];
-            u += src[(size_t)q * kTpTileElems + 1024];
+            u += src[(size_t)q * kTpTileElems + 16];
         }
         static_cast<uint16_t*>(y_out)[(int64_t)gr * n + gn] =
             f32_to_bf16_rne(g / (1.0f + expf(-g)) * u);
     } else {
-        const int gn = (tile % tiles_n) * kTpTileN + (wave & 3) * 64 + 32 * j + (lane & 31);
+        const int gn = (tile % tiles_n) * kTpTileN + wave * 32 + (lane & 31);
         if (gr >= m || gn >= n) return;
         float acc = 0.0f;
         for (int q = 0; q < split; ++q) acc += src[(size_t)q * kTpTileElems];
@@ -805,38 +790,38 @@ __global__ __launch_bounds__(256) void q4_tall_reduce_kernel(const float* __rest
 }
 
 // The same for kTpOutSwigluOperand: a workgroup takes four rows-of-registers (e = 4 eq .. + 3)
-// of one (row half, i) of a tile across all four wave columns, i.e. eight rows of the tile with
-// all their 128 outputs, so that it can add up their group sums: thread (wave column wq, lane)
+// of one block i of a tile across all eight waves, i.e. eight rows of the tile with
+// all their 128 outputs, so that it can add up their group sums: thread (wave, h, output of the wave)
 // sums the parts of the gate and the up product of its result in part order, applies the
 // activation and writes the bf16 value in pair order; chunk and group sums as in the product
 // kernel.  grid: 16 workgroups per tile.
 __global__ __launch_bounds__(256) void q4_tall_reduce_operand_kernel(
     const float* __restrict__ partials, void* __restrict__ y_out, int m, int n, int tiles_n,
     int full_tiles, int split, int out_pairs) {
-    __shared__ float red[4][4][8];  // [wave column][chunk of it][row of the eight]
+    __shared__ float red[16][8];  // [chunk of the group][row of the eight]
     const int t = blockIdx.x >> 4;
-    const int half = (blockIdx.x >> 3) & 1, i = (blockIdx.x >> 2) & 1, eq = blockIdx.x & 3;
-    const int wq = threadIdx.x >> 6, lane = threadIdx.x & 63, r = lane & 31, h = lane >> 5;
+    const int i = (blockIdx.x >> 2) & 3, eq = blockIdx.x & 3;
+    const int wave = threadIdx.x >> 5, h = (threadIdx.x >> 4) & 1, c = threadIdx.x & 15;
     const int tile = full_tiles + t;
     const int row0 = (tile / tiles_n) * kTpTileM, col0 = (tile % tiles_n) * (kTpTileN / 2);
-    const int gn = col0 + 32 * wq + r;
+    const int gn = col0 + 16 * wave + c;
     uint16_t* const xo = static_cast<uint16_t*>(y_out);
     float* const so = reinterpret_cast<float*>(static_cast<char*>(y_out) + tall_sums_offset(m, n));
-    const float* src = partials + (size_t)t * split * kTpTileElems +
-                       (size_t)(half * 4 + wq) * 4096 + (size_t)i * 2048 + lane;
+    const float* src = partials + (size_t)t * split * kTpTileElems + (size_t)wave * 4096 +
+                       (size_t)i * 1024 + h * 32 + c;
 #pragma unroll
     for (int el = 0; el < 4; ++el) {
         const int e = 4 * eq + el;
         float g = 0.0f, u = 0.0f;
         for (int q = 0; q < split; ++q) {
             g += src[(size_t)q * kTpTileElems + e * 64];
-            u += src[(size_t)q * kTpTileElems + 1024 + e * 64];
+            u += src[(size_t)q * kTpTileElems + e * 64 + 16];
         }
-        const int row = 64 * half + 32 * i + 8 * (e >> 2) + 4 * h + (e & 3);
+        const int row = 32 * i + 8 * (e >> 2) + 4 * h + (e & 3);
         const uint16_t b = f32_to_bf16_rne(g / (1.0f + expf(-g)) * u);
         xo[(int64_t)(row0 + row) * n + (gn & ~7) + tp_pair_slot(gn & 7)] = b;
         const float cs = tp_chunk_sum_across_lanes(__uint_as_float((unsigned)b << 16));
-        if ((r & 7) == 0) red[wq][r >> 3][2 * el + h] = cs;
+        if ((c & 7) == 0) red[2 * wave + (c >> 3)][2 * el + h] = cs;
     }
     __syncthreads();
     if (threadIdx.x < 8) {
@@ -845,8 +830,8 @@ __global__ __launch_bounds__(256) void q4_tall_reduce_operand_kernel(
 #pragma unroll
         for (int a = 0; a < 4; ++a)
 #pragma unroll
-            for (int c = 0; c < 4; ++c) cs[a][c] = red[a][c][threadIdx.x];
-        const int row = 64 * half + 32 * i + 8 * (e >> 2) + 4 * hh + (e & 3);
+            for (int b = 0; b < 4; ++b) cs[a][b] = red[4 * a + b][threadIdx.x];
+        const int row = 32 * i + 8 * (e >> 2) + 4 * hh + (e & 3);
         so[tall_sum_index(row0 + row, col0 >> 7, n, out_pairs)] = tp_group_sum(cs);
     }
 }
