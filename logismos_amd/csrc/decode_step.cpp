@@ -17,14 +17,13 @@ constexpr int kChunkRows = 32;  // rows the prepared layout and the decode GEMMs
 constexpr int kTallRows = 97;
 
 struct Workspace {
-    char* xn;        // prepared activations of width hidden, one per 32-row chunk (input of qkv /
-                     // gate_up; a chunk's buffer carries its normed rows from the end of one
-                     // layer to the start of the next)
-    char* qkv;       // f32  [Jqkv][rows][(hq+2hkv)*d]   split-K parts of one chunk
+    char* xn;        // prepared activations of width hidden, one buffer per 32-row chunk (input of
+                     // qkv / gate_up; they carry the normed rows from the end of one layer to
+                     // the start of the next)
+    char* qkv;       // f32  [Jqkv][rows][(hq+2hkv)*d]   split-K parts of a pass
     char* q;         // f16  [T][hq*d]
-    char* attn_b;    // prepared activations of width hq*d of one chunk (input of the o projection)
-    char* attn_out;  // bf16 [T][hq*d]: attention output of a step that is not one chunk of
-                     // decode rows (those go straight into attn_b)
+    char* attn_b;    // prepared activations of width hq*d (input of the o projection)
+    char* attn_out;  // bf16 [T][hq*d]: attention output where it does not go straight into attn_b
     char* proj;      // f32  [max(Jo,Jdown)][rows][hidden]  (o projection, then down projection)
     char* gate_up;   // f32  [Jgu][rows][2*inter]
     char* act;       // prepared activations of width inter (input of the down projection)
@@ -45,7 +44,7 @@ struct Workspace {
     char* last_xn;    // prepared activations of one chunk of them
     bool tall;
     size_t xn_stride;
-    int chunks, rows;  // rows: rows of a full chunk (= T when there is one chunk)
+    int chunks;        // of 32 rows
     int j_qkv, j_o, j_gu, j_down;
     size_t total;
 };
@@ -94,10 +93,9 @@ Workspace carve(const logismos_decode_config_t& c, int num_seqs, int t, int num_
         return w;
     }
     w.chunks = (t + kChunkRows - 1) / kChunkRows;
-    w.rows = t < kChunkRows ? t : kChunkRows;
-    const int b = w.rows;
+    const int b = t < kChunkRows ? t : kChunkRows;
     // the number of K parts depends on the batch only through its tile height (<= 16 rows or
-    // more), so a ragged last chunk of a long step may plan fewer parts than a full one: size
+    // more), so a ragged last chunk taken by itself may plan fewer parts than a full one: size
     // for the larger and let every launch use its own count
     auto parts = [&](int n, int k) {
         int j = logismos_qgemm_q4g128_splitk_xprep_parts(b, n, k);
@@ -110,15 +108,20 @@ Workspace carve(const logismos_decode_config_t& c, int num_seqs, int t, int num_
     w.j_gu = parts(2 * c.intermediate, c.hidden);
     w.j_down = parts(c.hidden, c.intermediate);
     const int j_proj = w.j_o > w.j_down ? w.j_o : w.j_down;
-    w.xn_stride = align256(logismos_q4_xprep_bytes(b, c.hidden));
-    w.xn = take(w.xn_stride * w.chunks);
-    w.qkv = take((size_t)w.j_qkv * b * (qd + 2 * kvd) * 4);
+    // prepared activations of all rows: one buffer, or one per chunk of 32
+    auto xprep = [&](int k) {
+        return w.chunks == 1 ? align256(logismos_q4_xprep_bytes(b, k))
+                             : w.chunks * lg::xprep_rows_stride(k);
+    };
+    w.xn_stride = lg::xprep_rows_stride(c.hidden);
+    w.xn = take(xprep(c.hidden));
+    w.qkv = take((size_t)w.j_qkv * t * (qd + 2 * kvd) * 4);
     w.q = take((size_t)t * qd * 2);
-    w.attn_b = take(logismos_q4_xprep_bytes(b, (int)qd));
+    w.attn_b = take(xprep((int)qd));
     w.attn_out = take((size_t)t * qd * 2);
-    w.proj = take((size_t)j_proj * b * c.hidden * 4);
-    w.gate_up = take((size_t)w.j_gu * b * 2 * c.intermediate * 4);
-    w.act = take(logismos_q4_xprep_bytes(b, c.intermediate));
+    w.proj = take((size_t)j_proj * t * c.hidden * 4);
+    w.gate_up = take((size_t)w.j_gu * t * 2 * c.intermediate * 4);
+    w.act = take(xprep(c.intermediate));
     w.attn_ws =
         take(logismos_paged_attn_workspace_bytes(num_seqs, c.num_q_heads, c.head_dim, num_splits));
     if (c.vocab > 0) {
@@ -214,6 +217,20 @@ bool few_rows(const logismos_decode_config_t& c, const logismos_decode_layer_t* 
                                            qd + 2 * c.num_kv_heads * c.head_dim, W->scale, W->zero))
                 return false;
     return true;
+}
+
+// Whether the last chunk of a step of 33 to 96 rows goes through the projections by itself.  Tiles of
+// 16 rows (and other K parts) add up in another order than the 32-row chunks beside them.  In front
+// of 3-bit K/V rows a last bit flips whole codes: over chunks that read mostly their own new rows another
+// order of the same sums moves the hidden state of 36 layers by up to 19 %, over decode rows, which
+// read encoded rows that are there already, by 1.8 %.
+bool split_last_chunk(const logismos_decode_config_t& c, int max_q, int last_rows) {
+    if (!c.kv_turbo3 || max_q == 1) return false;
+    const int qd = c.num_q_heads * c.head_dim, kvd = c.num_kv_heads * c.head_dim;
+    return !(lg::qgemm_q4_splitk_same_sums(last_rows, qd + 2 * kvd, c.hidden) &&
+             lg::qgemm_q4_splitk_same_sums(last_rows, c.hidden, qd) &&
+             lg::qgemm_q4_splitk_same_sums(last_rows, 2 * c.intermediate, c.hidden) &&
+             lg::qgemm_q4_splitk_same_sums(last_rows, c.hidden, c.intermediate));
 }
 
 #define LG_TRY(call)                                  \
@@ -354,7 +371,10 @@ extern "C" logismos_status_t logismos_launch_decode_step(const logismos_decode_c
     const int kvd = c.num_kv_heads * c.head_dim;
     const int width = qd + 2 * kvd;
     const float scale = 1.0f / sqrtf((float)c.head_dim);
-    const bool one_chunk = w.chunks == 1;
+    // Steps of up to 96 rows: every launch takes all rows, except where a last chunk of few rows by
+    // itself would add up in another order and that order matters (see below).
+    const int last_rows = t - (w.chunks - 1) * kChunkRows;
+    const bool one_pass = !w.tall && (w.chunks == 1 || !split_last_chunk(c, max_q, last_rows));
     // tokens for last rows: the normed rows of the whole batch, in the caller's buffer or in
     // the workspace, are gathered afterwards
     char* const norm_dst = batch->out_bf16 ? static_cast<char*>(batch->out_bf16)
@@ -378,12 +398,8 @@ extern "C" logismos_status_t logismos_launch_decode_step(const logismos_decode_c
     };
     // attention writes the o projection's input (the prepared layout's groups of 128 are whole
     // heads only at head_dim 128)
-    const bool direct = one_chunk && max_q == 1 && c.head_dim == 128;
+    const bool direct = one_pass && c.head_dim == 128;
     float* const h = static_cast<float*>(batch->hidden_f32);
-    auto rows_of = [&](int ch) {
-        const int r0 = ch * kChunkRows;
-        return t - r0 < kChunkRows ? t - r0 : kChunkRows;
-    };
 
     if (tokens_in)
         LG_TRY(logismos_launch_embed_lookup_bf16(batch->embed_table_bf16, batch->token_ids,
@@ -519,23 +535,32 @@ extern "C" logismos_status_t logismos_launch_decode_step(const logismos_decode_c
     if (few_rows(c, layers, t)) {
         LG_TRY(few_rows_layers(c, layers, batch, w, t, max_q, direct, stream));
     } else {
+        // All rows in one launch of every operator, the projections in chunks of 32 side by side (48
+        // rows of the 4096-wide layers, chunk after chunk: 19 launches a layer, 117 us beside the
+        // attention; 10 launches now).  Two passes where the last chunk stays by itself.
+        hipStream_t st = static_cast<hipStream_t>(stream);
+        struct {
+            int row0, rows;
+            char* xn;
+        } passes[2] = {{0, one_pass ? t : t - last_rows, w.xn},
+                       {t - last_rows, last_rows, w.xn + (w.chunks - 1) * w.xn_stride}};
+        const int num_passes = one_pass ? 1 : 2;
         // The normed input of a layer's first half is produced where the residual stream is
-        // completed: before layer 0 here, afterwards by the add + norm that folds a chunk's down
+        // completed: before layer 0 here, afterwards by the add + norm that folds a pass's down
         // projection into h (with the NEXT layer's gains).
-        for (int ch = 0; ch < w.chunks; ++ch)
-            LG_TRY(logismos_launch_add_rms_norm_f32p_xprep(
-                h + (int64_t)ch * kChunkRows * c.hidden, nullptr, 0, layers[0].norm1_w_f32,
-                w.xn + ch * w.xn_stride, rows_of(ch), c.hidden, c.rms_eps, stream));
+        for (int i = 0; i < num_passes; ++i)
+            LG_TRY(lg::add_rms_norm_xprep_rows(h + (int64_t)passes[i].row0 * c.hidden, nullptr, 0,
+                                               layers[0].norm1_w_f32, passes[i].xn, passes[i].rows,
+                                               c.hidden, c.rms_eps, st));
         for (int l = 0; l < c.num_layers; ++l) {
             const logismos_decode_layer_t& L = layers[l];
             const bool last_layer = l + 1 == c.num_layers;
-            // ---- first half, chunk by chunk: q/k/v projection, RoPE, K/V rows into the pools
-            for (int ch = 0; ch < w.chunks; ++ch) {
-                const int r0 = ch * kChunkRows, rows = rows_of(ch);
-                LG_TRY(logismos_launch_qgemm_q4g128_f32_splitk_xprep(
-                    w.xn + ch * w.xn_stride, L.qkv.qw, L.qkv.scale, L.qkv.zero, w.qkv, rows, width,
-                    c.hidden, stream));
-                const int j = logismos_qgemm_q4g128_splitk_xprep_parts(rows, width, c.hidden);
+            // ---- first half: q/k/v projection, RoPE, K/V rows into the pools
+            for (int i = 0; i < num_passes; ++i) {
+                const int r0 = passes[i].row0, rows = passes[i].rows;
+                LG_TRY(lg::qgemm_q4_splitk_rows(passes[i].xn, L.qkv.qw, L.qkv.scale, L.qkv.zero, w.qkv,
+                                                rows, width, c.hidden, st));
+                const int j = lg::qgemm_q4_splitk_rows_parts(rows, width, c.hidden);
                 const auto rope_kv_write = c.kv_turbo3 ? logismos_launch_rope_kv_write_f32p_turbo3_bias
                                                        : logismos_launch_rope_kv_write_f32p_bias;
                 LG_TRY(rope_kv_write(w.qkv, j, L.qkv_bias_f32, batch->positions + r0,
@@ -544,48 +569,44 @@ extern "C" logismos_status_t logismos_launch_decode_step(const logismos_decode_c
                                      L.v_pool_f16, rows, c.num_q_heads, c.num_kv_heads, c.head_dim,
                                      c.max_pos, stream));
             }
-            // ---- attention over the whole ragged batch.  One chunk of decode rows: the result
-            // goes straight into the prepared layout of the o projection; otherwise bf16 rows that
-            // each chunk prepares for itself.
+            // ---- attention over the whole ragged batch.  One pass: the result goes straight into
+            // the prepared layout of the o projection; otherwise bf16 rows that each pass prepares
+            // for itself.
             LG_TRY(lg::paged_attn_launch(
                 w.q, L.k_pool_f16, L.v_pool_f16, batch->block_tables, batch->cu_seqlens,
                 batch->context_lens, direct ? w.attn_b : w.attn_out,
                 w.attn_ws, num_seqs, t, max_q, c.num_q_heads, c.num_kv_heads, c.head_dim, c.block_size,
                 c.max_blocks_per_seq, batch->num_splits, scale, 1, LOGISMOS_ATTN_PHASE_ALL,
                 direct ? 2 : 1, c.kv_turbo3 ? 1 : 0, stream));
-            // ---- second half, chunk by chunk
-            for (int ch = 0; ch < w.chunks; ++ch) {
-                const int r0 = ch * kChunkRows, rows = rows_of(ch);
-                float* hc = h + (int64_t)r0 * c.hidden;
+            // ---- second half
+            for (int i = 0; i < num_passes; ++i) {
+                const int r0 = passes[i].row0, rows = passes[i].rows;
+                char* const xn = passes[i].xn;
+                float* hp = h + (int64_t)r0 * c.hidden;
                 if (!direct)
-                    LG_TRY(logismos_launch_q4_prepare_x_bf16(w.attn_out + (size_t)r0 * qd * 2, w.attn_b,
-                                                             rows, qd, stream));
-                LG_TRY(logismos_launch_qgemm_q4g128_f32_splitk_xprep(
-                    w.attn_b, L.o.qw, L.o.scale, L.o.zero, w.proj, rows, c.hidden, qd, stream));
-                LG_TRY(logismos_launch_add_rms_norm_f32p_xprep(
-                    hc, w.proj, logismos_qgemm_q4g128_splitk_xprep_parts(rows, c.hidden, qd),
-                    L.norm2_w_f32, w.xn + ch * w.xn_stride, rows, c.hidden, c.rms_eps, stream));
-                LG_TRY(logismos_launch_qgemm_q4g128_f32_splitk_xprep(
-                    w.xn + ch * w.xn_stride, L.gate_up.qw, L.gate_up.scale, L.gate_up.zero, w.gate_up,
-                    rows, 2 * c.intermediate, c.hidden, stream));
-                LG_TRY(logismos_launch_silu_mul_f32p_xprep(
-                    w.gate_up,
-                    logismos_qgemm_q4g128_splitk_xprep_parts(rows, 2 * c.intermediate, c.hidden), w.act,
-                    rows, c.intermediate, stream));
-                LG_TRY(logismos_launch_qgemm_q4g128_f32_splitk_xprep(
-                    w.act, L.down.qw, L.down.scale, L.down.zero, w.proj, rows, c.hidden, c.intermediate,
-                    stream));
-                const int j_down =
-                    logismos_qgemm_q4g128_splitk_xprep_parts(rows, c.hidden, c.intermediate);
+                    LG_TRY(lg::q4_prepare_x_rows(w.attn_out + (size_t)r0 * qd * 2, w.attn_b, rows, qd,
+                                                 st));
+                LG_TRY(lg::qgemm_q4_splitk_rows(w.attn_b, L.o.qw, L.o.scale, L.o.zero, w.proj, rows,
+                                                c.hidden, qd, st));
+                LG_TRY(lg::add_rms_norm_xprep_rows(
+                    hp, w.proj, lg::qgemm_q4_splitk_rows_parts(rows, c.hidden, qd), L.norm2_w_f32, xn,
+                    rows, c.hidden, c.rms_eps, st));
+                LG_TRY(lg::qgemm_q4_splitk_rows(xn, L.gate_up.qw, L.gate_up.scale, L.gate_up.zero,
+                                                w.gate_up, rows, 2 * c.intermediate, c.hidden, st));
+                LG_TRY(lg::silu_mul_xprep_rows(
+                    w.gate_up, lg::qgemm_q4_splitk_rows_parts(rows, 2 * c.intermediate, c.hidden),
+                    w.act, rows, c.intermediate, st));
+                LG_TRY(lg::qgemm_q4_splitk_rows(w.act, L.down.qw, L.down.scale, L.down.zero, w.proj,
+                                                rows, c.hidden, c.intermediate, st));
+                const int j_down = lg::qgemm_q4_splitk_rows_parts(rows, c.hidden, c.intermediate);
                 if (!last_layer) {
                     // fold the down projection into h and norm for the next layer's first half
-                    LG_TRY(logismos_launch_add_rms_norm_f32p_xprep(
-                        hc, w.proj, j_down, layers[l + 1].norm1_w_f32, w.xn + ch * w.xn_stride, rows,
-                        c.hidden, c.rms_eps, stream));
-                } else if (!one_chunk) {
-                    // last layer of a multi-chunk step: the final norm of this chunk's rows
+                    LG_TRY(lg::add_rms_norm_xprep_rows(hp, w.proj, j_down, layers[l + 1].norm1_w_f32,
+                                                       xn, rows, c.hidden, c.rms_eps, st));
+                } else if (!one_pass) {
+                    // last layer of two passes: the final norm of this pass's rows
                     LG_TRY(logismos_launch_add_rms_norm_f32p(
-                        hc, w.proj, j_down, batch->final_norm_w_f32,
+                        hp, w.proj, j_down, batch->final_norm_w_f32,
                         norm_dst + (size_t)r0 * c.hidden * 2, rows, c.hidden, c.rms_eps, stream));
                 } else {
                     res_parts = j_down;
@@ -593,7 +614,7 @@ extern "C" logismos_status_t logismos_launch_decode_step(const logismos_decode_c
             }
         }
     }
-    if (!one_chunk) return last_only ? project_last_rows() : 0;
+    if (!one_pass) return last_only ? project_last_rows() : 0;
     if (last_only) {
         LG_TRY(logismos_launch_add_rms_norm_f32p(batch->hidden_f32, w.proj, res_parts,
                                                  batch->final_norm_w_f32, norm_dst, t, c.hidden,

@@ -59,6 +59,24 @@ hipError_t qgemm_q4_regx_launch(const RegxPlan& plan, const void* xprep, const v
                                 const void* scale, const void* zero, void* part, int b, int n,
                                 int k, hipStream_t stream);
 
+// The prepared layout and its operators for any number of rows (q4_common.hpp: buffers of 32 rows
+// one behind the other): what the exported entry points of the same names do for up to 32.  The
+// products come as [part][rows][n].
+hipError_t qgemm_q4_splitk_rows(const void* x_prepared, const void* qw, const void* scale,
+                                const void* zero, void* parts_f32, int rows, int n, int k,
+                                hipStream_t stream);
+int qgemm_q4_splitk_rows_parts(int rows, int n, int k);
+size_t xprep_rows_stride(int k);  // bytes between two buffers of 32 rows
+// Whether a chunk of `rows` rows by itself adds up in the same order as one of 32.
+bool qgemm_q4_splitk_same_sums(int rows, int n, int k);
+hipError_t q4_prepare_x_rows(const void* x_bf16, void* x_prepared, int rows, int k,
+                             hipStream_t stream);
+hipError_t add_rms_norm_xprep_rows(void* h_f32, const void* parts_f32, int num_parts,
+                                   const void* w_f32, void* x_prepared, int rows, int n, float eps,
+                                   hipStream_t stream);
+hipError_t silu_mul_xprep_rows(const void* parts_f32, int num_parts, void* x_prepared, int rows,
+                               int inter, hipStream_t stream);
+
 // Q4G128 GEMM for a tall x (qgemm_q4_tall.hip): 128 x 128 output tiles, x through LDS, the
 // matrix cores as the bound.  x bf16 [b][K], y bf16 [b][N], bias fp32 [N] or null.
 bool qgemm_q4_tall_applies(int b, int n, int k);

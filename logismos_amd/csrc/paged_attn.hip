@@ -294,15 +294,12 @@ __device__ __forceinline__ void attn_write_zero_row(const AttnParams& p, int t, 
     if (c >= G) return;
     half8_t z = {0, 0, 0, 0, 0, 0, 0, 0};
     if (p.out_bf16 == 2) {
-        const int bp = xprep_bp(p.out_rows);
+        const XprepRow at = xprep_row(p.out, p.out_rows, p.hq * kHeadDim, t);
         const int head = kvh * G + c;
 #pragma unroll
         for (int j = 0; j < 4; ++j)
-            reinterpret_cast<half8_t*>(p.out)[(int64_t)(head * 16 + tg + 4 * j) * bp + t] = z;
-        if (tg == 0)
-            reinterpret_cast<float*>(reinterpret_cast<char*>(p.out) +
-                                     xprep_xg_offset(p.out_rows, p.hq * kHeadDim))[(int64_t)head * bp + t] =
-                0.0f;
+            at.xp[(int64_t)(head * 16 + tg + 4 * j) * at.bp] = __builtin_bit_cast(uint4_t, z);
+        if (tg == 0) at.xg[(int64_t)head * at.bp] = 0.0f;
     } else {
         _Float16* o = p.out + ((int64_t)t * p.hq + kvh * G + c) * kHeadDim;
 #pragma unroll
@@ -711,12 +708,9 @@ __device__ __forceinline__ void attn_partition(const AttnParams& p, int s, int t
             if (p.out_bf16 == 2) {
                 // a head is one group of 128: the 16 lanes of this row hold its 16 chunks
                 const float gs = row16_sum(sum8_bf16(o));
-                const int bp = xprep_bp(p.out_rows);
-                reinterpret_cast<uint4_t*>(p.out)[(int64_t)(head * 16 + c) * bp + t] = pair_order(o);
-                if (c == 0)
-                    reinterpret_cast<float*>(
-                        reinterpret_cast<char*>(p.out) +
-                        xprep_xg_offset(p.out_rows, p.hq * kHeadDim))[(int64_t)head * bp + t] = gs;
+                const XprepRow at = xprep_row(p.out, p.out_rows, p.hq * kHeadDim, t);
+                at.xp[(int64_t)(head * 16 + c) * at.bp] = pair_order(o);
+                if (c == 0) at.xg[(int64_t)head * at.bp] = gs;
             } else {
                 *reinterpret_cast<uint4_t*>(p.out + ((int64_t)t * p.hq + head) * kHeadDim + 8 * c) = o;
             }
@@ -1013,12 +1007,9 @@ __global__ __launch_bounds__(256) void paged_attn_merge_kernel(const AttnParams 
             const int c = threadIdx.x;
             const uint4_t o = reinterpret_cast<const uint4_t*>(sout)[c];
             const float gs = row16_sum(sum8_bf16(o));
-            const int bp = xprep_bp(p.out_rows);
-            reinterpret_cast<uint4_t*>(p.out)[(int64_t)(h * 16 + c) * bp + t0] = pair_order(o);
-            if (c == 0)
-                reinterpret_cast<float*>(
-                    reinterpret_cast<char*>(p.out) +
-                    xprep_xg_offset(p.out_rows, p.hq * kHeadDim))[(int64_t)h * bp + t0] = gs;
+            const XprepRow at = xprep_row(p.out, p.out_rows, p.hq * kHeadDim, t0);
+            at.xp[(int64_t)(h * 16 + c) * at.bp] = pair_order(o);
+            if (c == 0) at.xg[(int64_t)h * at.bp] = gs;
         }
     }
 }
@@ -1551,14 +1542,9 @@ __global__ __launch_bounds__(64 * kPfWaves) void paged_attn_prefill_kernel(const
             if (p.out_bf16 == 2) {
                 const float gs = row16_sum(sum8_bf16(o));
                 if (valid) {
-                    const int bp = xprep_bp(p.out_rows);
-                    reinterpret_cast<uint4_t*>(p.out)[(int64_t)(head * 16 + chunk) * bp + t] =
-                        pair_order(o);
-                    if (chunk == 0)
-                        reinterpret_cast<float*>(
-                            reinterpret_cast<char*>(p.out) +
-                            xprep_xg_offset(p.out_rows, p.hq * kHeadDim))[(int64_t)head * bp + t] =
-                            gs;
+                    const XprepRow at = xprep_row(p.out, p.out_rows, p.hq * kHeadDim, t);
+                    at.xp[(int64_t)(head * 16 + chunk) * at.bp] = pair_order(o);
+                    if (chunk == 0) at.xg[(int64_t)head * at.bp] = gs;
                 }
             } else if (valid) {
                 *reinterpret_cast<uint4_t*>(p.out + ((int64_t)t * p.hq + head) * kHeadDim +

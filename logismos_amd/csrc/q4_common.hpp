@@ -54,6 +54,30 @@ __host__ __device__ inline size_t xprep_bytes(int b, int k) {
     return xprep_xg_offset(b, k) + (size_t)(k / 128) * xprep_bp(b) * 4;
 }
 
+// More than 32 rows: one such buffer of 32 rows behind the other, xprep_chunk_stride bytes apart
+// (BP = 32 for the last one too).
+constexpr int kXprepChunkRows = 32;
+__host__ __device__ inline size_t xprep_chunk_stride(int k) {
+    return (xprep_bytes(kXprepChunkRows, k) + 255) & ~(size_t)255;
+}
+// Where row t of `rows` rows lies: chunk c of it is xp[c * bp], group g's sum xg[g * bp].
+struct XprepRow {
+    uint4_t* xp;
+    float* xg;
+    int bp;
+};
+__device__ __forceinline__ XprepRow xprep_row(void* base, int rows, int k, int64_t t) {
+    char* b = static_cast<char*>(base);
+    int bp = xprep_bp(rows);
+    if (rows > kXprepChunkRows) {
+        b += (size_t)(t / kXprepChunkRows) * xprep_chunk_stride(k);
+        t %= kXprepChunkRows;
+        bp = kXprepChunkRows;
+    }
+    return {reinterpret_cast<uint4_t*>(b) + t,
+            reinterpret_cast<float*>(b + (size_t)(k / 8) * bp * 16) + t, bp};
+}
+
 // Workspace of the Q4G128 GEMM for many rows (qgemm_q4_tallp.hip), first part: what its first
 // pass -- or the operator that produces x -- writes.
 //   xp  bf16  [m_pad][K]  x in pair order per 16-byte chunk, rows >= m zero, m_pad = m rounded

@@ -38,6 +38,8 @@
 
 #include <hip/hip_fp16.h>
 
+#include <algorithm>
+
 namespace lg {
 
 constexpr int kRegxWaves = 8;
@@ -389,6 +391,9 @@ __global__ __launch_bounds__(64 * kRegxWaves) void qgemm_q4g128_regx_kernel(
 // 2 * GS ring reads, 8 * GS MFMAs into one 16-register accumulator per group, GS / 2 fp32
 // MFMAs (32 x 32 x 2) for the zero-point term.  The first two tiles of a batch of three go to
 // the exchange buffers at once, the third waits in registers.
+// More than 32 rows: blockIdx.z is the chunk of 32, x_stride the distance of two chunks' x (in
+// 16-byte words).  The chunks of a column of tiles run on one XCD side by side and read its weights
+// through that L2.
 __host__ __device__ constexpr int regx32_tile_bytes(int gs) { return 32 * gs * 64 + 32 * gs * 4; }
 __host__ __device__ constexpr int regx32_lds_bytes(int gs, int ring) {
     return kRegxWaves * ring * regx32_tile_bytes(gs) + 2 * kRegxWaves * 4096;
@@ -400,7 +405,8 @@ template <int GS, bool PLAIN>
 __global__ __launch_bounds__(64 * kRegxWaves) void qgemm_q4g128_regx32_kernel(
     const uint4_t* __restrict__ xprep, const uint8_t* __restrict__ qw,
     const __half* __restrict__ scale, const __half* __restrict__ zero, float* __restrict__ part,
-    int b, int n, int k, int tiles_per_worker, int ring, const float* __restrict__ bias) {
+    int total_rows, int n, int k, int tiles_per_worker, int ring, int x_stride,
+    const float* __restrict__ bias) {
     static_assert(GS == 2 || GS == 4, "slices of 2 or 4 groups");
     constexpr int BP = 32;
     constexpr int W = kRegxWaves;
@@ -421,6 +427,8 @@ __global__ __launch_bounds__(64 * kRegxWaves) void qgemm_q4g128_regx32_kernel(
     const int tiles = (n + 31) >> 5;
     const int t_begin = blockIdx.x * tiles_per_worker;
     if (t_begin >= tiles) return;
+    const int row0 = 32 * blockIdx.z, b = min(total_rows - row0, 32);
+    xprep += (size_t)blockIdx.z * (unsigned)x_stride;
     const int my_tiles = min(tiles, t_begin + tiles_per_worker) - t_begin;
 
     const int lane = threadIdx.x & 63;
@@ -492,7 +500,7 @@ __global__ __launch_bounds__(64 * kRegxWaves) void qgemm_q4g128_regx32_kernel(
                 for (int d = 0; d < 4; ++d)
                     xr[i][h2][d] = xprep[(16 * (g0 + i) + 8 * h2 + 4 * kh + d) * BP + r32];
         const float* xg_src = reinterpret_cast<const float*>(
-            reinterpret_cast<const char*>(xprep) + xprep_xg_offset(b, k));
+            reinterpret_cast<const char*>(xprep) + (size_t)(k / 8) * BP * 16);
 #pragma unroll
         for (int e = 0; e < GS / 2; ++e) xs[e] = xg_src[(g0 + 2 * e + kh) * BP + r32];
     }
@@ -543,7 +551,7 @@ __global__ __launch_bounds__(64 * kRegxWaves) void qgemm_q4g128_regx32_kernel(
     const int m0 = 2 * (2 * wave + kh);
     const unsigned red_rd = red_base + (unsigned)((m0 >> 3) * 1024 + (((m0 >> 2) & 1) * 32 + r32) * 16 + (m0 & 3) * 4);
 
-    float* pbase = part + (int64_t)j * b * n;
+    float* pbase = part + ((int64_t)j * total_rows + row0) * n;
 
     int slot = 0;
     for (int s0 = 0; s0 < my_tiles; s0 += TM) {
@@ -702,11 +710,13 @@ static hipError_t launch_regx32(const void* xprep, const void* qw, const void* s
         reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,
         160 * 1024);
     if (opt != hipSuccess) return opt;
-    dim3 grid((tiles + tpw - 1) / tpw, (k / 128) / (kRegxWaves * GS));
+    dim3 grid((tiles + tpw - 1) / tpw, (k / 128) / (kRegxWaves * GS), (b + 31) / 32);
+    // (the chunks of a column on one XCD: workgroups go round the eight in the order of their ids)
+    if (grid.z > 1) grid.x = (grid.x + 7) / 8 * 8;
     kern<<<grid, dim3(64 * kRegxWaves), lds, stream>>>(
         static_cast<const uint4_t*>(xprep), static_cast<const uint8_t*>(qw),
         static_cast<const __half*>(scale), static_cast<const __half*>(zero),
-        static_cast<float*>(part), b, n, k, tpw, ring, bias);
+        static_cast<float*>(part), b, n, k, tpw, ring, (int)(xprep_chunk_stride(k) / 16), bias);
     return hipGetLastError();
 }
 
@@ -715,7 +725,7 @@ static hipError_t qgemm_q4_regx32_launch(const void* xprep, const void* qw, cons
                                          int k, int gs, int tpw, int ring, bool plain,
                                          hipStream_t stream) {
     if (gs != 2 && gs != 4) return hipErrorInvalidValue;
-    if (b <= 16 || b > 32) return hipErrorInvalidValue;
+    if (b <= 16 || (plain && b > 32)) return hipErrorInvalidValue;
     if ((k / 128) % (kRegxWaves * gs) != 0 || tpw < 1 || ring < 1 || ring > kRegxMaxRing)
         return hipErrorInvalidValue;
     if (regx32_lds_bytes(gs, ring) > 160 * 1024) return hipErrorInvalidValue;
@@ -769,10 +779,12 @@ static hipError_t qgemm_q4_regx16_launch(const void* xprep, const void* qw, cons
 // of at least 1024 rows.  Measured at batch 32 on 24576 x 4096, 4096 x 12288, 6144 x 4096
 // and 4096 x 4096: slices of two groups win up to K = 4096, four beyond; a ring deeper than
 // one tile (two for the 16-row kernel's short slices) gains nothing.
+// More than 32 rows: the plan of 32 with every chunk on its share of the compute units.
 RegxPlan regx_plan(int b, int n, int k) {
     RegxPlan p{0, 0, 0, 0, 0};
     const int groups = k / 128;
-    if (b < 3 || b > 32 || n < 1024 || k % 128 != 0) return p;
+    const int chunks = (b + 31) / 32;
+    if (b < 3 || n < 1024 || k % 128 != 0) return p;
     int gs = 0;
     if (k <= 4096 && groups % (kRegxWaves * 2) == 0) gs = 2;
     else if (groups % (kRegxWaves * 4) == 0) gs = 4;
@@ -783,7 +795,7 @@ RegxPlan regx_plan(int b, int n, int k) {
     p.rows = b <= 16 ? 16 : 32;
     p.ring = (p.rows == 16 && gs == 2) ? 2 : 1;
     const int tiles = (n + p.rows - 1) / p.rows;
-    const int columns = device_cu_count() / p.parts > 0 ? device_cu_count() / p.parts : 1;
+    const int columns = std::max(1, device_cu_count() / (p.parts * chunks));
     p.tpw = (tiles + columns - 1) / columns;
     return p;
 }

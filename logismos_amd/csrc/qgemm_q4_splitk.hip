@@ -40,17 +40,21 @@ template <int BT, int GP, int TW, bool PREP>
 __global__ __launch_bounds__(kSplitkThreads) void qgemm_q4g128_splitk_kernel(
     const uint16_t* __restrict__ x, const uint8_t* __restrict__ qw,
     const __half* __restrict__ scale, const __half* __restrict__ zero, float* __restrict__ part,
-    int b, int n, int k) {
+    int total_rows, int n, int k, int x_stride) {
     extern __shared__ uint4_t lds[];
     constexpr int BP = BT * 16;
     // xl: PREP ? [GP*16 chunks][BP] (the prepared layout itself) : [BP][QS], QS == 1 (mod 16)
     constexpr int QS = GP * 16 + 1;
     constexpr int ROWS = kSplitkWaves * TW * 16;
     const int groups = k >> 7;
+    // (prepared x of more than 32 rows: blockIdx.z is the chunk of 32)
+    const int chunk0 = 32 * blockIdx.z, b = min(total_rows - chunk0, 32);
+    if constexpr (PREP) x += (size_t)blockIdx.z * (unsigned)x_stride * 8;
     const int j = blockIdx.y;
     const int g0 = j * GP;
     const int gcount = min(GP, groups - g0);
     const int64_t row0 = (int64_t)blockIdx.x * ROWS;
+    if (row0 >= n) return;  // (a padded grid)
     const int rows_here = (int)min((int64_t)ROWS, (int64_t)n - row0);
 
     uint4_t* xl = lds;                                      // [BP][QS]
@@ -88,7 +92,7 @@ __global__ __launch_bounds__(kSplitkThreads) void qgemm_q4g128_splitk_kernel(
     if constexpr (PREP) {
         static_assert(GP * BP <= kSplitkThreads, "one group sum per thread");
         const float* xg_src = reinterpret_cast<const float*>(
-            reinterpret_cast<const char*>(x) + xprep_xg_offset(b, k));
+            reinterpret_cast<const char*>(x) + (size_t)(k / 8) * BP * 16);
         const int t = (int)threadIdx.x < gcount * BP ? (int)threadIdx.x : 0;
         xgd = xg_src[(int64_t)g0 * BP + t];
     }
@@ -202,7 +206,7 @@ __global__ __launch_bounds__(kSplitkThreads) void qgemm_q4g128_splitk_kernel(
             __builtin_amdgcn_sched_barrier(0);
         }
         if (r < rows_here) {
-            float* pbase = part + (int64_t)j * b * n + row0;  // uniform
+            float* pbase = part + ((int64_t)j * total_rows + chunk0) * n + row0;  // uniform
 #pragma unroll
             for (int bt = 0; bt < BT; ++bt)
 #pragma unroll
@@ -278,11 +282,12 @@ static hipError_t launch_splitk(const void* x, const void* qw, const void* scale
             160 * 1024 - 1024);
         if (opt != hipSuccess) return opt;
     }
-    dim3 grid((tiles + kSplitkWaves * TW - 1) / (kSplitkWaves * TW), plan.parts);
+    dim3 grid((tiles + kSplitkWaves * TW - 1) / (kSplitkWaves * TW), plan.parts, (b + 31) / 32);
+    if (grid.z > 1) grid.x = (grid.x + 7) / 8 * 8;  // (the chunks of a column on one XCD)
     kern<<<grid, dim3(kSplitkThreads), lds, stream>>>(
         static_cast<const uint16_t*>(x), static_cast<const uint8_t*>(qw),
         static_cast<const __half*>(scale), static_cast<const __half*>(zero),
-        static_cast<float*>(part), b, n, k);
+        static_cast<float*>(part), b, n, k, (int)(xprep_chunk_stride(k) / 16));
     return hipGetLastError();
 }
 
@@ -322,12 +327,13 @@ static logismos_status_t splitk_dispatch(const void* x, bool prepared, const voi
                                          const void* scale_f16, const void* zero_f16,
                                          void* parts_f32, int b, int n, int k,
                                          logismos_stream_t stream) {
-    if (b > 32 || logismos_check_qgemm_q4g128_shape(b, n, k, nullptr, 0) != 0)
+    if ((b > 32 && !prepared) || logismos_check_qgemm_q4g128_shape(b, n, k, nullptr, 0) != 0)
         return hipErrorInvalidValue;
     if (!x || !qw_u8 || !scale_f16 || !zero_f16 || !parts_f32) return hipErrorInvalidValue;
     if ((reinterpret_cast<uintptr_t>(qw_u8) & 15u) || (reinterpret_cast<uintptr_t>(x) & 15u))
         return hipErrorInvalidValue;
-    const lg::SplitkPlan plan = lg::splitk_plan(b, n, k);
+    // (more than 32 rows: chunks of 32, all on the plan of 32)
+    const lg::SplitkPlan plan = lg::splitk_plan(b < 32 ? b : 32, n, k);
     hipStream_t st = static_cast<hipStream_t>(stream);
     if (prepared) {
         if (const lg::RegxPlan rp = lg::regx_plan(b, n, k); rp.parts > 0)
@@ -357,7 +363,27 @@ extern "C" logismos_status_t logismos_launch_qgemm_q4g128_f32_splitk(
 extern "C" logismos_status_t logismos_launch_qgemm_q4g128_f32_splitk_xprep(
     const void* x_prepared, const void* qw_u8, const void* scale_f16, const void* zero_f16,
     void* parts_f32, int b, int n, int k, logismos_stream_t stream) {
+    if (b > 32) return hipErrorInvalidValue;
     return splitk_dispatch(x_prepared, true, qw_u8, scale_f16, zero_f16, parts_f32, b, n, k, stream);
+}
+
+hipError_t lg::qgemm_q4_splitk_rows(const void* x_prepared, const void* qw, const void* scale,
+                                    const void* zero, void* parts_f32, int rows, int n, int k,
+                                    hipStream_t stream) {
+    return static_cast<hipError_t>(
+        splitk_dispatch(x_prepared, true, qw, scale, zero, parts_f32, rows, n, k, stream));
+}
+
+int lg::qgemm_q4_splitk_rows_parts(int rows, int n, int k) {
+    return logismos_qgemm_q4g128_splitk_xprep_parts(rows < 32 ? rows : 32, n, k);
+}
+
+size_t lg::xprep_rows_stride(int k) { return xprep_chunk_stride(k); }
+
+bool lg::qgemm_q4_splitk_same_sums(int rows, int n, int k) {
+    if (rows <= 16) return false;  // (tiles of 16 rows multiply in steps of 32 columns)
+    if (regx_plan(32, n, k).parts > 0) return true;
+    return splitk_plan(rows, n, k).gp == splitk_plan(32, n, k).gp;
 }
 
 extern "C" size_t logismos_q4_xprep_bytes(int b, int k) {
@@ -369,7 +395,6 @@ namespace lg {
 // bf16 x [b][k] -> prepared form; one thread per 8-element chunk
 __global__ __launch_bounds__(256) void q4_prepare_x_kernel(const uint16_t* __restrict__ x,
                                                            void* __restrict__ xprep, int b, int k) {
-    const int bp = xprep_bp(b);
     const int chunks = k >> 3;
     const int idx = blockIdx.x * 256 + threadIdx.x;  // chunk-major inside a batch row
     const int bi = idx / chunks, c = idx - bi * chunks;
@@ -378,25 +403,29 @@ __global__ __launch_bounds__(256) void q4_prepare_x_kernel(const uint16_t* __res
     if (live) d = *reinterpret_cast<const uint4_t*>(x + (int64_t)bi * k + (int64_t)c * 8);
     const float gs = row16_sum(sum8_bf16(d));
     if (live) {
-        reinterpret_cast<uint4_t*>(xprep)[(int64_t)c * bp + bi] = pair_order(d);
-        if ((threadIdx.x & 15) == 0)
-            reinterpret_cast<float*>(reinterpret_cast<char*>(xprep) +
-                                     xprep_xg_offset(b, k))[(int64_t)(c >> 4) * bp + bi] = gs;
+        const XprepRow at = xprep_row(xprep, b, k, bi);
+        at.xp[(int64_t)c * at.bp] = pair_order(d);
+        if ((threadIdx.x & 15) == 0) at.xg[(int64_t)(c >> 4) * at.bp] = gs;
     }
 }
 }  // namespace lg
 
-extern "C" logismos_status_t logismos_launch_q4_prepare_x_bf16(const void* x_bf16, void* x_prepared,
-                                                               int b, int k,
-                                                               logismos_stream_t stream) {
-    if (b <= 0 || b > 32 || k <= 0 || k % 128 != 0 || (int64_t)b * k > (int64_t)INT32_MAX)
+hipError_t lg::q4_prepare_x_rows(const void* x_bf16, void* x_prepared, int b, int k,
+                                 hipStream_t stream) {
+    if (b <= 0 || k <= 0 || k % 128 != 0 || (int64_t)b * k > (int64_t)INT32_MAX)
         return hipErrorInvalidValue;
     if (!x_bf16 || !x_prepared || (reinterpret_cast<uintptr_t>(x_bf16) & 15u) ||
         (reinterpret_cast<uintptr_t>(x_prepared) & 15u))
         return hipErrorInvalidValue;
     const int items = b * (k / 8);
-    lg::q4_prepare_x_kernel<<<dim3((items + 255) / 256), dim3(256), 0,
-                              static_cast<hipStream_t>(stream)>>>(
+    lg::q4_prepare_x_kernel<<<dim3((items + 255) / 256), dim3(256), 0, stream>>>(
         static_cast<const uint16_t*>(x_bf16), x_prepared, b, k);
     return hipGetLastError();
+}
+
+extern "C" logismos_status_t logismos_launch_q4_prepare_x_bf16(const void* x_bf16, void* x_prepared,
+                                                               int b, int k,
+                                                               logismos_stream_t stream) {
+    if (b > 32) return hipErrorInvalidValue;
+    return lg::q4_prepare_x_rows(x_bf16, x_prepared, b, k, static_cast<hipStream_t>(stream));
 }

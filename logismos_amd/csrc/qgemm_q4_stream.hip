@@ -35,7 +35,7 @@ template <int BT>
 __global__ __launch_bounds__(64 * kStreamWaves) void qgemm_q4g128_stream_kernel(
     const uint4_t* __restrict__ xprep, const uint8_t* __restrict__ qw,
     const __half* __restrict__ scale, const __half* __restrict__ zero, float* __restrict__ part,
-    int b, int n, int k, int tiles_per_worker) {
+    int total_rows, int n, int k, int tiles_per_worker, int x_stride) {
     extern __shared__ uint4_t lds[];
     constexpr int BP = BT * 16;
     constexpr int GP = kStreamGP;
@@ -46,6 +46,9 @@ __global__ __launch_bounds__(64 * kStreamWaves) void qgemm_q4g128_stream_kernel(
     const int tiles = (n + 15) >> 4;
     const int t_begin = blockIdx.x * tiles_per_worker;
     if (t_begin >= tiles) return;
+    // (more than 32 rows: blockIdx.z is the chunk of 32)
+    const int chunk0 = 32 * blockIdx.z, b = min(total_rows - chunk0, 32);
+    xprep += (size_t)blockIdx.z * (unsigned)x_stride;
     const int t_end = min(tiles, t_begin + tiles_per_worker);
 
     uint4_t* xl = lds;                                          // [GP*16 chunks][BP]
@@ -67,7 +70,7 @@ __global__ __launch_bounds__(64 * kStreamWaves) void qgemm_q4g128_stream_kernel(
 #pragma unroll
     for (int u = 0; u < U; ++u) xd[u] = xb[u * NT + (int)threadIdx.x];
     const float* xg_src = reinterpret_cast<const float*>(
-        reinterpret_cast<const char*>(xprep) + xprep_xg_offset(b, k));
+        reinterpret_cast<const char*>(xprep) + (size_t)(k / 8) * BP * 16);
     const float xgd = xg_src[(int64_t)g0 * BP + ((int)threadIdx.x < GP * BP ? (int)threadIdx.x : 0)];
     __builtin_amdgcn_sched_barrier(0);
 
@@ -97,7 +100,7 @@ __global__ __launch_bounds__(64 * kStreamWaves) void qgemm_q4g128_stream_kernel(
     if ((int)threadIdx.x < GP * BP) xg[threadIdx.x] = xgd;
     __syncthreads();
 
-    float* pbase = part + (int64_t)j * b * n;  // uniform
+    float* pbase = part + ((int64_t)j * total_rows + chunk0) * n;  // uniform
     auto compute_tile = [&](int t, const StreamTile& tl) {
         float4_t ysum[BT];
 #pragma unroll
@@ -181,7 +184,10 @@ int stream_steps(int b, int n, int k) {
     // workgroups do as well
     if ((long)tiles * parts / cus < 10) return 0;
     int steps = 1;
-    while ((long)((tiles + steps * kStreamWaves - 1) / (steps * kStreamWaves)) * parts > cus) ++steps;
+    const int share = cus * 32 / (b <= 32 ? 32 : (b + 31) / 32 * 32);  // of one chunk of rows
+    while (steps < tiles &&
+           (long)((tiles + steps * kStreamWaves - 1) / (steps * kStreamWaves)) * parts > share)
+        ++steps;
     return steps;
 }
 
@@ -200,11 +206,12 @@ static hipError_t launch_stream(const void* xprep, const void* qw, const void* s
             160 * 1024 - 1024);
         if (opt != hipSuccess) return opt;
     }
-    dim3 grid((tiles + tpw - 1) / tpw, (k / 128) / kStreamGP);
+    dim3 grid((tiles + tpw - 1) / tpw, (k / 128) / kStreamGP, (b + 31) / 32);
+    if (grid.z > 1) grid.x = (grid.x + 7) / 8 * 8;  // (the chunks of a column on one XCD)
     kern<<<grid, dim3(64 * kStreamWaves), lds, stream>>>(
         static_cast<const uint4_t*>(xprep), static_cast<const uint8_t*>(qw),
         static_cast<const __half*>(scale), static_cast<const __half*>(zero),
-        static_cast<float*>(part), b, n, k, tpw);
+        static_cast<float*>(part), b, n, k, tpw, (int)(xprep_chunk_stride(k) / 16));
     return hipGetLastError();
 }
 

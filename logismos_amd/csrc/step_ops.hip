@@ -211,9 +211,9 @@ __global__ __launch_bounds__(kPrepThreads) void add_rms_norm_xprep_kernel(
 #pragma unroll
     for (int i = 0; i < kPrepThreads / 64; ++i) total += part[i];
     const float inv = 1.0f / sqrtf(total / (float)n + eps);
-    const int bp = xprep_bp(rows);
     uint4_t* xp = reinterpret_cast<uint4_t*>(xprep);
-    float* xg = reinterpret_cast<float*>(reinterpret_cast<char*>(xprep) + xprep_xg_offset(rows, n));
+    XprepRow at{};
+    if constexpr (!TALL) at = xprep_row(xprep, rows, n, row);
 #pragma unroll
     for (int p = 0; p < kPrepMaxPasses; ++p) {
         const int c = p * kPrepThreads + (int)threadIdx.x;  // chunk index
@@ -238,8 +238,8 @@ __global__ __launch_bounds__(kPrepThreads) void add_rms_norm_xprep_kernel(
                                              tall_sums_offset(rows, n))
                         [tall_sum_index(row, c >> 4, n, pairs)] = gs;
             } else {
-                xp[(int64_t)c * bp + row] = pair_order(o);
-                if ((threadIdx.x & 15) == 0) xg[(int64_t)(c >> 4) * bp + row] = gs;
+                at.xp[(int64_t)c * at.bp] = pair_order(o);
+                if ((threadIdx.x & 15) == 0) at.xg[(int64_t)(c >> 4) * at.bp] = gs;
             }
         }
     }
@@ -292,11 +292,9 @@ __global__ __launch_bounds__(256) void silu_mul_xprep_kernel(const float* __rest
     }
     const float gs = row16_sum(sum8_bf16(o));
     if (live) {
-        const int bp = xprep_bp(rows);
-        reinterpret_cast<uint4_t*>(xprep)[(int64_t)c * bp + t] = pair_order(o);
-        if ((threadIdx.x & 15) == 0)
-            reinterpret_cast<float*>(reinterpret_cast<char*>(xprep) +
-                                     xprep_xg_offset(rows, inter))[(int64_t)(c >> 4) * bp + t] = gs;
+        const XprepRow at = xprep_row(xprep, rows, inter, t);
+        at.xp[(int64_t)c * at.bp] = pair_order(o);
+        if ((threadIdx.x & 15) == 0) at.xg[(int64_t)(c >> 4) * at.bp] = gs;
     }
 }
 
@@ -942,19 +940,25 @@ extern "C" logismos_status_t logismos_launch_greedy_f32(const void* logits_f32, 
     return hipGetLastError();
 }
 
-extern "C" logismos_status_t logismos_launch_add_rms_norm_f32p_xprep(
-    void* h_f32, const void* parts_f32, int num_parts, const void* w_f32, void* x_prepared, int rows,
-    int n, float eps, logismos_stream_t stream) {
-    if (rows <= 0 || rows > 32 || n <= 0 || n % 128 != 0 ||
-        n > 8 * lg::kPrepThreads * lg::kPrepMaxPasses)
+hipError_t lg::add_rms_norm_xprep_rows(void* h_f32, const void* parts_f32, int num_parts,
+                                       const void* w_f32, void* x_prepared, int rows, int n,
+                                       float eps, hipStream_t stream) {
+    if (rows <= 0 || n <= 0 || n % 128 != 0 || n > 8 * lg::kPrepThreads * lg::kPrepMaxPasses)
         return hipErrorInvalidValue;
     if (!h_f32 || !w_f32 || !x_prepared || num_parts < 0 || (num_parts > 0 && !parts_f32))
         return hipErrorInvalidValue;
-    lg::add_rms_norm_xprep_kernel<false, false><<<dim3(rows), dim3(lg::kPrepThreads), 0,
-                                           static_cast<hipStream_t>(stream)>>>(
+    lg::add_rms_norm_xprep_kernel<false, false><<<dim3(rows), dim3(lg::kPrepThreads), 0, stream>>>(
         static_cast<float*>(h_f32), static_cast<const float*>(parts_f32), num_parts,
         (int64_t)rows * n, static_cast<const float*>(w_f32), x_prepared, rows, n, eps, 0);
     return hipGetLastError();
+}
+
+extern "C" logismos_status_t logismos_launch_add_rms_norm_f32p_xprep(
+    void* h_f32, const void* parts_f32, int num_parts, const void* w_f32, void* x_prepared, int rows,
+    int n, float eps, logismos_stream_t stream) {
+    if (rows > 32) return hipErrorInvalidValue;
+    return lg::add_rms_norm_xprep_rows(h_f32, parts_f32, num_parts, w_f32, x_prepared, rows, n, eps,
+                                       static_cast<hipStream_t>(stream));
 }
 
 hipError_t lg::add_rms_norm_tall(void* h_f32, const void* parts_f32, int num_parts,
@@ -989,20 +993,26 @@ extern "C" logismos_status_t logismos_launch_add_rms_norm_f32p_tall(
                                  pairs_per_load, static_cast<hipStream_t>(stream));
 }
 
-extern "C" logismos_status_t logismos_launch_silu_mul_f32p_xprep(const void* parts_f32,
-                                                                 int num_parts, void* x_prepared,
-                                                                 int rows, int inter,
-                                                                 logismos_stream_t stream) {
-    if (rows <= 0 || rows > 32 || inter <= 0 || inter % 128 != 0 || num_parts <= 0 ||
+hipError_t lg::silu_mul_xprep_rows(const void* parts_f32, int num_parts, void* x_prepared, int rows,
+                                   int inter, hipStream_t stream) {
+    if (rows <= 0 || inter <= 0 || inter % 128 != 0 || num_parts <= 0 ||
         (int64_t)rows * inter * 2 > (int64_t)INT32_MAX)
         return hipErrorInvalidValue;
     if (!parts_f32 || !x_prepared) return hipErrorInvalidValue;
     const int items = rows * (inter / 8);
-    lg::silu_mul_xprep_kernel<<<dim3((items + 255) / 256), dim3(256), 0,
-                                static_cast<hipStream_t>(stream)>>>(
+    lg::silu_mul_xprep_kernel<<<dim3((items + 255) / 256), dim3(256), 0, stream>>>(
         static_cast<const float*>(parts_f32), num_parts, (int64_t)rows * 2 * inter, x_prepared, rows,
         inter);
     return hipGetLastError();
+}
+
+extern "C" logismos_status_t logismos_launch_silu_mul_f32p_xprep(const void* parts_f32,
+                                                                 int num_parts, void* x_prepared,
+                                                                 int rows, int inter,
+                                                                 logismos_stream_t stream) {
+    if (rows > 32) return hipErrorInvalidValue;
+    return lg::silu_mul_xprep_rows(parts_f32, num_parts, x_prepared, rows, inter,
+                                   static_cast<hipStream_t>(stream));
 }
 
 static logismos_status_t embed_lookup_launch(const void* table, const void* ids_u32, void* out_f32,

@@ -1,0 +1,58 @@
+"""Steps of 33 to 96 packed rows: every operator takes all rows in one launch, the projections in
+chunks of 32 rows side by side, the last one with 1 to 32 rows.  Against the oracle, on each of the
+projection kernels (x in registers: K a multiple of 2048; streaming: 8 groups and many tiles; split
+over K: the rest), with decode rows, chunks, and 3-bit pools (whose last chunk of up to 16 rows stays
+by itself when there are chunks)."""
+import numpy as np
+import pytest
+
+from tests import workloads
+from tests.test_gpu_decode_step import _rel_l2, _run_both
+
+pytestmark = pytest.mark.gpu
+
+WIDTHS = [
+    (2048, 16, 4, 128, 2048),   # x in registers
+    (1024, 8, 2, 128, 16384),   # streaming gate/up projection, x in registers behind it
+    (896, 14, 2, 64, 1152),     # 7 and 9 groups, heads of 64
+    (384, 3, 1, 128, 640),      # fewer rows than a workgroup takes
+]
+
+
+def _check(cfg, layers, batch, rel, kv_ok=True):
+    r, got, want, lay, bat = _run_both(cfg, layers, batch)
+    assert _rel_l2(got, want) < rel
+    assert _rel_l2(r.h.to_numpy(np.float32, bat["h"].shape), bat["h"]) < rel
+    return got, want
+
+
+@pytest.mark.parametrize("rows", [33, 34, 48, 49, 64, 65, 96])
+@pytest.mark.parametrize("hidden,hq,hkv,d,inter", WIDTHS)
+def test_decode_rows(rows, hidden, hq, hkv, d, inter):
+    rng = np.random.default_rng(rows * 7 + hidden)
+    cfg, layers, batch = workloads.decode_step_problem(
+        rng, num_layers=2, hidden=hidden, hq=hq, hkv=hkv, d=d, inter=inter,
+        ctx=rng.integers(1, 60, size=rows), qkv_bias=bool(rows & 1))
+    # the decode batch's bounds (tests/test_gpu_decode_step.py), two layers
+    got, want = _check(cfg, layers, batch, 8e-3)
+    assert np.all(np.abs(got - want) <= 2e-2 + 3e-2 * np.abs(want))
+
+
+@pytest.mark.parametrize("new", [[1, 31, 1], [20, 1, 1, 30], [1, 64, 1, 1]])
+@pytest.mark.parametrize("hidden,hq,hkv,d,inter", WIDTHS[:3])
+def test_chunks_beside_decode_rows(new, hidden, hq, hkv, d, inter):
+    rng = np.random.default_rng(sum(new) + hidden)
+    cfg, layers, batch = workloads.decode_step_problem(
+        rng, num_layers=2, hidden=hidden, hq=hq, hkv=hkv, d=d, inter=inter,
+        ctx=[n + 9 * i for i, n in enumerate(new)], new_tokens=new)
+    got, want = _check(cfg, layers, batch, 8e-3)
+    assert np.all(np.abs(got - want) <= 2e-2 + 3e-2 * np.abs(want))
+
+
+@pytest.mark.parametrize("new", [[1] * 40, [1, 30, 2, 4], [1, 40, 20]])  # one pass, two, one
+def test_three_bit_pools(new):
+    rng = np.random.default_rng(len(new))
+    cfg, layers, batch = workloads.decode_step_problem(
+        rng, num_layers=1, hidden=512, hq=4, hkv=2, inter=1024,
+        ctx=[n + 40 + i for i, n in enumerate(new)], new_tokens=new, kv_turbo3=True)
+    _check(cfg, layers, batch, 1e-2)  # the bound of the steps over 3-bit pools
