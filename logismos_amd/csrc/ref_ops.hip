@@ -346,70 +346,137 @@ __global__ __launch_bounds__(256) void matmul_mfma_fp16_kernel(const _Float16* _
 }
 
 // The same product for rows that are whole 16-byte pieces (n and k multiples of 8): a workgroup
-// of four waves owns a TM x TN tile, each wave a quarter.  A [TM x KS] and B [KS x TN] slabs go to
-// LDS as they lie in memory; the B operand -- eight consecutive k of one column -- comes out of
-// the row-major slab through the transposing LDS read (two ds_read_b64_tr_b16: inside 16 lanes,
-// lane L receives element L % 4 of the 8-byte pieces that the lanes L / 4 + 4 i point at, so
-// lanes pointing at 4 k x 16 columns come back with 4 k of one column each).  A slab is asked
-// for one slab ahead of its LDS store, two ahead of its products; LDS is double buffered, one
-// barrier per slab.
-//
-// What bounds it at an encoder's sizes: a slab is a chain store -> barrier -> operand read ->
-// products of about 0.5 us whatever its size, so small matrices take small tiles (more
-// workgroups share a compute unit and fill each other's waits) and long slabs.  The kernel
-// above, one 128 x 128 tile per compute unit and 32 columns per slab, takes 0.9 us per slab.
-// us, this kernel / the one above:  2036 x 1536 x 1536 22.9 / 44.0 (419 TFLOP/s),
-// 16 x 1536 x 1536 10.4 / 33.1, 128 x 4096 x 4096 26.7 / 102.8, 4096^3 211 / 259,
-// 8192 x 8192 x 4096 735 / 816 (748 TFLOP/s).
-template <int TM, int TN, int KS>
-__global__ __launch_bounds__(256) void matmul_tiled_fp16_kernel(const _Float16* __restrict__ a,
-                                                                const _Float16* __restrict__ b,
-                                                                _Float16* __restrict__ d, int m,
-                                                                int n, int k) {
-    typedef short short4_t __attribute__((ext_vector_type(4)));
-    typedef __attribute__((address_space(3))) short4_t lds_short4_t;
-    constexpr int AS = KS + 8;                     // halfs per LDS row of A: operand reads conflict-free
-    constexpr int BS = TN + 16;                    // ... and of B
-    constexpr int AP = TM * KS / 8 / 256;        // pieces per thread
-    constexpr int BP = TN * KS / 8 / 256;
-    constexpr int MB = TM / 64, NB = TN / 64;      // 32 x 32 blocks per wave and direction
-    __shared__ __attribute__((aligned(16))) _Float16 as[2][TM * AS];
-    __shared__ __attribute__((aligned(16))) _Float16 bs[2][KS * BS];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int row0 = blockIdx.y * TM, col0 = blockIdx.x * TN;
-    const int wr = (wave >> 1) * (TM / 2), wc = (wave & 1) * (TN / 2);
+// owns a 32 MB WR x 32 NB WC tile, its WR x WC waves 32 MB x 32 NB each.  Slabs of 64 columns of A
+// (TM rows of 128 bytes) and 64 rows of B (TN columns) go from global memory straight into a ring of
+// BUFS buffers in LDS (global_load_lds, 1 KiB of consecutive LDS per request), BUFS - 1 slabs ahead,
+// two requests behind each of the last two steps of 16 columns.  As in the tiled Q4 GEMM the wait and
+// the barrier stand in the middle of a slab and the first operands of the next slab are read in its
+// last step.  Rows cannot be padded; the 16-byte chunks of a row are swizzled instead: A's by half
+// the row index (a ds_read_b128 of 32 rows x 2 chunks touches every bank once per 16 lanes), B's in
+// pairs (the transposing read takes 4 rows x 32 bytes per 16 lanes).  The B operand -- eight
+// consecutive k of one column -- is two ds_read_b64_tr_b16: inside 16 lanes, lane L receives element
+// L % 4 of the 8-byte pieces that the lanes L / 4 + 4 i point at, so lanes pointing at 4 k x 16 columns
+// come back with 4 k of one column each.  LDS is only touched through inline assembly inside the
+// loop: the compiler would order every access it can see behind all outstanding requests.
+typedef __attribute__((address_space(3))) void* mm_lds_ptr_t;
+#define LG_INLINE __attribute__((always_inline))
+template <int MB, int NB, int WR, int WC, int BUFS>
+__global__ __launch_bounds__(64 * WR * WC) void matmul_ring_fp16_kernel(
+    const _Float16* __restrict__ a, const _Float16* __restrict__ b, _Float16* __restrict__ d, int m,
+    int n, int k, int tiles_m, int tiles_n, int vec_out) {
+    constexpr int W = WR * WC, TM = 32 * MB * WR, TN = 32 * NB * WC, KS = 64;
+    constexpr int kA = TM * KS * 2, kBuf = kA + KS * TN * 2;   // bytes
+    constexpr int RA = TM / 8 / W, RB = TN / 8 / W;            // requests per wave and slab
+    static_assert(RA * W * 8 == TM && RB * W * 8 == TN , "whole requests");
+    static_assert(TN == 64 || TN == 128, "the swizzle of B");
+    constexpr int kReq = RA + RB;
+    extern __shared__ uint4_t mm_lds[];
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int r = lane & 31, h = lane >> 5;
 
-    // pieces of this thread: eight k of rows of A, eight columns of k rows of B
-    const int a_row = tid / (KS / 8), a_k = (tid % (KS / 8)) * 8;
-    const int b_col = (tid % (TN / 8)) * 8, b_k = tid / (TN / 8);
-    constexpr int AR = 256 / (KS / 8), BK = 256 / (TN / 8);  // rows between a thread's pieces
-    unsigned a_off[AP];
+    // Workgroups go round the eight XCDs in the order of their ids: each XCD takes a run of tiles,
+    // four row tiles by as many column tiles as that makes, and reads its part of A and B once.
+    const int tiles = tiles_m * tiles_n;
+    int t = blockIdx.x;
+    {
+        const int per = tiles / 8, more = tiles % 8, xcd = t % 8;
+        t = xcd * per + min(xcd, more) + t / 8;
+    }
+    const int band = t / (4 * tiles_n), in_band = t - band * 4 * tiles_n;
+    const int band_rows = min(4, tiles_m - 4 * band);
+    const int row0 = (4 * band + in_band % band_rows) * TM, col0 = (in_band / band_rows) * TN;
+
+    const unsigned lds_base = (unsigned)(uintptr_t)(mm_lds_ptr_t)mm_lds;
+    // ---- requests: q of A covers rows 8 (RA wave + q) .. + 7, lane -> row + lane / 8, position lane
+    // % 8, which holds chunk (position ^ row / 2 % 8); q of B covers 1 KiB of rows of TN columns.  What
+    // lies past m, n or k re-reads what is there (past k it is taken as zero below, past m and n it
+    // only reaches results that are not stored).
+    constexpr int BR = 512 / TN;                        // rows of B per request
+    auto b_swizzle = [](int row) { return TN == 128 ? 2 * (row & 3) : 2 * ((row >> 1) & 1); };
+    unsigned a_row[RA], b_col[RB];
+    int a_chunk[RA], b_row[RB];
 #pragma unroll
-    for (int u = 0; u < AP; ++u) a_off[u] = (unsigned)min(row0 + a_row + AR * u, m - 1) * (unsigned)k;
-    const bool col_in = col0 + b_col < n;
-    half8_t ra[AP], rb[BP];
-    const half8_t zero = {0, 0, 0, 0, 0, 0, 0, 0};
-    auto gload = [&](int k0) {
-        const int gk = k0 + a_k;
+    for (int q = 0; q < RA; ++q) {
+        const int row = 8 * (RA * wave + q) + (lane >> 3);
+        a_chunk[q] = 8 * ((lane & 7) ^ ((row >> 1) & 7));
+        a_row[q] = (unsigned)min(row0 + row, m - 1) * (unsigned)k;
+    }
 #pragma unroll
-        for (int u = 0; u < AP; ++u)
-            ra[u] = gk < k ? *reinterpret_cast<const half8_t*>(a + (a_off[u] + (unsigned)gk)) : zero;
-#pragma unroll
-        for (int u = 0; u < BP; ++u) {
-            const int gr = k0 + b_k + BK * u;
-            rb[u] = gr < k && col_in
-                             ? *reinterpret_cast<const half8_t*>(b + ((unsigned)gr * (unsigned)n + (unsigned)(col0 + b_col)))
-                             : zero;
-        }
+    for (int q = 0; q < RB; ++q) {
+        b_row[q] = BR * (RB * wave + q) + lane / (TN / 8);
+        b_col[q] = (unsigned)min(col0 + 8 * ((lane % (TN / 8)) ^ b_swizzle(b_row[q])), n - 8);
+    }
+    auto request = [&](const void* src, unsigned off, unsigned dst) LG_INLINE {
+        asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
+                     :
+                     : "v"(off), "s"(src), "s"(dst)
+                     : "memory");
     };
-    auto lstore = [&](int buf) {
+    auto request_a = [&](int s, int buf_off) LG_INLINE {
 #pragma unroll
-        for (int u = 0; u < AP; ++u)
-            *reinterpret_cast<half8_t*>(&as[buf][(a_row + AR * u) * AS + a_k]) = ra[u];
+        for (int q = 0; q < RA; ++q)
+            request(a, (a_row[q] + (unsigned)min(s * KS + a_chunk[q], k - 8)) * 2u,
+                    __builtin_amdgcn_readfirstlane(lds_base + (unsigned)buf_off + (unsigned)(RA * wave + q) * 1024u));
+    };
+    auto request_b = [&](int s, int buf_off) LG_INLINE {
 #pragma unroll
-        for (int u = 0; u < BP; ++u)
-            *reinterpret_cast<half8_t*>(&bs[buf][(b_k + BK * u) * BS + b_col]) = rb[u];
+        for (int q = 0; q < RB; ++q)
+            request(b, ((unsigned)min(s * KS + b_row[q], k - 1) * (unsigned)n + b_col[q]) * 2u,
+                    __builtin_amdgcn_readfirstlane(lds_base + (unsigned)buf_off + kA + (unsigned)(RB * wave + q) * 1024u));
+    };
+
+    // ---- operand reads.  A: lane (r, h) at step kk (16 columns) wants chunk 2 kk + h of row wr + 32 i +
+    // r.  B: rows 16 kk + 8 h + lane % 16 / 4 and four on, columns wc + 32 j + 16 (lane / 16 % 2) + 4 (lane % 4).
+    const int wr = (wave / WC) * 32 * MB, wc = (wave % WC) * 32 * NB;
+    const unsigned a_base = lds_base + (unsigned)(wr + r) * 128u;
+    const unsigned a_pos = (unsigned)(h ^ ((r >> 1) & 7)) * 16u;
+    const int s16 = lane & 15, b_k = 8 * h + (s16 >> 2);
+    unsigned b_base[NB];
+#pragma unroll
+    for (int j = 0; j < NB; ++j) {
+        const int col = wc + 32 * j + 16 * ((lane >> 4) & 1) + 4 * (s16 & 3);
+        b_base[j] = lds_base + kA + (unsigned)b_k * (TN * 2u) +
+                    (unsigned)((col >> 3) ^ b_swizzle(b_k)) * 16u + (unsigned)(col & 4) * 2u;
+    }
+    half8_t av[2][MB];
+    uint2_t bl[2][NB], bh[2][NB];  // rows 0 .. 3 and 4 .. 7 of the lane's eight
+    auto read_step = [&](auto kk_c, int buf_off) LG_INLINE {
+        constexpr int KK = decltype(kk_c)::value, P = KK & 1;
+        const unsigned aa = (a_base + (a_pos ^ (32u * KK))) + (unsigned)buf_off;
+        static_for<MB>([&](auto i_c) LG_INLINE {
+            constexpr int at = decltype(i_c)::value * 32 * 128;
+            half8_t& dst = av[P][decltype(i_c)::value];
+            const unsigned from = aa;
+            asm volatile("ds_read_b128 %0, %1 offset:%c2" : "=&v"(dst) : "v"(from), "n"(at) : "memory");
+        });
+        static_for<NB>([&](auto j_c) LG_INLINE {
+            constexpr int J = decltype(j_c)::value;
+            uint2_t& lo = bl[P][J];
+            uint2_t& hi = bh[P][J];
+            const unsigned from = b_base[J] + (unsigned)buf_off;
+            // (four rows on: the swizzle repeats every four rows)
+            asm volatile("ds_read_b64_tr_b16 %0, %2 offset:%c3\n\tds_read_b64_tr_b16 %1, %2 offset:%c4"
+                         : "=&v"(lo), "=&v"(hi)
+                         : "v"(from), "n"(KK * 16 * TN * 2), "n"((KK * 16 + 4) * TN * 2)
+                         : "memory");
+        });
+    };
+    auto step_landed = [&](auto kk_c) LG_INLINE {
+        constexpr int P = decltype(kk_c)::value & 1;
+        half8_t& a0 = av[P][0];
+        uint2_t& l0 = bl[P][0];
+        uint2_t& h0 = bh[P][0];
+        asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(a0), "+v"(l0), "+v"(h0)::"memory");
+        static_for<MB - 1>([&](auto i_c) LG_INLINE {
+            half8_t& x = av[P][decltype(i_c)::value + 1];
+            asm volatile("" : "+v"(x)::"memory");
+        });
+        static_for<NB - 1>([&](auto j_c) LG_INLINE {
+            uint2_t& x = bl[P][decltype(j_c)::value + 1];
+            uint2_t& y = bh[P][decltype(j_c)::value + 1];
+            asm volatile("" : "+v"(x), "+v"(y)::"memory");
+        });
     };
     float16_t acc[MB][NB];
 #pragma unroll
@@ -418,78 +485,158 @@ __global__ __launch_bounds__(256) void matmul_tiled_fp16_kernel(const _Float16* 
         for (int j = 0; j < NB; ++j)
 #pragma unroll
             for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.0f;
-    const int s16 = lane & 15;
-    const int b_lane = (8 * h + (s16 >> 2)) * BS + wc + 16 * ((lane >> 4) & 1) + 4 * (s16 & 3);
-    auto multiply = [&](int buf) {
+    const int slabs = (k + KS - 1) / KS;
+    auto multiply = [&](auto kk_c, int s) LG_INLINE {
+        constexpr int KK = decltype(kk_c)::value, P = KK & 1;
+        uint4_t bv[NB];
 #pragma unroll
-        for (int kk = 0; kk < KS; kk += 16) {
-            half8_t av[MB], bv[NB];
+        for (int j = 0; j < NB; ++j) bv[j] = uint4_t{bl[P][j][0], bl[P][j][1], bh[P][j][0], bh[P][j][1]};
+        if (s * KS + KS > k) {
+            // past k: zeros on both sides (what lies there may be an infinity)
+            const bool in = s * KS + 16 * KK + 8 * h < k;
 #pragma unroll
-            for (int i = 0; i < MB; ++i)
-                av[i] = *reinterpret_cast<const half8_t*>(&as[buf][(wr + 32 * i + r) * AS + kk + 8 * h]);
+            for (int i = 0; i < MB; ++i) {
+                uint4_t v = __builtin_bit_cast(uint4_t, av[P][i]);
 #pragma unroll
-            for (int j = 0; j < NB; ++j) {
-                const _Float16* src = &bs[buf][b_lane + kk * BS + 32 * j];
-                short4_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_short4_t*)src);
-                short4_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_short4_t*)(src + 4 * BS));
-                typedef short short8_t __attribute__((ext_vector_type(8)));
-                bv[j] = __builtin_bit_cast(half8_t, (short8_t)__builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+                for (int e = 0; e < 4; ++e) v[e] = in ? v[e] : 0u;
+                av[P][i] = __builtin_bit_cast(half8_t, v);
             }
 #pragma unroll
-            for (int i = 0; i < MB; ++i)
+            for (int j = 0; j < NB; ++j)
 #pragma unroll
-                for (int j = 0; j < NB; ++j)
-                    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(av[i], bv[j], acc[i][j], 0, 0, 0);
+                for (int e = 0; e < 4; ++e) bv[j][e] = in ? bv[j][e] : 0u;
         }
+#pragma unroll
+        for (int i = 0; i < MB; ++i)
+#pragma unroll
+            for (int j = 0; j < NB; ++j)
+                acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(av[P][i], __builtin_bit_cast(half8_t, bv[j]),
+                                                                   acc[i][j], 0, 0, 0);
     };
-    // slab s is multiplied out of buffer s % 2; slab s + 1 goes from its registers to the other
-    // buffer, whose last reader was slab s - 1, before the last barrier
-    const int slabs = (k + KS - 1) / KS;
-    gload(0);
-    lstore(0);
-    if (slabs > 1) gload(KS);
-    __syncthreads();
+
+    // ---- the first BUFS - 1 slabs, then slab by slab
+#pragma unroll
+    for (int u = 0; u < BUFS - 1; ++u)
+        if (u < slabs) {
+            request_a(u, u * kBuf);
+            request_b(u, u * kBuf);
+        }
+    if (slabs >= BUFS - 1) asm volatile("s_waitcnt vmcnt(%0)" ::"n"((BUFS - 2) * kReq) : "memory");
+    else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    read_step(ic<0>{}, 0);
+    step_landed(ic<0>{});
+    int buf_off = 0;
     for (int s = 0; s < slabs; ++s) {
-        multiply(s & 1);
-        if (s + 1 < slabs) lstore((s + 1) & 1);
-        if (s + 2 < slabs) gload((s + 2) * KS);
-        __syncthreads();
+        const int next_off = buf_off + kBuf == BUFS * kBuf ? 0 : buf_off + kBuf;
+        const int last_off = buf_off == 0 ? (BUFS - 1) * kBuf : buf_off - kBuf;  // of slab s - 1
+        const bool more = s + 1 < slabs, ahead = s + BUFS - 1 < slabs;
+        read_step(ic<1>{}, buf_off);
+        __builtin_amdgcn_sched_barrier(0);
+        multiply(ic<0>{}, s);
+        __builtin_amdgcn_sched_barrier(0);
+        step_landed(ic<1>{});
+        read_step(ic<2>{}, buf_off);
+        __builtin_amdgcn_sched_barrier(0);
+        multiply(ic<1>{}, s);
+        __builtin_amdgcn_sched_barrier(0);
+        step_landed(ic<2>{});
+        if (more) {
+            // slab s + 1 has landed (its requests are the oldest of BUFS - 2 slabs'; this wave's
+            // requests complete in the order they were issued), behind the barrier everybody's has,
+            // and everybody has left slab s - 1, whose buffer slab s + BUFS - 1 takes
+            if (s + BUFS - 2 < slabs) asm volatile("s_waitcnt vmcnt(%0)" ::"n"((BUFS - 3) * kReq) : "memory");
+            else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+            __builtin_amdgcn_s_barrier();
+        }
+        read_step(ic<3>{}, buf_off);
+        if (ahead) request_a(s + BUFS - 1, last_off);
+        __builtin_amdgcn_sched_barrier(0);
+        multiply(ic<2>{}, s);
+        __builtin_amdgcn_sched_barrier(0);
+        step_landed(ic<3>{});
+        if (more) read_step(ic<0>{}, next_off);
+        if (ahead) request_b(s + BUFS - 1, last_off);
+        __builtin_amdgcn_sched_barrier(0);
+        multiply(ic<3>{}, s);
+        __builtin_amdgcn_sched_barrier(0);
+        if (more) step_landed(ic<0>{});
+        buf_off = next_off;
     }
+
     // lane (h, r) holds column r, rows 8 * (e / 4) + 4h + e % 4 of each 32 x 32 block
+    if (!vec_out) {
+#pragma unroll
+        for (int i = 0; i < MB; ++i)
+#pragma unroll
+            for (int j = 0; j < NB; ++j) {
+                const int gc = col0 + wc + 32 * j + r;
+                if (gc >= n) continue;
+#pragma unroll
+                for (int e = 0; e < 16; ++e) {
+                    const int gr = row0 + wr + 32 * i + 8 * (e >> 2) + 4 * h + (e & 3);
+                    if (gr < m) d[(int64_t)gr * n + gc] = (_Float16)acc[i][j][e];
+                }
+            }
+        return;
+    }
+    // ... through LDS, and out in 16-byte pieces
+    __syncthreads();  // the ring is done with once every wave has read its last operands
+    constexpr int kPitch = TN + 8;
+    _Float16* const out = reinterpret_cast<_Float16*>(mm_lds);
 #pragma unroll
     for (int i = 0; i < MB; ++i)
 #pragma unroll
-        for (int j = 0; j < NB; ++j) {
-            const int gc = col0 + wc + 32 * j + r;
-            if (gc >= n) continue;
+        for (int j = 0; j < NB; ++j)
 #pragma unroll
-            for (int e = 0; e < 16; ++e) {
-                const int gr = row0 + wr + 32 * i + 8 * (e >> 2) + 4 * h + (e & 3);
-                if (gr < m) d[(int64_t)gr * n + gc] = (_Float16)acc[i][j][e];
-            }
-        }
+            for (int e = 0; e < 16; ++e)
+                out[(wr + 32 * i + 8 * (e >> 2) + 4 * h + (e & 3)) * kPitch + wc + 32 * j + r] = (_Float16)acc[i][j][e];
+    __syncthreads();
+    constexpr int kPieces = TN / 8;
+#pragma unroll
+    for (int u = 0; u < TM * kPieces / (64 * W); ++u) {
+        const int id = u * 64 * W + tid, row = id / kPieces, c = id % kPieces;
+        const int gr = row0 + row, gc = col0 + 8 * c;
+        if (gr < m && gc < n)
+            *reinterpret_cast<uint4_t*>(d + (int64_t)gr * n + gc) = *reinterpret_cast<const uint4_t*>(out + row * kPitch + 8 * c);
+    }
 }
 
-template <int TM, int TN, int KS>
-static hipError_t matmul_tiled_launch(const void* a, const void* b, void* d, int m, int n, int k,
-                                      hipStream_t st) {
-    matmul_tiled_fp16_kernel<TM, TN, KS><<<dim3((n + TN - 1) / TN, (m + TM - 1) / TM), dim3(256), 0, st>>>(
-        static_cast<const _Float16*>(a), static_cast<const _Float16*>(b), static_cast<_Float16*>(d), m, n, k);
+template <int MB, int NB, int WR, int WC, int BUFS>
+static hipError_t matmul_ring_launch(const void* a, const void* b, void* d, int m, int n, int k,
+                                     hipStream_t st) {
+    constexpr int TM = 32 * MB * WR, TN = 32 * NB * WC;
+    constexpr int lds = BUFS * (TM + TN) * 128;
+    const auto kernel = matmul_ring_fp16_kernel<MB, NB, WR, WC, BUFS>;
+    static const hipError_t opt = hipFuncSetAttribute(
+        reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+    if (opt != hipSuccess) return opt;
+    const int tm = (m + TM - 1) / TM, tn = (n + TN - 1) / TN;
+    const int vec_out = (reinterpret_cast<uintptr_t>(d) & 15u) == 0;
+    kernel<<<dim3((unsigned)((int64_t)tm * tn)), dim3(64 * WR * WC), lds, st>>>(
+        static_cast<const _Float16*>(a), static_cast<const _Float16*>(b), static_cast<_Float16*>(d), m, n, k,
+        tm, tn, vec_out);
     return hipGetLastError();
 }
 
-// 128 x 128 tiles once two of them fall on every compute unit (4096 x 2048 x 4096: 110 us, 154 on
-// 64 x 64); below that 64 x 64, with slabs of 128 while there are at most two such tiles per
-// compute unit (500 x 1024 x 1200: 9.6 us, 10.0 with 64) and of 64 where more of them share its
-// LDS (2036 x 1536 x 1536, three per unit: 22.9 us, 26.7 with 128).
+// The largest tile of which there are enough: 256 x 128 from three quarters of the compute units on,
+// 128 x 128 and 64 x 128 from six tenths, else 64 x 64.  us, 256 x 128 / 128 x 128 / 64 x 128 / 64 x 64
+// (tiles of the first) and what the kernel with a slab in registers on its way to two buffers took:
+//   4096 x 4096 x 4096 (512)  140 / 167 / 235 / 245, 172      1700 x 4096 x 4096 (224)  68 / 80 / 117 / 113, 114
+//   4096 x 2048 x 1000 (256)  25.6 / 26.9 / 36.8 / 38.9, 27.7  2500 x 1024 x 2048 (80)  29.4 / 20.6 / 30.6 / 28.2, 25.9
+//   2036 x 1536 x 1536 (96)   25.2 / 21.2 / 27.3 / 28.0, 23.3  1000 x 4096 x 768 (128)  15.4 / 12.1 / 16.1 / 16.1, 14.9
+//   1300 x 1536 x 1000 (72)   16.8 / 12.1 / 10.6 / 11.1, 11.2  4096 x 512 x 776 (64)    14.2 / 10.5 / 8.8 / 9.6, 13.6
+//   500 x 1024 x 1200 (16)    17.9 / 12.6 / 10.4 / 9.1, 9.3    294 x 1536 x 3560 (24)   53.6 / 32.4 / 25.9 / 22.8, 22.7
+// What bounds it: the operands' way from L2 (9 TB/s at 2036 x 1536 x 1536, 151 MB on 128 x 128 tiles), where
+// tiles are few a slab's chain of four dependent steps, 0.27 us on 64 x 64, 0.43 on 128 x 128.
 static hipError_t matmul_tiled(const void* a, const void* b, void* d, int m, int n, int k, void* stream) {
     hipStream_t st = static_cast<hipStream_t>(stream);
     const int64_t cus = device_cu_count();
-    const int64_t big = (int64_t)((m + 127) / 128) * ((n + 127) / 128);
-    const int64_t small = (int64_t)((m + 63) / 64) * ((n + 63) / 64);
-    if (big >= 2 * cus) return matmul_tiled_launch<128, 128, 64>(a, b, d, m, n, k, st);
-    if (small <= 2 * cus) return matmul_tiled_launch<64, 64, 128>(a, b, d, m, n, k, st);
-    return matmul_tiled_launch<64, 64, 64>(a, b, d, m, n, k, st);
+    auto tiles = [&](int tm, int tn) { return (int64_t)((m + tm - 1) / tm) * ((n + tn - 1) / tn); };
+    if (4 * tiles(256, 128) >= 3 * cus) return matmul_ring_launch<2, 2, 4, 2, 3>(a, b, d, m, n, k, st);
+    if (10 * tiles(128, 128) >= 6 * cus) return matmul_ring_launch<2, 1, 2, 4, 5>(a, b, d, m, n, k, st);
+    if (10 * tiles(64, 128) >= 6 * cus) return matmul_ring_launch<1, 1, 2, 4, 5>(a, b, d, m, n, k, st);
+    return matmul_ring_launch<1, 1, 2, 2, 5>(a, b, d, m, n, k, st);
 }
 
 // `check_matmul_shape` (crates/kernels/src/matmul/mod.rs:89-117)

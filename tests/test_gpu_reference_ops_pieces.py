@@ -1,6 +1,8 @@
 """The forms of the reference's launchers that work on whole 16-byte pieces, at the edges of their
 tiles, slabs and registers, with the reference's metric and tolerance
 (tests/test_gpu_reference_ops.py)."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -18,6 +20,39 @@ pytestmark = pytest.mark.gpu
 def test_matmul_of_whole_pieces(m, n, k):
     got, want = _matmul("wmma", m, n, k, 5)
     _parity(got, want)
+
+
+@pytest.mark.parametrize("m,n,k", [
+    (640, 2056, 72), (700, 1992, 320),                    # 64 x 128
+    (1409, 1672, 392), (1536, 1664, 328),                 # 128 x 128
+    (1793, 3464, 200), (2048, 3080, 256), (1900, 3336, 8)])  # 256 x 128
+def test_matmul_tiles(m, n, k):
+    # ragged last tiles and slabs, fewer and more slabs than the ring holds.  Bound: the rounding to
+    # fp16, and of each of the k fp32 sums at most one unit of what their terms add up to
+    rng = np.random.default_rng(m)
+    a, b = _f16(rng, m, k), _f16(rng, k, n)
+    da, db, d = hip.DeviceBuffer.from_numpy(a), hip.DeviceBuffer.from_numpy(b), hip.DeviceBuffer(m * n * 2)
+    kernels.launch_matmul_fp16("wmma", da, db, d, m, n, k)
+    hip.synchronize()
+    got = d.to_numpy(np.float16, (m, n)).astype(np.float64)
+    a, b = a.astype(np.float64), b.astype(np.float64)
+    want = a @ b
+    assert np.all(np.abs(got - want) <= 2.0 ** -11 * np.abs(want) + 2.0 ** -25
+                  + k * 2.0 ** -23 * (np.abs(a) @ np.abs(b)))
+
+
+@pytest.mark.parametrize("m,n,k", [(70, 136, 72), (1500, 1608, 72)])
+def test_matmul_into_rows_off_sixteen_bytes(m, n, k):
+    rng = np.random.default_rng(m)
+    a, b = _f16(rng, m, k), _f16(rng, k, n)
+    da, db = hip.DeviceBuffer.from_numpy(a), hip.DeviceBuffer.from_numpy(b)
+    d = hip.DeviceBuffer(m * n * 2 + 16)  # (the whole of it is read back)
+    d2 = hip.DeviceBuffer(m * n * 2)
+    kernels.launch_matmul_fp16("wmma", da, db, C.c_void_p(d.ptr.value + 2), m, n, k)
+    kernels.launch_matmul_fp16("wmma", da, db, d2, m, n, k)
+    hip.synchronize()
+    got = d.to_numpy(np.uint16, (m * n + 8,))[1:1 + m * n]
+    assert np.array_equal(got, d2.to_numpy(np.uint16, (m * n,)))
 
 
 def test_matmul_leaves_out_what_lies_behind_k():
