@@ -128,15 +128,18 @@ __global__ __launch_bounds__(kNormThreads) void add_rms_norm_kernel(
 
 // The step's form of the same operator: y arrives as fp32 split-K parts and the
 // normed row leaves in the prepared layout of the next Q4G128 GEMM (pair order
-// + per-group sums).  512 threads per row, eight consecutive elements (one
-// 16-byte chunk of the output) per thread and pass; n % 128 == 0.
-constexpr int kPrepThreads = 512;
-constexpr int kPrepMaxPasses = 4;  // rows up to 16384 wide
+// + per-group sums).  A workgroup per row, eight consecutive elements (one
+// 16-byte chunk of the output) per thread and pass; n % 128 == 0.  128 threads up to 1024 columns,
+// 256 up to 2048, 512 in one pass up to 4096 and in four beyond: over many rows a workgroup's idle
+// threads and the registers of passes that it does not have keep other rows off its compute unit
+// (1030 rows of 896: 9.2 -> 6.6 us, 10.5 -> 7.4 with nine parts; of 4096: 13.4 -> 11.8).  The sum
+// of squares adds up alike: threads past the row only ever add zeros.
+constexpr int kPrepMaxWidth = 8 * 512 * 4;
 
 // TALL: the normed rows leave as the operand of the tiled GEMM for many rows instead
 // (q4_common.hpp: row-major in pair order, `pairs` pairs of groups per block of sums; the grid
 // covers the rows padded to the GEMM's 128-row tiles, and a padding row is written as zeros).
-template <bool TALL, bool SUM_FIRST>
+template <bool TALL, bool SUM_FIRST, int kPrepThreads, int kPrepMaxPasses>
 __global__ __launch_bounds__(kPrepThreads) void add_rms_norm_xprep_kernel(
     float* __restrict__ h, const float* __restrict__ yp, int num_parts, int64_t part_stride,
     const float* __restrict__ w, void* __restrict__ xprep, int rows, int n, float eps,
@@ -243,6 +246,22 @@ __global__ __launch_bounds__(kPrepThreads) void add_rms_norm_xprep_kernel(
             }
         }
     }
+}
+
+template <bool TALL, bool SUM_FIRST>
+static hipError_t add_rms_norm_xprep_launch(int grid, float* h, const float* parts, int num_parts,
+                                            const float* w, void* out, int rows, int n, float eps,
+                                            int pairs, hipStream_t st) {
+    const int64_t stride = (int64_t)rows * n;
+#define LG_NORM(T, P)                                                                          \
+    add_rms_norm_xprep_kernel<TALL, SUM_FIRST, T, P>                                           \
+        <<<dim3(grid), dim3(T), 0, st>>>(h, parts, num_parts, stride, w, out, rows, n, eps, pairs)
+    if (n <= 1024) LG_NORM(128, 1);
+    else if (n <= 2048) LG_NORM(256, 1);
+    else if (n <= 4096) LG_NORM(512, 1);
+    else LG_NORM(512, 4);
+#undef LG_NORM
+    return hipGetLastError();
 }
 
 // act = silu(gate) * up from the fp32 parts of the gate_up GEMM, written in the
@@ -400,27 +419,29 @@ __global__ __launch_bounds__(64) void rope_kv_write_kernel(
     }
 }
 
-// The same operator for many rows (a prefill chunk's worth and more), 128-wide heads, fp16
+// The same operator for many rows (a prefill chunk's worth and more), heads a multiple of 8 wide, fp16
 // pools, fp32 parts in: one thread per four consecutive rotation pairs (i .. i + 3 with
-// i + 64 .. i + 67), 16-byte loads and 8-byte stores, 16 heads of a token per workgroup.  The
+// i + D / 2 ..), 16-byte loads and 8-byte stores (1030 tokens x 18 heads of 64: 7.4 -> 4.9 us).  The
 // kernel above is one 64-thread workgroup per (token, head) with 4-byte accesses: at 8240
 // tokens x 48 heads that is 400 k workgroups for 300 MB.  Same sums in the same order, same
 // rotation, same rounding.
 constexpr int kRopeRowsKernelFrom = 64;  // tokens from which the many-row kernel is used
+template <bool D128>
 __global__ __launch_bounds__(256) void rope_kv_write_rows_kernel(
     const float* __restrict__ qkv_parts, int num_parts, int64_t part_stride,
     const int32_t* __restrict__ positions, const float* __restrict__ cos_t,
     const float* __restrict__ sin_t, const int64_t* __restrict__ slot_mapping,
     __half* __restrict__ q_out, __half* __restrict__ k_pool, __half* __restrict__ v_pool, int hq,
-    int hkv, int max_pos, const float* __restrict__ bias, int64_t total_quads) {
+    int hkv, int max_pos, const float* __restrict__ bias, int64_t total_quads, int head_dim) {
     const int64_t gid = (int64_t)blockIdx.x * 256 + threadIdx.x;
     if (gid >= total_quads) return;
     const int heads = hq + 2 * hkv;
-    const int i = 4 * (int)(gid & 15);
-    const int64_t th = gid >> 4;
+    const int D = D128 ? 128 : head_dim, HALF = D / 2, quads = HALF / 4;
+    const int64_t th = D128 ? gid >> 4 : (int64_t)((unsigned)gid / (unsigned)quads);
+    const int i = 4 * (int)(gid - th * quads);
     const int64_t t = th / heads;
     const int head = (int)(th - t * heads);
-    const int64_t off = th * 128;
+    const int64_t off = th * D;
     float4_t x0 = {0.0f, 0.0f, 0.0f, 0.0f}, x1 = x0;
     for_part_rounds<4>(num_parts, [&](auto nc, int q0) {
         constexpr int N = decltype(nc)::value;
@@ -429,7 +450,7 @@ __global__ __launch_bounds__(256) void rope_kv_write_rows_kernel(
         for (int u = 0; u < N; ++u) {
             const float* src = qkv_parts + (int64_t)(q0 + u) * part_stride + off + i;
             a[u] = *reinterpret_cast<const float4_t*>(src);
-            b[u] = *reinterpret_cast<const float4_t*>(src + 64);
+            b[u] = *reinterpret_cast<const float4_t*>(src + HALF);
         }
 #pragma unroll
         for (int u = 0; u < N; ++u)
@@ -440,8 +461,8 @@ __global__ __launch_bounds__(256) void rope_kv_write_rows_kernel(
             }
     });
     if (bias) {
-        const float4_t b0 = *reinterpret_cast<const float4_t*>(bias + head * 128 + i);
-        const float4_t b1 = *reinterpret_cast<const float4_t*>(bias + head * 128 + i + 64);
+        const float4_t b0 = *reinterpret_cast<const float4_t*>(bias + head * D + i);
+        const float4_t b1 = *reinterpret_cast<const float4_t*>(bias + head * D + i + HALF);
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
             x0[e] += b0[e];
@@ -459,8 +480,8 @@ __global__ __launch_bounds__(256) void rope_kv_write_rows_kernel(
     if (head < hq + hkv) {
         int pos = positions[t];
         pos = pos < 0 ? 0 : (pos >= max_pos ? max_pos - 1 : pos);
-        const float4_t c = *reinterpret_cast<const float4_t*>(cos_t + (int64_t)pos * 64 + i);
-        const float4_t sn = *reinterpret_cast<const float4_t*>(sin_t + (int64_t)pos * 64 + i);
+        const float4_t c = *reinterpret_cast<const float4_t*>(cos_t + (int64_t)pos * HALF + i);
+        const float4_t sn = *reinterpret_cast<const float4_t*>(sin_t + (int64_t)pos * HALF + i);
         float4_t y0, y1;
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
@@ -471,20 +492,20 @@ __global__ __launch_bounds__(256) void rope_kv_write_rows_kernel(
         }
         __half* dst;
         if (head < hq) {
-            dst = q_out + (t * hq + head) * 128;
+            dst = q_out + (t * hq + head) * D;
         } else {
             const int64_t slot = slot_mapping[t];
             if (slot < 0) return;
-            dst = k_pool + (slot * hkv + (head - hq)) * 128;
+            dst = k_pool + (slot * hkv + (head - hq)) * D;
         }
         store4(dst + i, y0);
-        store4(dst + i + 64, y1);
+        store4(dst + i + HALF, y1);
     } else {
         const int64_t slot = slot_mapping[t];
         if (slot < 0) return;
-        __half* dst = v_pool + (slot * hkv + (head - hq - hkv)) * 128;
+        __half* dst = v_pool + (slot * hkv + (head - hq - hkv)) * D;
         store4(dst + i, x0);
-        store4(dst + i + 64, x1);
+        store4(dst + i + HALF, x1);
     }
 }
 
@@ -778,7 +799,7 @@ extern "C" logismos_status_t logismos_launch_rope_kv_write_f32p_bias(
     if (!qkv_parts_f32 || !positions || !cos_f32 || !sin_f32 || !slot_mapping || !q_out_f16 ||
         !k_pool_f16 || !v_pool_f16)
         return hipErrorInvalidValue;
-    // many rows of 128-wide heads: the kernel with 16-byte accesses (everything it reads and
+    // many rows: the kernel with 16-byte accesses (everything it reads and
     // writes 16-byte aligned)
     const uintptr_t align = reinterpret_cast<uintptr_t>(qkv_parts_f32) |
                             reinterpret_cast<uintptr_t>(bias_f32) |
@@ -787,16 +808,17 @@ extern "C" logismos_status_t logismos_launch_rope_kv_write_f32p_bias(
                             reinterpret_cast<uintptr_t>(q_out_f16) |
                             reinterpret_cast<uintptr_t>(k_pool_f16) |
                             reinterpret_cast<uintptr_t>(v_pool_f16);
-    if (head_dim == 128 && total_tokens >= lg::kRopeRowsKernelFrom && (align & 15u) == 0 &&
-        ((int64_t)total_tokens * width) % 4 == 0) {
-        const int64_t quads = (int64_t)total_tokens * (num_q_heads + 2 * num_kv_heads) * 16;
-        lg::rope_kv_write_rows_kernel<<<dim3((unsigned)((quads + 255) / 256)), dim3(256), 0,
+    if (head_dim % 8 == 0 && total_tokens >= lg::kRopeRowsKernelFrom && (align & 15u) == 0) {
+        const int64_t quads = (int64_t)total_tokens * width / 8;
+        const auto kernel = head_dim == 128 ? lg::rope_kv_write_rows_kernel<true>
+                                            : lg::rope_kv_write_rows_kernel<false>;
+        kernel<<<dim3((unsigned)((quads + 255) / 256)), dim3(256), 0,
                                         static_cast<hipStream_t>(stream)>>>(
             static_cast<const float*>(qkv_parts_f32), num_parts, (int64_t)total_tokens * width,
             positions, static_cast<const float*>(cos_f32), static_cast<const float*>(sin_f32),
             slot_mapping, static_cast<__half*>(q_out_f16), static_cast<__half*>(k_pool_f16),
             static_cast<__half*>(v_pool_f16), num_q_heads, num_kv_heads, max_pos,
-            static_cast<const float*>(bias_f32), quads);
+            static_cast<const float*>(bias_f32), quads, head_dim);
         return hipGetLastError();
     }
     dim3 grid(num_q_heads + 2 * num_kv_heads, total_tokens);
@@ -943,14 +965,13 @@ extern "C" logismos_status_t logismos_launch_greedy_f32(const void* logits_f32, 
 hipError_t lg::add_rms_norm_xprep_rows(void* h_f32, const void* parts_f32, int num_parts,
                                        const void* w_f32, void* x_prepared, int rows, int n,
                                        float eps, hipStream_t stream) {
-    if (rows <= 0 || n <= 0 || n % 128 != 0 || n > 8 * lg::kPrepThreads * lg::kPrepMaxPasses)
+    if (rows <= 0 || n <= 0 || n % 128 != 0 || n > lg::kPrepMaxWidth)
         return hipErrorInvalidValue;
     if (!h_f32 || !w_f32 || !x_prepared || num_parts < 0 || (num_parts > 0 && !parts_f32))
         return hipErrorInvalidValue;
-    lg::add_rms_norm_xprep_kernel<false, false><<<dim3(rows), dim3(lg::kPrepThreads), 0, stream>>>(
-        static_cast<float*>(h_f32), static_cast<const float*>(parts_f32), num_parts,
-        (int64_t)rows * n, static_cast<const float*>(w_f32), x_prepared, rows, n, eps, 0);
-    return hipGetLastError();
+    return lg::add_rms_norm_xprep_launch<false, false>(
+        rows, static_cast<float*>(h_f32), static_cast<const float*>(parts_f32), num_parts,
+        static_cast<const float*>(w_f32), x_prepared, rows, n, eps, 0, stream);
 }
 
 extern "C" logismos_status_t logismos_launch_add_rms_norm_f32p_xprep(
@@ -967,7 +988,7 @@ hipError_t lg::add_rms_norm_tall(void* h_f32, const void* parts_f32, int num_par
     if (rows <= 0 || n <= 0 || num_parts < 0 ||
         (pairs_per_load != 1 && pairs_per_load != 2 && pairs_per_load != 4) ||
         n % (pairs_per_load == 1 ? 128 : 256 * pairs_per_load) != 0 ||
-        n > 8 * lg::kPrepThreads * lg::kPrepMaxPasses)
+        n > lg::kPrepMaxWidth)
         return hipErrorInvalidValue;
     const int rows_pad = lg::tall_padded_rows(rows);
     if ((int64_t)rows_pad * n * 2 > (int64_t)INT32_MAX) return hipErrorInvalidValue;
@@ -976,13 +997,10 @@ hipError_t lg::add_rms_norm_tall(void* h_f32, const void* parts_f32, int num_par
     if ((reinterpret_cast<uintptr_t>(h_f32) | reinterpret_cast<uintptr_t>(parts_f32) |
          reinterpret_cast<uintptr_t>(w_f32) | reinterpret_cast<uintptr_t>(workspace)) & 15u)
         return hipErrorInvalidValue;
-    const auto kernel = sum_first && num_parts > 1 ? lg::add_rms_norm_xprep_kernel<true, true>
-                                                   : lg::add_rms_norm_xprep_kernel<true, false>;
-    kernel<<<dim3(rows_pad), dim3(lg::kPrepThreads), 0, stream>>>(
-        static_cast<float*>(h_f32), static_cast<const float*>(parts_f32), num_parts,
-        (int64_t)rows * n, static_cast<const float*>(w_f32), workspace, rows, n, eps,
-        pairs_per_load);
-    return hipGetLastError();
+    const auto launch = sum_first && num_parts > 1 ? lg::add_rms_norm_xprep_launch<true, true>
+                                                   : lg::add_rms_norm_xprep_launch<true, false>;
+    return launch(rows_pad, static_cast<float*>(h_f32), static_cast<const float*>(parts_f32), num_parts,
+                  static_cast<const float*>(w_f32), workspace, rows, n, eps, pairs_per_load, stream);
 }
 
 extern "C" logismos_status_t logismos_launch_add_rms_norm_f32p_tall(
