@@ -744,6 +744,11 @@ hipError_t paged_attn_anydim_launch(const AttnParams& params, int head_dim, int 
     if (p.hq % p.hkv != 0 || p.hq / p.hkv > 16) return hipErrorInvalidValue;
     if (total_tokens > 65520 || p.num_seqs > 65535 || p.hkv > 65535) return hipErrorInvalidValue;
     if (p.out_bf16 != 0 && p.out_bf16 != 1) return hipErrorInvalidValue;
+    if ((phases & LOGISMOS_ATTN_PHASE_PREFILL) && max_seqlen_q > 1 &&
+        paged_attn_chunk64_applies(p, head_dim)) {
+        if (const hipError_t e = paged_attn_chunk64_launch(p, total_tokens, max_seqlen_q, stream)) return e;
+        phases &= ~LOGISMOS_ATTN_PHASE_PREFILL;
+    }
     if (phases & (LOGISMOS_ATTN_PHASE_DECODE | LOGISMOS_ATTN_PHASE_PREFILL)) {
         switch (head_dim / 32) {
             case 1: launch_rows<1>(p, total_tokens, max_seqlen_q, phases, stream); break;

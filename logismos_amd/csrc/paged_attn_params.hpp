@@ -84,6 +84,11 @@ inline bool small_decode_batch(int num_seqs, int num_kv_heads, int block_size,
 hipError_t paged_attn_anydim_launch(const AttnParams& p, int head_dim, int total_tokens,
                                     int max_seqlen_q, int phases, hipStream_t stream);
 
+// Rows of sequences with several new tokens at 64-wide heads (paged_attn_chunk64.hip).
+bool paged_attn_chunk64_applies(const AttnParams& p, int head_dim);
+hipError_t paged_attn_chunk64_launch(const AttnParams& p, int total_tokens, int max_seqlen_q,
+                                     hipStream_t stream);
+
 // Partition count for that kernel (pure host arithmetic).
 int paged_attn_anydim_num_splits(int num_seqs, int num_kv_heads, int head_dim, int block_size,
                                  int max_blocks_per_seq);
