@@ -396,9 +396,10 @@ extern "C" logismos_status_t logismos_launch_decode_step(const logismos_decode_c
         }
         return 0;
     };
-    // attention writes the o projection's input (the prepared layout's groups of 128 are whole
-    // heads only at head_dim 128)
-    const bool direct = one_pass && c.head_dim == 128;
+    // attention writes the o projection's input
+    const bool direct = one_pass && lg::paged_attn_prepared_out(c.head_dim, c.num_q_heads, c.num_kv_heads,
+                                                                c.block_size, c.max_blocks_per_seq, max_q,
+                                                                batch->num_splits);
     float* const h = static_cast<float*>(batch->hidden_f32);
 
     if (tokens_in)

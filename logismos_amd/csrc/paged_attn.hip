@@ -1876,8 +1876,8 @@ logismos_status_t lg::paged_attn_launch(
 
     hipStream_t st = static_cast<hipStream_t>(stream);
     if (head_dim != lg::kHeadDim) {
-        // turbo3 head rows and the prepared output layout are defined for 128-wide heads
-        if (kv_turbo3 || out_bf16 == 2) return hipErrorInvalidValue;
+        // turbo3 head rows are 128 wide
+        if (kv_turbo3) return hipErrorInvalidValue;
         p.num_workers = 0;
         return lg::paged_attn_anydim_launch(p, head_dim, total_tokens, max_seqlen_q, phases, st);
     }

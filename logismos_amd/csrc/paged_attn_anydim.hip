@@ -47,7 +47,7 @@
 namespace lg {
 
 constexpr int kAnyWaves = 8;           // waves of a workgroup: KV heads x tile phases
-constexpr int kAnyLdsBytes = 48 * 1024;  // for the accumulators of the phases beyond the first
+constexpr int kAnyLdsBytes = 48 * 1024;  // for the accumulators of the phases (beyond the first)
 constexpr int kAnyWgHeads = 8;           // KV heads per workgroup at most
 constexpr int kAnyPhases = 8;            // tile phases per head at most
 
@@ -119,14 +119,15 @@ __device__ __forceinline__ int seq_of_row(const int32_t* cu, int num_seqs, int t
 
 // The work of one workgroup on the keys [key_begin, key_end) (not empty) of sequence s for the
 // ntok query tokens from packed row t on: scores, softmax, P.V, the merge of the tile phases,
-// and either the finished rows (single) or the partial (m, l, acc) at workspace slot `slot`.
+// and either the finished rows (single; into out_rows in LDS, a row per head, if given) or the partial
+// (m, l, acc) at workspace slot `slot`.
 // Called by every wave of the workgroup (it holds two barriers).
 template <int NJ, bool NT>
 __device__ __forceinline__ void anydim_range(const AttnParams& p, int G, int wg_heads, int phases,
                                              int cols, int s, int t, int ntok, int vis_first,
                                              int visible, int key_begin, int key_end, bool single,
                                              int64_t slot, float (*sm_m)[16], float (*sm_l)[16],
-                                             float* sm_acc) {
+                                             float* sm_acc, unsigned short* out_rows = nullptr) {
     constexpr int D = 32 * NJ;
     constexpr int E = 2 * NJ;
     constexpr bool kLines = NJ % 2 == 0;  // head rows are whole 128-byte lines
@@ -327,56 +328,90 @@ __device__ __forceinline__ void anydim_range(const AttnParams& p, int G, int wg_
         }
     }
 
-    // ---- the states of a head's phases into its phase 0: M = max m_f, factors 2^(m_f - M).
-    // A wave without a tile has m = -inf, l = 0, acc = 0 and factor 0; phase 0 always has one.
     float lsum = l + lane_xor_f32<16>(l);
     lsum += lane_xor_f32<32>(lsum);
-    if (tg == 0) {
-        sm_m[wave][c] = m;
-        sm_l[wave][c] = lsum;
-    }
-    __syncthreads();
-    float mall = m, lall = 0.0f;
-    for (int f = 0; f < phases; ++f) mall = fmaxf(mall, sm_m[f * wg_heads + wg_head][c]);
-    const float mall_ref = mall == -INFINITY ? 0.0f : mall;
-    for (int f = 0; f < phases; ++f)
-        lall += fast_exp2(sm_m[f * wg_heads + wg_head][c] - mall_ref) *
-                sm_l[f * wg_heads + wg_head][c];
-    const float fown = fast_exp2(m - mall_ref);
-    float fr[4];
+    auto out_row_of = [&](int tq, int head) {
+        return reinterpret_cast<unsigned short*>(p.out) + ((int64_t)(t + tq) * p.hq + head) * D;
+    };
+    if (phases > 1) {
+        // ---- The states of a head's phases meet in LDS: M = max m_f, factors 2^(m_f - M).  A wave
+        // without a tile has m = -inf, l = 0, acc = 0 and factor 0; phase 0 always has one.  Every
+        // phase leaves its scaled accumulators there, and all threads add them up, phase by phase
+        // (by the waves of phase 0 alone, 32 results a lane and phase one behind the other, the
+        // sums took 2.5 us of a 9 us launch).
+        if (tg == 0) {
+            sm_m[wave][c] = m;
+            sm_l[wave][c] = lsum;
+        }
+        __syncthreads();
+        float mall = m, lall = 0.0f;
+        for (int f = 0; f < phases; ++f) mall = fmaxf(mall, sm_m[f * wg_heads + wg_head][c]);
+        const float mall_ref = mall == -INFINITY ? 0.0f : mall;
+        for (int f = 0; f < phases; ++f)
+            lall += fast_exp2(sm_m[f * wg_heads + wg_head][c] - mall_ref) *
+                    sm_l[f * wg_heads + wg_head][c];
+        const float fown = fast_exp2(m - mall_ref);
+        float fr[4];
 #pragma unroll
-    for (int r = 0; r < 4; ++r) fr[r] = lane_read_f32(fown, (lane & 48) | (4 * tg + r));
-    if (phase > 0) {
+        for (int r = 0; r < 4; ++r) fr[r] = lane_read_f32(fown, (lane & 48) | (4 * tg + r));
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
             const int h = 4 * tg + r;  // the column these accumulator rows belong to
             if (h >= ncols) continue;
-            float* dst = sm_acc + (((phase - 1) * wg_heads + wg_head) * cols + h) * D + E * c;
-#pragma unroll
-            for (int e = 0; e < E; ++e) dst[e] = acc[e][r] * fr[r];
+            float* dst = sm_acc + ((phase * wg_heads + wg_head) * cols + h) * D;
+            static_for<E>([&](auto ec) {
+                constexpr int e = decltype(ec)::value;
+                dst[v_chunk_pos(E, e, c) + (e - v_chunk_start(E, e))] = acc[e][r] * fr[r];
+            });
         }
+        __syncthreads();
+        if (phase == 0 && tg == 0) {
+            sm_m[wave][c] = mall;
+            sm_l[wave][c] = lall;
+        }
+        __syncthreads();
+        const int pairs = wg_heads * ncols * (D / 2);
+        for (int i = threadIdx.x; i < pairs; i += 64 * wg_heads * phases) {
+            const int col = i / (D / 2), d = 2 * (i - col * (D / 2));
+            const int wh = col / ncols, h = col - wh * ncols;
+            float a0 = 0.0f, a1 = 0.0f;
+            const float* src = sm_acc + (wh * cols + h) * D + d;
+            for (int f = 0; f < phases; ++f) {
+                a0 += src[0];
+                a1 += src[1];
+                src += wg_heads * cols * D;
+            }
+            const int htok = h / G, head = (blockIdx.y * wg_heads + wh) * G + (h - htok * G);
+            const float lh = sm_l[wh][h];
+            if (single) {
+                const float inv = lh > 0.0f ? 1.0f / lh : 0.0f;  // a token that sees no key: zeros
+                unsigned short* dst = out_rows ? out_rows + (wh * G + h) * D : out_row_of(htok, head);
+                *reinterpret_cast<unsigned*>(dst + d) =
+                    (unsigned)attn_out_elem(a0 * inv, p.out_bf16) |
+                    ((unsigned)attn_out_elem(a1 * inv, p.out_bf16) << 16);
+            } else {
+                const int64_t idx = slot * p.hq + head;
+                *reinterpret_cast<float2*>(p.ws_acc + idx * D + d) = float2{a0, a1};
+                if (d == 0) {
+                    p.ws_ml[idx * 2] = sm_m[wh][h];
+                    p.ws_ml[idx * 2 + 1] = lh;
+                }
+            }
+        }
+        __syncthreads();  // (a worker of the balanced kernel goes on to its next piece)
+        return;
     }
-    __syncthreads();
-    if (phase > 0) return;
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
         const int h = 4 * tg + r;
-        const float mh = lane_read_f32(mall, (lane & 48) | h);
-        const float lh = lane_read_f32(lall, (lane & 48) | h);
+        const float mh = lane_read_f32(m, (lane & 48) | h);
+        const float lh = lane_read_f32(lsum, (lane & 48) | h);
         if (h >= ncols) continue;
-#pragma unroll
-        for (int e = 0; e < E; ++e) {
-            float a = acc[e][r] * fr[r];
-            for (int f = 0; f < phases - 1; ++f)
-                a += sm_acc[((f * wg_heads + wg_head) * cols + h) * D + E * c + e];
-            acc[e][r] = a;
-        }
         const int htok = h / G;
         const int head = kvh * G + (h - htok * G);
         if (single) {
             const float inv = lh > 0.0f ? 1.0f / lh : 0.0f;  // a token that sees no key: zeros
-            unsigned short* dst = reinterpret_cast<unsigned short*>(p.out) +
-                                  ((int64_t)(t + htok) * p.hq + head) * D;
+            unsigned short* dst = out_rows ? out_rows + (wg_head * G + h) * D : out_row_of(htok, head);
             static_for<E / 2>([&](auto ec) {
                 constexpr int e = 2 * decltype(ec)::value;
                 const unsigned w = (unsigned)attn_out_elem(acc[e][r] * inv, p.out_bf16) |
@@ -408,7 +443,7 @@ __global__ __launch_bounds__(64 * kAnyWaves) void paged_attn_anydim_kernel(const
                                                                            int phases, int cols) {
     constexpr int D = 32 * NJ;
     __shared__ float sm_m[kAnyWaves][16], sm_l[kAnyWaves][16];  // [phase * wg_heads + head]
-    extern __shared__ float sm_acc[];  // [phases - 1][wg_heads][cols][D]
+    extern __shared__ float sm_acc[];  // [phases][wg_heads][cols][D]
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int wg_head = wave % wg_heads, phase = wave / wg_heads;
     const int kvh = blockIdx.y * wg_heads + wg_head;
@@ -451,7 +486,7 @@ __global__ __launch_bounds__(64 * kAnyWaves) void paged_attn_anydim_kernel(const
     if (decode_row && p.num_splits > 1) {
         key_begin = split * p.part_tokens;
         key_end = min(visible, key_begin + p.part_tokens);
-        single = visible <= p.part_tokens;
+        single = visible <= p.part_tokens && p.out_bf16 != 2;  // (2: the merge writes every row)
     } else if (split != 0) {
         return;
     }
@@ -474,6 +509,52 @@ __global__ __launch_bounds__(64 * kAnyWaves) void paged_attn_anydim_kernel(const
                             sm_l, sm_acc);
 }
 
+// Decode rows whose contexts are short (kAnyWholeKeys): a workgroup of up to sixteen waves takes the
+// whole context of one sequence for wg_heads KV heads, so that there are no partials and no merge.  A
+// compute unit takes in 25 bytes a clock, so longer contexts are better off in partitions.  24 layers of
+// 14 / 2 heads of 64, us a step, whole / in partitions with their merge: one sequence of 128 keys 579 / 577,
+// of 250 590 / 634, of 380 644 / 618; 8 sequences 613 / 612, 617 / 655, 688 / 672.
+// p.out_bf16 == 2: the rows leave in the prepared layout of the following Q4G128 GEMM (a
+// workgroup's heads are whole groups of 128 columns).
+// grid (1, KV-head groups, sequences).
+constexpr int kAnyWholeWaves = 16;
+constexpr int kAnyWholeKeys = 256;  // longest context a block table may hold
+template <int NJ>
+__global__ __launch_bounds__(64 * kAnyWholeWaves) void paged_attn_anydim_whole_kernel(
+    const AttnParams p, int G, int wg_heads, int phases) {
+    constexpr int D = 32 * NJ;
+    __shared__ float sm_m[kAnyWholeWaves][16], sm_l[kAnyWholeWaves][16];
+    __shared__ __attribute__((aligned(16))) unsigned short rows[2 * 16 * D];
+    extern __shared__ float sm_acc[];  // [phases][wg_heads][G][D]
+    const int s = blockIdx.z;
+    const int t = p.cu_seqlens_q[s];
+    if (p.cu_seqlens_q[s + 1] - t != 1) return;
+    const int ctx = p.context_lens[s];
+    const int width = wg_heads * G * D;  // this workgroup's columns of the row
+    const int64_t col0 = (int64_t)blockIdx.y * width;
+    const bool prepared = p.out_bf16 == 2;
+    if (ctx <= 0) {
+        if (prepared)
+            for (int i = threadIdx.x; i < width; i += blockDim.x) rows[i] = 0;
+        else
+            for (int i = threadIdx.x; i < width; i += blockDim.x)
+                reinterpret_cast<unsigned short*>(p.out)[(int64_t)t * p.hq * D + col0 + i] = 0;
+    } else {
+        anydim_range<NJ, false>(p, G, wg_heads, phases, G, s, t, 1, ctx, ctx, 0, ctx, true, 0, sm_m, sm_l,
+                                sm_acc, prepared ? rows : nullptr);
+    }
+    if (!prepared) return;
+    __syncthreads();
+    const int c = threadIdx.x;
+    if (c >= width / 8) return;  // (whole rows of 16 lanes: a multiple of 128 columns)
+    const uint4_t o = reinterpret_cast<const uint4_t*>(rows)[c];
+    const float gs = row16_sum(sum8_bf16(o));
+    const XprepRow at = xprep_row(p.out, p.out_rows, p.hq * D, t);
+    const int64_t chunk = col0 / 8 + c;
+    at.xp[chunk * at.bp] = pair_order(o);
+    if ((c & 15) == 0) at.xg[(chunk >> 4) * at.bp] = gs;
+}
+
 // Decode rows, balanced: the 16-key tiles of all decode sequences form one stream (each
 // sequence preceded by kSeqStartUnits units for starting it); worker w (grid.x) takes the units
 // [wR, (w + 1)R), R = ceil(total / workers), whichever sequences they belong to, so every
@@ -485,7 +566,7 @@ __global__ __launch_bounds__(64 * kAnyWaves) void paged_attn_anydim_balanced_ker
     const AttnParams p, int G, int wg_heads, int phases) {
     __shared__ int pt[kMaxBalancedSeqs + 1];  // exclusive prefix of the sequences' units
     __shared__ float sm_m[kAnyWaves][16], sm_l[kAnyWaves][16];
-    extern __shared__ float sm_acc[];  // [phases - 1][wg_heads][G][D]
+    extern __shared__ float sm_acc[];  // [phases][wg_heads][G][D]
     const int lane = threadIdx.x & 63;
     const int S = p.num_seqs;
     if (threadIdx.x < 64) {
@@ -538,7 +619,7 @@ __global__ __launch_bounds__(64 * kAnyWaves) void paged_attn_anydim_balanced_ker
         const int tile_hi = seg_end - seq_begin - kSeqStartUnits;
         if (tile_hi > tile_lo) {
             const int ctx = p.context_lens[s];
-            const bool single = tile_lo == 0 && seg_end == seq_end;
+            const bool single = tile_lo == 0 && seg_end == seq_end && p.out_bf16 != 2;
             // (inlined: as a call the body needs its frame in scratch memory; four tile buffers
             // instead of two measured no faster at head_dim 64, 46.8 vs 45.6 us)
             // Non-temporal K/V loads where every request covers whole 128-byte lines: head_dim
@@ -551,6 +632,104 @@ __global__ __launch_bounds__(64 * kAnyWaves) void paged_attn_anydim_balanced_ker
                              (int64_t)w + s, sm_m, sm_l, sm_acc);
         }
         ucur = seg_end;
+    }
+}
+
+// Partials of sequence s (0: no key) and the slot of the first one.  Called by 256 threads (it holds a
+// barrier).
+__device__ __forceinline__ int anydim_partials(const AttnParams& p, int s, int ctx, int64_t& slot0) {
+    const int tid = threadIdx.x;
+    if (p.num_workers <= 0) {
+        slot0 = (int64_t)s * p.num_splits;
+        return ctx <= 0 ? 0 : (ctx + p.part_tokens - 1) / p.part_tokens;
+    }
+    // balanced split: where this sequence sits in the stream of units
+    __shared__ int red[2][4];
+    int before = 0, total = 0;
+    for (int i = tid; i < p.num_seqs; i += 256) {
+        const int nt = decode_tiles(p, i);
+        total += nt;
+        before += i < s ? nt : 0;
+    }
+#pragma unroll
+    for (int mask = 32; mask >= 1; mask >>= 1) {
+        total += __shfl_xor(total, mask, 64);
+        before += __shfl_xor(before, mask, 64);
+    }
+    if ((tid & 63) == 0) {
+        red[0][tid >> 6] = total;
+        red[1][tid >> 6] = before;
+    }
+    __syncthreads();
+    total = red[0][0] + red[0][1] + red[0][2] + red[0][3];
+    before = red[1][0] + red[1][1] + red[1][2] + red[1][3];
+    if (ctx <= 0) return 0;
+    // its tiles are the units [before + kSeqStartUnits, before + nt)
+    const int nt = (ctx + kTileKeys - 1) / kTileKeys + kSeqStartUnits;
+    const int R = worker_tiles(total, p.num_workers);
+    const int w_first = (before + kSeqStartUnits) / R;
+    slot0 = (int64_t)w_first + s;
+    return (before + nt - 1) / R - w_first + 1;
+}
+
+// The same as the operand of the following Q4G128 GEMM (p.out_bf16 == 2, head widths that divide 128;
+// then every decode row has its partials here, also a single one): a workgroup takes the 128 columns of
+// one group, i.e. 128 / D heads; thread = (stripe of four, element pair).  One launch less, 2.4 us a
+// layer for one sequence of 14 heads of 64.  grid (groups, num_seqs).
+__global__ __launch_bounds__(256) void paged_attn_anydim_merge_prepared_kernel(const AttnParams p, int D) {
+    __shared__ float sm_w[8][2];           // [head of the group][max m, sum]
+    __shared__ float sm_a[4][128], sm_l[4][64];
+    __shared__ __attribute__((aligned(16))) unsigned short row[128];
+    const int s = blockIdx.y, tid = threadIdx.x;
+    const int t = p.cu_seqlens_q[s];
+    if (p.cu_seqlens_q[s + 1] - t != 1) return;
+    int64_t slot0 = 0;
+    const int parts = anydim_partials(p, s, p.context_lens[s], slot0);
+    const int heads = 128 / D, head0 = blockIdx.x * heads;
+    // every head's maximum: a wave a head
+    for (int i = tid >> 6; i < heads; i += 4) {
+        float mmax = -INFINITY;
+        for (int q = tid & 63; q < parts; q += 64)
+            mmax = fmaxf(mmax, p.ws_ml[((slot0 + q) * p.hq + head0 + i) * 2]);
+#pragma unroll
+        for (int o = 1; o < 64; o <<= 1) mmax = fmaxf(mmax, shfl_xor_f32(mmax, o));
+        if ((tid & 63) == 0) sm_w[i][0] = mmax;
+    }
+    __syncthreads();
+    const int stripe = tid >> 6, pair = tid & 63;
+    const int hd = 2 * pair / D, d = 2 * pair - hd * D, head = head0 + hd;
+    const float mmax = sm_w[hd][0];
+    float a0 = 0.0f, a1 = 0.0f, lt = 0.0f;
+    for (int q = stripe; q < parts; q += 4) {
+        const int64_t idx = (slot0 + q) * p.hq + head;
+        const float w = fast_exp2(p.ws_ml[idx * 2] - mmax);
+        lt += w * p.ws_ml[idx * 2 + 1];
+        const float2 a = *reinterpret_cast<const float2*>(p.ws_acc + idx * D + d);
+        a0 += w * a.x;
+        a1 += w * a.y;
+    }
+    sm_a[stripe][2 * pair] = a0;
+    sm_a[stripe][2 * pair + 1] = a1;
+    sm_l[stripe][pair] = lt;
+    __syncthreads();
+    if (stripe == 0) {
+#pragma unroll
+        for (int j = 1; j < 4; ++j) {
+            a0 += sm_a[j][2 * pair];
+            a1 += sm_a[j][2 * pair + 1];
+            lt += sm_l[j][pair];
+        }
+        const float inv = lt > 0.0f ? 1.0f / lt : 0.0f;  // no key: zeros
+        *reinterpret_cast<unsigned*>(row + 2 * pair) =
+            (unsigned)attn_out_elem(a0 * inv, 1) | ((unsigned)attn_out_elem(a1 * inv, 1) << 16);
+        asm volatile("" ::: "memory");  // (one wave: its LDS accesses stay in this order)
+        const uint4_t o = reinterpret_cast<const uint4_t*>(row)[tid & 15];
+        const float gs = row16_sum(sum8_bf16(o));
+        if (tid < 16) {
+            const XprepRow at = xprep_row(p.out, p.out_rows, p.hq * D, t);
+            at.xp[(int64_t)(blockIdx.x * 16 + tid) * at.bp] = pair_order(o);
+            if (tid == 0) at.xg[(int64_t)blockIdx.x * at.bp] = gs;
+        }
     }
 }
 
@@ -567,45 +746,14 @@ __global__ __launch_bounds__(256) void paged_attn_anydim_merge_kernel(const Attn
     if (p.cu_seqlens_q[s + 1] - t != 1) return;
     const int ctx = p.context_lens[s];
     const int tid = threadIdx.x;
-    int parts;      // partials of this sequence
-    int64_t slot0;  // of its first partial
-    if (p.num_workers > 0) {
-        // balanced split: where this sequence sits in the stream of units
-        __shared__ int red[2][4];
-        int before = 0, total = 0;
-        for (int i = tid; i < p.num_seqs; i += 256) {
-            const int nt = decode_tiles(p, i);
-            total += nt;
-            before += i < s ? nt : 0;
-        }
-#pragma unroll
-        for (int mask = 32; mask >= 1; mask >>= 1) {
-            total += __shfl_xor(total, mask, 64);
-            before += __shfl_xor(before, mask, 64);
-        }
-        if ((tid & 63) == 0) {
-            red[0][tid >> 6] = total;
-            red[1][tid >> 6] = before;
-        }
-        __syncthreads();
-        total = red[0][0] + red[0][1] + red[0][2] + red[0][3];
-        before = red[1][0] + red[1][1] + red[1][2] + red[1][3];
-        if (ctx <= 0) {
-            // the stream has no tile of this row and nobody wrote it: a row of zeros
-            if (2 * tid < D)
-                *reinterpret_cast<unsigned*>(reinterpret_cast<unsigned short*>(p.out) +
-                                             ((int64_t)t * p.hq + head) * D + 2 * tid) = 0u;
-            return;
-        }
-        // its tiles are the units [before + kSeqStartUnits, before + nt)
-        const int nt = (ctx + kTileKeys - 1) / kTileKeys + kSeqStartUnits;
-        const int R = worker_tiles(total, p.num_workers);
-        const int w_first = (before + kSeqStartUnits) / R;
-        parts = (before + nt - 1) / R - w_first + 1;
-        slot0 = (int64_t)w_first + s;
-    } else {
-        parts = ctx <= 0 ? 0 : (ctx + p.part_tokens - 1) / p.part_tokens;
-        slot0 = (int64_t)s * p.num_splits;
+    int64_t slot0 = 0;  // of its first partial
+    const int parts = anydim_partials(p, s, ctx, slot0);
+    if (parts == 0 && p.num_workers > 0) {
+        // the stream has no tile of this row and nobody wrote it: a row of zeros
+        if (2 * tid < D)
+            *reinterpret_cast<unsigned*>(reinterpret_cast<unsigned short*>(p.out) +
+                                         ((int64_t)t * p.hq + head) * D + 2 * tid) = 0u;
+        return;
     }
     if (parts <= 1) return;  // zero or one partial: already final
     float mmax = -INFINITY;
@@ -648,36 +796,78 @@ __global__ __launch_bounds__(256) void paged_attn_anydim_merge_kernel(const Attn
                                  ((int64_t)t * p.hq + head) * D + 2 * pair) = w;
 }
 
+// Whether the decode rows of a launch take whole contexts (heads of up to 64: the accumulators of
+// sixteen waves), and then the KV heads of a workgroup.
+static int anydim_whole_heads(int head_dim, int hq, int hkv, int block_size, int max_blocks_per_seq) {
+    if (head_dim > 64 || (int64_t)block_size * max_blocks_per_seq > kAnyWholeKeys) return 0;
+    return hkv % 2 == 0 ? 2 : 1;
+}
+
+bool paged_attn_prepared_out(int head_dim, int hq, int hkv, int block_size, int max_blocks_per_seq,
+                             int max_seqlen_q, int num_splits) {
+    if (head_dim == 128) return true;
+    if (max_seqlen_q != 1 || (int64_t)hq * head_dim % 128 != 0) return false;
+    if (const int heads = anydim_whole_heads(head_dim, hq, hkv, block_size, max_blocks_per_seq))
+        return (int64_t)hq / hkv * heads * head_dim % 128 == 0;
+    return 128 % head_dim == 0 && num_splits > 1;  // the merge writes it
+}
+
+// Tile phases of a workgroup (a power of two) with `waves` waves at most, and the LDS they meet in.
+struct AnyPhases {
+    int count;
+    size_t lds;
+};
+static AnyPhases anydim_phases(int wg_heads, int cols, int head_dim, int waves) {
+    const size_t bytes = (size_t)wg_heads * cols * head_dim * sizeof(float);
+    int n = 1;
+    while (n * 2 <= kAnyPhases && n * 2 * wg_heads <= waves &&
+           (size_t)(n * 2 - 1) * bytes <= (size_t)kAnyLdsBytes)
+        n *= 2;
+    return {n, n > 1 ? n * bytes : 0};
+}
+constexpr int kAnyMaxLds = 2 * kAnyLdsBytes;  // (2 n / (2 n - 1) of the budget at most)
+template <typename K>
+static hipError_t anydim_allow_lds(K kernel) {
+    return hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
+                               hipFuncAttributeMaxDynamicSharedMemorySize, kAnyMaxLds);
+}
+
 template <int NJ>
-static void launch_rows(const AttnParams& p, int total_tokens, int max_seqlen_q, int phases,
-                 hipStream_t stream) {
+static hipError_t launch_whole(const AttnParams& p, int wg_heads, hipStream_t stream) {
     const int g = p.hq / p.hkv;
-    // waves of a workgroup: KV heads first, the rest as tile phases (a power of two) as far as
+    static const hipError_t opt = anydim_allow_lds(paged_attn_anydim_whole_kernel<NJ>);
+    if (opt != hipSuccess) return opt;
+    const AnyPhases ph = anydim_phases(wg_heads, g, 32 * NJ, kAnyWholeWaves);
+    paged_attn_anydim_whole_kernel<NJ>
+        <<<dim3(1, p.hkv / wg_heads, p.num_seqs), dim3(64 * wg_heads * ph.count), ph.lds, stream>>>(
+            p, g, wg_heads, ph.count);
+    return hipGetLastError();
+}
+
+template <int NJ>
+static hipError_t launch_rows(const AttnParams& p, int total_tokens, int max_seqlen_q, int phases,
+                              hipStream_t stream) {
+    const int g = p.hq / p.hkv;
+    static const hipError_t opt = anydim_allow_lds(paged_attn_anydim_kernel<NJ>);
+    static const hipError_t opt_b = anydim_allow_lds(paged_attn_anydim_balanced_kernel<NJ>);
+    if (opt != hipSuccess || opt_b != hipSuccess) return opt != hipSuccess ? opt : opt_b;
+    // waves of a workgroup: KV heads first, the rest as tile phases as far as
     // their accumulators fit the LDS budget
     const int wg_heads = anydim_wg_heads(p.hkv);
     // (cols: the columns a wave's accumulators cover -- a decode row's group, or the
     // 16 / G tokens of a chunk times the group)
     auto launch = [&](int grid_x, int grid_z, int decode_rows, int cols, int wg_heads) {
-        const size_t phase_bytes = (size_t)wg_heads * cols * (32 * NJ) * sizeof(float);
-        int tile_phases = 1;
-        while (tile_phases * 2 <= kAnyPhases && tile_phases * 2 * wg_heads <= kAnyWaves &&
-               (size_t)(tile_phases * 2 - 1) * phase_bytes <= (size_t)kAnyLdsBytes)
-            tile_phases *= 2;
-        const size_t lds = (size_t)(tile_phases - 1) * phase_bytes;
+        const AnyPhases ph = anydim_phases(wg_heads, cols, 32 * NJ, kAnyWaves);
         paged_attn_anydim_kernel<NJ>
-            <<<dim3(grid_x, p.hkv / wg_heads, grid_z), dim3(64 * wg_heads * tile_phases), lds,
-               stream>>>(p, g, decode_rows, wg_heads, tile_phases, cols);
+            <<<dim3(grid_x, p.hkv / wg_heads, grid_z), dim3(64 * wg_heads * ph.count), ph.lds, stream>>>(
+                p, g, decode_rows, wg_heads, ph.count, cols);
     };
     if (phases & LOGISMOS_ATTN_PHASE_DECODE) {
         if (p.num_workers > 0) {
-            const size_t phase_bytes = (size_t)wg_heads * g * (32 * NJ) * sizeof(float);
-            int tile_phases = 1;
-            while (tile_phases * 2 <= kAnyPhases && tile_phases * 2 * wg_heads <= kAnyWaves &&
-                   (size_t)(tile_phases * 2 - 1) * phase_bytes <= (size_t)kAnyLdsBytes)
-                tile_phases *= 2;
+            const AnyPhases ph = anydim_phases(wg_heads, g, 32 * NJ, kAnyWaves);
             paged_attn_anydim_balanced_kernel<NJ>
-                <<<dim3(p.num_workers, p.hkv / wg_heads), dim3(64 * wg_heads * tile_phases),
-                   (size_t)(tile_phases - 1) * phase_bytes, stream>>>(p, g, wg_heads, tile_phases);
+                <<<dim3(p.num_workers, p.hkv / wg_heads), dim3(64 * wg_heads * ph.count), ph.lds, stream>>>(
+                    p, g, wg_heads, ph.count);
         } else {
             launch(p.num_splits, p.num_seqs, 1, g, wg_heads);
         }
@@ -687,6 +877,7 @@ static void launch_rows(const AttnParams& p, int total_tokens, int max_seqlen_q,
     if ((phases & LOGISMOS_ATTN_PHASE_PREFILL) && max_seqlen_q > 1)
         launch(1, (total_tokens + 16 / g - 1) / (16 / g) * (16 / g), 0, (16 / g) * g,
                wg_heads % 2 == 0 ? 2 : 1);
+    return hipGetLastError();
 }
 
 // Workers of a balanced launch per group of KV heads: one workgroup per CU (narrow heads fit
@@ -743,27 +934,46 @@ hipError_t paged_attn_anydim_launch(const AttnParams& params, int head_dim, int 
     if (head_dim <= 0 || head_dim % 32 != 0 || head_dim > 256) return hipErrorInvalidValue;
     if (p.hq % p.hkv != 0 || p.hq / p.hkv > 16) return hipErrorInvalidValue;
     if (total_tokens > 65520 || p.num_seqs > 65535 || p.hkv > 65535) return hipErrorInvalidValue;
-    if (p.out_bf16 != 0 && p.out_bf16 != 1) return hipErrorInvalidValue;
+    const int whole = phases & LOGISMOS_ATTN_PHASE_DECODE && phases & LOGISMOS_ATTN_PHASE_MERGE
+                          ? anydim_whole_heads(head_dim, p.hq, p.hkv, p.block_size, p.max_blocks_per_seq)
+                          : 0;
+    if (p.out_bf16 == 2 &&
+        !(phases == LOGISMOS_ATTN_PHASE_ALL &&
+          paged_attn_prepared_out(head_dim, p.hq, p.hkv, p.block_size, p.max_blocks_per_seq,
+                                  max_seqlen_q, p.num_splits)))
+        return hipErrorInvalidValue;
+    if (p.out_bf16 < 0 || p.out_bf16 > 2) return hipErrorInvalidValue;
+    if (whole > 0) {
+        if (const hipError_t e = head_dim == 32 ? launch_whole<1>(p, whole, stream)
+                                                : launch_whole<2>(p, whole, stream))
+            return e;
+        phases &= ~(LOGISMOS_ATTN_PHASE_DECODE | LOGISMOS_ATTN_PHASE_MERGE);
+    }
     if ((phases & LOGISMOS_ATTN_PHASE_PREFILL) && max_seqlen_q > 1 &&
         paged_attn_chunk64_applies(p, head_dim)) {
         if (const hipError_t e = paged_attn_chunk64_launch(p, total_tokens, max_seqlen_q, stream)) return e;
         phases &= ~LOGISMOS_ATTN_PHASE_PREFILL;
     }
     if (phases & (LOGISMOS_ATTN_PHASE_DECODE | LOGISMOS_ATTN_PHASE_PREFILL)) {
+        hipError_t e = hipSuccess;
         switch (head_dim / 32) {
-            case 1: launch_rows<1>(p, total_tokens, max_seqlen_q, phases, stream); break;
-            case 2: launch_rows<2>(p, total_tokens, max_seqlen_q, phases, stream); break;
-            case 3: launch_rows<3>(p, total_tokens, max_seqlen_q, phases, stream); break;
-            case 4: launch_rows<4>(p, total_tokens, max_seqlen_q, phases, stream); break;
-            case 5: launch_rows<5>(p, total_tokens, max_seqlen_q, phases, stream); break;
-            case 6: launch_rows<6>(p, total_tokens, max_seqlen_q, phases, stream); break;
-            case 7: launch_rows<7>(p, total_tokens, max_seqlen_q, phases, stream); break;
-            default: launch_rows<8>(p, total_tokens, max_seqlen_q, phases, stream); break;
+            case 1: e = launch_rows<1>(p, total_tokens, max_seqlen_q, phases, stream); break;
+            case 2: e = launch_rows<2>(p, total_tokens, max_seqlen_q, phases, stream); break;
+            case 3: e = launch_rows<3>(p, total_tokens, max_seqlen_q, phases, stream); break;
+            case 4: e = launch_rows<4>(p, total_tokens, max_seqlen_q, phases, stream); break;
+            case 5: e = launch_rows<5>(p, total_tokens, max_seqlen_q, phases, stream); break;
+            case 6: e = launch_rows<6>(p, total_tokens, max_seqlen_q, phases, stream); break;
+            case 7: e = launch_rows<7>(p, total_tokens, max_seqlen_q, phases, stream); break;
+            default: e = launch_rows<8>(p, total_tokens, max_seqlen_q, phases, stream); break;
         }
+        if (e != hipSuccess) return e;
     }
     if ((phases & LOGISMOS_ATTN_PHASE_MERGE) && p.num_splits > 1) {
-        dim3 grid(p.hq, p.num_seqs);
-        paged_attn_anydim_merge_kernel<<<grid, dim3(256), 0, stream>>>(p, head_dim);
+        if (p.out_bf16 == 2)
+            paged_attn_anydim_merge_prepared_kernel<<<dim3(p.hq * head_dim / 128, p.num_seqs), dim3(256),
+                                                      0, stream>>>(p, head_dim);
+        else
+            paged_attn_anydim_merge_kernel<<<dim3(p.hq, p.num_seqs), dim3(256), 0, stream>>>(p, head_dim);
     }
     return hipGetLastError();
 }
