@@ -368,9 +368,10 @@ bool paged_attn_chunk64_applies(const AttnParams& p, int head_dim) {
 hipError_t paged_attn_chunk64_launch(const AttnParams& p, int total_tokens, int max_seqlen_q,
                                      hipStream_t stream) {
     // By how many groups of 128 columns there are (if all rows are chunks').  us of a launch, CW = 4 / 2 /
-    // 1 (the general kernel 34 / 27 at the first two):
-    //   2 x 512 tokens (112 groups), contexts to 1500: 29.8 / 20.8 / 26.0
-    //   8 x 512 (448), contexts to 4600: 116 / 131 / 157      1 x 20 (2), a context of 4000: 46 / 30 / 23
+    // 1, the general kernel:
+    //   8 x 512 tokens (448 groups), contexts to 4600: 116 / 131 / 157, 257
+    //   2 x 512 (112), contexts to 1500:               29.8 / 20.8 / 26.0, 36
+    //   1 x 20 (2), a context of 4000:                 46 / 30 / 23, 34
     const int64_t groups = (int64_t)total_tokens * p.hq / 128;
     const int64_t cus = device_cu_count();
     if (groups >= cus) return launch_chunk64<4, 1>(p, max_seqlen_q, stream);

@@ -206,9 +206,9 @@ __device__ __forceinline__ float tp_group_sum(const float (&cs)[4][4]) {
 // ODD (W = 1): an odd number of groups.  Rows of scales are then only 2-byte aligned and come
 // as halves; the last pair has one group.  The zero-point term is taken off group by group, halfway
 // through a group's columns: error against 64 bits at 896 columns 5.3e-7, 9.7e-7 with a term per pair
-// as below, 6.5e-7 on the kernel of qgemm_q4_tall.hip.  1030 rows x 896 (seven groups): 9728 gate/up rows with the activation 43.6 us, 52.6
-// + 11.0 on the kernel of qgemm_q4_tall.hip with the activation behind it; 1152 rows of q/k/v
-// 13.3 (24.5), both on the smaller tiles of `tp_less`.
+// as below, 6.5e-7 on the kernel of qgemm_q4_tall.hip.  1030 rows x 896 (seven groups): 9728 gate/up
+// rows with the activation 39.7 us, 52.6 + 11.0 on the kernel of qgemm_q4_tall.hip with the activation
+// behind it; 1152 rows of q/k/v 13.5 (24.5), both on the smaller tiles of `tp_less`.
 template <int OUT, int W, bool ODD, class T>
 __global__ __launch_bounds__(64 * T::kWaves) void qgemm_q4g128_tallp_kernel(
     const uint16_t* __restrict__ xp, const float* __restrict__ xs, const uint8_t* __restrict__ qw,
@@ -859,20 +859,18 @@ static TpPlan tp_big_plan(int m, int n, int k, int block_groups, int cus) {
                    cus);
 }
 
-// Whether a launch takes the smaller tiles.  A 128 x 256 tile costs about 7 us + 2 us per group
-// whatever else runs, a 64 x 128 one 4 us + 1 us (a chain of requests, barriers and operand reads,
-// not arithmetic), so with few groups of K and few tiles the smaller ones win by filling the chip.
-// us, 128 x 256 / 64 x 128 (the first with the sum of its K parts):
-//   K  768, 1152 columns:  100 rows 19.1 / 11.0, 1030 20.2 / 11.6, 2060 20.7 / 15.5, 4120 22.2 / 24.7
-//   K 1536, 1536 columns:  100 rows 13.0 / 15.5,  520 19.3 / 16.9, 2060 29.5 / 23.7, 4120 31.3 / 40.2
-//   K 4096, 4096 columns:  300 rows 29.8 / 31.4, 1030 58.8 / 63.7
-// hence: at most 16 groups, all tiles resident at once (two per compute unit), and where the big
-// tiles could be split over K at least 20 of them.  A next product's operand is written by
-// 64 x 256 tiles, one per compute unit, whose round takes five eighths of a big one's (a last round
-// that is split over K about six of them):
-//   K  768, 4864 outputs:  200 rows 18.9 / 12.7,  520 19.9 / 24.4, 1030 38.2 / 36.2, 2060 56.7 / 69.7
-//   K 1536, 8960 outputs:  100 rows 24.9 / 19.2,  200 28.4 / 37.3,  500 50.2 / 58.6, 1030 82.9 / 91.0
-//   K 2048, 6144 outputs:  700 rows 59.3 / 66.3 (288 tiles: one round and 32 split ones)
+// Whether a launch takes the smaller tiles.  A 128 x 256 tile takes about 1.8 us a group of 128 columns
+// whatever else runs, so with few groups of K and few tiles the smaller ones win by filling the chip.
+// us, 128 x 256 / 64 x 128 (the first with the sum of its K parts, both at K 896 with the first pass
+// over x):
+//   K  896, 1152 columns:  100 rows 23.2 / 13.9, 1030 26.4 / 17.0, 2060 29.1 / 21.7, 4120 32.4 / 33.3
+//   K 1536, 2048 columns:  100 rows 13.1 / 13.4,  520 20.6 / 14.4, 1030 23.6 / 17.1, 2060 28.5 / 29.7
+// hence: at most 16 groups (at 32 a small tile's chain costs what the large one's parts do), all tiles
+// resident at once (two per compute unit), and where the big tiles could be split over K at least 20 of
+// them.  A next product's operand is written by 64 x 256 tiles, one per compute unit, whose round takes
+// five eighths of a big one's (a last round that is split over K about six of them):
+//   K  896, 4864 outputs:  195 rows 23.4 / 15.7,  520 25.2 / 28.2, 1030 45.8 / 40.8, 2060 69.4 / 77.4
+//   K 1536, 8960 outputs:  100 rows 23.6 / 16.8,  195 25.5 / 31.9,  300 28.3 / 33.9, 2060 148 / 168
 // Whole large tiles in front of split ones keep the large tiles (none of the above is lost by it), so
 // that a launch on the smaller ones adds up all of its tiles alike.
 template <int OUT>
