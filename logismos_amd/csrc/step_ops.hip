@@ -136,6 +136,22 @@ __global__ __launch_bounds__(kNormThreads) void add_rms_norm_kernel(
 // of squares adds up alike: threads past the row only ever add zeros.
 constexpr int kPrepMaxWidth = 8 * 512 * 4;
 
+// The row of a workgroup where rows leave in the prepared layout: 16 bytes of a row lie next to 16 of the
+// next one, so that the rows of a line are written from one XCD (workgroups go round the eight in
+// turn): of each chunk of 32 rows a run of neighbours.  -1: none (the last run may be short).  48 rows of
+// 4096: 4.8 -> 4.6 us a launch.
+constexpr int kXcds = 8;
+__host__ __device__ inline int norm_run(int rows_in_chunk) { return (rows_in_chunk + kXcds - 1) / kXcds; }
+__device__ __forceinline__ int norm_row(int b, int rows) {
+    const int base = b / kXprepChunkRows * kXprepChunkRows;
+    const int have = min(rows - base, kXprepChunkRows), run = norm_run(have);
+    const int i = b - base, r = i % kXcds * run + i / kXcds;
+    return r < have ? base + r : -1;
+}
+static int norm_grid(int rows) {
+    return rows / kXprepChunkRows * kXprepChunkRows + kXcds * norm_run(rows % kXprepChunkRows);
+}
+
 // TALL: the normed rows leave as the operand of the tiled GEMM for many rows instead
 // (q4_common.hpp: row-major in pair order, `pairs` pairs of groups per block of sums; the grid
 // covers the rows padded to the GEMM's 128-row tiles, and a padding row is written as zeros).
@@ -144,7 +160,10 @@ __global__ __launch_bounds__(kPrepThreads) void add_rms_norm_xprep_kernel(
     float* __restrict__ h, const float* __restrict__ yp, int num_parts, int64_t part_stride,
     const float* __restrict__ w, void* __restrict__ xprep, int rows, int n, float eps,
     int pairs) {
-    const int64_t row = blockIdx.x;
+    const int64_t row = TALL ? (int64_t)blockIdx.x : norm_row(blockIdx.x, rows);
+    if constexpr (!TALL) {
+        if (row < 0) return;
+    }
     if constexpr (TALL) {
         if (row >= rows) {
             uint4_t* xt = reinterpret_cast<uint4_t*>(xprep) + row * (n >> 3);
@@ -265,15 +284,17 @@ static hipError_t add_rms_norm_xprep_launch(int grid, float* h, const float* par
 }
 
 // act = silu(gate) * up from the fp32 parts of the gate_up GEMM, written in the
-// prepared layout of the down projection.  One thread per 8 outputs.
+// prepared layout of the down projection.  One thread per 8 outputs, a workgroup per 16 rows of a group of
+// 128 columns: 16 bytes of a row lie next to 16 of the next one, and a workgroup of one row's chunks
+// wrote a sixteenth of every line it touched (48 rows of 12288: 5.7 -> 5.0 us; with the norms' order of rows
+// steps of 17 to 96 rows 0.4-1.5 % faster).
 __global__ __launch_bounds__(256) void silu_mul_xprep_kernel(const float* __restrict__ parts,
                                                              int num_parts, int64_t part_stride,
                                                              void* __restrict__ xprep, int rows,
                                                              int inter) {
-    const int chunks = inter >> 3;
-    const int idx = blockIdx.x * 256 + threadIdx.x;
-    const int t = idx / chunks, c = idx - t * chunks;
-    const bool live = t < rows;  // uniform over groups of 16 threads (inter % 128 == 0)
+    const int c = blockIdx.x * 16 + (threadIdx.x & 15);
+    const int t = blockIdx.y * 16 + (threadIdx.x >> 4);
+    const bool live = t < rows;  // uniform over groups of 16 threads
     uint4_t o = {0u, 0u, 0u, 0u};
     if (live) {
         float g[8], u[8];
@@ -970,7 +991,7 @@ hipError_t lg::add_rms_norm_xprep_rows(void* h_f32, const void* parts_f32, int n
     if (!h_f32 || !w_f32 || !x_prepared || num_parts < 0 || (num_parts > 0 && !parts_f32))
         return hipErrorInvalidValue;
     return lg::add_rms_norm_xprep_launch<false, false>(
-        rows, static_cast<float*>(h_f32), static_cast<const float*>(parts_f32), num_parts,
+        lg::norm_grid(rows), static_cast<float*>(h_f32), static_cast<const float*>(parts_f32), num_parts,
         static_cast<const float*>(w_f32), x_prepared, rows, n, eps, 0, stream);
 }
 
@@ -1017,8 +1038,7 @@ hipError_t lg::silu_mul_xprep_rows(const void* parts_f32, int num_parts, void* x
         (int64_t)rows * inter * 2 > (int64_t)INT32_MAX)
         return hipErrorInvalidValue;
     if (!parts_f32 || !x_prepared) return hipErrorInvalidValue;
-    const int items = rows * (inter / 8);
-    lg::silu_mul_xprep_kernel<<<dim3((items + 255) / 256), dim3(256), 0, stream>>>(
+    lg::silu_mul_xprep_kernel<<<dim3(inter / 128, (rows + 15) / 16), dim3(256), 0, stream>>>(
         static_cast<const float*>(parts_f32), num_parts, (int64_t)rows * 2 * inter, x_prepared, rows,
         inter);
     return hipGetLastError();
