@@ -1,7 +1,6 @@
 """The norm and the activation that write the prepared layout at every kind of row count: each row exactly
-once, bit for bit what the plain activation gives (the norm
-within a rounding of the oracle), and nothing in the places of
-rows that there are not."""
+once, the norm within a rounding of the oracle, the activation bit for bit the plain one's, and nothing in
+the places of rows that there are not."""
 import numpy as np
 import pytest
 
