@@ -867,7 +867,8 @@ static TpPlan tp_big_plan(int m, int n, int k, int block_groups, int cus) {
 //   K 1536, 2048 columns:  100 rows 13.1 / 13.4,  520 20.6 / 14.4, 1030 23.6 / 17.1, 2060 28.5 / 29.7
 // hence: at most 16 groups (at 32 a small tile's chain costs what the large one's parts do), all tiles
 // resident at once (two per compute unit), and where the big tiles could be split over K at least 20 of
-// them.  A next product's operand is written by 64 x 256 tiles, one per compute unit, whose round takes
+// them (2048 columns at 200 rows are 16: 15.1 / 13.7 us by themselves, but in a step the parts go to the
+// next operator without a sum of their own, and 28 layers of 1536 take 3418 / 3491 us).  A next product's operand is written by 64 x 256 tiles, one per compute unit, whose round takes
 // five eighths of a big one's (a last round that is split over K about six of them):
 //   K  896, 4864 outputs:  195 rows 23.4 / 15.7,  520 25.2 / 28.2, 1030 45.8 / 40.8, 2060 69.4 / 77.4
 //   K 1536, 8960 outputs:  100 rows 23.6 / 16.8,  195 25.5 / 31.9,  300 28.3 / 33.9, 2060 148 / 168
