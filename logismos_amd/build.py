@@ -12,6 +12,7 @@ from __future__ import annotations
 
 import glob
 import os
+import re
 import shutil
 import subprocess
 import sys
@@ -52,6 +53,24 @@ EXTRA_FLAGS = {
     "qgemm_q4g32.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
 }
 
+# Kernels that ask for operands in one assembly statement and wait for them in a later one, so that
+# work lies between the two.  A register that the compiler moved to memory (or copied) in between
+# would keep what it held before the read, with no error: a build in which one of them spills is refused.
+READS_IN_FLIGHT = ("qgemm_q4g128_tallp_kernel", "matmul_ring_fp16_kernel", "paged_attn_chunk64_kernel")
+
+
+def spills(remarks: str) -> list[str]:
+    """The kernels of READS_IN_FLIGHT that use scratch memory, from the compiler's
+    kernel-resource-usage remarks."""
+    found, name = [], ""
+    for line in remarks.splitlines():
+        if m := re.search(r"remark: Function Name: (\S+)", line):
+            name = m.group(1)
+        elif m := re.search(r"remark:\s+(VGPRs Spill|ScratchSize \[bytes/lane\]): ([1-9]\d*)", line):
+            if any(k in name for k in READS_IN_FLIGHT):
+                found.append(f"{name}: {m.group(1)} {m.group(2)}")
+    return found
+
 
 def hipcc() -> str:
     exe = os.environ.get("HIPCC") or shutil.which("hipcc") or "/opt/rocm/bin/hipcc"
@@ -66,12 +85,16 @@ def sources() -> list[str]:
 
 def _compile(src: str) -> str:
     obj = os.path.join(OBJDIR, os.path.basename(src) + ".o")
-    cmd = [hipcc(), *HIPCC_FLAGS, *EXTRA_FLAGS.get(os.path.basename(src), []), "-x", "hip", "-c",
-           src, "-o", obj]
+    cmd = [hipcc(), *HIPCC_FLAGS, *EXTRA_FLAGS.get(os.path.basename(src), []),
+           "-Rpass-analysis=kernel-resource-usage", "-fno-caret-diagnostics", "-x", "hip", "-c", src,
+           "-o", obj]
     r = subprocess.run(cmd, capture_output=True, text=True)
     if r.returncode != 0:
         raise RuntimeError(f"hipcc failed for {src}:\n{r.stderr}")
-    noise = ("packed-fp32-ops", "is not a recognized feature")
+    if bad := spills(r.stderr):
+        os.remove(obj)
+        raise RuntimeError(f"{src}: registers spilled where reads are in flight:\n" + "\n".join(bad))
+    noise = ("packed-fp32-ops", "is not a recognized feature", "[-Rpass-analysis=")
     warn = [ln for ln in r.stderr.splitlines() if ln.strip() and not any(n in ln for n in noise)]
     if warn:
         sys.stderr.write("\n".join(warn) + "\n")

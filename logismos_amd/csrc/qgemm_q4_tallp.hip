@@ -71,7 +71,6 @@ namespace lg {
 #define LG_INLINE __attribute__((always_inline))
 
 typedef __attribute__((address_space(3))) void* tp_lds_ptr_t;
-typedef const __attribute__((address_space(1))) void* tp_glb_ptr_t;
 
 // A workgroup's tile: 32 * BLOCKS rows of x by 32 weight rows for each of its WAVES waves.
 // CUTS: adds up in the parts a 128 x 256 tile would be split into (32 more registers; the code for it
@@ -197,6 +196,16 @@ __device__ __forceinline__ float tp_group_sum(const float (&cs)[4][4]) {
 #pragma unroll
     for (int q = 0; q < 4; ++q) quad[q] = (cs[0][q] + cs[2][q]) + (cs[1][q] + cs[3][q]);
     return (quad[0] + quad[2]) + (quad[1] + quad[3]);
+}
+
+// The lane's number, computed where it is asked for: to the compiler a new value, so that a lane constant
+// that is needed once per block or behind the loop holds no register inside it.  Without it six of the
+// 128 x 256 instances are short of 1 to 7 registers, and a register that goes to scratch while a read
+// into it is in flight would hold what was there before (the build refuses spills in this kernel).
+__device__ __forceinline__ int tp_lane_again() {
+    int v;
+    asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=v"(v));
+    return v;
 }
 
 // out_pairs (kTpOutSwigluOperand): the following launch's W.  (kTpOutF32): 1 where the K parts are
@@ -333,15 +342,20 @@ __global__ __launch_bounds__(64 * T::kWaves) void qgemm_q4g128_tallp_kernel(
     struct Small {
         TpRegs<unsigned, W> s, z;
         TpRegs<float, WX> xs[MI];
-        unsigned s_hi;  // ODD: s and s_hi the scales of the pair's two groups, z the zero of
-                        // this lane's group of the pair
+        unsigned s_hi;  // ODD, on its way: the scale of the pair's second group (then the high half
+                        // of s); z is the zero of this lane's group of the pair
     };
-    const unsigned soff = (unsigned)weight_row(wc + r) * (unsigned)groups_row * 2u;
-    const unsigned xsoff = (unsigned)((h * kTallTileRows + (row0 % kTallTileRows) + r) * W) * 4u;
+    // (kept where registers are left: with small loads for every pair of groups it is 1-2 % of 4000 x
+    // 1536 x 8960 to compute their offsets anew)
+    constexpr bool kLaneAgain = T::kBig && (ODD || (W > 1 && OUT != kTpOutSwigluOperand));
+    auto lane_for_loads = [&]() LG_INLINE { return kLaneAgain ? tp_lane_again() : lane; };
     // the sums of the WX pairs from group g on
     auto gload_sums = [&](int g, Small& v) LG_INLINE {
         const float* xb = xs + ((size_t)(row0 / kTallTileRows) * ((groups_row + BL - 1) / BL) + g / BL) *
                                    (2 * kTallTileRows * W) + (g % BL) / 2;
+        const int ln = lane_for_loads();
+        const unsigned xsoff =
+            (unsigned)(((ln >> 5) * kTallTileRows + (row0 % kTallTileRows) + (ln & 31)) * W) * 4u;
         // (the row tiles 32 W floats apart, as immediates)
         static_for<MI>([&](auto i_c) LG_INLINE {
             constexpr int at = decltype(i_c)::value * 32 * W * 4;
@@ -357,10 +371,12 @@ __global__ __launch_bounds__(64 * T::kWaves) void qgemm_q4g128_tallp_kernel(
     auto gload_small = [&](int g, Small& v) LG_INLINE {
         const __half* sb = scale + g;
         const __half* zb = zero + g;
+        const int ln = lane_for_loads();
+        const unsigned soff = (unsigned)weight_row(wc + (ln & 31)) * (unsigned)groups_row * 2u;
         if constexpr (ODD) {
             // (a missing second group re-reads the first)
             const unsigned second = soff + (g + 1 < groups_row ? 2u : 0u);
-            const unsigned own = h ? second : soff;
+            const unsigned own = ln & 32 ? second : soff;
             asm volatile("global_load_ushort %0, %1, %2" : "=&v"(v.s.raw) : "v"(soff), "s"(sb) : "memory");
             asm volatile("global_load_ushort %0, %1, %2" : "=&v"(v.s_hi) : "v"(second), "s"(sb) : "memory");
             asm volatile("global_load_ushort %0, %1, %2" : "=&v"(v.z.raw) : "v"(own), "s"(zb) : "memory");
@@ -385,7 +401,10 @@ __global__ __launch_bounds__(64 * T::kWaves) void qgemm_q4g128_tallp_kernel(
                      :
                      : "memory");
         if constexpr (MI == 4) asm volatile("" : "+v"(v.xs[MI - 2].raw), "+v"(v.xs[MI - 1].raw)::"memory");
-        if constexpr (ODD) asm volatile("" : "+v"(v.s_hi)::"memory");
+        if constexpr (ODD) {
+            asm volatile("" : "+v"(v.s_hi)::"memory");
+            v.s.raw |= v.s_hi << 16;
+        }
     };
     // The next block's values are loaded over a block's behind their last use; they are waited for
     // in the middle of the next group, and first used behind that.
@@ -590,8 +609,7 @@ __global__ __launch_bounds__(64 * T::kWaves) void qgemm_q4g128_tallp_kernel(
         }
         __builtin_amdgcn_sched_barrier(0);
         const unsigned sd = cur.s[U >> 1];
-        const unsigned short sb =
-            (unsigned short)(ODD ? (par ? cur.s_hi : sd) : (par ? (sd >> 16) : sd));
+        const unsigned short sb = (unsigned short)(par ? (sd >> 16) : sd);
         const float sf = __half2float(__builtin_bit_cast(__half, sb));
 #pragma unroll
         for (int i = 0; i < MI; ++i) {
@@ -652,23 +670,24 @@ __global__ __launch_bounds__(64 * T::kWaves) void qgemm_q4g128_tallp_kernel(
             for (int e = 0; e < 16; ++e) yacc[i][e] = parts_sum[i][e] + yacc[i][e];
     }
 
+    const int lane_e = tp_lane_again(), r_e = lane_e & 31, h_e = lane_e >> 5, tid_e = 64 * wave + lane_e;
     if (OUT == kTpOutF32 && T::kBig && part >= 0 && out_pairs != 0) {
         // a part of a launch whose consumer adds up the parts: rows of an [m][n] matrix each
         float* dst = partials + (size_t)(part % split) * ((size_t)m * n);
-        const int gn = col0 + wc + r;
+        const int gn = col0 + wc + r_e;
         if (gn >= n) return;
 #pragma unroll
         for (int i = 0; i < MI; ++i)
 #pragma unroll
             for (int e = 0; e < 16; ++e) {
-                const int gr = row0 + 32 * i + 8 * (e >> 2) + 4 * h + (e & 3);
+                const int gr = row0 + 32 * i + 8 * (e >> 2) + 4 * h_e + (e & 3);
                 if (gr < m) dst[(int64_t)gr * n + gn] = yacc[i][e];
             }
         return;
     }
     if (T::kBig && part >= 0) {
         // a part of a tile: the wave's 128 x 32 results as they lie in registers, lane fastest
-        float* dst = partials + (size_t)part * kTpTileElems + (size_t)wave * 4096 + lane;
+        float* dst = partials + (size_t)part * kTpTileElems + (size_t)wave * 4096 + lane_e;
 #pragma unroll
         for (int i = 0; i < MI; ++i)
 #pragma unroll
@@ -689,7 +708,7 @@ __global__ __launch_bounds__(64 * T::kWaves) void qgemm_q4g128_tallp_kernel(
                 yacc[i][e + 8] = __uint_as_float(sw[1]);  // up
             }
         // the row of result e (0 .. 7) of block i
-        auto row_of = [&](int i, int e) { return 32 * i + 8 * (e >> 2) + (r & 16) + 4 * h + (e & 3); };
+        auto row_of = [&](int i, int e) { return 32 * i + 8 * (e >> 2) + (r_e & 16) + 4 * h_e + (e & 3); };
         auto activation = [&](int i, int e) {
             const float g = yacc[i][e], u = yacc[i][e + 8];
             return f32_to_bf16_rne(g / (1.0f + expf(-g)) * u);
@@ -709,18 +728,18 @@ __global__ __launch_bounds__(64 * T::kWaves) void qgemm_q4g128_tallp_kernel(
             for (int i = 0; i < MI; ++i)
 #pragma unroll
                 for (int e = 0; e < 8; ++e)
-                    tile_b[row_of(i, e) * kPitch + 16 * wave + (r & 15)] = activation(i, e);
+                    tile_b[row_of(i, e) * kPitch + 16 * wave + (r_e & 15)] = activation(i, e);
             __syncthreads();
 #pragma unroll
             for (int u = 0; u < T::kM / 32; ++u) {
-                const int row = 32 * u + (tid >> 4), c = tid & 15;
+                const int row = 32 * u + (tid_e >> 4), c = tid_e & 15;
                 const uint4_t v = *reinterpret_cast<const uint4_t*>(tile_b + row * kPitch + 8 * c);
                 const float gs = row16_sum(sum8_bf16(v));
                 *reinterpret_cast<uint4_t*>(xo + (int64_t)(row0 + row) * n + col0 + 8 * c) = pair_order(v);
                 if (c == 0) so[tall_sum_index(row0 + row, col0 >> 7, n, out_pairs)] = gs;
             }
         } else {
-            const int gn = col0 + (wc >> 1) + (r & 15);
+            const int gn = col0 + (wc >> 1) + (r_e & 15);
             if (gn >= n) return;
 #pragma unroll
             for (int i = 0; i < MI; ++i)
@@ -732,14 +751,17 @@ __global__ __launch_bounds__(64 * T::kWaves) void qgemm_q4g128_tallp_kernel(
         }
         return;
     }
-    const int gn = col0 + wc + r;
+    const int gn = col0 + wc + r_e;
     if (gn >= n) return;
-    const float bv_n = bias ? bias[gn] : 0.0f;
+    float bv_n = bias ? bias[gn] : 0.0f;
+    // (waited for here: left to the compiler the wait stands in front of every store, and behind the
+    // stores before it: 281 us instead of 263 for 4096 x 4096 at 8240 rows)
+    asm volatile("" : "+v"(bv_n));
 #pragma unroll
     for (int i = 0; i < MI; ++i)
 #pragma unroll
         for (int e = 0; e < 16; ++e) {
-            const int gr = row0 + 32 * i + 8 * (e >> 2) + 4 * h + (e & 3);
+            const int gr = row0 + 32 * i + 8 * (e >> 2) + 4 * h_e + (e & 3);
             if (gr < m) {
                 if constexpr (OUT == kTpOutF32)
                     static_cast<float*>(y_out)[(int64_t)gr * n + gn] = yacc[i][e] + bv_n;
