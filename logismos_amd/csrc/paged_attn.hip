@@ -1742,8 +1742,9 @@ extern "C" logismos_status_t logismos_launch_paged_attn_decode_fp16_xprep(
     const int32_t* cu_seqlens_q, const int32_t* context_lens, void* out_prepared, void* workspace,
     int num_seqs, int num_q_heads, int num_kv_heads, int head_dim, int block_size,
     int max_blocks_per_seq, int num_splits, float scale, logismos_stream_t stream) {
-    // the prepared layout holds at most 32 rows
-    if (num_seqs > 32) return hipErrorInvalidValue;
+    // the prepared layout holds at most 32 rows; what the step does at narrow heads depends on its own
+    // num_splits and block tables and is no contract of this entry point
+    if (num_seqs > 32 || head_dim != lg::kHeadDim) return hipErrorInvalidValue;
     return lg::paged_attn_launch(q_f16, k_pool_f16, v_pool_f16, block_tables, cu_seqlens_q,
                                  context_lens, out_prepared, workspace, num_seqs, num_seqs, 1,
                                  num_q_heads, num_kv_heads, head_dim, block_size,
