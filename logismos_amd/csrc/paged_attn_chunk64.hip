@@ -50,12 +50,13 @@ constexpr int kC64Tile = kC64Keys * 64 * 2;  // bytes of a tile of K (or V)
 constexpr int c64_bufs(int kp) { return kp == 4 ? 2 : 4; }
 
 template <int CW, int KP>
-__global__ __launch_bounds__(256) void paged_attn_chunk64_kernel(const AttnParams p, int G, int block_shift) {
+__global__ __launch_bounds__(256, KP == 1 ? 2 : 1) void paged_attn_chunk64_kernel(const AttnParams p, int G, int block_shift) {
     static_assert(CW * KP == 4, "four waves");
     constexpr int kBuf = 2 * kC64Tile;       // K, then V
     constexpr int kReq = kC64Keys / 8 / CW;  // requests of K (and of V) per wave and tile
     constexpr int kBufs = c64_bufs(KP), kRing = kBufs * kBuf;
     extern __shared__ uint4_t c64_lds[];     // KP rings
+    __shared__ unsigned odd_waves[4];
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int cw = wave % CW, phase = wave / CW;
@@ -79,6 +80,7 @@ __global__ __launch_bounds__(256) void paged_attn_chunk64_kernel(const AttnParam
     const int last_tok = min(n_new - 1, ((group + 1) * 32 * CW - 1) / G);
     const int visible = p.causal ? ctx - n_new + last_tok + 1 : ctx;  // of the workgroup's last
     const int first_vis = p.causal ? ctx - n_new + min(c0, cols - 1) / G + 1 : ctx;  // of the wave's first
+    const int last_vis = p.causal ? ctx - n_new + min(c0 + 31, cols - 1) / G + 1 : ctx;  // ... and last
 
     // the queries as the B operand: column col, elements 16 st + 8 h .. + 7
     half8_t qb[4];
@@ -149,14 +151,16 @@ __global__ __launch_bounds__(256) void paged_attn_chunk64_kernel(const AttnParam
     }
 
     float m = -INFINITY, l = 0.0f;
-    float16_t o[2];
-#pragma unroll
-    for (int dt = 0; dt < 2; ++dt)
-#pragma unroll
-        for (int e = 0; e < 16; ++e) o[dt][e] = 0.0f;
+    float16_t o[2] = {};
 
     const unsigned k_swz = (unsigned)((col >> 1) & 7);
-    auto tile_step = [&](int step, int buf) LG_INLINE {
+    // CAREFUL: a key that a column does not see has the probability 0 there, and 0 times an infinity or NaN
+    // of its V row is a NaN.  The first walk over the keys takes no notice; if its results are not all
+    // finite, a second one takes a pass of its own for every number of keys that a column of the wave
+    // sees in a tile.  (Looked for in the V rows of the tiles in which a column ends, non-finite values
+    // cost 1 to 7 % of a launch.)
+    auto tile_step = [&](auto careful_c, int step, int buf) LG_INLINE {
+        constexpr bool CAREFUL = decltype(careful_c)::value != 0;
         const unsigned off = (unsigned)buf * kBuf;
         half8_t ka[2][4];  // [32 keys][16 elements]
         {
@@ -245,21 +249,54 @@ __global__ __launch_bounds__(256) void paged_attn_chunk64_kernel(const AttnParam
             uint2_t(&hi)[2] = vh[decltype(kb_c)::value];
             asm volatile("" : "+v"(lo[0]), "+v"(hi[0]), "+v"(lo[1]), "+v"(hi[1])::"memory");
         });
+        // O += V^T . P^T of the tile (ALL), or of its keys in front of key `keys` + 4 h of it
+        auto products = [&](auto all_c, int keys, float16_t(&acc)[2]) LG_INLINE {
+            static_for<4>([&](auto kb_c) LG_INLINE {
+                constexpr int kb = decltype(kb_c)::value;
+                uint4_t v[2];
 #pragma unroll
-        for (int kb = 0; kb < 4; ++kb) {
-            half8_t va[2];
+                for (int dt = 0; dt < 2; ++dt) v[dt] = uint4_t{vl[kb][dt][0], vl[kb][dt][1], vh[kb][dt][0], vh[kb][dt][1]};
+                if constexpr (!decltype(all_c)::value) {
 #pragma unroll
-            for (int dt = 0; dt < 2; ++dt)
-                va[dt] = __builtin_bit_cast(
-                    half8_t, uint4_t{vl[kb][dt][0], vl[kb][dt][1], vh[kb][dt][0], vh[kb][dt][1]});
+                    for (int w = 0; w < 4; ++w) {
+                        const int at = 16 * kb + 2 * w + (w > 1 ? 4 : 0);  // (and 4 h: its first key)
+                        const unsigned m = keys >= at + 2 ? ~0u : keys == at + 1 ? 0xffffu : 0u;
+                        v[0][w] &= m;
+                        v[1][w] &= m;
+                    }
+                }
+                half8_t va[2];
 #pragma unroll
-            for (int dt = 0; dt < 2; ++dt) o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(va[dt], __builtin_bit_cast(half8_t, pa[kb]), o[dt], 0, 0, 0);
+                for (int dt = 0; dt < 2; ++dt) va[dt] = __builtin_bit_cast(half8_t, v[dt]);
 #pragma unroll
-            for (int dt = 0; dt < 2; ++dt) o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(va[dt], __builtin_bit_cast(half8_t, pb[kb]), o[dt], 0, 0, 0);
+                for (int dt = 0; dt < 2; ++dt)
+                    acc[dt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(va[dt], __builtin_bit_cast(half8_t, pa[kb]), acc[dt], 0, 0, 0);
+#pragma unroll
+                for (int dt = 0; dt < 2; ++dt)
+                    acc[dt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(va[dt], __builtin_bit_cast(half8_t, pb[kb]), acc[dt], 0, 0, 0);
+            });
+        };
+        if (!CAREFUL || key0 + kC64Keys <= first_vis) {
+            products(ic<1>{}, kC64Keys, o);
+        } else {
+            for (int seen = first_vis; seen <= last_vis; ++seen) {
+                float16_t t[2] = {o[0], o[1]};
+                products(ic<0>{}, seen - key0 - 4 * h, t);
+#pragma unroll
+                for (int dt = 0; dt < 2; ++dt)
+#pragma unroll
+                    for (int e = 0; e < 16; ++e) o[dt][e] = vis == seen ? t[dt][e] : o[dt][e];
+            }
         }
     };
 
-    if (steps > 0) {
+    auto walk = [&](auto careful_c) LG_INLINE {
+        m = -INFINITY;
+        l = 0.0f;
+#pragma unroll
+        for (int dt = 0; dt < 2; ++dt)
+#pragma unroll
+            for (int e = 0; e < 16; ++e) o[dt][e] = 0.0f;
         for (int u = 0; u < kBufs - 1; ++u)
             if (u < steps) {
                 load_ids(u);
@@ -278,15 +315,29 @@ __global__ __launch_bounds__(256) void paged_attn_chunk64_kernel(const AttnParam
                 request_tile(i + kBufs - 1, (buf + kBufs - 1) & (kBufs - 1));
                 load_ids(i + kBufs);
             }
-            if (i * KP + phase < tiles) tile_step(i, buf);
+            if (i * KP + phase < tiles) tile_step(careful_c, i, buf);
             buf = (buf + 1) & (kBufs - 1);
+        }
+    };
+    if (steps > 0) {
+        walk(ic<0>{});
+        float odd = 0.0f;  // NaN if a result is not finite
+#pragma unroll
+        for (int dt = 0; dt < 2; ++dt)
+#pragma unroll
+            for (int e = 0; e < 16; ++e) odd = fmaf(o[dt][e], 0.0f, odd);
+        if (lane == 0) odd_waves[wave] = 0u;
+        if (odd != odd) odd_waves[wave] = 1u;
+        __syncthreads();  // (and behind it the rings are free)
+        if (__builtin_amdgcn_readfirstlane(odd_waves[0] | odd_waves[1] | odd_waves[2] | odd_waves[3]) != 0) {
+            walk(ic<1>{});
+            __syncthreads();
         }
     }
 
     l += lane_xor_f32<32>(l);
     if constexpr (KP > 1) {
         // the phases' states into phase 0's; a phase without a key of the column has m = -inf, l = 0, o = 0
-        __syncthreads();
         float* const sm = reinterpret_cast<float*>(c64_lds);  // [phase - 1][cw][34][lane]
         if (phase > 0) {
             float* dst = sm + (size_t)((phase - 1) * CW + cw) * 34 * 64 + lane;
