@@ -45,7 +45,6 @@ struct Workspace {
     bool tall;
     size_t xn_stride;
     int chunks;        // of 32 rows
-    int j_qkv, j_o, j_gu, j_down;
     size_t total;
 };
 
@@ -94,20 +93,19 @@ Workspace carve(const logismos_decode_config_t& c, int num_seqs, int t, int num_
     }
     w.chunks = (t + kChunkRows - 1) / kChunkRows;
     const int b = t < kChunkRows ? t : kChunkRows;
-    // the number of K parts depends on the batch only through its tile height (<= 16 rows or
-    // more), so a ragged last chunk taken by itself may plan fewer parts than a full one: size
-    // for the larger and let every launch use its own count
-    auto parts = [&](int n, int k) {
-        int j = logismos_qgemm_q4g128_splitk_xprep_parts(b, n, k);
-        const int last = t - (w.chunks - 1) * kChunkRows;
-        const int jl = logismos_qgemm_q4g128_splitk_xprep_parts(last, n, k);
-        return j > jl ? j : jl;
+    // fp32 rows that the K parts of a product take: those of all rows on the plan of a chunk, and of a
+    // ragged last chunk by itself, which may have more parts (few rows are split further).  The most
+    // over all smaller batches too, so that a workspace for many rows is one for fewer.
+    auto part_rows = [&](int n, int k) {
+        int most = 0;
+        for (int rows = 1; rows <= b; ++rows) {
+            const int r = logismos_qgemm_q4g128_splitk_xprep_parts(rows, n, k) * rows;
+            most = r > most ? r : most;
+        }
+        const int all = logismos_qgemm_q4g128_splitk_xprep_parts(b, n, k) * t;
+        return (size_t)(all > most ? all : most);
     };
-    w.j_qkv = parts((int)(qd + 2 * kvd), c.hidden);
-    w.j_o = parts(c.hidden, (int)qd);
-    w.j_gu = parts(2 * c.intermediate, c.hidden);
-    w.j_down = parts(c.hidden, c.intermediate);
-    const int j_proj = w.j_o > w.j_down ? w.j_o : w.j_down;
+    const size_t o_rows = part_rows(c.hidden, (int)qd), down_rows = part_rows(c.hidden, c.intermediate);
     // prepared activations of all rows: one buffer, or one per chunk of 32
     auto xprep = [&](int k) {
         return w.chunks == 1 ? align256(logismos_q4_xprep_bytes(b, k))
@@ -115,12 +113,12 @@ Workspace carve(const logismos_decode_config_t& c, int num_seqs, int t, int num_
     };
     w.xn_stride = lg::xprep_rows_stride(c.hidden);
     w.xn = take(xprep(c.hidden));
-    w.qkv = take((size_t)w.j_qkv * t * (qd + 2 * kvd) * 4);
+    w.qkv = take(part_rows((int)(qd + 2 * kvd), c.hidden) * (qd + 2 * kvd) * 4);
     w.q = take((size_t)t * qd * 2);
     w.attn_b = take(xprep((int)qd));
     w.attn_out = take((size_t)t * qd * 2);
-    w.proj = take((size_t)j_proj * t * c.hidden * 4);
-    w.gate_up = take((size_t)w.j_gu * t * 2 * c.intermediate * 4);
+    w.proj = take((o_rows > down_rows ? o_rows : down_rows) * c.hidden * 4);
+    w.gate_up = take(part_rows(2 * c.intermediate, c.hidden) * 2 * c.intermediate * 4);
     w.act = take(xprep(c.intermediate));
     w.attn_ws =
         take(logismos_paged_attn_workspace_bytes(num_seqs, c.num_q_heads, c.head_dim, num_splits));
