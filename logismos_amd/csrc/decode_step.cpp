@@ -395,9 +395,9 @@ extern "C" logismos_status_t logismos_launch_decode_step(const logismos_decode_c
         return 0;
     };
     // attention writes the o projection's input
-    const bool direct = one_pass && lg::paged_attn_prepared_out(c.head_dim, c.num_q_heads, c.num_kv_heads,
-                                                                c.block_size, c.max_blocks_per_seq, max_q,
-                                                                batch->num_splits);
+    const bool direct = one_pass && lg::paged_attn_prepared_out(num_seqs, c.head_dim, c.num_q_heads,
+                                                                c.num_kv_heads, c.block_size,
+                                                                c.max_blocks_per_seq, max_q, batch->num_splits);
     float* const h = static_cast<float*>(batch->hidden_f32);
 
     if (tokens_in)

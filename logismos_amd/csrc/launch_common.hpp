@@ -33,8 +33,8 @@ logismos_status_t paged_attn_launch(
 
 // Whether that launch can write the prepared layout of a following Q4G128 GEMM (out_bf16 == 2; bf16
 // rows otherwise).
-bool paged_attn_prepared_out(int head_dim, int hq, int hkv, int block_size, int max_blocks_per_seq,
-                             int max_seqlen_q, int num_splits);
+bool paged_attn_prepared_out(int num_seqs, int head_dim, int hq, int hkv, int block_size,
+                             int max_blocks_per_seq, int max_seqlen_q, int num_splits);
 
 // Streaming Q4G128 GEMM over prepared activations (qgemm_q4_stream.hip): steps per worker
 // for this shape (0: not applicable, use the split-K kernel) and the launch.  K parts are

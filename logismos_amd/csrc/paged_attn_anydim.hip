@@ -797,17 +797,30 @@ __global__ __launch_bounds__(256) void paged_attn_anydim_merge_kernel(const Attn
 }
 
 // Whether the decode rows of a launch take whole contexts (heads of up to 64: the accumulators of
-// sixteen waves), and then the KV heads of a workgroup.
-static int anydim_whole_heads(int head_dim, int hq, int hkv, int block_size, int max_blocks_per_seq) {
-    if (head_dim > 64 || (int64_t)block_size * max_blocks_per_seq > kAnyWholeKeys) return 0;
-    return hkv % 2 == 0 ? 2 : 1;
+// sixteen waves), and then the KV heads of a workgroup.  Two such workgroups fill a compute unit.  Up to
+// one per unit no launch is slower than on partitions; more of them take turns, and each adds its phases
+// up for two heads, where the partition kernel's workgroup streams up to eight heads in one go.  us, whole /
+// partitions, tables and contexts of 48, 128, 256 keys:
+//   64 sequences, 16 / 16 heads of 64 (512 of them)    9.1 / 7.8   14.9 / 12.6   18.6 / 22.9
+//   256 sequences, 8 / 8 heads of 64 (1024)            16.9 / 7.6   29.5 / 21.3   34.5 / 30.7
+//   256 sequences, 8 / 8 heads of 32 (1024)            10.3 / 7.9   14.0 / 16.7   17.6 / 22.0
+//   1024 sequences, 14 / 2 heads of 64 (1024)          19.7 / 17.0  31.8 / 58.1   36.8 / 67.6
+//   1024 sequences, 3 / 3 heads of 64 (3072)           24.3 / 13.2  35.7 / 47.5   41.1 / 64.0
+// hence beyond one per unit: tables of at least 128 keys, and heads of 32 or up to three KV heads.
+static int anydim_whole_heads(int num_seqs, int head_dim, int hkv, int block_size, int max_blocks_per_seq) {
+    const int64_t keys = (int64_t)block_size * max_blocks_per_seq;
+    if (head_dim > 64 || keys > kAnyWholeKeys) return 0;
+    const int heads = hkv % 2 == 0 ? 2 : 1;
+    if ((int64_t)num_seqs * (hkv / heads) > device_cu_count() && !(keys >= 128 && (head_dim == 32 || hkv <= 3)))
+        return 0;
+    return heads;
 }
 
-bool paged_attn_prepared_out(int head_dim, int hq, int hkv, int block_size, int max_blocks_per_seq,
-                             int max_seqlen_q, int num_splits) {
+bool paged_attn_prepared_out(int num_seqs, int head_dim, int hq, int hkv, int block_size,
+                             int max_blocks_per_seq, int max_seqlen_q, int num_splits) {
     if (head_dim == 128) return true;
     if (max_seqlen_q != 1 || (int64_t)hq * head_dim % 128 != 0) return false;
-    if (const int heads = anydim_whole_heads(head_dim, hq, hkv, block_size, max_blocks_per_seq))
+    if (const int heads = anydim_whole_heads(num_seqs, head_dim, hkv, block_size, max_blocks_per_seq))
         return (int64_t)hq / hkv * heads * head_dim % 128 == 0;
     return 128 % head_dim == 0 && num_splits > 1;  // the merge writes it
 }
@@ -935,12 +948,12 @@ hipError_t paged_attn_anydim_launch(const AttnParams& params, int head_dim, int 
     if (p.hq % p.hkv != 0 || p.hq / p.hkv > 16) return hipErrorInvalidValue;
     if (total_tokens > 65520 || p.num_seqs > 65535 || p.hkv > 65535) return hipErrorInvalidValue;
     const int whole = phases & LOGISMOS_ATTN_PHASE_DECODE && phases & LOGISMOS_ATTN_PHASE_MERGE
-                          ? anydim_whole_heads(head_dim, p.hq, p.hkv, p.block_size, p.max_blocks_per_seq)
+                          ? anydim_whole_heads(p.num_seqs, head_dim, p.hkv, p.block_size, p.max_blocks_per_seq)
                           : 0;
     if (p.out_bf16 == 2 &&
         !(phases == LOGISMOS_ATTN_PHASE_ALL &&
-          paged_attn_prepared_out(head_dim, p.hq, p.hkv, p.block_size, p.max_blocks_per_seq,
-                                  max_seqlen_q, p.num_splits)))
+          paged_attn_prepared_out(p.num_seqs, head_dim, p.hq, p.hkv, p.block_size,
+                                  p.max_blocks_per_seq, max_seqlen_q, p.num_splits)))
         return hipErrorInvalidValue;
     if (p.out_bf16 < 0 || p.out_bf16 > 2) return hipErrorInvalidValue;
     if (whole > 0) {

@@ -85,8 +85,8 @@ hipError_t paged_attn_anydim_launch(const AttnParams& p, int head_dim, int total
                                     int max_seqlen_q, int phases, hipStream_t stream);
 
 // Whether a launch of all phases can write the prepared layout (out_bf16 == 2).
-bool paged_attn_prepared_out(int head_dim, int hq, int hkv, int block_size, int max_blocks_per_seq,
-                             int max_seqlen_q, int num_splits);
+bool paged_attn_prepared_out(int num_seqs, int head_dim, int hq, int hkv, int block_size,
+                             int max_blocks_per_seq, int max_seqlen_q, int num_splits);
 
 // Rows of sequences with several new tokens at 64-wide heads (paged_attn_chunk64.hip).
 bool paged_attn_chunk64_applies(const AttnParams& p, int head_dim);
