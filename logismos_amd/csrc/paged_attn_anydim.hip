@@ -48,15 +48,7 @@ namespace lg {
 
 constexpr int kAnyWaves = 8;           // waves of a workgroup: KV heads x tile phases
 constexpr int kAnyLdsBytes = 48 * 1024;  // for the accumulators of the phases (beyond the first)
-constexpr int kAnyWgHeads = 8;           // KV heads per workgroup at most
 constexpr int kAnyPhases = 8;            // tile phases per head at most
-
-// KV heads per workgroup: the largest divisor of hkv up to kAnyWgHeads
-static int anydim_wg_heads(int hkv) {
-    for (int w = kAnyWgHeads; w > 1; --w)
-        if (hkv % w == 0) return w;
-    return 1;
-}
 
 template <int NJ>
 struct AnyTile {
@@ -963,7 +955,7 @@ hipError_t paged_attn_anydim_launch(const AttnParams& params, int head_dim, int 
         phases &= ~(LOGISMOS_ATTN_PHASE_DECODE | LOGISMOS_ATTN_PHASE_MERGE);
     }
     if ((phases & LOGISMOS_ATTN_PHASE_PREFILL) && max_seqlen_q > 1 &&
-        paged_attn_chunk64_applies(p, head_dim)) {
+        paged_attn_chunk64_applies(p, head_dim, total_tokens, max_seqlen_q)) {
         if (const hipError_t e = paged_attn_chunk64_launch(p, total_tokens, max_seqlen_q, stream)) return e;
         phases &= ~LOGISMOS_ATTN_PHASE_PREFILL;
     }

@@ -410,24 +410,50 @@ static hipError_t launch_chunk64(const AttnParams& p, int max_seqlen_q, hipStrea
     return hipGetLastError();
 }
 
-bool paged_attn_chunk64_applies(const AttnParams& p, int head_dim) {
+// Which split a launch takes, from what the host knows: the tokens of the longest chunk, all packed rows and
+// the block tables' length.  If all rows came in chunks of that length there would be `chunks` of them.
+// us, the general kernel / CW = 4 / 2 / 1:
+//   8 x 512 tokens, contexts to 4600, 14 / 2 heads: 257 / 116 / 131 / 157; 2 x 512 to 1500: 36 / 29.8 / 20.8 / 26.0
+//   1 x 20, a context of 4000, 14 / 2:              34 / 46 / 30 / 23
+//   1 x 512 at 8000, 16 / 16:                       101 / 160 / 99 / 68 (256 workgroups at CW = 1: one round)
+//   1 x 2000 at 6000, 16 / 2:                       316 / 151 / 161 / 207
+//   1 x 128 and 1 x 32 alone, 14 / 2:               8.8 / 8.5 / 7.6 / 7.9 and 7.6 / 7.2 / 7.5 / 7.9
+//   200 x 2 at 300, 8 / 8:                          34 / 44 / 54 / 54;  64 x 2 at 300: 18.1 / 19.1 / 20.4 / 20.5
+//   1 x 32 at 16000, 8 / 1:                         95 / 296 / 178 / 114;  1 x 512 at 8000: 55 / 159 / 97 / 65
+//   1 x 2000 alone, 8 / 1:                          40 / 44 / 29 / 26
+constexpr int kC64General = 0;
+static int chunk64_columns(const AttnParams& p, int64_t total_tokens, int64_t max_seqlen_q) {
+    const int64_t g = p.hq / p.hkv, cols = max_seqlen_q * g, cus = device_cu_count();
+    const int64_t keys = (int64_t)p.block_size * p.max_blocks_per_seq;
+    const int64_t chunks_hkv = total_tokens * p.hkv;  // (chunks x hkv x max_seqlen_q)
+    auto workgroups = [&](int64_t cw) { return chunks_hkv * ((cols + 32 * cw - 1) / (32 * cw)) / max_seqlen_q; };
+    // The general kernel: where a KV head has all eight of its waves, which walk a long context faster
+    // than four here, as long as its tiles of 16 columns are about one per unit; and where a whole chunk is
+    // one such tile and there are more chunks than units (a tile of 32 columns here is half empty).
+    const int64_t tile = 16 / g;
+    if (anydim_wg_heads(p.hkv) % 2 == 1 && keys > 512 &&
+        (total_tokens + tile - 1) / tile * p.hkv <= cus + cus / 4)
+        return kC64General;
+    if (max_seqlen_q <= tile && workgroups(1) > cus) return kC64General;
+    if (keys <= kC64Keys) return 4;  // (a key phase needs a tile)
+    if (total_tokens * p.hq / 128 >= cus && cols > 32) return 4;
+    if (keys <= 2 * kC64Keys) return 2;
+    return workgroups(1) <= cus || cols <= 32 ? 1 : 2;
+}
+
+bool paged_attn_chunk64_applies(const AttnParams& p, int head_dim, int total_tokens, int max_seqlen_q) {
     const uintptr_t at = reinterpret_cast<uintptr_t>(p.k_pool) | reinterpret_cast<uintptr_t>(p.v_pool) |
                          reinterpret_cast<uintptr_t>(p.q) | reinterpret_cast<uintptr_t>(p.out);
-    return head_dim == 64 && (at & 15u) == 0;
+    return head_dim == 64 && (at & 15u) == 0 && chunk64_columns(p, total_tokens, max_seqlen_q) != kC64General;
 }
 
 hipError_t paged_attn_chunk64_launch(const AttnParams& p, int total_tokens, int max_seqlen_q,
                                      hipStream_t stream) {
-    // By how many groups of 128 columns there are (if all rows are chunks').  us of a launch, CW = 4 / 2 /
-    // 1, the general kernel:
-    //   8 x 512 tokens (448 groups), contexts to 4600: 116 / 131 / 157, 257
-    //   2 x 512 (112), contexts to 1500:               29.8 / 20.8 / 26.0, 36
-    //   1 x 20 (2), a context of 4000:                 46 / 30 / 23, 34
-    const int64_t groups = (int64_t)total_tokens * p.hq / 128;
-    const int64_t cus = device_cu_count();
-    if (groups >= cus) return launch_chunk64<4, 1>(p, max_seqlen_q, stream);
-    if (groups >= cus / 4) return launch_chunk64<2, 2>(p, max_seqlen_q, stream);
-    return launch_chunk64<1, 4>(p, max_seqlen_q, stream);
+    switch (chunk64_columns(p, total_tokens, max_seqlen_q)) {
+        case 4: return launch_chunk64<4, 1>(p, max_seqlen_q, stream);
+        case 2: return launch_chunk64<2, 2>(p, max_seqlen_q, stream);
+        default: return launch_chunk64<1, 4>(p, max_seqlen_q, stream);
+    }
 }
 
 }  // namespace lg

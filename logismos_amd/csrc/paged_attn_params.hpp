@@ -88,8 +88,15 @@ hipError_t paged_attn_anydim_launch(const AttnParams& p, int head_dim, int total
 bool paged_attn_prepared_out(int num_seqs, int head_dim, int hq, int hkv, int block_size,
                              int max_blocks_per_seq, int max_seqlen_q, int num_splits);
 
+// KV heads per workgroup of that kernel: the largest divisor of hkv up to eight.
+inline int anydim_wg_heads(int hkv) {
+    int w = 8;
+    while (hkv % w != 0) --w;
+    return w;
+}
+
 // Rows of sequences with several new tokens at 64-wide heads (paged_attn_chunk64.hip).
-bool paged_attn_chunk64_applies(const AttnParams& p, int head_dim);
+bool paged_attn_chunk64_applies(const AttnParams& p, int head_dim, int total_tokens, int max_seqlen_q);
 hipError_t paged_attn_chunk64_launch(const AttnParams& p, int total_tokens, int max_seqlen_q,
                                      hipStream_t stream);
 
