@@ -20,6 +20,8 @@
 #include <hip/hip_fp16.h>
 #include <math.h>
 
+#include <algorithm>
+
 namespace lg {
 
 constexpr int kRowThreads = 256;
@@ -606,11 +608,16 @@ template <int MB, int NB, int WR, int WC, int BUFS>
 static hipError_t matmul_ring_launch(const void* a, const void* b, void* d, int m, int n, int k,
                                      hipStream_t st) {
     constexpr int TM = 32 * MB * WR, TN = 32 * NB * WC;
-    constexpr int lds = BUFS * (TM + TN) * 128;
+    constexpr int kMost = BUFS * (TM + TN) * 128;
     const auto kernel = matmul_ring_fp16_kernel<MB, NB, WR, WC, BUFS>;
     static const hipError_t opt = hipFuncSetAttribute(
-        reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+        reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, kMost);
     if (opt != hipSuccess) return opt;
+    // few slabs: the ring is no longer than they are (and the product's way out needs its tile), so that
+    // more workgroups share a compute unit
+    const int slabs = (k + 63) / 64;
+    const int lds = std::max(std::min(slabs, BUFS) * (TM + TN) * 128, TM * (TN + 8) * 2);
+    static_assert(TM * (TN + 8) * 2 <= kMost, "the tile fits the ring");
     const int tm = (m + TM - 1) / TM, tn = (n + TN - 1) / TN;
     const int vec_out = (reinterpret_cast<uintptr_t>(d) & 15u) == 0;
     kernel<<<dim3((unsigned)((int64_t)tm * tn)), dim3(64 * WR * WC), lds, st>>>(
@@ -619,24 +626,52 @@ static hipError_t matmul_ring_launch(const void* a, const void* b, void* d, int 
     return hipGetLastError();
 }
 
-// The largest tile of which there are enough: 256 x 128 from three quarters of the compute units on,
-// 128 x 128 and 64 x 128 from six tenths, else 64 x 64.  us, 256 x 128 / 128 x 128 / 64 x 128 / 64 x 64
-// (tiles of the first) and what the kernel with a slab in registers on its way to two buffers took:
-//   4096 x 4096 x 4096 (512)  140 / 167 / 235 / 245, 172      1700 x 4096 x 4096 (224)  68 / 80 / 117 / 113, 114
-//   4096 x 2048 x 1000 (256)  25.6 / 26.9 / 36.8 / 38.9, 27.7  2500 x 1024 x 2048 (80)  29.4 / 20.6 / 30.6 / 28.2, 25.9
-//   2036 x 1536 x 1536 (96)   25.2 / 21.2 / 27.3 / 28.0, 23.3  1000 x 4096 x 768 (128)  15.4 / 12.1 / 16.1 / 16.1, 14.9
-//   1300 x 1536 x 1000 (72)   16.8 / 12.1 / 10.6 / 11.1, 11.2  4096 x 512 x 776 (64)    14.2 / 10.5 / 8.8 / 9.6, 13.6
-//   500 x 1024 x 1200 (16)    17.9 / 12.6 / 10.4 / 9.1, 9.3    294 x 1536 x 3560 (24)   53.6 / 32.4 / 25.9 / 22.8, 22.7
-// What bounds it: the operands' way from L2 (9 TB/s at 2036 x 1536 x 1536, 151 MB on 128 x 128 tiles), where
-// tiles are few a slab's chain of four dependent steps, 0.27 us on 64 x 64, 0.43 on 128 x 128.
+// Which tile: the one whose rounds take the least.  A compute unit holds as many workgroups of a tile as
+// the ring (min(slabs, buffers) slabs of LDS) and the registers allow; a round of r of them takes the tile's
+// ramp and, per slab of 64 columns, the longer of its own chain of dependent steps and r times its share of
+// the unit.  `once`, `ramp`, `chain` and `share` in us, fitted to 663 shapes (64 to 5000 rows, 512 to 4096
+// columns, K 64 to 4096): the tile taken is 0.8 % off the fastest of the six on the mean.  Counting tiles only,
+// a nearly empty second round went unseen (264 tiles of 64 x 128 for 2100 x 1024).  us, the tile taken / by
+// count / the kernel with a slab in registers on its way to two buffers:
+//   2036 x 1536 x 1536  17.6 / 18.2 / 21.7   2100 x 1024 x 768  10.4 / 15.2 / 11.5   4096 x 4096 x 768  34.2 / 34.9 / 40.0
+//   1300 x 3072 x 4096  52.5 / 76.3 / 67.4   2900 x 768 x 4096  37.3 / 57.8 / 48.3   700 x 3072 x 256   5.7 / 8.5 / 6.1
+//   2036 x 512 x 768    7.2 / 7.3 / 7.3      3200 x 768 x 64    4.3 / 5.9 / 4.2
+// Up to three slabs the shorter rings only.  (One or two slabs, no ring to speak of: 15 of the 663 shapes are up
+// to 0.46 us behind the kernel of two buffers.)
+// What bounds it: the operands' way from L2 where tiles are many, where they are few a slab's chain of four
+// dependent steps, 0.3 us on 64 x 64, 0.5 on 128 x 128.
+struct MatmulTile {
+    int rows, cols, bufs, most;  // most: workgroups of a compute unit by its registers
+    float once, ramp, chain, share;
+    decltype(&matmul_ring_launch<2, 2, 4, 2, 3>) launch;
+};
+static float matmul_time(const MatmulTile& t, int64_t m, int64_t n, int64_t slabs, int64_t cus) {
+    const int64_t lds = std::max(std::min<int64_t>(slabs, t.bufs) * (t.rows + t.cols) * 128,
+                                 (int64_t)t.rows * (t.cols + 8) * 2);
+    const int64_t held = std::min<int64_t>(160 * 1024 / lds, t.most);
+    const int64_t tiles = ((m + t.rows - 1) / t.rows) * ((n + t.cols - 1) / t.cols);
+    const int64_t per_cu = (tiles + cus - 1) / cus;
+    auto round = [&](int64_t r) { return t.ramp + (float)slabs * std::max(t.chain, (float)r * t.share); };
+    return t.once + (float)(per_cu / held) * round(held) + (per_cu % held ? round(per_cu % held) : 0.0f);
+}
 static hipError_t matmul_tiled(const void* a, const void* b, void* d, int m, int n, int k, void* stream) {
-    hipStream_t st = static_cast<hipStream_t>(stream);
-    const int64_t cus = device_cu_count();
-    auto tiles = [&](int tm, int tn) { return (int64_t)((m + tm - 1) / tm) * ((n + tn - 1) / tn); };
-    if (4 * tiles(256, 128) >= 3 * cus) return matmul_ring_launch<2, 2, 4, 2, 3>(a, b, d, m, n, k, st);
-    if (10 * tiles(128, 128) >= 6 * cus) return matmul_ring_launch<2, 1, 2, 4, 5>(a, b, d, m, n, k, st);
-    if (10 * tiles(64, 128) >= 6 * cus) return matmul_ring_launch<1, 1, 2, 4, 5>(a, b, d, m, n, k, st);
-    return matmul_ring_launch<1, 1, 2, 2, 5>(a, b, d, m, n, k, st);
+    static const MatmulTile tiles[] = {
+        {256, 128, 3, 2, 0.0f, 4.86f, 0.29f, 0.77f, matmul_ring_launch<2, 2, 4, 2, 3>},
+        {128, 128, 5, 3, 0.46f, 3.55f, 0.52f, 0.53f, matmul_ring_launch<2, 1, 2, 4, 5>},
+        {64, 128, 5, 4, 1.67f, 1.87f, 0.41f, 0.41f, matmul_ring_launch<1, 1, 2, 4, 5>},
+        {64, 64, 5, 8, 2.05f, 1.35f, 0.33f, 0.23f, matmul_ring_launch<1, 1, 2, 2, 5>},
+        {64, 128, 3, 4, 1.10f, 2.38f, 0.44f, 0.36f, matmul_ring_launch<1, 1, 2, 4, 3>},
+        {64, 64, 3, 8, 2.09f, 1.22f, 0.38f, 0.22f, matmul_ring_launch<1, 1, 2, 2, 3>},
+    };
+    const int64_t slabs = ((int64_t)k + 63) / 64, cus = device_cu_count();
+    const MatmulTile* best = nullptr;
+    float best_time = 0.0f;
+    for (const MatmulTile& t : tiles) {
+        if (slabs <= 3 && t.bufs == 5 && t.rows == 64) continue;
+        const float time = matmul_time(t, m, n, slabs, cus);
+        if (!best || time < best_time) best = &t, best_time = time;
+    }
+    return best->launch(a, b, d, m, n, k, static_cast<hipStream_t>(stream));
 }
 
 // `check_matmul_shape` (crates/kernels/src/matmul/mod.rs:89-117)
