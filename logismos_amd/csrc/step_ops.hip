@@ -446,7 +446,17 @@ __global__ __launch_bounds__(64) void rope_kv_write_kernel(
 // kernel above is one 64-thread workgroup per (token, head) with 4-byte accesses: at 8240
 // tokens x 48 heads that is 400 k workgroups for 300 MB.  Same sums in the same order, same
 // rotation, same rounding.
-constexpr int kRopeRowsKernelFrom = 64;  // tokens from which the many-row kernel is used
+// From 64 tokens on at heads of 128 and more, else from 2400 (token, head) pairs on: its three microseconds
+// do not fall with the work, and the kernel above takes fewer pairs of narrow heads in less.  us, this one /
+// the one above: 14 + 4 heads of 64, 64 tokens 2.9 / 2.6, 128 (2304 pairs) 2.9 / 2.9, 200 2.9 / 3.2; 8 + 16 of
+// 32, 64 2.9 / 2.7, 100 2.9 / 3.0; 8 + 8 of 96, 64 2.9 / 2.5, 160 3.0 / 3.0; 2 + 2 of 32, 600 2.95 / 3.2;
+// 8 + 8 of 256, 64 tokens 2.7 / 3.2.
+constexpr int kRopeRowsKernelFrom = 64;
+constexpr int kRopeRowsKernelPairs = 2400;
+static bool rope_rows_kernel(int64_t tokens, int heads, int head_dim) {
+    return head_dim % 8 == 0 && tokens >= kRopeRowsKernelFrom &&
+           (head_dim >= 128 || tokens * heads >= kRopeRowsKernelPairs);
+}
 template <bool D128>
 __global__ __launch_bounds__(256) void rope_kv_write_rows_kernel(
     const float* __restrict__ qkv_parts, int num_parts, int64_t part_stride,
@@ -829,7 +839,7 @@ extern "C" logismos_status_t logismos_launch_rope_kv_write_f32p_bias(
                             reinterpret_cast<uintptr_t>(q_out_f16) |
                             reinterpret_cast<uintptr_t>(k_pool_f16) |
                             reinterpret_cast<uintptr_t>(v_pool_f16);
-    if (head_dim % 8 == 0 && total_tokens >= lg::kRopeRowsKernelFrom && (align & 15u) == 0) {
+    if (lg::rope_rows_kernel(total_tokens, num_q_heads + 2 * num_kv_heads, head_dim) && (align & 15u) == 0) {
         const int64_t quads = (int64_t)total_tokens * width / 8;
         const auto kernel = head_dim == 128 ? lg::rope_kv_write_rows_kernel<true>
                                             : lg::rope_kv_write_rows_kernel<false>;

@@ -1,6 +1,7 @@
-"""The many-row rotation + K/V write (64 tokens and more) at head widths other than 128: bit for bit
-the per-head kernel that launches of fewer tokens take, from split-K parts with a bias, with a token
-that has no slot.  Widths that are no multiple of 8 stay on the per-head kernel."""
+"""The many-row rotation + K/V write (64 tokens and more at heads of 128 and wider, 2400 (token, head)
+pairs and more at narrower ones) at head widths other than 128: bit for bit the per-head kernel that
+launches of fewer tokens take, from split-K parts with a bias, with a token that has no slot.  Widths
+that are no multiple of 8 stay on the per-head kernel."""
 import numpy as np
 import pytest
 
@@ -10,10 +11,11 @@ from logismos_amd import hip, kernels
 pytestmark = pytest.mark.gpu
 
 
+@pytest.mark.parametrize("t", [131, 266, 267])  # 9 heads: 2394 and 2403 pairs
 @pytest.mark.parametrize("d", [8, 24, 64, 96, 256, 12])
-def test_same_bits_as_the_per_head_kernel(d):
+def test_same_bits_as_the_per_head_kernel(d, t):
     rng = np.random.default_rng(d)
-    t, hq, hkv, rows, max_pos = 131, 7, 1, 160, 300
+    hq, hkv, rows, max_pos = 7, 1, t + 29, 300
     width = (hq + 2 * hkv) * d
     parts = rng.standard_normal((2, t, width), np.float32)
     bias = rng.standard_normal(width).astype(np.float32)
