@@ -783,8 +783,12 @@ __global__ __launch_bounds__(256) void q4_tall_reduce_kernel(const float* __rest
                                                             int split) {
     static_assert(OUT != kTpOutSwigluOperand, "q4_tall_reduce_operand_kernel");
     constexpr int kPerTile = OUT == kTpOutSwiglu ? kTpTileElems / 2 : kTpTileElems;
-    const int t = blockIdx.x / (kPerTile / 256);
-    int idx = (blockIdx.x % (kPerTile / 256)) * 256 + threadIdx.x;
+    // a tile's workgroups by its blocks of 32 rows first: of a tile whose rows end early the first ones
+    // have work and the rest none (every other run of them, with the waves first: 280 to 320 rows of
+    // 1536 x 8960 in 14 parts 9.8 us, 6.3 this way)
+    constexpr int kWgs = kPerTile / 256, kSub = kWgs / 32;  // kSub: of a wave's block
+    const int t = blockIdx.x / kWgs, b = blockIdx.x % kWgs;
+    int idx = (((b / kSub) % 8 * 4 + b / (8 * kSub)) * kSub + b % kSub) * 256 + threadIdx.x;
     if constexpr (OUT == kTpOutSwiglu) idx = ((idx >> 4) << 5) | (idx & 15);  // the gate's lanes
     const int lane = idx & 63, e = (idx >> 6) & 15, i = (idx >> 10) & 3, wave = idx >> 12;
     const int tile = full_tiles + t;
