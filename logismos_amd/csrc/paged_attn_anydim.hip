@@ -483,8 +483,9 @@ __global__ __launch_bounds__(64 * kAnyWaves) void paged_attn_anydim_kernel(const
         return;
     }
     if (visible <= 0) {
-        // no visible key for any of the tokens: rows of zeros (written once)
-        if (split == 0)
+        // no visible key for any of the tokens: rows of zeros (written once; in the prepared layout by
+        // the merge)
+        if (split == 0 && p.out_bf16 != 2)
             for (int tq = 0; tq < ntok; ++tq) {
                 _Float16* out_row = p.out + ((int64_t)(t + tq) * p.hq + (int64_t)kvh * G) * D;
                 for (int i = lane + 64 * phase; i < G * D; i += 64 * phases)
@@ -664,67 +665,6 @@ __device__ __forceinline__ int anydim_partials(const AttnParams& p, int s, int c
     return (before + nt - 1) / R - w_first + 1;
 }
 
-// The same as the operand of the following Q4G128 GEMM (p.out_bf16 == 2, head widths that divide 128;
-// then every decode row has its partials here, also a single one): a workgroup takes the 128 columns of
-// one group, i.e. 128 / D heads; thread = (stripe of four, element pair).  One launch less, 2.4 us a
-// layer for one sequence of 14 heads of 64.  grid (groups, num_seqs).
-__global__ __launch_bounds__(256) void paged_attn_anydim_merge_prepared_kernel(const AttnParams p, int D) {
-    __shared__ float sm_w[8][2];           // [head of the group][max m, sum]
-    __shared__ float sm_a[4][128], sm_l[4][64];
-    __shared__ __attribute__((aligned(16))) unsigned short row[128];
-    const int s = blockIdx.y, tid = threadIdx.x;
-    const int t = p.cu_seqlens_q[s];
-    if (p.cu_seqlens_q[s + 1] - t != 1) return;
-    int64_t slot0 = 0;
-    const int parts = anydim_partials(p, s, p.context_lens[s], slot0);
-    const int heads = 128 / D, head0 = blockIdx.x * heads;
-    // every head's maximum: a wave a head
-    for (int i = tid >> 6; i < heads; i += 4) {
-        float mmax = -INFINITY;
-        for (int q = tid & 63; q < parts; q += 64)
-            mmax = fmaxf(mmax, p.ws_ml[((slot0 + q) * p.hq + head0 + i) * 2]);
-#pragma unroll
-        for (int o = 1; o < 64; o <<= 1) mmax = fmaxf(mmax, shfl_xor_f32(mmax, o));
-        if ((tid & 63) == 0) sm_w[i][0] = mmax;
-    }
-    __syncthreads();
-    const int stripe = tid >> 6, pair = tid & 63;
-    const int hd = 2 * pair / D, d = 2 * pair - hd * D, head = head0 + hd;
-    const float mmax = sm_w[hd][0];
-    float a0 = 0.0f, a1 = 0.0f, lt = 0.0f;
-    for (int q = stripe; q < parts; q += 4) {
-        const int64_t idx = (slot0 + q) * p.hq + head;
-        const float w = fast_exp2(p.ws_ml[idx * 2] - mmax);
-        lt += w * p.ws_ml[idx * 2 + 1];
-        const float2 a = *reinterpret_cast<const float2*>(p.ws_acc + idx * D + d);
-        a0 += w * a.x;
-        a1 += w * a.y;
-    }
-    sm_a[stripe][2 * pair] = a0;
-    sm_a[stripe][2 * pair + 1] = a1;
-    sm_l[stripe][pair] = lt;
-    __syncthreads();
-    if (stripe == 0) {
-#pragma unroll
-        for (int j = 1; j < 4; ++j) {
-            a0 += sm_a[j][2 * pair];
-            a1 += sm_a[j][2 * pair + 1];
-            lt += sm_l[j][pair];
-        }
-        const float inv = lt > 0.0f ? 1.0f / lt : 0.0f;  // no key: zeros
-        *reinterpret_cast<unsigned*>(row + 2 * pair) =
-            (unsigned)attn_out_elem(a0 * inv, 1) | ((unsigned)attn_out_elem(a1 * inv, 1) << 16);
-        asm volatile("" ::: "memory");  // (one wave: its LDS accesses stay in this order)
-        const uint4_t o = reinterpret_cast<const uint4_t*>(row)[tid & 15];
-        const float gs = row16_sum(sum8_bf16(o));
-        if (tid < 16) {
-            const XprepRow at = xprep_row(p.out, p.out_rows, p.hq * D, t);
-            at.xp[(int64_t)(blockIdx.x * 16 + tid) * at.bp] = pair_order(o);
-            if (tid == 0) at.xg[(int64_t)blockIdx.x * at.bp] = gs;
-        }
-    }
-}
-
 // Decode rows with more than one partition: out = sum_p w_p acc_p / sum_p w_p l_p,
 // w_p = 2^(m_p - max m).  grid (hq, num_seqs), 256 threads: thread = (stripe, element pair),
 // stripe j sums the partitions j, j + S, ...; the stripes are added through LDS.
@@ -788,6 +728,81 @@ __global__ __launch_bounds__(256) void paged_attn_anydim_merge_kernel(const Attn
                                  ((int64_t)t * p.hq + head) * D + 2 * pair) = w;
 }
 
+// The same as the operand of the following Q4G128 GEMM (p.out_bf16 == 2, head widths that divide 128;
+// then every decode row has its partials here, also a single one): a workgroup takes the 128 columns of
+// one group, i.e. 128 / D heads; thread = (wave, element pair), and a wave takes a fourth of the stripes
+// above, each in an accumulator of its own, so that the bits are those of the rows above.  One launch
+// less, 2.4 us a layer for one sequence of 14 heads of 64.  grid (groups, num_seqs).
+template <int D>
+__global__ __launch_bounds__(256) void paged_attn_anydim_merge_prepared_kernel(const AttnParams p) {
+    constexpr int S = 512 / D, N = S / 4;  // stripes, and those of a wave (w, w + 4, ..)
+    __shared__ float sm_m[4];              // [head of the group] max m
+    __shared__ float sm_a[S][128], sm_l[S][128 / D];
+    __shared__ __attribute__((aligned(16))) unsigned short row[128];
+    const int s = blockIdx.y, tid = threadIdx.x;
+    const int t = p.cu_seqlens_q[s];
+    if (p.cu_seqlens_q[s + 1] - t != 1) return;
+    int64_t slot0 = 0;
+    const int parts = anydim_partials(p, s, p.context_lens[s], slot0);
+    constexpr int heads = 128 / D;
+    const int head0 = blockIdx.x * heads;
+    // every head's maximum: a wave a head
+    if (const int i = tid >> 6; i < heads) {
+        float mmax = -INFINITY;
+        for (int q = tid & 63; q < parts; q += 64)
+            mmax = fmaxf(mmax, p.ws_ml[((slot0 + q) * p.hq + head0 + i) * 2]);
+#pragma unroll
+        for (int o = 1; o < 64; o <<= 1) mmax = fmaxf(mmax, shfl_xor_f32(mmax, o));
+        if ((tid & 63) == 0) sm_m[i] = mmax;
+    }
+    __syncthreads();
+    const int wave = tid >> 6, pair = tid & 63;
+    const int hd = 2 * pair / D, d = 2 * pair - hd * D, head = head0 + hd;
+    const float mmax = sm_m[hd];
+    float a0[N], a1[N], lt[N];
+#pragma unroll
+    for (int u = 0; u < N; ++u) a0[u] = a1[u] = lt[u] = 0.0f;
+    for (int q0 = wave; q0 < parts; q0 += S) {
+#pragma unroll
+        for (int u = 0; u < N; ++u) {
+            const int q = q0 + 4 * u;
+            if (q >= parts) break;
+            const int64_t idx = (slot0 + q) * p.hq + head;
+            const float w = fast_exp2(p.ws_ml[idx * 2] - mmax);
+            lt[u] += w * p.ws_ml[idx * 2 + 1];
+            const float2 a = *reinterpret_cast<const float2*>(p.ws_acc + idx * D + d);
+            a0[u] += w * a.x;
+            a1[u] += w * a.y;
+        }
+    }
+#pragma unroll
+    for (int u = 0; u < N; ++u) {
+        sm_a[wave + 4 * u][2 * pair] = a0[u];
+        sm_a[wave + 4 * u][2 * pair + 1] = a1[u];
+        if (d == 0) sm_l[wave + 4 * u][hd] = lt[u];
+    }
+    __syncthreads();
+    if (wave != 0) return;
+    float x0 = a0[0], x1 = a1[0], l = sm_l[0][hd];
+#pragma unroll
+    for (int j = 1; j < S; ++j) {
+        x0 += sm_a[j][2 * pair];
+        x1 += sm_a[j][2 * pair + 1];
+        l += sm_l[j][hd];
+    }
+    const float inv = l > 0.0f ? 1.0f / l : 0.0f;  // no key: zeros
+    *reinterpret_cast<unsigned*>(row + 2 * pair) =
+        (unsigned)attn_out_elem(x0 * inv, 1) | ((unsigned)attn_out_elem(x1 * inv, 1) << 16);
+    asm volatile("" ::: "memory");  // (one wave: its LDS accesses stay in this order)
+    const uint4_t o = reinterpret_cast<const uint4_t*>(row)[tid & 15];
+    const float gs = row16_sum(sum8_bf16(o));
+    if (tid < 16) {
+        const XprepRow at = xprep_row(p.out, p.out_rows, p.hq * D, t);
+        at.xp[(int64_t)(blockIdx.x * 16 + tid) * at.bp] = pair_order(o);
+        if (tid == 0) at.xg[(int64_t)blockIdx.x * at.bp] = gs;
+    }
+}
+
 // Whether the decode rows of a launch take whole contexts (heads of up to 64: the accumulators of
 // sixteen waves), and then the KV heads of a workgroup.  Two such workgroups fill a compute unit.  Up to
 // one per unit no launch is slower than on partitions; more of them take turns, and each adds its phases
@@ -814,7 +829,7 @@ bool paged_attn_prepared_out(int num_seqs, int head_dim, int hq, int hkv, int bl
     if (max_seqlen_q != 1 || (int64_t)hq * head_dim % 128 != 0) return false;
     if (const int heads = anydim_whole_heads(num_seqs, head_dim, hkv, block_size, max_blocks_per_seq))
         return (int64_t)hq / hkv * heads * head_dim % 128 == 0;
-    return 128 % head_dim == 0 && num_splits > 1;  // the merge writes it
+    return (head_dim == 32 || head_dim == 64) && num_splits > 1;  // the merge writes it
 }
 
 // Tile phases of a workgroup (a power of two) with `waves` waves at most, and the LDS they meet in.
@@ -974,10 +989,11 @@ hipError_t paged_attn_anydim_launch(const AttnParams& params, int head_dim, int 
         if (e != hipSuccess) return e;
     }
     if ((phases & LOGISMOS_ATTN_PHASE_MERGE) && p.num_splits > 1) {
-        if (p.out_bf16 == 2)
-            paged_attn_anydim_merge_prepared_kernel<<<dim3(p.hq * head_dim / 128, p.num_seqs), dim3(256),
-                                                      0, stream>>>(p, head_dim);
-        else
+        if (p.out_bf16 == 2) {
+            const auto merge = head_dim == 32 ? paged_attn_anydim_merge_prepared_kernel<32>
+                                              : paged_attn_anydim_merge_prepared_kernel<64>;
+            merge<<<dim3(p.hq * head_dim / 128, p.num_seqs), dim3(256), 0, stream>>>(p);
+        } else
             paged_attn_anydim_merge_kernel<<<dim3(p.hq, p.num_seqs), dim3(256), 0, stream>>>(p, head_dim);
     }
     return hipGetLastError();
