@@ -7,6 +7,7 @@ import numpy as np
 import pytest
 
 from tests import workloads
+from tests.gpu_harness import DecodeStepRunner
 from tests.test_gpu_decode_step import _rel_l2, _run_both
 
 pytestmark = pytest.mark.gpu
@@ -56,3 +57,30 @@ def test_three_bit_pools(new):
         rng, num_layers=1, hidden=512, hq=4, hkv=2, inter=1024,
         ctx=[n + 40 + i for i, n in enumerate(new)], new_tokens=new, kv_turbo3=True)
     _check(cfg, layers, batch, 1e-2)  # the bound of the steps over 3-bit pools
+
+
+@pytest.mark.parametrize("rows", [64, 96])
+@pytest.mark.parametrize("hidden,hq,hkv,d,inter", WIDTHS)
+def test_whole_chunks_are_steps_of_32_rows(rows, hidden, hq, hkv, d, inter):
+    """Every chunk's rows, bit for bit, as a step of those 32 rows by themselves: a norm, rotation or
+    activation that took another row's value, group sum or place in a later chunk's buffer would not be.
+    (One key per sequence: attention is that key's value however a batch is split.)"""
+    rng = np.random.default_rng(rows + hidden)
+    cfg, layers, batch = workloads.decode_step_problem(
+        rng, num_layers=2, hidden=hidden, hq=hq, hkv=hkv, d=d, inter=inter, ctx=np.ones(rows, np.int32),
+        qkv_bias=True)
+
+    def run(r0, r1):
+        part = dict(batch, cu_seqlens=np.arange(r1 - r0 + 1, dtype=np.int32))
+        for name in ("h", "block_tables", "context_lens", "positions", "slots"):
+            part[name] = batch[name][r0:r1]
+        r = DecodeStepRunner(cfg, layers, part)
+        r.launch()
+        pools = [p.to_numpy(np.uint16, L["k_pool"].shape)[part["slots"]]
+                 for kv, L in zip(r.pools, layers) for p in kv]
+        return r.result_bits(), r.h.to_numpy(np.uint32, (r1 - r0, hidden)), *pools
+
+    whole = run(0, rows)
+    for r0 in range(0, rows, 32):
+        for got, want in zip(whole, run(r0, r0 + 32)):
+            assert np.array_equal(got[r0:r0 + 32], want)

@@ -46,13 +46,15 @@ def test_matmul_into_rows_off_sixteen_bytes(m, n, k):
     rng = np.random.default_rng(m)
     a, b = _f16(rng, m, k), _f16(rng, k, n)
     da, db = hip.DeviceBuffer.from_numpy(a), hip.DeviceBuffer.from_numpy(b)
-    d = hip.DeviceBuffer(m * n * 2 + 16)  # (the whole of it is read back)
+    d = hip.DeviceBuffer(m * n * 2 + 16)
+    d.fill(0xA5)
     d2 = hip.DeviceBuffer(m * n * 2)
     kernels.launch_matmul_fp16("wmma", da, db, C.c_void_p(d.ptr.value + 2), m, n, k)
     kernels.launch_matmul_fp16("wmma", da, db, d2, m, n, k)
     hip.synchronize()
-    got = d.to_numpy(np.uint16, (m * n + 8,))[1:1 + m * n]
-    assert np.array_equal(got, d2.to_numpy(np.uint16, (m * n,)))
+    got = d.to_numpy(np.uint16, (m * n + 8,))
+    assert np.array_equal(got[1:1 + m * n], d2.to_numpy(np.uint16, (m * n,)))
+    assert got[0] == 0xA5A5 and (got[1 + m * n:] == 0xA5A5).all()  # and nothing beside them
 
 
 def test_matmul_leaves_out_what_lies_behind_k():
