@@ -891,17 +891,25 @@ static TpPlan tp_big_plan(int m, int n, int k, int block_groups, int cus) {
 // over x):
 //   K  896, 1152 columns:  100 rows 23.2 / 13.9, 1030 26.4 / 17.0, 2060 29.1 / 21.7, 4120 32.4 / 33.3
 //   K 1536, 2048 columns:  100 rows 13.1 / 13.4,  520 20.6 / 14.4, 1030 23.6 / 17.1, 2060 28.5 / 29.7
-// hence: at most 16 groups (at 32 a small tile's chain costs what the large one's parts do), all tiles
-// resident at once (two per compute unit), and where the big tiles could be split over K at least 20 of
-// them (2048 columns at 200 rows are 16: 15.1 / 13.7 us by themselves, but in a step the parts go to the
-// next operator without a sum of their own, and 28 layers of 1536 take 3418 / 3491 us).  A next product's operand is written by 64 x 256 tiles, one per compute unit, whose round takes
+// hence: at most 16 groups (at 32 a small tile's chain costs what the large one's parts do) and all tiles
+// resident at once (two per compute unit).  Where the big tiles could be split over K, it matters who adds
+// up the parts:
+// * the next operator of a step, which reads its operand anyway: at least 20 big tiles (28 layers of 1536,
+//   200 rows, 2048 columns of q/k/v, which are 16: 3418 us a step, 3491 on small ones);
+// * a launch of its own, 4 us: always in two parts and for fp32 results, else from ten big tiles on.  1440
+//   products of 16 to 1000 rows, 256 to 4608 columns, the first pass over x included:
+//     K 1280, 2 parts:  128 x 256 fp32 16.2 / 12.8, 300 x 256 bf16 16.6 / 14.1;  K 2048, 2 parts:  128 x 256 bf16 19.4 / 17.5
+//     K 1536, 3 parts:  128 x 256 fp32 14.3 / 14.0, bf16 14.2 / 14.9, with SwiGLU 11.5 / 12.4 (from ten tiles on:
+//     128 x 2560 16.5 / 14.2, 16.4 / 15.1, 13.1 / 12.6; 200 x 2048 18.1 / 14.7, 18.0 / 15.7, 13.8 / 12.6)
+// A next product's operand is written by 64 x 256 tiles, one per compute unit, whose round takes
 // five eighths of a big one's (a last round that is split over K about six of them):
 //   K  896, 4864 outputs:  195 rows 23.4 / 15.7,  520 25.2 / 28.2, 1030 45.8 / 40.8, 2060 69.4 / 77.4
 //   K 1536, 8960 outputs:  100 rows 23.6 / 16.8,  195 25.5 / 31.9,  300 28.3 / 33.9, 2060 148 / 168
 // Whole large tiles in front of split ones keep the large tiles (none of the above is lost by it), so
 // that a launch on the smaller ones adds up all of its tiles alike.
+// parts_out: the launch may leave its K parts to the next operator.
 template <int OUT>
-static bool tp_less(int m, int n, int k, int block_groups, int cus) {
+static bool tp_less(int m, int n, int k, int block_groups, int cus, bool parts_out) {
     const int groups = k >> 7;
     if (groups > 16) return false;
     auto tiles = [&](int rows, int tm, int tn) {
@@ -917,7 +925,9 @@ static bool tp_less(int m, int n, int k, int block_groups, int cus) {
     }
     const int div = tp_is_swiglu(OUT) ? 2 : 1;
     if (tiles(m, TpSmall<false>::kM, TpSmall<false>::kN / div) > 2 * cus) return false;
-    return tiles(m, TpBig::kM, TpBig::kN / div) >= 20 || plan.split == 1;
+    const int64_t big = tiles(m, TpBig::kM, TpBig::kN / div);
+    if (parts_out) return plan.split == 1 || big >= 20;
+    return plan.split <= 2 || OUT == kTpOutF32 || big >= 10;
 }
 
 template <int OUT, int W, bool ODD, class T>
@@ -967,7 +977,7 @@ static hipError_t tallp_launch(const uint16_t* xp, const float* xs, float* parti
     using LessCuts = std::conditional_t<operand, TpHalf<true>, TpSmall<true>>;
     const int cus = device_cu_count();
     if (cus <= 0) return hipErrorInvalidDevice;
-    if (tp_less<OUT>(m, n, k, 2 * W, cus)) {
+    if (tp_less<OUT>(m, n, k, 2 * W, cus, OUT == kTpOutF32 && out_pairs != 0)) {
         if (tp_big_plan<OUT>(m, n, k, 2 * W, cus).split > 1)
             return tallp_launch_tile<OUT, W, ODD, LessCuts>(xp, xs, partials, qw, scale, zero, bias, y,
                                                             m, n, k, st, out_pairs);
@@ -1055,7 +1065,7 @@ static int tallp_parts(const void* scale_f16, const void* zero_f16, int m, int n
     const int cus = device_cu_count();
     if (cus <= 0) return 1;
     const int block_groups = ((k >> 7) & 1) ? 2 : 2 * tp_pairs_per_load(k, scale_f16, zero_f16);
-    if (tp_less<kTpOutF32>(m, n, k, block_groups, cus)) return 1;
+    if (tp_less<kTpOutF32>(m, n, k, block_groups, cus, true)) return 1;
     const int tiles = ((m + kTpTileM - 1) / kTpTileM) * ((n + kTpTileN - 1) / kTpTileN);
     const TpPlan plan = tp_plan(tiles, k >> 7, block_groups, cus);
     return plan.full == 0 ? plan.split : 1;

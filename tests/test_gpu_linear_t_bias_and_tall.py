@@ -203,7 +203,9 @@ def test_q4g128_workspace_kernel_ragged_shapes(b, n, k, with_bias):
     # how many pairs of groups a lane loads scales / zeros / sums for at once (a multiple of
     # 1024: four, 1536 = 3 x 512: two, else one), each with one and with several such blocks;
     # every one of these launches is smaller than the device, so its tiles are split over K
-    # (evenly or not: 24 groups in parts of 8, 12 in parts of 4) and summed by the reduce kernel
+    # (evenly or not: 24 groups in parts of 8, 12 in parts of 4) and summed by the reduce kernel, or
+    # smaller ones that take all of K and add up in the same parts (the fp32 product at 12 groups,
+    # where the bf16 one is split)
     rng = np.random.default_rng(b + 7 * n + 13 * k)
     qw, s, z = _q4(rng, n, k)
     xb = O.f32_to_bf16_bits(rng.standard_normal((b, k), np.float32))
