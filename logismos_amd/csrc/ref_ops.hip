@@ -488,12 +488,13 @@ __global__ __launch_bounds__(64 * WR * WC) void matmul_ring_fp16_kernel(
 #pragma unroll
             for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.0f;
     const int slabs = (k + KS - 1) / KS;
-    auto multiply = [&](auto kk_c, int s) LG_INLINE {
+    // (LAST: the slab is the last one, which may end past k)
+    auto multiply = [&](auto kk_c, auto last_c, int s) LG_INLINE {
         constexpr int KK = decltype(kk_c)::value, P = KK & 1;
         uint4_t bv[NB];
 #pragma unroll
         for (int j = 0; j < NB; ++j) bv[j] = uint4_t{bl[P][j][0], bl[P][j][1], bh[P][j][0], bh[P][j][1]};
-        if (s * KS + KS > k) {
+        if (decltype(last_c)::value && s * KS + KS > k) {
             // past k: zeros on both sides (what lies there may be an infinity)
             const bool in = s * KS + 16 * KK + 8 * h < k;
 #pragma unroll
@@ -528,22 +529,25 @@ __global__ __launch_bounds__(64 * WR * WC) void matmul_ring_fp16_kernel(
     __builtin_amdgcn_s_barrier();
     read_step(ic<0>{}, 0);
     step_landed(ic<0>{});
-    int buf_off = 0;
-    for (int s = 0; s < slabs; ++s) {
+    // MORE: there is a slab behind this one.  (A constant: whether a read is waited for has to be known where
+    // it is asked for, or the compiler may join the two ways with a copy of what is still in flight.)
+    auto slab = [&](auto more_c, int s, int buf_off) LG_INLINE {
+        constexpr bool more = decltype(more_c)::value != 0;
+        constexpr ic<!more> last{};
         const int next_off = buf_off + kBuf == BUFS * kBuf ? 0 : buf_off + kBuf;
         const int last_off = buf_off == 0 ? (BUFS - 1) * kBuf : buf_off - kBuf;  // of slab s - 1
-        const bool more = s + 1 < slabs, ahead = s + BUFS - 1 < slabs;
+        const bool ahead = more && s + BUFS - 1 < slabs;
         read_step(ic<1>{}, buf_off);
         __builtin_amdgcn_sched_barrier(0);
-        multiply(ic<0>{}, s);
+        multiply(ic<0>{}, last, s);
         __builtin_amdgcn_sched_barrier(0);
         step_landed(ic<1>{});
         read_step(ic<2>{}, buf_off);
         __builtin_amdgcn_sched_barrier(0);
-        multiply(ic<1>{}, s);
+        multiply(ic<1>{}, last, s);
         __builtin_amdgcn_sched_barrier(0);
         step_landed(ic<2>{});
-        if (more) {
+        if constexpr (more) {
             // slab s + 1 has landed (its requests are the oldest of BUFS - 2 slabs'; this wave's
             // requests complete in the order they were issued), behind the barrier everybody's has,
             // and everybody has left slab s - 1, whose buffer slab s + BUFS - 1 takes
@@ -554,17 +558,20 @@ __global__ __launch_bounds__(64 * WR * WC) void matmul_ring_fp16_kernel(
         read_step(ic<3>{}, buf_off);
         if (ahead) request_a(s + BUFS - 1, last_off);
         __builtin_amdgcn_sched_barrier(0);
-        multiply(ic<2>{}, s);
+        multiply(ic<2>{}, last, s);
         __builtin_amdgcn_sched_barrier(0);
         step_landed(ic<3>{});
-        if (more) read_step(ic<0>{}, next_off);
+        if constexpr (more) read_step(ic<0>{}, next_off);
         if (ahead) request_b(s + BUFS - 1, last_off);
         __builtin_amdgcn_sched_barrier(0);
-        multiply(ic<3>{}, s);
+        multiply(ic<3>{}, last, s);
         __builtin_amdgcn_sched_barrier(0);
-        if (more) step_landed(ic<0>{});
-        buf_off = next_off;
-    }
+        if constexpr (more) step_landed(ic<0>{});
+        return next_off;
+    };
+    int buf_off = 0;
+    for (int s = 0; s + 1 < slabs; ++s) buf_off = slab(ic<1>{}, s, buf_off);
+    slab(ic<0>{}, slabs - 1, buf_off);
 
     // lane (h, r) holds column r, rows 8 * (e / 4) + 4h + e % 4 of each 32 x 32 block
     if (!vec_out) {
@@ -629,46 +636,60 @@ static hipError_t matmul_ring_launch(const void* a, const void* b, void* d, int 
 // Which tile: the one whose rounds take the least.  A compute unit holds as many workgroups of a tile as
 // the ring (min(slabs, buffers) slabs of LDS) and the registers allow; a round of r of them takes the tile's
 // ramp and, per slab of 64 columns, the longer of its own chain of dependent steps and r times its share of
-// the unit.  `once`, `ramp`, `chain` and `share` in us, fitted to 663 shapes (64 to 5000 rows, 512 to 4096
-// columns, K 64 to 4096): the tile taken is 0.8 % off the fastest of the six on the mean.  Counting tiles only,
-// a nearly empty second round went unseen (264 tiles of 64 x 128 for 2100 x 1024).  us, the tile taken / by
-// count / the kernel with a slab in registers on its way to two buffers:
-//   2036 x 1536 x 1536  17.6 / 18.2 / 21.7   2100 x 1024 x 768  10.4 / 15.2 / 11.5   4096 x 4096 x 768  34.2 / 34.9 / 40.0
-//   1300 x 3072 x 4096  52.5 / 76.3 / 67.4   2900 x 768 x 4096  37.3 / 57.8 / 48.3   700 x 3072 x 256   5.7 / 8.5 / 6.1
-//   2036 x 512 x 768    7.2 / 7.3 / 7.3      3200 x 768 x 64    4.3 / 5.9 / 4.2
-// Up to three slabs the shorter rings only.  (One or two slabs, no ring to speak of: 15 of the 663 shapes are up
-// to 0.46 us behind the kernel of two buffers.)
+// the unit.  The share is larger by `uneven` where the rows of A or B are not whole 128-byte lines: what a
+// request asks for lies in more of them, the more so the narrower the tile.  All in us, fitted to 2380 shapes
+// (64 to 5000 rows, 512 to 4096 columns, K 64 to 4096, half of them uneven): the tile taken is 2.1 % off the
+// fastest of the six on the mean.  us, 256 x 128 / 128 x 128 / 64 x 128 / 64 x 64 (the last two on the better of
+// their rings):
+//   3200 x 768 x 2048   28.2 / 16.9 / 19.5 / 18.4   2100 x 1024 x 512   9.1 / 6.6 / 6.6 / 5.9
+//   1700 x 4096 x 512   12.3 / 13.4 / 14.4 / 16.2   200 x 4096 x 512    8.6 / 6.2 / 4.4 / 4.3
+// A shorter ring (three buffers) lets more workgroups share a unit.  Where the longer one holds all there are, it
+// is taken: at a long K the shorter one waits for memory (200 x 3072 x 3560 26.0 / 17.0, 700 x 512 x 3560 25.5 /
+// 16.5).  Up to three slabs there is no difference but the code; the shorter one then.
 // What bounds it: the operands' way from L2 where tiles are many, where they are few a slab's chain of four
-// dependent steps, 0.3 us on 64 x 64, 0.5 on 128 x 128.
+// dependent steps, 0.24 us on 64 x 64, 0.34 on 128 x 128.
 struct MatmulTile {
     int rows, cols, bufs, most;  // most: workgroups of a compute unit by its registers
-    float once, ramp, chain, share;
+    float once, ramp, chain, share, uneven;
     decltype(&matmul_ring_launch<2, 2, 4, 2, 3>) launch;
+    int64_t held(int64_t slabs) const {  // workgroups of a unit
+        const int64_t lds = std::max(std::min<int64_t>(slabs, bufs) * (rows + cols) * 128,
+                                     (int64_t)rows * (cols + 8) * 2);
+        return std::min<int64_t>(160 * 1024 / lds, most);
+    }
+    float time(int64_t per_cu, int64_t slabs, bool whole_lines) const {
+        const int64_t h = held(slabs);
+        const float part = whole_lines ? share : share * (1.0f + uneven);
+        auto round = [&](int64_t r) { return ramp + (float)slabs * std::max(chain, (float)r * part); };
+        return once + (float)(per_cu / h) * round(h) + (per_cu % h ? round(per_cu % h) : 0.0f);
+    }
 };
-static float matmul_time(const MatmulTile& t, int64_t m, int64_t n, int64_t slabs, int64_t cus) {
-    const int64_t lds = std::max(std::min<int64_t>(slabs, t.bufs) * (t.rows + t.cols) * 128,
-                                 (int64_t)t.rows * (t.cols + 8) * 2);
-    const int64_t held = std::min<int64_t>(160 * 1024 / lds, t.most);
-    const int64_t tiles = ((m + t.rows - 1) / t.rows) * ((n + t.cols - 1) / t.cols);
-    const int64_t per_cu = (tiles + cus - 1) / cus;
-    auto round = [&](int64_t r) { return t.ramp + (float)slabs * std::max(t.chain, (float)r * t.share); };
-    return t.once + (float)(per_cu / held) * round(held) + (per_cu % held ? round(per_cu % held) : 0.0f);
-}
 static hipError_t matmul_tiled(const void* a, const void* b, void* d, int m, int n, int k, void* stream) {
     static const MatmulTile tiles[] = {
-        {256, 128, 3, 2, 0.0f, 4.86f, 0.29f, 0.77f, matmul_ring_launch<2, 2, 4, 2, 3>},
-        {128, 128, 5, 3, 0.46f, 3.55f, 0.52f, 0.53f, matmul_ring_launch<2, 1, 2, 4, 5>},
-        {64, 128, 5, 4, 1.67f, 1.87f, 0.41f, 0.41f, matmul_ring_launch<1, 1, 2, 4, 5>},
-        {64, 64, 5, 8, 2.05f, 1.35f, 0.33f, 0.23f, matmul_ring_launch<1, 1, 2, 2, 5>},
-        {64, 128, 3, 4, 1.10f, 2.38f, 0.44f, 0.36f, matmul_ring_launch<1, 1, 2, 4, 3>},
-        {64, 64, 3, 8, 2.09f, 1.22f, 0.38f, 0.22f, matmul_ring_launch<1, 1, 2, 2, 3>},
+        {256, 128, 3, 2, 0.0f, 3.71f, 0.25f, 0.90f, 0.19f, matmul_ring_launch<2, 2, 4, 2, 3>},
+        {128, 128, 5, 3, 0.02f, 3.56f, 0.34f, 0.48f, 0.13f, matmul_ring_launch<2, 1, 2, 4, 5>},
+        {64, 128, 5, 4, 0.67f, 1.97f, 0.32f, 0.32f, 0.10f, matmul_ring_launch<1, 1, 2, 4, 5>},
+        {64, 128, 3, 4, 1.15f, 1.72f, 0.50f, 0.32f, 0.10f, matmul_ring_launch<1, 1, 2, 4, 3>},
+        {64, 64, 5, 8, 1.48f, 1.10f, 0.24f, 0.24f, 0.20f, matmul_ring_launch<1, 1, 2, 2, 5>},
+        {64, 64, 3, 8, 1.55f, 1.15f, 0.22f, 0.18f, 0.27f, matmul_ring_launch<1, 1, 2, 2, 3>},
     };
     const int64_t slabs = ((int64_t)k + 63) / 64, cus = device_cu_count();
+    const bool whole_lines = n % 64 == 0 && k % 64 == 0;
     const MatmulTile* best = nullptr;
     float best_time = 0.0f;
+    bool all_held = false;  // of the tile in front, on the longer ring
     for (const MatmulTile& t : tiles) {
-        if (slabs <= 3 && t.bufs == 5 && t.rows == 64) continue;
-        const float time = matmul_time(t, m, n, slabs, cus);
+        const int64_t count = (((int64_t)m + t.rows - 1) / t.rows) * (((int64_t)n + t.cols - 1) / t.cols);
+        const int64_t per_cu = (count + cus - 1) / cus;
+        if (t.rows == 64) {
+            if (t.bufs == 5) {
+                if (slabs <= 3) continue;
+                all_held = per_cu <= t.held(slabs);
+            } else if (slabs > 3 && all_held) {
+                continue;
+            }
+        }
+        const float time = t.time(per_cu, slabs, whole_lines);
         if (!best || time < best_time) best = &t, best_time = time;
     }
     return best->launch(a, b, d, m, n, k, static_cast<hipStream_t>(stream));
