@@ -5,6 +5,9 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+// A lambda with two call sites is a function of its own otherwise, its captures in scratch.
+#define LG_INLINE __attribute__((always_inline))
+
 namespace lg {
 
 typedef _Float16 half8_t __attribute__((ext_vector_type(8)));
@@ -155,5 +158,16 @@ __device__ __forceinline__ float shfl_xor_f32(float v, int mask) {
 }
 
 __device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
+
+// 16 bytes per lane from src + off straight into LDS: lane 0's at byte dst, the others behind it in the order
+// of the lanes (1 KiB per wave).  As assembly: 32-bit offsets with a scalar base (the builtin widens each to a 64-bit
+// address in two more registers), and dst may be computed.  M0, which holds dst, is reserved to the
+// compiler -- it cannot be named as overwritten -- which sets it right in front of each use of its own.
+__device__ __forceinline__ void request_lds16(const void* src, unsigned off, unsigned dst) {
+    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
+                 :
+                 : "v"(off), "s"(src), "s"(dst)
+                 : "memory");
+}
 
 }  // namespace lg

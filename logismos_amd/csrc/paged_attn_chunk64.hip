@@ -5,7 +5,7 @@
 //
 // * A tile is 64 keys: 8 KiB of K and of V, straight from the pools into LDS (global_load_lds, 16
 //   bytes per lane, eight keys per request; block_size is a multiple of 16, so a request lies in one
-//   block), a ring of four tiles (two where every wave has its own), requested that far ahead.  The
+//   block), a ring of four tiles (two where every wave has its own), requested three (one) ahead.  The
 //   16-byte chunks of a row are swizzled by its index so that the operand reads below touch every
 //   bank once.
 // * Scores transposed: S^T = K . Q^T on v_mfma_f32_32x32x16_f16 (A = K from LDS, B = the queries, in
@@ -34,7 +34,6 @@
 namespace lg {
 
 typedef __attribute__((address_space(3))) void* c64_lds_ptr_t;
-#define LG_INLINE __attribute__((always_inline))
 
 // Lengths and block ids are the same for a whole wave and are not written while the kernel runs: read
 // through the constant address space they come as scalar loads.  (As vector loads, which is what the
@@ -133,10 +132,8 @@ __global__ __launch_bounds__(256, KP == 1 ? 2 : 1) void paged_attn_chunk64_kerne
             const unsigned dst = __builtin_amdgcn_readfirstlane(ring + (unsigned)buf * kBuf + (unsigned)k8 * 128u);
             const char* ks = kp + base;
             const char* vs = vp + base;
-            asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
-                         :: "v"(ko), "s"(ks), "s"(dst) : "memory");
-            asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
-                         :: "v"(vo), "s"(vs), "s"(dst + kC64Tile) : "memory");
+            request_lds16(ks, ko, dst);
+            request_lds16(vs, vo, dst + kC64Tile);
         }
     };
 

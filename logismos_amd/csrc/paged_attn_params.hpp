@@ -28,8 +28,8 @@ struct AttnParams {
     float scale_log2e;
     int causal;
     // 0: fp16 [T][hq][head_dim]; 1: bf16, same shape; 2: the prepared layout of the following
-    // Q4G128 GEMM (x = [out_rows][hq*128], see q4_common.hpp) -- what the step executor uses
-    // at head_dim 128
+    // Q4G128 GEMM (x = [out_rows][hq*head_dim], see q4_common.hpp) -- what the step executor uses
+    // where paged_attn_prepared_out says so
     int out_bf16;
     int out_rows;
 };

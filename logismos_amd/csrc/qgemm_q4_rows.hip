@@ -5,9 +5,9 @@
 //   activations and the weights of one projection; each launch costs its boundary, one trip to
 //   memory and its drain whatever it computes, so the chain's length is the step's time.  With
 //   fp32 K parts between the operators a layer is ten launches; here it is six (five with one
-//   attention partition; one more for heads of other widths than 128 or a chunk in the batch, whose
-//   attention rows are prepared for the o projection by a launch of their own, and one more over
-//   3-bit pools, where rotation and encoding follow the projection):
+//   attention partition; one more where attention cannot write the o projection's operand -- heads of
+//   other widths than 128 with a chunk in the batch, or not 32 or 64 wide -- and a launch of its own
+//   prepares its rows, and one more over 3-bit pools, where rotation and encoding follow the projection):
 //     rows_norm<QKV>   RMSNorm of the residual rows, q/k/v projection, bias, rotation, q out,
 //                      K/V rows into the pools
 //     attention, merge
@@ -46,7 +46,7 @@
 //   hidden  896, 14 / 2 heads of 64, MLP 4864, one row       16.5 (40)
 //   hidden 1536, 12 / 2 heads of 128, MLP 8960, 16 rows      29.8 (52)
 //   hidden 4096, 32 / 8 heads of 128, MLP 12288, one row     36.7 (62)
-// Whole steps: 24 layers of the first 1323 -> 784 us, 28 of the second 1796 -> 1172, 36 of the third
+// Whole steps: 24 layers of the first 1323 -> 784 us (674 since attention writes the operand), 28 of the second 1796 -> 1172, 36 of the third
 // 2769 -> 1882.
 #include "device_utils.hpp"
 #include "launch_common.hpp"

@@ -23,8 +23,8 @@
 //   the MFMA operands stay conflict-free;
 // * a wave takes ALL rows of the tile by 32 weight rows, so that no two waves unpack the same nibbles:
 //   56 vector instructions of unpack per 32 MFMAs instead of the 112 of 64 x 64 parts, for an LDS
-//   operand read per MFMA instead of one per two (16-byte reads come at 256 bytes per clock: 1100 of
-//   the 3600 cycles a group takes);
+//   operand read per MFMA instead of one per two (at 256 bytes per clock, the rate of 16-byte reads, these
+//   take 1100 clocks by count, of the 3600 that a group's 1.75 us are at about 2.05 GHz);
 // * the requests go out one per step of 16 columns.  Issued together behind the barrier, all eight
 //   waves waited in front of the texture addresser (48 requests x 16 cycles) with the matrix pipe
 //   idle: a build without any requests was 15 % faster, and this one gets most of that back.
@@ -66,9 +66,6 @@
 #include <type_traits>
 
 namespace lg {
-
-// (a lambda with two call sites is a function of its own otherwise, its captures in scratch)
-#define LG_INLINE __attribute__((always_inline))
 
 typedef __attribute__((address_space(3))) void* tp_lds_ptr_t;
 
@@ -162,9 +159,9 @@ struct TpRegs<T, 1> {
 };
 
 // What a launch writes.  kTpOutSwiglu: the weights are a gate/up pair [gate rows | up rows]
-// (2 n rows) and y [m][n] is bf16 silu(gate) * up -- a workgroup tile takes 128 gate rows and
-// the 128 up rows of the same outputs, a wave's first 32 columns the gate and its other 32 the
-// up values of the same 32 outputs, so a lane holds both products of a result and the fp32
+// (2 n rows) and y [m][n] is bf16 silu(gate) * up -- a workgroup tile takes as many gate rows as
+// up rows of the same outputs, a wave's first 16 columns the gate and its other 16 the up values of
+// the same 16 outputs, which the two halves of a row of 32 lanes exchange at the end, so that the fp32
 // gate/up products (a gigabyte at 8240 rows of a 12288-wide MLP) never go to memory.
 // kTpOutSwigluOperand: the same product, written as the operand of a following launch of this
 // kernel over K = n (n a multiple of 256): y is that launch's workspace -- the bf16 values in
@@ -285,28 +282,19 @@ __global__ __launch_bounds__(64 * T::kWaves) void qgemm_q4g128_tallp_kernel(
         const int piece = (lane & 3) ^ ((row >> 2) & 3);
         woff[q] = (unsigned)weight_row(row) * (unsigned)(k >> 1) + (unsigned)piece * 16u;
     }
-    // As assembly: the 32-bit offsets above with a scalar base (the builtin widens each to a
-    // 64-bit address in two more registers); M0 holds the LDS address of lane 0's 16 bytes and
-    // nothing else in this kernel uses M0.
-    auto request = [&](const char* src, unsigned off, unsigned dst) LG_INLINE {
-        asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
-                     :
-                     : "v"(off), "s"(src), "s"(dst)
-                     : "memory");
-    };
     // request q of group g's x and weights, into the buffer at byte `buf_off` of the ring
     auto request_x = [&](auto q_c, int g, int buf_off) LG_INLINE {
         constexpr int Q = decltype(q_c)::value;
         // (scalar registers for sure: a value the compiler takes for lane-dependent would be
         // handed to the statement in vector registers)
-        request(reinterpret_cast<const char*>(xp) + ((size_t)g * 256 + (size_t)Q * 8 * (unsigned)k),
+        request_lds16(reinterpret_cast<const char*>(xp) + ((size_t)g * 256 + (size_t)Q * 8 * (unsigned)k),
                 xoff ^ (64u * Q),
                 __builtin_amdgcn_readfirstlane(lds_base + (unsigned)buf_off +
                                                (unsigned)(wave * kXReq + Q) * 1024u));
     };
     auto request_w = [&](auto q_c, int g, int buf_off) LG_INLINE {
         constexpr int Q = decltype(q_c)::value;
-        request(reinterpret_cast<const char*>(qw) + (size_t)g * 64, woff[Q],
+        request_lds16(reinterpret_cast<const char*>(qw) + (size_t)g * 64, woff[Q],
                 __builtin_amdgcn_readfirstlane(lds_base + (unsigned)buf_off + kSlab +
                                                (unsigned)(wave * 2 + Q) * 1024u));
     };
@@ -772,9 +760,9 @@ __global__ __launch_bounds__(64 * T::kWaves) void qgemm_q4g128_tallp_kernel(
 }
 
 // Sums the `split` fp32 parts of each tile of the last round, in part order, adds the bias and
-// writes y.  One thread per result; a part's element index is (wave, i, j, e, lane) as the
-// product kernel left it.  (SwiGLU: j = 0 is the gate and j = 1 the up product of the same
-// result; one thread takes both.)
+// writes y.  One thread per result; a part's element index is (wave, i, e, lane) as the
+// product kernel left it.  (SwiGLU: lane % 32 < 16 is the gate and the lane 16 on the up product of the
+// same result; one thread takes both.)
 template <int OUT>
 __global__ __launch_bounds__(256) void q4_tall_reduce_kernel(const float* __restrict__ partials,
                                                             const float* __restrict__ bias,

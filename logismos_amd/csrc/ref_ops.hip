@@ -361,7 +361,6 @@ __global__ __launch_bounds__(256) void matmul_mfma_fp16_kernel(const _Float16* _
 // come back with 4 k of one column each.  LDS is only touched through inline assembly inside the
 // loop: the compiler would order every access it can see behind all outstanding requests.
 typedef __attribute__((address_space(3))) void* mm_lds_ptr_t;
-#define LG_INLINE __attribute__((always_inline))
 template <int MB, int NB, int WR, int WC, int BUFS>
 __global__ __launch_bounds__(64 * WR * WC) void matmul_ring_fp16_kernel(
     const _Float16* __restrict__ a, const _Float16* __restrict__ b, _Float16* __restrict__ d, int m,
@@ -409,22 +408,16 @@ __global__ __launch_bounds__(64 * WR * WC) void matmul_ring_fp16_kernel(
         b_row[q] = BR * (RB * wave + q) + lane / (TN / 8);
         b_col[q] = (unsigned)min(col0 + 8 * ((lane % (TN / 8)) ^ b_swizzle(b_row[q])), n - 8);
     }
-    auto request = [&](const void* src, unsigned off, unsigned dst) LG_INLINE {
-        asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
-                     :
-                     : "v"(off), "s"(src), "s"(dst)
-                     : "memory");
-    };
     auto request_a = [&](int s, int buf_off) LG_INLINE {
 #pragma unroll
         for (int q = 0; q < RA; ++q)
-            request(a, (a_row[q] + (unsigned)min(s * KS + a_chunk[q], k - 8)) * 2u,
+            request_lds16(a, (a_row[q] + (unsigned)min(s * KS + a_chunk[q], k - 8)) * 2u,
                     __builtin_amdgcn_readfirstlane(lds_base + (unsigned)buf_off + (unsigned)(RA * wave + q) * 1024u));
     };
     auto request_b = [&](int s, int buf_off) LG_INLINE {
 #pragma unroll
         for (int q = 0; q < RB; ++q)
-            request(b, ((unsigned)min(s * KS + b_row[q], k - 1) * (unsigned)n + b_col[q]) * 2u,
+            request_lds16(b, ((unsigned)min(s * KS + b_row[q], k - 1) * (unsigned)n + b_col[q]) * 2u,
                     __builtin_amdgcn_readfirstlane(lds_base + (unsigned)buf_off + kA + (unsigned)(RB * wave + q) * 1024u));
     };
 
