@@ -739,9 +739,9 @@ typedef struct {
     /* A mixed batch (chunked prefill + decode): total_tokens = cu_seqlens[num_seqs] packed
      * rows and the largest number of new tokens of a sequence; 0 / 0 means one new token per
      * sequence.  Every per-row array above (hidden_f32, out_bf16, positions, slot_mapping) then
-     * has total_tokens rows, in packed order.  Up to 96 rows go through the projections 32 at
-     * a time, every pass streaming the layer's weights once; from 97 rows on every projection
-     * is one launch of the tiled matrix-core GEMM over all rows (`linear_t` over `seq` rows,
+     * has total_tokens rows, in packed order.  Every projection takes all rows in one launch: up
+     * to 96 of them as chunks of 32 side by side (over 3-bit pools, with prompt chunks, a last
+     * one of few rows may follow by itself), from 97 on in the tiled matrix-core GEMM (`linear_t` over `seq` rows,
      * crates/transformers/src/mlp.rs:104-111).  The attention takes the whole ragged batch in
      * one launch either way.  token_ids takes any number of rows; lm_head, as described
      * above (a token for every packed row), needs total_tokens <= 32. */
