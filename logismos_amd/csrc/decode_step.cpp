@@ -94,16 +94,18 @@ Workspace carve(const logismos_decode_config_t& c, int num_seqs, int t, int num_
     w.chunks = (t + kChunkRows - 1) / kChunkRows;
     const int b = t < kChunkRows ? t : kChunkRows;
     // fp32 rows that the K parts of a product take: those of all rows on the plan of a chunk, and of a
-    // ragged last chunk by itself, which may have more parts (few rows are split further).  The most
-    // over all smaller batches too, so that a workspace for many rows is one for fewer.
+    // ragged last chunk by itself, which may have more parts (few rows are split further).  The size
+    // asked for (no base) holds the most over all smaller batches too, so that a workspace for many rows
+    // is one for fewer; a launch lays out what its batch takes, which is no more (32 plans of four products
+    // are 3 to 6 us of a host core).
+    const int last = t - (w.chunks - 1) * kChunkRows;
     auto part_rows = [&](int n, int k) {
-        int most = 0;
-        for (int rows = 1; rows <= b; ++rows) {
+        int most = logismos_qgemm_q4g128_splitk_xprep_parts(b, n, k) * t;
+        for (int rows = base ? last : 1; rows <= (base ? last : b); ++rows) {
             const int r = logismos_qgemm_q4g128_splitk_xprep_parts(rows, n, k) * rows;
             most = r > most ? r : most;
         }
-        const int all = logismos_qgemm_q4g128_splitk_xprep_parts(b, n, k) * t;
-        return (size_t)(all > most ? all : most);
+        return (size_t)most;
     };
     const size_t o_rows = part_rows(c.hidden, (int)qd), down_rows = part_rows(c.hidden, c.intermediate);
     // prepared activations of all rows: one buffer, or one per chunk of 32

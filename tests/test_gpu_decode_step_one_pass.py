@@ -6,6 +6,7 @@ by itself when there are chunks)."""
 import numpy as np
 import pytest
 
+from logismos_amd import hip
 from tests import workloads
 from tests.gpu_harness import DecodeStepRunner
 from tests.test_gpu_decode_step import _rel_l2, _run_both
@@ -84,3 +85,21 @@ def test_whole_chunks_are_steps_of_32_rows(rows, hidden, hq, hkv, d, inter):
     for r0 in range(0, rows, 32):
         for got, want in zip(whole, run(r0, r0 + 32)):
             assert np.array_equal(got[r0:r0 + 32], want)
+
+
+@pytest.mark.parametrize("new", [[1] * 17, [1] * 33, [1] * 65, [1, 30, 2, 4]])  # (the last over 3-bit pools: two passes)
+@pytest.mark.parametrize("hidden,hq,hkv,d,inter", WIDTHS)
+def test_nothing_behind_the_workspace(new, hidden, hq, hkv, d, inter):
+    rng = np.random.default_rng(hidden)
+    cfg, layers, batch = workloads.decode_step_problem(
+        rng, num_layers=1, hidden=hidden, hq=hq, hkv=hkv, d=d, inter=inter, ctx=[n + 5 for n in new],
+        new_tokens=new, kv_turbo3=max(new) > 1 and d == 128)
+    r = DecodeStepRunner(cfg, layers, batch)
+    r.launch()
+    want, size = r.result_bits(), r.ws.nbytes
+    r = DecodeStepRunner(cfg, layers, batch)
+    r.ws = hip.DeviceBuffer(size + 4096)
+    r.ws.fill(0xA5)
+    r.launch()
+    assert np.array_equal(r.result_bits(), want)
+    assert (r.ws.to_numpy(np.uint8, (size + 4096,))[size:] == 0xA5).all()
