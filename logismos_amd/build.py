@@ -47,6 +47,7 @@ EXTRA_FLAGS = {
     "qgemm_q4_splitk.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
     "qgemm_q4_stream.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
     "qgemm_q4_greedy.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
+    "decode_resident.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
     "qgemm_q4_rows.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
     "ref_ops.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
     "paged_attn_chunk64.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],

@@ -1,0 +1,23 @@
+// The layers of a decode step of one row as one resident launch (decode_resident.hip).
+#pragma once
+
+#include "../../include/logismos_decode.h"
+
+#include <hip/hip_runtime.h>
+#include <stddef.h>
+
+namespace lg {
+
+// Bytes of the step's workspace that the launch uses: 0 where the geometry is not one of its own.
+size_t decode_resident_bytes(const logismos_decode_config_t& c);
+
+// Whether a step of t rows over these operands runs there.
+bool decode_resident_applies(const logismos_decode_config_t& c, const logismos_decode_layer_t* layers,
+                             const logismos_decode_batch_t& b, int t);
+
+// All layers: residual stream in and out in b.hidden_f32, K/V rows into the pools.  workgroups: how many are
+// launched (0: as many as the work is cut for; fewer do the same work with the same result).
+hipError_t decode_resident_launch(const logismos_decode_config_t& c, const logismos_decode_layer_t* layers,
+                                  const logismos_decode_batch_t& b, void* region, int workgroups, hipStream_t st);
+
+}  // namespace lg

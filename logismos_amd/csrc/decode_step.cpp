@@ -3,6 +3,7 @@
 // does not have yet (crates/decoders/src/lib.rs is a scaffold), written against
 // the launchers of this library only.  Nothing is allocated, nothing
 // synchronises; a caller may capture the whole step into a HIP graph.
+#include "decode_resident.hpp"
 #include "launch_common.hpp"
 #include "q4_rows.hpp"
 
@@ -42,6 +43,8 @@ struct Workspace {
                       // steps; a many-row step has t_xn free by then)
     char* last_rows;  // bf16 [num_seqs][hidden]: the normed last rows, gathered
     char* last_xn;    // prepared activations of one chunk of them
+    char* resident;   // of the resident launch; in every step's workspace, so that one for many rows
+                      // is one for few
     bool tall;
     size_t xn_stride;
     int chunks;        // of 32 rows
@@ -62,6 +65,7 @@ Workspace carve(const logismos_decode_config_t& c, int num_seqs, int t, int num_
     const size_t qd = (size_t)c.num_q_heads * c.head_dim;
     const size_t kvd = (size_t)c.num_kv_heads * c.head_dim;
     w.tall = t >= kTallRows;
+    w.resident = take(lg::decode_resident_bytes(c));
     if (w.tall) {
         w.attn_ws = take(
             logismos_paged_attn_workspace_bytes(num_seqs, c.num_q_heads, c.head_dim, num_splits));
@@ -533,7 +537,10 @@ extern "C" logismos_status_t logismos_launch_decode_step(const logismos_decode_c
         return last_only ? project_last_rows() : 0;
     }
     int res_parts = 0;  // split-K parts of the last down projection not yet folded into h
-    if (few_rows(c, layers, t)) {
+    if (lg::decode_resident_applies(c, layers, *batch, t)) {
+        LG_TRY(lg::decode_resident_launch(c, layers, *batch, w.resident, 0,
+                                          static_cast<hipStream_t>(stream)));
+    } else if (few_rows(c, layers, t)) {
         LG_TRY(few_rows_layers(c, layers, batch, w, t, max_q, direct, stream));
     } else {
         // All rows in one launch of every operator, the projections in chunks of 32 side by side (48

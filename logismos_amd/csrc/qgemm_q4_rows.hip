@@ -60,12 +60,6 @@ namespace lg {
 
 namespace {
 
-__device__ __forceinline__ unsigned pack_bf16(float lo, float hi) {
-    typedef float f2 __attribute__((ext_vector_type(2)));
-    const f2 v = {lo, hi};
-    return __builtin_bit_cast(unsigned, __builtin_convertvector(v, bf16x2_t));
-}
-
 // A tile is two runs of eight weight rows, `rows_tile_first` and `rows_tile_apart` further on:
 // for the rotation the two halves of its pairs, for the SwiGLU the gate and the up rows of the
 // same outputs.
@@ -86,18 +80,6 @@ __device__ __forceinline__ int rows_tile_apart(const RowsEpilogueArgs& e) {
     return EPI == kRowsSilu ? e.inter : (EPI == kRowsQkv ? e.head_dim >> 1 : 8);
 }
 
-// The unpack's magic number and the ones of the sum MFMA, kept in registers.
-struct RowsConst {
-    unsigned magic;
-    bf16x8_t ones;
-    __device__ __forceinline__ RowsConst() {
-        unsigned one;
-        asm volatile("v_mov_b32 %0, 0x43004300" : "=v"(magic));
-        asm volatile("v_mov_b32 %0, 0x3f803f80" : "=v"(one));
-        ones = __builtin_bit_cast(bf16x8_t, uint4_t{one, one, one, one});
-    }
-};
-
 // Sum of x over a group of K, per batch row, in the layout of the products.
 __device__ __forceinline__ float4_t rows_group_sum(const uint4_t (&x)[4], const RowsConst& c) {
     float4_t s = {0.0f, 0.0f, 0.0f, 0.0f};
@@ -105,31 +87,6 @@ __device__ __forceinline__ float4_t rows_group_sum(const uint4_t (&x)[4], const 
     for (int s4 = 0; s4 < 4; ++s4)
         s = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, x[s4]), c.ones, s, 0, 0, 0);
     return s;
-}
-
-// y += one group of 128 columns of K: scale * (x . q - zero * sum(x)), nibbles as bf16 128 + q.
-__device__ __forceinline__ void rows_group(float4_t& y, const uint4_t& wv, const uint4_t (&x)[4],
-                                           const float4_t& xs, uint16_t scale, uint16_t zero,
-                                           const RowsConst& c) {
-    const float sf = __half2float(__ushort_as_half(scale));
-    const float zf = 128.0f + __half2float(__ushort_as_half(zero));
-    float4_t acc = {0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-    for (int s4 = 0; s4 < 4; ++s4) {
-        uint4_t h;
-#pragma unroll
-        for (int sft = 0; sft < 4; ++sft) h[sft] = ((wv[s4] >> (4 * sft)) & kNibMask) | c.magic;
-        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, x[s4]),
-                                                      __builtin_bit_cast(bf16x8_t, h), acc, 0, 0, 0);
-    }
-#pragma unroll
-    for (int e = 0; e < 4; ++e) y[e] = fmaf(sf, fmaf(-zf, xs[e], acc[e]), y[e]);
-}
-
-// Groups [first, first + count) of wave w when `groups` are dealt to `waves` evenly.
-__device__ __forceinline__ int2 rows_share(int groups, int waves, int w) {
-    const int each = groups / waves, more = groups - each * waves;
-    return int2{w * each + min(w, more), each + (w < more ? 1 : 0)};
 }
 
 // A wave's slices (GPW groups) of the 16 weight rows of a tile, 16 bytes per lane and request,

@@ -1,0 +1,134 @@
+"""A step of one row, whose layers are one resident launch (decode_resident.hip): edges of its lists and
+pieces against the oracle, any number of workgroups bit for bit, and against the route of 2 to 16 rows."""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+from logismos_amd import hip, kernels
+from tests import workloads
+from tests.gpu_harness import DecodeStepRunner
+from tests.test_gpu_decode_step import _rel_l2, _run_both
+
+pytestmark = pytest.mark.gpu
+
+SHAPES = [  # hidden, query heads, KV heads, head width, MLP width, context, rows per KV block
+    (128, 1, 1, 128, 128, 1, 16),          # one group of K: seven waves with nothing; parts without a tile
+    (384, 3, 3, 128, 256, 16, 32),         # a whole tile of keys
+    (896, 14, 2, 64, 4864, 17, 16),        # 7 and 38 groups: shares of four and one; the new key alone in its tile
+    (896, 14, 2, 64, 4864, 500, 48),       # four pieces, read by the o projection itself
+    (1536, 12, 2, 128, 8960, 129, 16),     # 12 and 70 groups: shares of two and one, nine; one piece and a key
+    (512, 16, 1, 64, 512, 1300, 16),       # the widest group of heads, eleven pieces merged
+    (2176, 17, 17, 128, 1152, 700, 16),    # no two heads share K and V; more than one tile per wave
+    (4096, 32, 8, 128, 1024, 2100, 16),    # the widest norm, seventeen pieces merged
+    (512, 8, 2, 64, 16384, 70, 64),        # the widest operand
+]
+
+
+def _problem(shape, layers=1, seed=0, bias=True):
+    hidden, hq, hkv, d, inter, ctx, block = shape
+    return workloads.decode_step_problem(
+        np.random.default_rng(seed + hidden + ctx), num_layers=layers, hidden=hidden, hq=hq, hkv=hkv, d=d,
+        inter=inter, ctx=[ctx], block_size=block, qkv_bias=bias)
+
+
+def _state(r, batch, layers):
+    out = r.result_bits().copy()
+    h = r.h.to_numpy(np.float32, batch["h"].shape)
+    pools = [[b.to_numpy(np.uint16, L["k_pool"].shape) for b in kv] for kv, L in zip(r.pools, layers)]
+    return out, h, pools
+
+
+def _lib():
+    # library-internal: size of the region, and the launch with a number of workgroups
+    lib = C.CDLL(kernels.library()._name)
+    size, launch = (getattr(lib, n) for n in (
+        "_ZN2lg21decode_resident_bytesERK24logismos_decode_config_t",
+        "_ZN2lg22decode_resident_launchERK24logismos_decode_config_tPK23logismos_decode_layer_t"
+        "RK23logismos_decode_batch_tPviP12ihipStream_t"))
+    size.restype = C.c_size_t
+    return size, launch
+
+
+@pytest.mark.parametrize("shape", SHAPES)
+def test_against_the_oracle(shape):
+    cfg, layers, batch = _problem(shape)
+    r, got, want, lay, bat = _run_both(cfg, layers, batch)
+    assert _lib()[0](C.byref(r.cfg)) > 0  # the resident launch takes it
+    # one layer: the decode batch's bounds (tests/test_gpu_decode_step.py)
+    assert _rel_l2(got, want) < 6e-3
+    assert np.all(np.abs(got - want) <= 1.5e-2 + 2e-2 * np.abs(want))
+    assert _rel_l2(r.h.to_numpy(np.float32, bat["h"].shape), bat["h"]) < 6e-3
+    for (kp, vp), L in zip(r.pools, lay):
+        for buf, ref in ((kp, L["k_pool"]), (vp, L["v_pool"])):
+            diff = np.abs(buf.to_numpy(np.float16, ref.shape).astype(np.float32) - ref.astype(np.float32))
+            assert np.all((diff <= 4e-3) | (diff <= 1e-2 * np.abs(ref.astype(np.float32))))
+
+
+@pytest.mark.parametrize("workgroups", [1, 7, 100, 255])
+@pytest.mark.parametrize("shape", [SHAPES[2], (512, 8, 2, 128, 1024, 900, 16)])
+def test_any_number_of_workgroups(shape, workgroups):
+    # the work is cut for all compute units; fewer workgroups take several parts each, phase by phase
+    cfg, layers, batch = _problem(shape, layers=3)
+    whole = DecodeStepRunner(cfg, layers, batch)
+    size, launch = _lib()
+    want = None
+    for n in (0, workgroups, workgroups):
+        r = DecodeStepRunner(cfg, layers, batch)
+        region = hip.DeviceBuffer(size(C.byref(r.cfg)))
+        region.fill(0xFF)
+        assert launch(C.byref(r.cfg), r.layers, C.byref(r.batch), region.ptr, n, None) == 0
+        hip.synchronize()
+        got = _state(r, batch, layers)
+        want = want or got
+        assert np.array_equal(got[1], want[1])
+        assert all(np.array_equal(a, b) for x, y in zip(got[2], want[2]) for a, b in zip(x, y))
+    whole.launch()
+    assert np.array_equal(_state(whole, batch, layers)[1], want[1])
+
+
+@pytest.mark.parametrize("slot", ["its own", "none", "another key's"])
+@pytest.mark.parametrize("shape", [SHAPES[3], (512, 8, 2, 128, 1024, 300, 16)])
+def test_against_the_route_of_more_rows(shape, slot):
+    # scales off 16 bytes take the fused launches of 2 to 16 rows.  The row may be appended nowhere, or
+    # where an earlier key stands: attention then sees what the pools hold.
+    cfg, layers, batch = _problem(shape, seed=5)
+    if slot != "its own":
+        table, bs = batch["block_tables"][0], cfg["block_size"]
+        batch["slots"] = np.array([-1 if slot == "none" else int(table[2]) * bs + 5], np.int64)
+    states = []
+    for off in (0, 4):
+        r = DecodeStepRunner(cfg, layers, batch)
+        if off:
+            for lay, L in zip(r.layers, layers):
+                s = np.ascontiguousarray(L["qkv"][1]).view(np.uint16).reshape(-1)
+                buf = hip.DeviceBuffer.from_numpy(np.concatenate([np.zeros(off // 2, np.uint16), s]))
+                r.keep.append(buf)
+                w = lay.qkv
+                lay.qkv = kernels.Q4Weight(w.qw, buf.ptr.value + off, w.zero)
+        r.launch()
+        states.append(_state(r, batch, layers))
+    (a, ha, pa), (b, hb, pb) = states
+    # the same operands and roundings, other orders of the fp32 sums: last bits of fp16 and bf16 values
+    assert _rel_l2(ha, hb) < 2e-3
+    for x, y, L in zip(pa, pb, layers):
+        for u, v, name in zip(x, y, ("k_pool", "v_pool")):
+            was = L[name].view(np.uint16)
+            changed = np.nonzero((u != was).any(axis=1))[0]
+            assert changed.tolist() == ([] if slot == "none" else [int(batch["slots"][0])])
+            assert np.allclose(u.view(np.float16).astype(np.float32), v.view(np.float16).astype(np.float32),
+                               atol=4e-3, rtol=4e-3)
+
+
+def test_no_key_is_seen():
+    # a context of 0: attention adds nothing, and the layers still follow one another (more workgroups have
+    # q/k/v tiles than tiles of the other projections); twice the same
+    cfg, layers, batch = _problem((1024, 32, 16, 128, 128, 9, 16), layers=4, seed=9)
+    batch["context_lens"] = np.zeros(1, np.int32)
+    states = []
+    for _ in range(2):
+        r = DecodeStepRunner(cfg, layers, batch)
+        r.launch()
+        states.append(_state(r, batch, layers))
+    assert np.isfinite(states[0][1]).all() and np.array_equal(states[0][1], states[1][1])
+    assert not np.array_equal(states[0][1], batch["h"])
