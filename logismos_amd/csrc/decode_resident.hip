@@ -70,7 +70,6 @@ constexpr int kMaxList = 512;       // batches of a wave's part of a layer
 constexpr int kNormChunks = 2;      // chunks of eight columns a front thread normalises
 constexpr int kDirectWords = 8192;  // partial words the o projection's workgroups read themselves
 constexpr int kPollBudget = 1 << 21;
-constexpr int kPace = 2;            // of 64 clocks, between two requests of a wave while words are waited for
 
 // the projections, in the order of a layer; attention stands between the first two
 enum { kQkv = 0, kO = 1, kGateUp = 2, kDown = 3 };
@@ -115,7 +114,7 @@ struct ResidentPlan {
     int slots;           // per streaming wave
     // LDS, bytes from the start
     unsigned group_inv[4];  // of the projections' groups of K: 2^20 / groups, rounded up
-    int lds_x, lds_xs, lds_red, lds_scale[2], lds_ssq, lds_misc;
+    int lds_x, lds_red, lds_scale[2], lds_ssq, lds_misc;
     // the region: bytes from its start
     unsigned at_step, at_pieces, at_starts, at_lists, at_h, at_qkv, at_part, at_x, at_act, bytes;
     char* region;
@@ -240,7 +239,6 @@ struct Stream {
     int64_t v_from_k = 0;  // from a layer's K pool to its V pool
     unsigned key = ~0u, off0 = 0, off1 = 0;
     int key_c = 0;
-    int passed = 0;  // operands that this workgroup has had
     int in = 0, out = 0, issued = 0, used = 0;
     // the computing side
     int now = -64, now_part = -1;
@@ -370,23 +368,13 @@ struct Stream {
                       (unsigned)uniform((int)(q.dst + (r == 2 ? q.c * 512 : r * 1024))));
         ++issued;
     }
-    // Fills the ring.  A compute unit's requests return in order, so while the front waves wait for words
-    // the ring is filled no faster than memory can: a poll behind 96 KiB of requests takes 4 us.
-    template <bool PACED>
     __device__ __forceinline__ void fill() {
-        const unsigned* const ready = reinterpret_cast<const unsigned*>(lds + arguments().lds_misc) + 3;
 #pragma unroll 1
         while (true) {
             const Next q = next();
             if (q.c == 0) return;
 #pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                send(q, r);
-                if (PACED && q.c == 4) {
-                    const unsigned had = __hip_atomic_load(ready, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-                    if (uniform((int)had) <= passed) __builtin_amdgcn_s_sleep(kPace);
-                }
-            }
+            for (int r = 0; r < 4; ++r) send(q, r);
         }
     }
     // several parts: the requests of a phase's range only, when it is its turn
@@ -397,7 +385,7 @@ struct Stream {
         at = r.x;
         end = r.y;
         have = -64;
-        fill<false>();
+        fill();
     }
     __device__ __forceinline__ char* next_slot() {
         char* s = lds + ring + out * kSlot;
@@ -427,17 +415,15 @@ struct Stream {
         const int G = proj_shape(p, wh, D).k >> 7, lane = here();
         const int row = lane & 15, quarter = lane >> 4;
         const char* const xsrc = lds + p.lds_x + quarter * 64;
-        const float* const xsum = reinterpret_cast<const float*>(lds + p.lds_xs);
         const char* const scales = lds + ((wh & 1) ? p.lds_scale[1] : p.lds_scale[0]) + (row >> 3) * 16 * G +
                                    (row & 7) * G * 2;
         float* const red = reinterpret_cast<float*>(lds + p.lds_red) + wave * 16 + lane;
         const RowsConst cst;
         uint4_t x[C][4];
-        float y = 0.0f;
+        float xs[C], y = 0.0f;
         int xg = -1;  // the group that x starts with
         unsigned what = of(now_what, r.x - now);
         block_barrier();  // operand and scales are there
-        ++passed;
 #pragma unroll 1
         for (int i = r.x;;) {
             const int c = what & 7, t = (what >> 4) & 15, g = (what >> 8) & 255;
@@ -450,6 +436,9 @@ struct Stream {
                         for (int s4 = 0; s4 < 4; ++s4)
                             x[u][s4] = *reinterpret_cast<const uint4_t*>(xsrc + (g + u) * 256 + s4 * 16);
                     }
+                    // (the matrix cores have time; a front wave's sums would be on the chain)
+#pragma unroll
+                    for (int u = 0; u < C; ++u) xs[u] = rows_group_sum(x[u], cst)[0];
                     xg = g;
                 }
                 const char* const sc = scales + t * 64 * G + g * 2;
@@ -457,12 +446,10 @@ struct Stream {
                 const char* const wsrc = next_slot() + row * 64 * c;
                 const int sw = swizzle(row, c);
                 uint4_t w[C];
-                float xs[C];
                 uint16_t scale[C], zero[C];
 #pragma unroll
                 for (int u = 0; u < C; ++u) {
                     w[u] = *reinterpret_cast<const uint4_t*>(wsrc + (((4 * u + quarter) ^ sw) * 16));
-                    xs[u] = xsum[g + u];
                     scale[u] = *reinterpret_cast<const uint16_t*>(sc + 2 * u);
                     zero[u] = *reinterpret_cast<const uint16_t*>(sc + 32 * G + 2 * u);
                 }
@@ -508,7 +495,7 @@ struct Stream {
         if (c == 4) multiply<4>(p, wh, v, r);
         else if (c == 2) multiply<2>(p, wh, v, r);
         else multiply<1>(p, wh, v, r);
-        fill<true>();
+        fill();
     }
 
     // ---- attention: this wave's tiles of the part's piece
@@ -523,7 +510,6 @@ struct Stream {
         const float scale = p.scale_log2e;
         char* const area = lds + p.lds_x;
         block_barrier();  // the queries and the token's K/V row are there
-        ++passed;
         {
             half8_t q[KV];
 #pragma unroll
@@ -606,7 +592,7 @@ struct Stream {
                     acc[e] = __builtin_amdgcn_mfma_f32_16x16x16f16(pa, __builtin_bit_cast(half4_t, b), acc[e], 0, 0, 0);
                     acc[e] = __builtin_amdgcn_mfma_f32_16x16x16f16(pb, __builtin_bit_cast(half4_t, b), acc[e], 0, 0, 0);
                 }
-                if (i + 1 < range_.y) fill<false>();
+                if (i + 1 < range_.y) fill();
             }
             sum += lane_xor_f32<16>(sum);
             sum += lane_xor_f32<32>(sum);
@@ -623,14 +609,14 @@ struct Stream {
                         *reinterpret_cast<float4_t*>(part_ + 32 + (4 * tg + r) * D + E * c + e) =
                             float4_t{acc[e][r], acc[e + 1][r], acc[e + 2][r], acc[e + 3][r]};
             block_barrier();  // the waves' parts are there
-            fill<true>();
+            fill();
         }
     }
 
     __device__ __forceinline__ void run() {
         if (alone) {
             end = range(arguments(), rank, kPhases - 1).y;
-            fill<false>();
+            fill();
         }
 #pragma unroll 1
         for (int l = 0; l < layers; ++l)
@@ -652,7 +638,7 @@ struct Front {
     const int parts, layers;
     const Words words;
     int budget = kPollBudget;
-    unsigned meets = 0, operands = 0;
+    unsigned meets = 0;
     const int pieces;  // of the context
     const bool many;   // more partials than the o projection's workgroups read themselves
     const int pos;
@@ -678,13 +664,6 @@ struct Front {
         while (__hip_atomic_load(count, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) < meets) {
         }
         asm volatile("" ::: "memory");
-    }
-    // tells the streaming waves, before the barrier, that no poll is under way
-    __device__ __forceinline__ void operand_ready() {
-        ++operands;
-        if (tid == 0)
-            __hip_atomic_store(reinterpret_cast<unsigned*>(lds + arguments().lds_misc) + 3, operands, __ATOMIC_RELAXED,
-                               __HIP_MEMORY_SCOPE_WORKGROUP);
     }
     // once more around a poll?
     __device__ __forceinline__ bool again(bool ok) {
@@ -759,7 +738,8 @@ struct Front {
                     if (i * kFrontThreads >= chunks) continue;
                     const unsigned at = at_h + (unsigned)min(i * kFrontThreads + tid, chunks - 1) * 64u;
 #pragma unroll
-                    for (int q = 0; q < 4; ++q) raw[i][q] = words.get2(at + q * 16);
+                    for (int q = 0; q < 4; ++q)
+                        raw[i][q] = words.get2(at + q * 16);
                 }
 #pragma unroll
                 for (int i = 0; i < kNormChunks; ++i) {
@@ -800,13 +780,9 @@ struct Front {
             put_operand(o, i * kFrontThreads + tid, chunks);
         }
     }
-    // chunk c (eight columns in pair order), and with the 15 lanes beside it its group's sum
+    // chunk c (eight columns in pair order)
     __device__ __forceinline__ void put_operand(const uint4_t& o, int c, int chunks) {
-        Plan& p = arguments();
-        const float s = row16_sum(sum8_bf16(o));
-        if (c >= chunks) return;
-        *reinterpret_cast<uint4_t*>(lds + p.lds_x + c * 16) = o;
-        if ((lane & 15) == 0) reinterpret_cast<float*>(lds + p.lds_xs)[c >> 4] = s;
+        if (c < chunks) *reinterpret_cast<uint4_t*>(lds + arguments().lds_x + c * 16) = o;
     }
 
     // ---- the operand: bf16 values that are there as words of two
@@ -823,8 +799,9 @@ struct Front {
                 for (int i = 0; i < R; ++i) {
                     if (c0 + i * kFrontThreads >= chunks) continue;
                     const unsigned ch = (unsigned)min(c0 + i * kFrontThreads + tid, chunks - 1);
-                    raw[i][0] = words.get2(at + ch * 32u);
-                    raw[i][1] = words.get2(at + ch * 32u + 16u);
+#pragma unroll
+                    for (int q = 0; q < 2; ++q)
+                        raw[i][q] = words.get2(at + ch * 32u + q * 16u);
                 }
 #pragma unroll
                 for (int i = 0; i < R; ++i) {
@@ -1006,7 +983,6 @@ struct Front {
                 for (int j = 0; j < 2; ++j)
                     *reinterpret_cast<uint2_t*>(area + to[j]) = uint2_t{raw[j][0], raw[j][2]};
             }
-            operand_ready();
             block_barrier();
             block_barrier();  // the waves' parts are there
             const float* const part = reinterpret_cast<const float*>(area + attn_part_at(D));
@@ -1080,7 +1056,6 @@ struct Front {
             }
             first = false;
             asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the scales
-            operand_ready();
             block_barrier();
             if (alone) fetch_next_scales(which, l);
             block_barrier();  // the streaming waves' parts are there
@@ -1151,7 +1126,7 @@ __global__ __launch_bounds__(kThreads) void decode_resident_kernel(const Residen
     extern __shared__ __attribute__((aligned(16))) char lds[];
     const int tid = threadIdx.x;
     const int wave = uniform(tid >> 6);
-    unsigned* const misc = reinterpret_cast<unsigned*>(lds + p.lds_misc);  // {front barrier, rank, n, operands so far}
+    unsigned* const misc = reinterpret_cast<unsigned*>(lds + p.lds_misc);  // {front barrier, rank, n}
     if (tid == 0) {
         unsigned* const ctl = reinterpret_cast<unsigned*>(p.region);  // {tickets, closed}
         const unsigned ticket = __hip_atomic_fetch_add(ctl, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -1171,7 +1146,7 @@ __global__ __launch_bounds__(kThreads) void decode_resident_kernel(const Residen
                 if (n == 0) n = now;
             }
         }
-        misc[0] = misc[3] = 0;
+        misc[0] = 0;
         misc[1] = ticket;
         misc[2] = n;
     }
@@ -1295,7 +1270,7 @@ bool resident_plan(const logismos_decode_config_t& c, ResidentPlan* p) {
     const int tiles[4] = {(int)(width / 16), c.hidden / 16, c.intermediate / 8, c.hidden / 16};
     const int ks[4] = {c.hidden, (int)qd, c.hidden, c.intermediate};
     // a wave's list: the batches of its share of K for every tile, and its K/V tiles
-    int list = 0, held = 1, scale[2] = {0, 0}, x = 0, kmax = 0;
+    int list = 0, held = 1, scale[2] = {0, 0}, x = 0;
     for (int i = 0; i < 4; ++i) {
         const int per = (tiles[i] + parts - 1) / parts, groups = ks[i] / 128;
         if (per > kMaxTilesHeld) return false;
@@ -1307,7 +1282,6 @@ bool resident_plan(const logismos_decode_config_t& c, ResidentPlan* p) {
         if (bytes > scale[i & 1]) scale[i & 1] = bytes;
         const int op = 2 * ks[i];
         if (op > x) x = op;
-        if (ks[i] > kmax) kmax = ks[i];
         p->group_inv[i] = ((1u << 20) + groups - 1) / groups;
     }
     {
@@ -1348,7 +1322,6 @@ bool resident_plan(const logismos_decode_config_t& c, ResidentPlan* p) {
     };
     p->lds_misc = lds(16);
     p->lds_ssq = lds(kFrontWaves * 4);
-    p->lds_xs = lds(kmax / 128 * 4);
     p->lds_red = lds(red);
     p->lds_x = lds(x);
     p->lds_scale[0] = lds(scale[0]);

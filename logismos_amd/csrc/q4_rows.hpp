@@ -76,6 +76,15 @@ struct RowsConst {
     }
 };
 
+// Sum of x over a group of K, per batch row, in the layout of the products.
+__device__ __forceinline__ float4_t rows_group_sum(const uint4_t (&x)[4], const RowsConst& c) {
+    float4_t s = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int s4 = 0; s4 < 4; ++s4)
+        s = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, x[s4]), c.ones, s, 0, 0, 0);
+    return s;
+}
+
 // x . q over one group of 128 columns of K, nibbles as bf16 128 + q.
 __device__ __forceinline__ float4_t rows_product(const uint4_t& wv, const uint4_t (&x)[4], const RowsConst& c) {
     float4_t acc = {0.0f, 0.0f, 0.0f, 0.0f};

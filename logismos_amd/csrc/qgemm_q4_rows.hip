@@ -80,15 +80,6 @@ __device__ __forceinline__ int rows_tile_apart(const RowsEpilogueArgs& e) {
     return EPI == kRowsSilu ? e.inter : (EPI == kRowsQkv ? e.head_dim >> 1 : 8);
 }
 
-// Sum of x over a group of K, per batch row, in the layout of the products.
-__device__ __forceinline__ float4_t rows_group_sum(const uint4_t (&x)[4], const RowsConst& c) {
-    float4_t s = {0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-    for (int s4 = 0; s4 < 4; ++s4)
-        s = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, x[s4]), c.ones, s, 0, 0, 0);
-    return s;
-}
-
 // A wave's slices (GPW groups) of the 16 weight rows of a tile, 16 bytes per lane and request,
 // as whole runs of 64 * GPW bytes; put down row by row (stride 4 * GPW + 1 pieces) and read back
 // as MFMA operands (lane = 16 rows x 4 pieces of a group).
