@@ -248,7 +248,7 @@ bool split_last_chunk(const logismos_decode_config_t& c, int max_q, int last_row
 logismos_status_t few_rows_layers(const logismos_decode_config_t& c,
                                   const logismos_decode_layer_t* layers,
                                   const logismos_decode_batch_t* batch, const Workspace& w, int t,
-                                  int max_q, bool direct, logismos_stream_t stream) {
+                                  int max_q, bool direct, int* res_parts, logismos_stream_t stream) {
     hipStream_t st = static_cast<hipStream_t>(stream);
     const int qd = c.num_q_heads * c.head_dim;
     const int width = qd + 2 * c.num_kv_heads * c.head_dim;
@@ -266,10 +266,16 @@ logismos_status_t few_rows_layers(const logismos_decode_config_t& c,
         a.k = k;
         return a;
     };
+    // the down projection in two parts leaves the second to the next layer's norm and o projection, and of
+    // the last layer to the final norm
+    const bool two = lg::qgemm_q4_rows_res_parts(c.hidden / 16, c.intermediate) == 2;
+    const float* const pending = two ? reinterpret_cast<const float*>(w.proj) : nullptr;
+    *res_parts = two ? 1 : 0;
     for (int l = 0; l < c.num_layers; ++l) {
         const logismos_decode_layer_t& L = layers[l];
         lg::RowsArgs a = with(L.qkv, width, c.hidden);
         a.gain = static_cast<const float*>(L.norm1_w_f32);
+        a.e.pending = l ? pending : nullptr;
         if (c.kv_turbo3) {
             // the encoder wants whole head rows: the product as it is, then the operator
             a.e.out_f32 = reinterpret_cast<float*>(w.qkv);
@@ -304,6 +310,7 @@ logismos_status_t few_rows_layers(const logismos_decode_config_t& c,
             LG_TRY(logismos_launch_q4_prepare_x_bf16(w.attn_out, w.attn_b, t, qd, stream));
         a = with(L.o, c.hidden, qd);
         a.xprep = reinterpret_cast<const lg::uint4_t*>(w.attn_b);
+        a.e.pending = l ? pending : nullptr;
         LG_TRY(lg::qgemm_q4_rows_launch(false, lg::kRowsRes, a, st));
         a = with(L.gate_up, 2 * c.intermediate, c.hidden);
         a.gain = static_cast<const float*>(L.norm2_w_f32);
@@ -312,6 +319,7 @@ logismos_status_t few_rows_layers(const logismos_decode_config_t& c,
         LG_TRY(lg::qgemm_q4_rows_launch(true, lg::kRowsSilu, a, st));
         a = with(L.down, c.hidden, c.intermediate);
         a.xprep = reinterpret_cast<const lg::uint4_t*>(w.act);
+        a.e.out_f32 = reinterpret_cast<float*>(w.proj);
         LG_TRY(lg::qgemm_q4_rows_launch(false, lg::kRowsRes, a, st));
     }
     return 0;
@@ -541,7 +549,7 @@ extern "C" logismos_status_t logismos_launch_decode_step(const logismos_decode_c
         LG_TRY(lg::decode_resident_launch(c, layers, *batch, w.resident, 0,
                                           static_cast<hipStream_t>(stream)));
     } else if (few_rows(c, layers, t)) {
-        LG_TRY(few_rows_layers(c, layers, batch, w, t, max_q, direct, stream));
+        LG_TRY(few_rows_layers(c, layers, batch, w, t, max_q, direct, &res_parts, stream));
     } else {
         // All rows in one launch of every operator, the projections in chunks of 32 side by side (48
         // rows of the 4096-wide layers, chunk after chunk: 19 launches a layer, 117 us beside the

@@ -25,7 +25,10 @@ enum RowsEpilogue {
 };
 
 struct RowsEpilogueArgs {
-    float* out_f32;  // kRowsF32
+    float* out_f32;  // kRowsF32; kRowsRes in two parts: the second part's products
+    // what is still to be added to the residual stream, [b][its width], or null: the norm reads the stream with
+    // it, kRowsRes adds it before its product
+    const float* pending;
     uint4_t* act;    // kRowsSilu
     int inter;
     // kRowsQkv; tiles_per_head_inv = ceil(2^20 / (head_dim / 16))
@@ -55,6 +58,8 @@ bool qgemm_q4_rows_applies(int b, int hidden, int widest, int qkv, const void* s
                            const void* zero);
 // norm: kRowsQkv, kRowsSilu, kRowsF32; otherwise kRowsRes.
 hipError_t qgemm_q4_rows_launch(bool norm, int epilogue, const RowsArgs& args, hipStream_t st);
+// Parts of K that kRowsRes takes for this product where out_f32 is given: of two, the second one's products go there.
+int qgemm_q4_rows_res_parts(int tiles, int k);
 
 // ---- device helpers of the kernels that multiply few rows by 16 weight rows at a time
 

@@ -173,11 +173,14 @@ struct RowsFinish {
     int64_t slot = -1;
     float bias = 0.0f;
 
+    template <bool PENDING = false>
     __device__ __forceinline__ void early(const RowsEpilogueArgs& e, const float* h, int tile,
                                           int tiles, int r, int n, bool ok) {
         if (!ok) return;
         if constexpr (EPI == kRowsRes) {
-            a = h[(unsigned)r * (unsigned)(16 * tiles) + (unsigned)(16 * tile + n)];
+            const unsigned at = (unsigned)r * (unsigned)(16 * tiles) + (unsigned)(16 * tile + n);
+            a = h[at];
+            if constexpr (PENDING) a += e.pending[at];
         } else if constexpr (EPI == kRowsQkv) {
             pos = e.positions[r];
             slot = e.slots[r];
@@ -272,8 +275,8 @@ struct RowsNormLds {
     }
 };
 
-// CR: chunks of the rows per lane.
-template <int EPI, int NW, int W, int GPW, int TN, int CR>
+// CR: chunks of the rows per lane.  PENDING: the stream is h with what is pending.
+template <int EPI, int NW, int W, int GPW, int TN, int CR, bool PENDING>
 __global__ __launch_bounds__(64 * NW) void qgemm_q4g128_rows_norm_kernel(
     const float* __restrict__ h, const float* __restrict__ gain, const uint8_t* __restrict__ qw,
     const __half* __restrict__ scale, const __half* __restrict__ zero, int b, int k, int tiles,
@@ -307,6 +310,17 @@ __global__ __launch_bounds__(64 * NW) void qgemm_q4g128_rows_norm_kernel(
             const int c = min((i * wpr + part) * 64 + lane, chunks - 1);
             hv[i][0] = *reinterpret_cast<const float4_t*>(hrow + 8 * c);
             hv[i][1] = *reinterpret_cast<const float4_t*>(hrow + 8 * c + 4);
+        }
+    }
+    if constexpr (PENDING) {
+        const float* prow = e.pending + (unsigned)(mine ? row : 0) * (unsigned)k;
+#pragma unroll
+        for (int i = 0; i < CR; ++i) {
+            if (i * wpr * 64 < chunks) {
+                const int c = min((i * wpr + part) * 64 + lane, chunks - 1);
+                hv[i][0] += *reinterpret_cast<const float4_t*>(prow + 8 * c);
+                hv[i][1] += *reinterpret_cast<const float4_t*>(prow + 8 * c + 4);
+            }
         }
     }
     const unsigned xrow = (unsigned)(2 * k + 16);  // bytes per row of x, off the banks' period
@@ -417,8 +431,11 @@ __global__ __launch_bounds__(64 * NW) void qgemm_q4g128_rows_norm_kernel(
 }
 
 // Projection of prepared rows: one tile per workgroup, the waves split the groups of K, SETS
-// groups of a wave in flight.
-template <int EPI, int W, int DW>
+// groups of a wave in flight.  K may be cut in two parts (grid y): the first adds to the residual stream, the
+// second's products are left to the operators behind it.  (Modes of their own: an argument that a launch does not
+// need is a load in front of everything else, 1.5 % of a step of 8 rows at width 4096.)
+enum RowsPrepMode { kPrepPlain = 0, kPrepPending = 1, kPrepTwoParts = 2 };
+template <int EPI, int W, int DW, int MODE>
 __global__ __launch_bounds__(64 * W) void qgemm_q4g128_rows_prep_kernel(
     const uint4_t* __restrict__ xprep, const uint8_t* __restrict__ qw, const __half* __restrict__ scale,
     const __half* __restrict__ zero, float* __restrict__ h, int b, int k, int tiles,
@@ -432,7 +449,10 @@ __global__ __launch_bounds__(64 * W) void qgemm_q4g128_rows_prep_kernel(
     const int G = k >> 7;
     const unsigned khalf = (unsigned)k >> 1;
     const int tile = blockIdx.x;
-    const int2 share = rows_share(G, W, wave);
+    const bool second = MODE == kPrepTwoParts && blockIdx.y != 0;
+    const int half = (G + 1) >> 1;
+    int2 share = rows_share(MODE != kPrepTwoParts ? G : (second ? G - half : half), W, wave);
+    if (second) share.x += half;
     const int end = share.x + share.y;
     char* const stage = lds + wave * Stage::BYTES;
 
@@ -454,7 +474,7 @@ __global__ __launch_bounds__(64 * W) void qgemm_q4g128_rows_prep_kernel(
     const int fr = (tid >> 4) & 15, fn = tid & 15;
     const bool fok = tid < 256 && fr < b;
     RowsFinish<EPI> fin;
-    fin.early(e, h, tile, tiles, fr, fn, fok);
+    fin.template early<MODE == kPrepPending>(e, h, tile, tiles, fr, fn, fok && !second);
     const RowsConst cst;
     float4_t y = {0.0f, 0.0f, 0.0f, 0.0f};
     scales.put(G, wave, lane, reinterpret_cast<unsigned*>(sz));
@@ -472,8 +492,11 @@ __global__ __launch_bounds__(64 * W) void qgemm_q4g128_rows_prep_kernel(
     }
     *reinterpret_cast<float4_t*>(stage + lane * 16) = y;
     __syncthreads();
-    if (tid < 256)
-        fin.finish(e, h, tile, tiles, fr, fn, rows_meet<W>(lds, Stage::BYTES, fr, fn), fok);
+    if (tid < 256) {
+        const float v = rows_meet<W>(lds, Stage::BYTES, fr, fn);
+        if (!second) fin.finish(e, h, tile, tiles, fr, fn, v, fok);
+        else if (fok) e.out_f32[(unsigned)fr * (unsigned)(16 * tiles) + (unsigned)(16 * tile + fn)] = v;
+    }
 }
 
 template <typename K>
@@ -482,9 +505,12 @@ hipError_t rows_opt_in(K kernel) {
                                hipFuncAttributeMaxDynamicSharedMemorySize, kRowsLds);
 }
 
-template <int EPI, int NW, int W, int GPW, int TN, int CR>
+template <int EPI, int NW, int W, int GPW, int TN, int CR, bool PENDING = false>
 hipError_t rows_norm_launch(const RowsArgs& a, hipStream_t st) {
-    const auto kernel = qgemm_q4g128_rows_norm_kernel<EPI, NW, W, GPW, TN, CR>;
+    // (only widths of up to 2048 have something pending, in front of the q/k/v projection)
+    if constexpr (!PENDING && EPI != kRowsSilu && W * GPW <= 16)
+        if (a.e.pending) return rows_norm_launch<EPI, NW, W, GPW, TN, CR, true>(a, st);
+    const auto kernel = qgemm_q4g128_rows_norm_kernel<EPI, NW, W, GPW, TN, CR, PENDING>;
     static const hipError_t opt_in = rows_opt_in(kernel);
     if (opt_in != hipSuccess) return opt_in;
     constexpr int tiles = TN * NW / W;
@@ -533,15 +559,21 @@ hipError_t rows_norm(const RowsArgs& a, hipStream_t st) {
     return rows_norm_by_b<EPI, 16, 16, 2>(a, st);
 }
 
-template <int W, int DW>
+template <int W, int DW, int MODE>
 hipError_t rows_prep_launch(const RowsArgs& a, hipStream_t st) {
-    const auto kernel = qgemm_q4g128_rows_prep_kernel<kRowsRes, W, DW>;
+    const auto kernel = qgemm_q4g128_rows_prep_kernel<kRowsRes, W, DW, MODE>;
     static const hipError_t opt_in = rows_opt_in(kernel);
     if (opt_in != hipSuccess) return opt_in;
     const int lds = W * RowsStage<1>::BYTES + 16 * (a.k >> 7) * 4;
-    kernel<<<dim3((unsigned)a.tiles), dim3(64 * W), (size_t)lds, st>>>(
+    kernel<<<dim3((unsigned)a.tiles, MODE == kPrepTwoParts ? 2u : 1u), dim3(64 * W), (size_t)lds, st>>>(
         a.xprep, a.qw, a.scale, a.zero, a.h, a.b, a.k, a.tiles, a.e);
     return hipGetLastError();
+}
+template <int W, int DW>
+hipError_t rows_prep(const RowsArgs& a, hipStream_t st) {
+    if (a.e.out_f32 && qgemm_q4_rows_res_parts(a.tiles, a.k) == 2) return rows_prep_launch<W, DW, kPrepTwoParts>(a, st);
+    if (a.e.pending) return rows_prep_launch<W, DW, kPrepPending>(a, st);
+    return rows_prep_launch<W, DW, kPrepPlain>(a, st);
 }
 
 }  // namespace
@@ -553,6 +585,15 @@ bool qgemm_q4_rows_applies(int b, int hidden, int widest, int qkv, const void* s
            widest <= kRowsMaxPrepWidth && qkv <= kRowsMaxQkv && (al & 3u) == 0;
 }
 
+// Two parts where a wave of one has more groups than it keeps in flight (16 waves of three groups), both
+// parts' workgroups, one to a compute unit, run at once, and the norm that takes the rest is one of the narrow ones
+// (up to 2048 columns): 1536 x 8960 is 96 workgroups of 70 groups.  28 layers of it, us per step, one part / two:
+// 2 rows 899 / 854, 8 rows 936 / 912, 12 rows 1055 / 1010, 16 rows 1157 / 1108.  (From 24 groups on, 896 x 4864
+// of 56 workgroups too: no difference.)
+int qgemm_q4_rows_res_parts(int tiles, int k) {
+    return (k >> 7) > 48 && tiles <= 128 && 2 * tiles <= device_cu_count() ? 2 : 1;
+}
+
 hipError_t qgemm_q4_rows_launch(bool norm, int epilogue, const RowsArgs& a, hipStream_t st) {
     if (norm) {
         if (epilogue == kRowsQkv) return rows_norm<kRowsQkv>(a, st);
@@ -560,10 +601,10 @@ hipError_t qgemm_q4_rows_launch(bool norm, int epilogue, const RowsArgs& a, hipS
         return rows_norm<kRowsF32>(a, st);
     }
     // DW: 4 * K / 128 dwords of scales over 64 * W / 4 lanes
-    if (a.k <= 2048) return rows_prep_launch<8, 1>(a, st);
-    if (a.k <= 8192) return rows_prep_launch<16, 1>(a, st);
-    if (a.k <= 16384) return rows_prep_launch<16, 2>(a, st);
-    return rows_prep_launch<16, 4>(a, st);
+    if (a.k <= 2048) return rows_prep<8, 1>(a, st);
+    if (a.k <= 8192) return rows_prep<16, 1>(a, st);
+    if (a.k <= 16384) return rows_prep<16, 2>(a, st);
+    return rows_prep<16, 4>(a, st);
 }
 
 }  // namespace lg
