@@ -65,7 +65,6 @@ Workspace carve(const logismos_decode_config_t& c, int num_seqs, int t, int num_
     const size_t qd = (size_t)c.num_q_heads * c.head_dim;
     const size_t kvd = (size_t)c.num_kv_heads * c.head_dim;
     w.tall = t >= kTallRows;
-    w.resident = take(lg::decode_resident_bytes(c));
     if (w.tall) {
         w.attn_ws = take(
             logismos_paged_attn_workspace_bytes(num_seqs, c.num_q_heads, c.head_dim, num_splits));
@@ -92,6 +91,7 @@ Workspace carve(const logismos_decode_config_t& c, int num_seqs, int t, int num_
             w.head_ws =
                 take(logismos_qgemm_q4g128_greedy_workspace_bytes(kChunkRows, c.vocab, c.hidden));
         }
+        w.resident = take(lg::decode_resident_bytes(c));
         w.total = off;
         return w;
     }
@@ -135,6 +135,7 @@ Workspace carve(const logismos_decode_config_t& c, int num_seqs, int t, int num_
         w.last_rows = take((size_t)num_seqs * c.hidden * 2);
         w.last_xn = take(logismos_q4_xprep_bytes(kChunkRows, c.hidden));
     }
+    w.resident = take(lg::decode_resident_bytes(c));
     w.total = off;
     return w;
 }
