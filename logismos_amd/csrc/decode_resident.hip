@@ -20,15 +20,15 @@
 // the context for one KV head per workgroup | (merge of the pieces) | o projection + residual | row
 // normed -> gate/up, SwiGLU | down projection + residual.
 //
-// What bounds it, from clock stamps at widths 896 / 4096 (us per layer 20 / 42): six exchanges of 2-4 us,
+// What bounds it, from clock stamps at widths 896 / 4096 (us per layer 20 / 40): six exchanges of 2-4 us,
 // of which the poll 1.3-2 and what follows it up to the barrier 1; products 0.6-2 / 1-8 (gate/up waits for memory:
 // 370 KiB per compute unit and layer at 23-27 B/ns); epilogues 0.6 each.  A compute unit's requests return in order, so
 // a poll also waits for what the streaming waves asked for before it.  Every instruction of a front wave is on the
 // chain: for two to four rows the same kernel was slower than the launches it replaces (0.81-1.01 of their speed),
 // hence one row.
 //
-// Steps of one row, us (six launches a layer / here): 24 layers of 896 at 500 keys 671 / 516, 28 of 1536 at 500 keys
-// 884 / 790, 36 of 4096 at 1500 keys 1883 / 1566.
+// Steps of one row, us (six launches a layer / here): 24 layers of 896 at 500 keys 674 / 502, 28 of 1536 at 4000 keys
+// 912 / 773, 36 of 4096 at 1500 keys 1885 / 1524.
 //
 // Work is cut for V workgroups (one per compute unit) before the launch: a small kernel writes, for each and
 // for each of its streaming waves, the list of a layer's batches (up to four groups of K of a tile, or a

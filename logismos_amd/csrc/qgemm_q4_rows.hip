@@ -1,4 +1,5 @@
-// Q4G128 projections of a step with few packed rows (up to 16), with what surrounds them folded
+// Q4G128 projections of a step with few packed rows (up to 16; one row over fp16 pools mostly takes
+// decode_resident.hip, which is 1.18 to 1.34 times as fast there), with what surrounds them folded
 // in: one launch is "norm -> projection -> what is done to each output".
 //
 //   A step of few rows is a chain of dependent launches whose inputs are a few KiB of
