@@ -887,6 +887,10 @@ struct Front {
         constexpr int TEAMS = kFrontThreads / D;
         const int team = tid / D, c = tid % D;
         float* const area = reinterpret_cast<float*>(lds + p.lds_red);  // [team]{M, L, o[D]}
+        // The area lies over the parts of the q/k/v product, which a wave with a tile of it may still be adding up:
+        // a workgroup without a piece of the context comes here without a barrier, and the words it waits for
+        // are those of another KV head.
+        if (n - 1 - rank < p.hq) meet();
 #pragma unroll 1
         for (int head = n - 1 - rank; head < p.hq; head += n) {
             const int kvh = head / p.group, hin = head - kvh * p.group, u0 = kvh * pieces;

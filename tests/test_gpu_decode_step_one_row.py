@@ -22,6 +22,8 @@ SHAPES = [  # hidden, query heads, KV heads, head width, MLP width, context, row
     (2176, 17, 17, 128, 1152, 700, 16),    # no two heads share K and V; more than one tile per wave
     (4096, 32, 8, 128, 1024, 2100, 16),    # the widest norm, seventeen pieces merged
     (512, 8, 2, 64, 16384, 70, 64),        # the widest operand
+    (512, 64, 8, 128, 512, 100, 16),       # one piece of a group's eight heads: 56 workgroups that merge a head have
+                                           # q/k/v tiles and no piece of the context
 ]
 
 
@@ -66,7 +68,7 @@ def test_against_the_oracle(shape):
 
 
 @pytest.mark.parametrize("workgroups", [1, 7, 100, 255])
-@pytest.mark.parametrize("shape", [SHAPES[2], (512, 8, 2, 128, 1024, 900, 16)])
+@pytest.mark.parametrize("shape", [SHAPES[2], (512, 8, 2, 128, 1024, 900, 16), SHAPES[9]])
 def test_any_number_of_workgroups(shape, workgroups):
     # the work is cut for all compute units; fewer workgroups take several parts each, phase by phase
     cfg, layers, batch = _problem(shape, layers=3)
