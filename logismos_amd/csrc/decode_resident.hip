@@ -1177,7 +1177,8 @@ __global__ __launch_bounds__(64 * kStreamWaves) void decode_resident_init_kernel
             words[i] = uint4_t{0, 0, 0, 0};
     }
     // the context in pieces: a tile per streaming wave, as long as there are parts
-    const int ctx = p.cu[1] - p.cu[0] == 1 ? p.ctx[0] : 0;
+    // (a list has room for the keys that the block table can hold, and the table no entries past them)
+    const int ctx = p.cu[1] - p.cu[0] == 1 ? min(p.ctx[0], p.max_blocks * p.block_size) : 0;
     Piece piece{0, 0, 0, 0};
     int pieces = 0, t0 = 0, t1 = 0;
     if (ctx > 0) {

@@ -134,3 +134,25 @@ def test_no_key_is_seen():
         states.append(_state(r, batch, layers))
     assert np.isfinite(states[0][1]).all() and np.array_equal(states[0][1], states[1][1])
     assert not np.array_equal(states[0][1], batch["h"])
+
+
+@pytest.mark.parametrize("shape", [(384, 3, 3, 128, 256, 80, 16), (512, 16, 1, 64, 512, 1296, 16)])
+def test_a_context_past_the_block_table(shape):
+    # context_lens is a device value that the host does not see: the lists of K/V tiles, whose room follows from
+    # the block table, take the keys that the table holds
+    states = []
+    for past in (0, 1, 100, 10 ** 6):
+        cfg, layers, batch = _problem(shape, layers=2)
+        assert batch["block_tables"].shape[1] * cfg["block_size"] == shape[5]
+        batch["context_lens"] = batch["context_lens"] + np.int32(past)
+        r = DecodeStepRunner(cfg, layers, batch)
+        size = _lib()[0](C.byref(r.cfg))
+        region = hip.DeviceBuffer(size + 4096)
+        region.fill(0x5A)
+        assert _lib()[1](C.byref(r.cfg), r.layers, C.byref(r.batch), region.ptr, 0, None) == 0
+        hip.synchronize()
+        assert (region.to_numpy(np.uint8, (4096,), size) == 0x5A).all()
+        states.append(_state(r, batch, layers))
+    for got in states[1:]:
+        assert np.array_equal(got[1], states[0][1])
+        assert all(np.array_equal(a, b) for x, y in zip(got[2], states[0][2]) for a, b in zip(x, y))
