@@ -882,7 +882,8 @@ struct Front {
         }
     }
     // ... or, with more of them, one head per workgroup, published as bf16 pairs
-    __device__ __forceinline__ void merge_pieces(unsigned tag) {
+    // (apart: a barrier lies between the q/k/v epilogue and here)
+    __device__ __forceinline__ void merge_pieces(unsigned tag, bool apart) {
         Plan& p = arguments();
         constexpr int TEAMS = kFrontThreads / D;
         const int team = tid / D, c = tid % D;
@@ -890,7 +891,7 @@ struct Front {
         // The area lies over the parts of the q/k/v product, which a wave with a tile of it may still be adding up:
         // a workgroup without a piece of the context comes here without a barrier, and the words it waits for
         // are those of another KV head.
-        if (n - 1 - rank < p.hq) meet();
+        if (!apart && n - 1 - rank < p.hq) meet();
 #pragma unroll 1
         for (int head = n - 1 - rank; head < p.hq; head += n) {
             const int kvh = head / p.group, hin = head - kvh * p.group, u0 = kvh * pieces;
@@ -947,14 +948,17 @@ struct Front {
     }
 
     // ---- attention: queries and the token's K and V row into LDS, the waves' parts out of it
-    __device__ __forceinline__ void attend(int l) {
+    // returns whether the workgroup had a piece
+    __device__ __forceinline__ bool attend(int l) {
         Plan& p = arguments();
         const unsigned tag = l + 1;
         const int G = p.group;
+        bool any = false;
 #pragma unroll 1
         for (int v = rank; v < parts; v += n) {
             const Piece* const pp = reinterpret_cast<const Piece*>(p.region + p.at_pieces) + v;
             if (uniform_load(&pp->count) == 0) continue;
+            any = true;
             const int unit = uniform_load(&pp->unit), kvh = uniform_load(&pp->kvh);
             char* const area = lds + p.lds_x;
             const int nq = G * (D / 4), total = nq + D / 2;  // runs of four values
@@ -1026,6 +1030,7 @@ struct Front {
             }
             meet();  // the area's readers are through
         }
+        return any;
     }
 
     // ---- a projection: its operand, then the epilogue, a weight row of a tile per lane
@@ -1117,8 +1122,8 @@ struct Front {
             for (int which = kQkv; which <= kDown; ++which) {
                 project(which, l);
                 if (which == kQkv) {
-                    attend(l);
-                    if (many) merge_pieces(l + 1);
+                    const bool any = attend(l);
+                    if (many) merge_pieces(l + 1, any);
                 }
             }
     }
