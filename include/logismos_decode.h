@@ -741,7 +741,8 @@ typedef struct {
      * sequence.  Every per-row array above (hidden_f32, out_bf16, positions, slot_mapping) then
      * has total_tokens rows, in packed order.  A step of one row over fp16 pools (heads of 64 or 128, hidden up
      * to 4096, scales, gains, pools and hidden_f32 on 16 bytes) is one launch for all layers, which other kernels may
-     * run beside.  Otherwise every projection takes all rows in one launch: up
+     * run beside; its workgroups wait for one another's results, and should such a wait run out (after seconds),
+     * hidden_f32 ends as NaN and no K/V row that follows from it is written.  Otherwise every projection takes all rows in one launch: up
      * to 96 of them as chunks of 32 side by side (over 3-bit pools, with prompt chunks, a last
      * one of few rows may follow by itself), from 97 on in the tiled matrix-core GEMM (`linear_t` over `seq` rows,
      * crates/transformers/src/mlp.rs:104-111).  The attention takes the whole ragged batch in

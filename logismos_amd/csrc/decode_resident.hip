@@ -38,7 +38,9 @@
 // the last one, or one that has waited 100 us, closes the step to the n workgroups that hold tickets so
 // far, which are all running; later ones leave.  Workgroup r does the parts r, r + n, ... of the V, so
 // results do not depend on n.  A tag is written by whoever owns the value in every case, whatever the
-// batch holds.  (A budget of polls bounds the kernel even so.)
+// batch holds.  A budget of polls bounds the kernel even so.  A wave that has spent it says so in the region, and
+// all that its workgroup publishes from there on is NaN, which every product behind it hands on: the residual stream
+// ends as NaN, and K/V rows that are NaN on that account are left out of the pools.
 //
 // A buffer of words is reused by the next layer without a wait: between two writes of a word lies the
 // whole chain of a layer, and the workgroups of every link read all of what the one before it wrote.
@@ -69,7 +71,7 @@ constexpr int kMaxTilesHeld = 15;   // tiles of a projection in a part
 constexpr int kMaxList = 512;       // batches of a wave's part of a layer
 constexpr int kNormChunks = 2;      // chunks of eight columns a front thread normalises
 constexpr int kDirectWords = 8192;  // partial words the o projection's workgroups read themselves
-constexpr int kPollBudget = 1 << 21;
+constexpr int kPollBudget = 1 << 21;  // of a wave and step: seconds, where a step's waits are some hundred polls
 
 // the projections, in the order of a layer; attention stands between the first two
 enum { kQkv = 0, kO = 1, kGateUp = 2, kDown = 3 };
@@ -123,6 +125,7 @@ struct ResidentPlan {
     const int32_t *block_tables, *cu, *ctx, *positions;
     const int64_t* slot_mapping;
     const float *cos_t, *sin_t;
+    int polls;  // after which a front wave gives up (at the end: further up it moves fields that are loaded together, 1.3 %)
 };
 
 #define LG_CONST __attribute__((address_space(4)))
@@ -637,7 +640,7 @@ struct Front {
     const int rank, n, tid, lane, wave;  // tid 0 .. 255
     const int parts, layers;
     const Words words;
-    int budget = kPollBudget;
+    int budget;
     unsigned meets = 0;
     const int pieces;  // of the context
     const bool many;   // more partials than the o projection's workgroups read themselves
@@ -648,7 +651,7 @@ struct Front {
 
     __device__ __forceinline__ Front(Plan& p, char* l, int r, int n_, int t)
         : lds(l), rank(r), n(n_), tid(t), lane(t & 63), wave(uniform(t >> 6)), parts(p.parts), layers(p.layers),
-          words(p.region, p.bytes), pieces(uniform_load(&info(p)->pieces)),
+          words(p.region, p.bytes), budget(p.polls), pieces(uniform_load(&info(p)->pieces)),
           many(pieces * p.hq * (D + 2) > kDirectWords), pos(uniform_load(p.positions)),
           slot(uniform_load(p.slot_mapping)), et(t >> 4), en(t & 15) {}
     static __device__ __forceinline__ const StepInfo* info(Plan& p) {
@@ -670,6 +673,28 @@ struct Front {
         asm volatile("" ::: "memory");
         if (__all(ok)) return false;
         return --budget > 0;
+    }
+    // Where a wave has words that it waited for, on the way to what follows from them (in the polls themselves it cost a
+    // step 1 to 2 %, here at most 0.7 %).
+    __device__ __forceinline__ void arrived() {
+        if (__builtin_expect(budget > 0, 1)) return;
+        if (lane == 0) {
+            __hip_atomic_store(gave_up_word(), 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            *whole() = NAN;
+        }
+        asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");  // known before anything that follows is
+    }
+    // 1, or NaN from where a wave of this workgroup has gone on without words that it waited for: a factor of all
+    // that the workgroup publishes
+    __device__ __forceinline__ float* whole() const {
+        return reinterpret_cast<float*>(lds + arguments().lds_misc) + 3;
+    }
+    static __device__ __forceinline__ unsigned* gave_up_word() {
+        return reinterpret_cast<unsigned*>(arguments().region) + 2;
+    }
+    // ... a wave of any workgroup
+    static __device__ __forceinline__ bool any_gave_up() {
+        return __hip_atomic_load(gave_up_word(), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0;
     }
 
     // ---- scales and zeros of a part's tiles: [tile][scales, zeros][eight rows][16 G bytes] straight into LDS
@@ -927,6 +952,7 @@ struct Front {
             area[team * (D + 2)] = M;
             area[team * (D + 2) + 1] = L;
             area[team * (D + 2) + 2 + c] = o;
+            arrived();
             meet();
             if (tid < D / 2) {
                 float mx = -INFINITY, den = 0.0f, o0 = 0.0f, o1 = 0.0f;
@@ -940,7 +966,7 @@ struct Front {
                     o0 += area[t * (D + 2) + 2 + 2 * tid] * a;
                     o1 += area[t * (D + 2) + 3 + 2 * tid] * a;
                 }
-                const float inv = 1.0f / den;
+                const float inv = *whole() / den;
                 words.put(p.at_x + (unsigned)(head * (D / 2) + tid) * 8u, pack_bf16(o0 * inv, o1 * inv), tag);
             }
             meet();
@@ -991,6 +1017,7 @@ struct Front {
                 for (int j = 0; j < 2; ++j)
                     *reinterpret_cast<uint2_t*>(area + to[j]) = uint2_t{raw[j][0], raw[j][2]};
             }
+            arrived();
             block_barrier();
             block_barrier();  // the waves' parts are there
             const float* const part = reinterpret_cast<const float*>(area + attn_part_at(D));
@@ -1025,7 +1052,7 @@ struct Front {
                 words.put(at + 24u + c * 8u, __float_as_uint(o1), tag);
                 if (c == 0) {
                     words.put(at, __float_as_uint(M), tag);
-                    words.put(at + 8u, __float_as_uint(L), tag);
+                    words.put(at + 8u, __float_as_uint(L * *whole()), tag);
                 }
             }
             meet();  // the area's readers are through
@@ -1064,6 +1091,7 @@ struct Front {
                 else take_row(which == kO ? p.at_x : p.at_act, s.k, l + 1);
             }
             first = false;
+            arrived();
             asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the scales
             block_barrier();
             if (alone) fetch_next_scales(which, l);
@@ -1073,6 +1101,7 @@ struct Front {
             float sum = red[0];
 #pragma unroll
             for (int w = 1; w < kStreamWaves; ++w) sum += red[w * 16];
+            sum *= *whole();
             const bool ok = et < count;
             if (which == kO || which == kDown) {
                 if (ok) {
@@ -1100,7 +1129,7 @@ struct Front {
                 const unsigned lo = __half_as_ushort(r16), hi = (unsigned)lane_xor_i32<1>((int)lo);
                 const int col = head * D + at + (en < 8 ? 0 : D / 2);
                 if (ok && (en & 1) == 0) words.put(p.at_qkv + (unsigned)col * 4u, lo | (hi << 16), l + 1);
-                if (ok && head >= p.hq && slot >= 0) {
+                if (ok && head >= p.hq && slot >= 0 && !(res != res && any_gave_up())) {
                     const bool is_k = head < p.hq + p.hkv;
                     __half* const kp = uniform_load(&p.table[l].k_pool);
                     __half* const vp = uniform_load(&p.table[l].v_pool);
@@ -1135,9 +1164,9 @@ __global__ __launch_bounds__(kThreads) void decode_resident_kernel(const Residen
     extern __shared__ __attribute__((aligned(16))) char lds[];
     const int tid = threadIdx.x;
     const int wave = uniform(tid >> 6);
-    unsigned* const misc = reinterpret_cast<unsigned*>(lds + p.lds_misc);  // {front barrier, rank, n}
+    unsigned* const misc = reinterpret_cast<unsigned*>(lds + p.lds_misc);  // {front barrier, rank, n, Front::whole}
     if (tid == 0) {
-        unsigned* const ctl = reinterpret_cast<unsigned*>(p.region);  // {tickets, closed}
+        unsigned* const ctl = reinterpret_cast<unsigned*>(p.region);  // {tickets, closed, a wave gave up}
         const unsigned ticket = __hip_atomic_fetch_add(ctl, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         unsigned n = 0;
         if (ticket == gridDim.x - 1) {
@@ -1158,6 +1187,7 @@ __global__ __launch_bounds__(kThreads) void decode_resident_kernel(const Residen
         misc[0] = 0;
         misc[1] = ticket;
         misc[2] = n;
+        misc[3] = __float_as_uint(1.0f);
     }
     __syncthreads();
     const int rank = uniform((int)misc[1]), n = uniform((int)misc[2]);
@@ -1202,7 +1232,7 @@ __global__ __launch_bounds__(64 * kStreamWaves) void decode_resident_init_kernel
         reinterpret_cast<Piece*>(p.region + p.at_pieces)[v] = piece;
         if (v == 0) {
             unsigned* const ctl = reinterpret_cast<unsigned*>(p.region);
-            ctl[0] = ctl[1] = 0;
+            ctl[0] = ctl[1] = ctl[2] = 0;
             reinterpret_cast<StepInfo*>(p.region + p.at_step)->pieces = pieces;
         }
     }
@@ -1401,10 +1431,11 @@ bool decode_resident_applies(const logismos_decode_config_t& c, const logismos_d
 }
 
 hipError_t decode_resident_launch(const logismos_decode_config_t& c, const logismos_decode_layer_t* layers,
-                                  const logismos_decode_batch_t& b, void* region, int workgroups,
-                                  hipStream_t st) {
+                                  const logismos_decode_batch_t& b, void* region, hipStream_t st,
+                                  const ResidentLimits& limits) {
     ResidentPlan p;
     if (!resident_plan(c, &p)) return hipErrorInvalidValue;
+    p.polls = limits.polls > 0 ? limits.polls : kPollBudget;
     ResidentLayer* const table = static_cast<ResidentLayer*>(region);
     p.region = static_cast<char*>(region) + table_bytes(c);
     p.table = table;
@@ -1416,8 +1447,19 @@ hipError_t decode_resident_launch(const logismos_decode_config_t& c, const logis
     p.slot_mapping = b.slot_mapping;
     p.cos_t = static_cast<const float*>(b.rope_cos_f32);
     p.sin_t = static_cast<const float*>(b.rope_sin_f32);
-    return c.head_dim == 64 ? resident_launch<64>(p, c, layers, table, workgroups, st)
-                            : resident_launch<128>(p, c, layers, table, workgroups, st);
+    return c.head_dim == 64 ? resident_launch<64>(p, c, layers, table, limits.workgroups, st)
+                            : resident_launch<128>(p, c, layers, table, limits.workgroups, st);
 }
 
 }  // namespace lg
+
+// The launch by itself, for the tests (the header does not declare it).
+extern "C" size_t lg_decode_resident_bytes(const logismos_decode_config_t* cfg) {
+    return lg::decode_resident_bytes(*cfg);
+}
+extern "C" logismos_status_t lg_decode_resident_launch(const logismos_decode_config_t* cfg,
+                                                       const logismos_decode_layer_t* layers,
+                                                       const logismos_decode_batch_t* batch, void* region,
+                                                       const lg::ResidentLimits* limits, logismos_stream_t stream) {
+    return lg::decode_resident_launch(*cfg, layers, *batch, region, static_cast<hipStream_t>(stream), *limits);
+}

@@ -15,9 +15,15 @@ size_t decode_resident_bytes(const logismos_decode_config_t& c);
 bool decode_resident_applies(const logismos_decode_config_t& c, const logismos_decode_layer_t* layers,
                              const logismos_decode_batch_t& b, int t);
 
-// All layers: residual stream in and out in b.hidden_f32, K/V rows into the pools.  workgroups: how many are
-// launched (0: as many as the work is cut for; fewer do the same work with the same result).
+// What tests set (0: what a step takes).
+struct ResidentLimits {
+    int workgroups;  // launched (fewer than the work is cut for do the same work with the same result)
+    int polls;       // of a wave, after which it gives up
+};
+
+// All layers: residual stream in and out in b.hidden_f32, K/V rows into the pools.
 hipError_t decode_resident_launch(const logismos_decode_config_t& c, const logismos_decode_layer_t* layers,
-                                  const logismos_decode_batch_t& b, void* region, int workgroups, hipStream_t st);
+                                  const logismos_decode_batch_t& b, void* region, hipStream_t st,
+                                  const ResidentLimits& limits = {});
 
 }  // namespace lg

@@ -547,8 +547,7 @@ extern "C" logismos_status_t logismos_launch_decode_step(const logismos_decode_c
     }
     int res_parts = 0;  // split-K parts of the last down projection not yet folded into h
     if (lg::decode_resident_applies(c, layers, *batch, t)) {
-        LG_TRY(lg::decode_resident_launch(c, layers, *batch, w.resident, 0,
-                                          static_cast<hipStream_t>(stream)));
+        LG_TRY(lg::decode_resident_launch(c, layers, *batch, w.resident, static_cast<hipStream_t>(stream)));
     } else if (few_rows(c, layers, t)) {
         LG_TRY(few_rows_layers(c, layers, batch, w, t, max_q, direct, &res_parts, stream));
     } else {

@@ -42,13 +42,14 @@ def _state(r, batch, layers):
 
 
 def _lib():
-    # library-internal: size of the region, and the launch with a number of workgroups
+    # library-internal: size of the region, and the launch with limits of its own
     lib = C.CDLL(kernels.library()._name)
-    size, launch = (getattr(lib, n) for n in (
-        "_ZN2lg21decode_resident_bytesERK24logismos_decode_config_t",
-        "_ZN2lg22decode_resident_launchERK24logismos_decode_config_tPK23logismos_decode_layer_t"
-        "RK23logismos_decode_batch_tPviP12ihipStream_t"))
+    size = lib.lg_decode_resident_bytes
     size.restype = C.c_size_t
+
+    def launch(cfg, layers, batch, region, workgroups=0, polls=0):
+        limits = (C.c_int * 2)(workgroups, polls)
+        return lib.lg_decode_resident_launch(cfg, layers, batch, region, limits, None)
     return size, launch
 
 
@@ -79,7 +80,7 @@ def test_any_number_of_workgroups(shape, workgroups):
         r = DecodeStepRunner(cfg, layers, batch)
         region = hip.DeviceBuffer(size(C.byref(r.cfg)))
         region.fill(0xFF)
-        assert launch(C.byref(r.cfg), r.layers, C.byref(r.batch), region.ptr, n, None) == 0
+        assert launch(C.byref(r.cfg), r.layers, C.byref(r.batch), region.ptr, n) == 0
         hip.synchronize()
         got = _state(r, batch, layers)
         want = want or got
@@ -149,10 +150,35 @@ def test_a_context_past_the_block_table(shape):
         size = _lib()[0](C.byref(r.cfg))
         region = hip.DeviceBuffer(size + 4096)
         region.fill(0x5A)
-        assert _lib()[1](C.byref(r.cfg), r.layers, C.byref(r.batch), region.ptr, 0, None) == 0
+        assert _lib()[1](C.byref(r.cfg), r.layers, C.byref(r.batch), region.ptr) == 0
         hip.synchronize()
         assert (region.to_numpy(np.uint8, (4096,), size) == 0x5A).all()
         states.append(_state(r, batch, layers))
     for got in states[1:]:
         assert np.array_equal(got[1], states[0][1])
         assert all(np.array_equal(a, b) for x, y in zip(got[2], states[0][2]) for a, b in zip(x, y))
+
+
+@pytest.mark.parametrize("shape", [SHAPES[3], SHAPES[5], SHAPES[7], SHAPES[9]])
+def test_a_wait_that_runs_out_shows(shape):
+    # every wave gives up at its first poll that does not find its words
+    cfg, layers, batch = _problem(shape, layers=3, bias=False)
+    r = DecodeStepRunner(cfg, layers, batch)
+    size, launch = _lib()
+    region = hip.DeviceBuffer(size(C.byref(r.cfg)))
+    assert launch(C.byref(r.cfg), r.layers, C.byref(r.batch), region.ptr, polls=1) == 0
+    hip.synchronize()
+    _, h, pools = _state(r, batch, layers)
+    assert np.isnan(h).all()
+    slot = int(batch["slots"][0])
+    for kv, L in zip(pools, layers):
+        for got, name in zip(kv, ("k_pool", "v_pool")):
+            assert not np.isnan(got.view(np.float16)).any()
+            assert set(np.nonzero((got != L[name].view(np.uint16)).any(axis=1))[0]) <= {slot}
+    # the next step over the same region is a step like any other
+    want = DecodeStepRunner(cfg, layers, batch)
+    want.launch()
+    r.h.copy_from_host(batch["h"].astype(np.float32))
+    assert launch(C.byref(r.cfg), r.layers, C.byref(r.batch), region.ptr) == 0
+    hip.synchronize()
+    assert np.array_equal(_state(r, batch, layers)[1], _state(want, batch, layers)[1])
