@@ -73,6 +73,10 @@ constexpr int kNormChunks = 2;      // chunks of eight columns a front thread no
 constexpr int kDirectWords = 8192;  // partial words the o projection's workgroups read themselves
 constexpr int kPollBudget = 1 << 21;  // of a wave and step: seconds, where a step's waits are some hundred polls
 
+// What a merge of pieces starts from: below every score, and finite, so that a piece whose keys all score -inf weighs
+// nothing (from -inf the difference of the two maxima is NaN).
+constexpr float kNoKey = -3.402823466e38f;
+
 // the projections, in the order of a layer; attention stands between the first two
 enum { kQkv = 0, kO = 1, kGateUp = 2, kDown = 3 };
 enum { kPhaseQkv = 0, kPhaseAttn = 1, kPhaseO = 2, kPhaseGateUp = 3, kPhaseDown = 4, kPhases = 5 };
@@ -864,7 +868,7 @@ struct Front {
             const int ch = min(c0 + tid, chunks - 1);
             const int head = ch / (D / 8), c = ch % (D / 8);
             const int kvh = head / p.group, hin = head - kvh * p.group, u0 = kvh * pieces;
-            float M = -INFINITY, L = 0.0f, o[8];
+            float M = kNoKey, L = 0.0f, o[8];
 #pragma unroll
             for (int e = 0; e < 8; ++e) o[e] = 0.0f;
 #pragma unroll 1
@@ -920,7 +924,7 @@ struct Front {
 #pragma unroll 1
         for (int head = n - 1 - rank; head < p.hq; head += n) {
             const int kvh = head / p.group, hin = head - kvh * p.group, u0 = kvh * pieces;
-            float M = -INFINITY, L = 0.0f, o = 0.0f;
+            float M = kNoKey, L = 0.0f, o = 0.0f;
             constexpr int R = 8;
 #pragma unroll 1
             for (int j0 = 0; j0 < pieces; j0 += R * TEAMS) {
@@ -960,8 +964,7 @@ struct Front {
                 for (int t = 0; t < TEAMS; ++t) mx = fmaxf(mx, area[t * (D + 2)]);
 #pragma unroll
                 for (int t = 0; t < TEAMS; ++t) {
-                    const float mt = area[t * (D + 2)];
-                    const float a = mt == -INFINITY ? 0.0f : fast_exp2(mt - mx);
+                    const float a = fast_exp2(area[t * (D + 2)] - mx);
                     den += area[t * (D + 2) + 1] * a;
                     o0 += area[t * (D + 2) + 2 + 2 * tid] * a;
                     o1 += area[t * (D + 2) + 3 + 2 * tid] * a;

@@ -182,3 +182,23 @@ def test_a_wait_that_runs_out_shows(shape):
     assert launch(C.byref(r.cfg), r.layers, C.byref(r.batch), region.ptr) == 0
     hip.synchronize()
     assert np.array_equal(_state(r, batch, layers)[1], _state(want, batch, layers)[1])
+
+
+@pytest.mark.parametrize("shape", [SHAPES[3], (512, 8, 2, 128, 512, 1300, 16), (512, 16, 1, 64, 512, 1300, 16)])
+def test_pieces_of_keys_that_have_no_weight(shape):
+    # every key of the first piece, then of all but the last two, has a score of -inf (K minus infinity where the
+    # queries are far above zero): such a piece weighs nothing beside the others, in whatever order they meet
+    hidden, hq, hkv, d, inter, ctx, block = shape
+    for keys in (128, ctx - 2):
+        cfg, layers, batch = _problem(shape, seed=11)
+        batch["cos"], batch["sin"] = np.ones_like(batch["cos"]), np.zeros_like(batch["sin"])
+        L = layers[0]
+        L["qkv_bias"][:hq * d:d] = 100.0
+        key = np.arange(keys)
+        rows = batch["block_tables"][0][key // block].astype(np.int64) * block + key % block
+        L["k_pool"][rows[:, None], np.arange(hkv) * d] = -np.inf
+        r, got, want, _, bat = _run_both(cfg, layers, batch)
+        assert _lib()[0](C.byref(r.cfg)) > 0
+        assert np.isfinite(want).all() and np.isfinite(got).all()
+        assert _rel_l2(got, want) < 6e-3
+        assert _rel_l2(r.h.to_numpy(np.float32, bat["h"].shape), bat["h"]) < 6e-3
