@@ -71,6 +71,7 @@ constexpr int kMaxTilesHeld = 15;   // tiles of a projection in a part
 constexpr int kMaxList = 512;       // batches of a wave's part of a layer
 constexpr int kNormChunks = 2;      // chunks of eight columns a front thread normalises
 constexpr int kDirectWords = 8192;  // partial words the o projection's workgroups read themselves
+constexpr int kCloseAfter = 10000;  // ticks of 10 ns that a workgroup waits for the others
 constexpr int kPollBudget = 1 << 21;  // of a wave and step: seconds, where a step's waits are some hundred polls
 
 // What a merge of pieces starts from: below every score, and finite, so that a piece whose keys all score -inf weighs
@@ -130,6 +131,7 @@ struct ResidentPlan {
     const int64_t* slot_mapping;
     const float *cos_t, *sin_t;
     int polls;  // after which a front wave gives up (at the end: further up it moves fields that are loaded together, 1.3 %)
+    unsigned all;  // tickets with which the step is closed at once
 };
 
 #define LG_CONST __attribute__((address_space(4)))
@@ -1172,15 +1174,15 @@ __global__ __launch_bounds__(kThreads) void decode_resident_kernel(const Residen
         unsigned* const ctl = reinterpret_cast<unsigned*>(p.region);  // {tickets, closed, a wave gave up}
         const unsigned ticket = __hip_atomic_fetch_add(ctl, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         unsigned n = 0;
-        if (ticket == gridDim.x - 1) {
-            __hip_atomic_compare_exchange_strong(ctl + 1, &n, gridDim.x, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
+        if (const unsigned all = p.all; ticket == all - 1) {
+            __hip_atomic_compare_exchange_strong(ctl + 1, &n, all, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
                                                  __HIP_MEMORY_SCOPE_AGENT);
-            if (n == 0) n = gridDim.x;
+            if (n == 0) n = all;
         }
         const unsigned long long start = __builtin_readsteadycounter();  // 100 MHz
         while (n == 0) {
             n = __hip_atomic_load(ctl + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            if (n == 0 && __builtin_readsteadycounter() - start > 10000) {
+            if (n == 0 && __builtin_readsteadycounter() - start > kCloseAfter) {
                 const unsigned now = __hip_atomic_load(ctl, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
                 __hip_atomic_compare_exchange_strong(ctl + 1, &n, now, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
                                                      __HIP_MEMORY_SCOPE_AGENT);
@@ -1406,8 +1408,7 @@ hipError_t resident_launch(const ResidentPlan& p, const logismos_decode_config_t
             p, table, l0, count, arg);
         if (const hipError_t e = hipGetLastError(); e != hipSuccess) return e;
     }
-    const int blocks = workgroups > 0 && workgroups < p.parts ? workgroups : p.parts;
-    kernel<<<dim3((unsigned)blocks), dim3(kThreads), kResLds, st>>>(p);
+    kernel<<<dim3((unsigned)workgroups), dim3(kThreads), kResLds, st>>>(p);
     return hipGetLastError();
 }
 
@@ -1439,6 +1440,8 @@ hipError_t decode_resident_launch(const logismos_decode_config_t& c, const logis
     ResidentPlan p;
     if (!resident_plan(c, &p)) return hipErrorInvalidValue;
     p.polls = limits.polls > 0 ? limits.polls : kPollBudget;
+    const int workgroups = limits.workgroups > 0 && limits.workgroups < p.parts ? limits.workgroups : p.parts;
+    p.all = limits.tickets > 0 && limits.tickets < workgroups ? limits.tickets : workgroups;
     ResidentLayer* const table = static_cast<ResidentLayer*>(region);
     p.region = static_cast<char*>(region) + table_bytes(c);
     p.table = table;
@@ -1450,8 +1453,8 @@ hipError_t decode_resident_launch(const logismos_decode_config_t& c, const logis
     p.slot_mapping = b.slot_mapping;
     p.cos_t = static_cast<const float*>(b.rope_cos_f32);
     p.sin_t = static_cast<const float*>(b.rope_sin_f32);
-    return c.head_dim == 64 ? resident_launch<64>(p, c, layers, table, limits.workgroups, st)
-                            : resident_launch<128>(p, c, layers, table, limits.workgroups, st);
+    return c.head_dim == 64 ? resident_launch<64>(p, c, layers, table, workgroups, st)
+                            : resident_launch<128>(p, c, layers, table, workgroups, st);
 }
 
 }  // namespace lg

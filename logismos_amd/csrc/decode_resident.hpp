@@ -19,6 +19,7 @@ bool decode_resident_applies(const logismos_decode_config_t& c, const logismos_d
 struct ResidentLimits {
     int workgroups;  // launched (fewer than the work is cut for do the same work with the same result)
     int polls;       // of a wave, after which it gives up
+    int tickets;     // with which the step is closed: the workgroups without one leave
 };
 
 // All layers: residual stream in and out in b.hidden_f32, K/V rows into the pools.

@@ -7,7 +7,7 @@ import pytest
 
 from logismos_amd import hip, kernels
 from tests import workloads
-from tests.gpu_harness import DecodeStepRunner
+from tests.gpu_harness import DecodeStepRunner, PagedAttnRunner
 from tests.test_gpu_decode_step import _rel_l2, _run_both
 
 pytestmark = pytest.mark.gpu
@@ -47,8 +47,8 @@ def _lib():
     size = lib.lg_decode_resident_bytes
     size.restype = C.c_size_t
 
-    def launch(cfg, layers, batch, region, workgroups=0, polls=0):
-        limits = (C.c_int * 2)(workgroups, polls)
+    def launch(cfg, layers, batch, region, workgroups=0, polls=0, tickets=0):
+        limits = (C.c_int * 3)(workgroups, polls, tickets)
         return lib.lg_decode_resident_launch(cfg, layers, batch, region, limits, None)
     return size, launch
 
@@ -88,6 +88,47 @@ def test_any_number_of_workgroups(shape, workgroups):
         assert all(np.array_equal(a, b) for x, y in zip(got[2], want[2]) for a, b in zip(x, y))
     whole.launch()
     assert np.array_equal(_state(whole, batch, layers)[1], want[1])
+
+
+@pytest.mark.parametrize("shape", [SHAPES[2], (512, 8, 2, 128, 1024, 900, 16), SHAPES[9]])
+def test_closed_before_all_workgroups_are_there(shape):
+    # the step is closed to the first so many that hold tickets, as after a wait for the others: those leave
+    cfg, layers, batch = _problem(shape, layers=3)
+    size, launch = _lib()
+    table = (3 * 136 + 255) // 256 * 256  # in front of the region: three layers' operands
+    want = None
+    for tickets in (0, 255, 100, 7, 1):
+        r = DecodeStepRunner(cfg, layers, batch)
+        region = hip.DeviceBuffer(size(C.byref(r.cfg)))
+        region.fill(0xFF)
+        assert launch(C.byref(r.cfg), r.layers, C.byref(r.batch), region.ptr, tickets=tickets) == 0
+        hip.synchronize()
+        assert region.to_numpy(np.uint32, (3,), table).tolist() == [256, tickets or 256, 0]
+        got = _state(r, batch, layers)
+        want = want or got
+        assert np.array_equal(got[1], want[1])
+        assert all(np.array_equal(a, b) for x, y in zip(got[2], want[2]) for a, b in zip(x, y))
+
+
+def test_beside_another_stream():
+    # prompt attention on another stream holds compute units for longer than a step waits for them
+    cfg, layers, batch = _problem(SHAPES[2], layers=3)
+    alone = DecodeStepRunner(cfg, layers, batch)
+    alone.launch()
+    want = _state(alone, batch, layers)
+    other = PagedAttnRunner(workloads.paged_case(np.random.default_rng(1), [64], [20000], hq=32, hkv=8,
+                                                 pool_period_rows=4096), stream=hip.Stream())
+    stream = hip.Stream()
+    steps = [DecodeStepRunner(cfg, layers, batch, stream=stream) for _ in range(6)]
+    hip.synchronize()
+    for _ in range(10):
+        other.launch()
+    for r in steps:
+        r.launch()
+    hip.synchronize()
+    for r in steps:
+        got = _state(r, batch, layers)
+        assert np.array_equal(got[0], want[0]) and np.array_equal(got[1], want[1])
 
 
 @pytest.mark.parametrize("slot", ["its own", "none", "another key's"])
