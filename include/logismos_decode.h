@@ -740,9 +740,10 @@ typedef struct {
      * rows and the largest number of new tokens of a sequence; 0 / 0 means one new token per
      * sequence.  Every per-row array above (hidden_f32, out_bf16, positions, slot_mapping) then
      * has total_tokens rows, in packed order.  A step of one row over fp16 pools (heads of 64 or 128, hidden up
-     * to 4096, scales, gains, pools and hidden_f32 on 16 bytes) is one launch for all layers, which other kernels may
-     * run beside; its workgroups wait for one another's results, and should such a wait run out (after seconds),
-     * hidden_f32 ends as NaN and no K/V row that follows from it is written.  Otherwise every projection takes all rows in one launch: up
+     * to 4096, scales, gains, pools and hidden_f32 on 16 bytes) is one launch for all layers that takes every compute unit it can
+     * get for the whole step (see logismos_launch_decode_step_per_operator); its workgroups wait for one another's
+     * results, and should such a wait run out (after seconds), hidden_f32 ends as NaN and no K/V row that follows
+     * from it is written.  Otherwise every projection takes all rows in one launch: up
      * to 96 of them as chunks of 32 side by side (over 3-bit pools, with prompt chunks, a last
      * one of few rows may follow by itself), from 97 on in the tiled matrix-core GEMM (`linear_t` over `seq` rows,
      * crates/transformers/src/mlp.rs:104-111).  The attention takes the whole ragged batch in
@@ -767,6 +768,19 @@ logismos_status_t logismos_launch_decode_step(const logismos_decode_config_t* cf
                                               const logismos_decode_layer_t* layers,
                                               const logismos_decode_batch_t* batch, void* workspace,
                                               logismos_stream_t stream);
+/* The same step, arguments and workspace with a launch per operator also where a step of one row would be one launch
+ * for all layers: for a program whose other streams have work for the device meanwhile.  The one launch takes the whole
+ * LDS of every compute unit it gets, so that other streams' kernels mostly wait until its 0.5 to 1.5 ms are
+ * over, and it waits up to 100 us for compute units that others hold before it does with fewer; operators
+ * launched one by one interleave with other work.  us per step, one launch / per operator, 24 layers of width 896 and 36 of
+ * 4096: alone 480 / 600 and 1525 / 1885; beside a second stream of the same steps 1030 / 620 and 3040 / 2390; beside a
+ * prompt's attention that holds 64 compute units for 1.7 ms at a time 790 / 670 and 2620 / 2650; beside GEMMs of 2048 rows
+ * 770 / 2850 and 2500 / 4100 (the GEMMs take 1.2 to 1.9 times as long / 1.0 to 1.1).  Results differ in
+ * the order of fp32 sums. */
+logismos_status_t logismos_launch_decode_step_per_operator(const logismos_decode_config_t* cfg,
+                                                           const logismos_decode_layer_t* layers,
+                                                           const logismos_decode_batch_t* batch, void* workspace,
+                                                           logismos_stream_t stream);
 
 /* ------------------------------------------------------------------------
  * Paged KV cache (host object over device pools)

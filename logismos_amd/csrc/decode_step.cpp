@@ -334,6 +334,10 @@ int batch_max_q(const logismos_decode_batch_t* b) {
     return b->max_seqlen_q > 0 ? b->max_seqlen_q : 1;
 }
 
+logismos_status_t launch_step(const logismos_decode_config_t* cfg, const logismos_decode_layer_t* layers,
+                              const logismos_decode_batch_t* batch, void* workspace, bool per_operator,
+                              logismos_stream_t stream);
+
 }  // namespace
 
 extern "C" size_t logismos_decode_step_workspace_bytes(const logismos_decode_config_t* cfg,
@@ -353,6 +357,22 @@ extern "C" logismos_status_t logismos_launch_decode_step(const logismos_decode_c
                                                          const logismos_decode_batch_t* batch,
                                                          void* workspace,
                                                          logismos_stream_t stream) {
+    return launch_step(cfg, layers, batch, workspace, false, stream);
+}
+extern "C" logismos_status_t logismos_launch_decode_step_per_operator(const logismos_decode_config_t* cfg,
+                                                                      const logismos_decode_layer_t* layers,
+                                                                      const logismos_decode_batch_t* batch,
+                                                                      void* workspace,
+                                                                      logismos_stream_t stream) {
+    return launch_step(cfg, layers, batch, workspace, true, stream);
+}
+
+namespace {
+
+// per_operator: no launch takes several operators that depend on one another's whole results.
+logismos_status_t launch_step(const logismos_decode_config_t* cfg, const logismos_decode_layer_t* layers,
+                              const logismos_decode_batch_t* batch, void* workspace, bool per_operator,
+                              logismos_stream_t stream) {
     if (!cfg || !layers || !batch || !workspace) return hipErrorInvalidValue;
     const int num_seqs = batch->num_seqs;
     const int t = batch_tokens(batch);
@@ -546,7 +566,7 @@ extern "C" logismos_status_t logismos_launch_decode_step(const logismos_decode_c
         return last_only ? project_last_rows() : 0;
     }
     int res_parts = 0;  // split-K parts of the last down projection not yet folded into h
-    if (lg::decode_resident_applies(c, layers, *batch, t)) {
+    if (!per_operator && lg::decode_resident_applies(c, layers, *batch, t)) {
         LG_TRY(lg::decode_resident_launch(c, layers, *batch, w.resident, static_cast<hipStream_t>(stream)));
     } else if (few_rows(c, layers, t)) {
         LG_TRY(few_rows_layers(c, layers, batch, w, t, max_q, direct, &res_parts, stream));
@@ -655,3 +675,5 @@ extern "C" logismos_status_t logismos_launch_decode_step(const logismos_decode_c
                                                  c.hidden, c.rms_eps, stream));
     return 0;
 }
+
+}  // namespace

@@ -114,6 +114,7 @@ _SIGNATURES = {
     "logismos_launch_rope_kv_write_f32p_turbo3_bias":
         (C.c_uint32, [_vp, _i] + [_vp] * 8 + [_i] * 5 + [_vp]),
     "logismos_launch_decode_step": (C.c_uint32, [_vp, _vp, _vp, _vp, _vp]),
+    "logismos_launch_decode_step_per_operator": (C.c_uint32, [_vp, _vp, _vp, _vp, _vp]),
     "logismos_qgemm_q4g128_splitk_parts": (C.c_int, [_i, _i, _i]),
     "logismos_qgemm_q4g128_splitk_xprep_parts": (C.c_int, [_i, _i, _i]),
     "logismos_launch_qgemm_q4g128_f32_splitk": (C.c_uint32, [_vp] * 5 + [_i, _i, _i, _vp]),
@@ -620,6 +621,12 @@ def decode_step_workspace_bytes(cfg: DecodeConfig, num_seqs: int, num_splits: in
 def launch_decode_step(cfg: DecodeConfig, layers, batch: DecodeBatch, workspace, stream=None) -> None:
     """`layers` is a ctypes array of DecodeLayer (host memory)."""
     _status("decode_step", library().logismos_launch_decode_step(
+        C.byref(cfg), C.cast(layers, _vp), C.byref(batch), _ptr(workspace), _raw(stream)))
+
+
+def launch_decode_step_per_operator(cfg: DecodeConfig, layers, batch: DecodeBatch, workspace, stream=None) -> None:
+    """The same step with a launch per operator also at one row: for a device shared with other streams."""
+    _status("decode_step_per_operator", library().logismos_launch_decode_step_per_operator(
         C.byref(cfg), C.cast(layers, _vp), C.byref(batch), _ptr(workspace), _raw(stream)))
 
 

@@ -164,6 +164,31 @@ def test_against_the_route_of_more_rows(shape, slot):
                                atol=4e-3, rtol=4e-3)
 
 
+@pytest.mark.parametrize("rows", [1, 2, 16, 40])
+def test_a_launch_per_operator(rows):
+    # at one row the route of 2 to 16 rows (what scales off 16 bytes take, bit for bit), otherwise the same step
+    cfg, layers, batch = workloads.decode_step_problem(
+        np.random.default_rng(rows), num_layers=2, hidden=512, hq=8, hkv=2, inter=768, ctx=[300] * rows, qkv_bias=True)
+    states = []
+    for per_operator in (False, True):
+        r = DecodeStepRunner(cfg, layers, batch)
+        if rows == 1 and not per_operator:
+            for lay, L in zip(r.layers, layers):
+                s = np.ascontiguousarray(L["o"][1]).view(np.uint16).reshape(-1)
+                buf = hip.DeviceBuffer.from_numpy(np.concatenate([np.zeros(2, np.uint16), s]))
+                r.keep.append(buf)
+                lay.o = kernels.Q4Weight(lay.o.qw, buf.ptr.value + 4, lay.o.zero)
+        call = kernels.launch_decode_step_per_operator if per_operator else kernels.launch_decode_step
+        call(r.cfg, r.layers, r.batch, r.ws)
+        out = r.result_bits().copy()
+        states.append((out, r.h.to_numpy(np.float32, batch["h"].shape), r.pools))
+    (a, ha, pa), (b, hb, pb) = states
+    assert np.array_equal(a, b) and np.array_equal(ha, hb)
+    for x, y, L in zip(pa, pb, layers):
+        for u, v in zip(x, y):
+            assert np.array_equal(u.to_numpy(np.uint16, L["k_pool"].shape), v.to_numpy(np.uint16, L["k_pool"].shape))
+
+
 def test_no_key_is_seen():
     # a context of 0: attention adds nothing, and the layers still follow one another (more workgroups have
     # q/k/v tiles than tiles of the other projections); twice the same
