@@ -1299,6 +1299,15 @@ bool resident_plan(const logismos_decode_config_t& c, ResidentPlan* p) {
     if (group > 16 || c.intermediate > 16384 || qd > 16384 || width > 32768) return false;
     const int cus = device_cu_count(), parts = cus < kMaxParts ? cus : kMaxParts;
     if (c.num_kv_heads > parts) return false;
+    // Long contexts: this kernel's attention reads K and V at 5.7 TB/s, the launches' at 7 (with one or two KV heads less),
+    // so that from some size on their stream outweighs the chain of launches.  us of eight layers with a full
+    // table, launches / here, at 256 | 384 | 512 MiB of K and V per layer: 32 KV heads of 128 762 / 740 | 916 / 926 |
+    // 1085 / 1117; 8 heads 795 / 737 | 963 / 935 | 1117 / 1133; 4 heads 711 / 661 | 887 / 860 | 1059 / 1058; 16 heads of
+    // 64 790 / 721 | 960 / 920 | 1112 / 1110; at 512 and 768 MiB 2 heads of 128 1184 / 1049 and 1520 / 1441, of 64
+    // 1017 / 997 and 1365 / 1383.  The host knows
+    // what the table can hold, not what it holds: the lines lie where a full one is still no slower.
+    const int64_t kv_bytes = 4 * (int64_t)c.num_kv_heads * d * c.block_size * c.max_blocks_per_seq;
+    if (kv_bytes > (c.num_kv_heads <= 2 ? (int64_t)512 : (int64_t)320) << 20) return false;
     *p = ResidentPlan{};
     p->layers = c.num_layers;
     p->hidden = c.hidden;

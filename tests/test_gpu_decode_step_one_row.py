@@ -164,6 +164,28 @@ def test_against_the_route_of_more_rows(shape, slot):
                                atol=4e-3, rtol=4e-3)
 
 
+@pytest.mark.parametrize("hq,hkv,d,mib", [(8, 2, 128, 512), (8, 4, 64, 320), (4, 4, 128, 320)])
+def test_tables_too_long_for_one_launch(hq, hkv, d, mib):
+    # past so many bytes of K and V that a layer's table can hold a step is launched operator by operator
+    cfg, layers, batch = _problem((512, hq, hkv, d, 512, 200, 16))
+    blocks = (mib << 20) // (4 * hkv * d * 16)
+    states = []
+    for more in (0, 1):
+        b = dict(batch)
+        b["block_tables"] = np.full((1, blocks + more), 0x3FFFFFF, np.int32)
+        b["block_tables"][0, :13] = batch["block_tables"][0, :13]
+        for name in ("cos", "sin"):
+            b[name] = np.resize(batch[name], (b["block_tables"].shape[1] * 16, d // 2))
+        r = DecodeStepRunner(cfg, layers, b)
+        assert (_lib()[0](C.byref(r.cfg)) > 0) == (more == 0)
+        for call in (kernels.launch_decode_step, kernels.launch_decode_step_per_operator):
+            r.h.copy_from_host(batch["h"].astype(np.float32))
+            call(r.cfg, r.layers, r.batch, r.ws)
+            states.append(_state(r, b, layers))
+    assert _rel_l2(states[0][1], states[1][1]) < 2e-3
+    assert np.array_equal(states[2][1], states[3][1]) and np.array_equal(states[2][0], states[3][0])
+
+
 @pytest.mark.parametrize("rows", [1, 2, 16, 40])
 def test_a_launch_per_operator(rows):
     # at one row the route of 2 to 16 rows (what scales off 16 bytes take, bit for bit), otherwise the same step
