@@ -70,7 +70,12 @@ constexpr int kMaxParts = 256;      // V: parts the work is cut into, and pieces
 constexpr int kMaxTilesHeld = 15;   // tiles of a projection in a part
 constexpr int kMaxList = 512;       // batches of a wave's part of a layer
 constexpr int kNormChunks = 2;      // chunks of eight columns a front thread normalises
-constexpr int kDirectWords = 8192;  // partial words the o projection's workgroups read themselves
+// The partials of the context's pieces: the o projection's workgroups read them themselves where a thread has one chunk of
+// eight columns and they are few words, otherwise a workgroup per head merges them, which is one exchange more.  us of 16
+// layers, read / merged: 512 columns of heads, 1 | 4 | 8 pieces 241 / 273 | 247 / 274 | 262 / 274; 896, 325 / 353 | 326 / 357 |
+// 341 / 340; 1536 (width 1536), 429 / 449 | 434 / 460; but 2048 (width 2048), 1 | 2 pieces 397 / 374 | 414 / 377 (width 1024, one
+// piece 297 / 308); 2560, 551 / 513 | 574 / 525; 4096, 692 / 640 | 780 / 716.
+constexpr int kDirectWords = 8192, kDirectColumns = 1536;
 constexpr int kCloseAfter = 10000;  // ticks of 10 ns that a workgroup waits for the others
 constexpr int kPollBudget = 1 << 21;  // of a wave and step: seconds, where a step's waits are some hundred polls
 
@@ -107,9 +112,9 @@ constexpr int kKvTile = 5;
 struct Piece {
     int count, unit, kvh, none;  // count: pieces of the context; 0: this part has none
 };
-// Of the step: pieces of the context (0: no key is seen).
+// Of the step: pieces of the context (0: no key is seen), and whether a workgroup per head merges them.
 struct StepInfo {
-    int pieces;
+    int pieces, merged;
 };
 
 struct ResidentPlan {
@@ -658,7 +663,7 @@ struct Front {
     __device__ __forceinline__ Front(Plan& p, char* l, int r, int n_, int t)
         : lds(l), rank(r), n(n_), tid(t), lane(t & 63), wave(uniform(t >> 6)), parts(p.parts), layers(p.layers),
           words(p.region, p.bytes), budget(p.polls), pieces(uniform_load(&info(p)->pieces)),
-          many(pieces * p.hq * (D + 2) > kDirectWords), pos(uniform_load(p.positions)),
+          many(uniform_load(&info(p)->merged)), pos(uniform_load(p.positions)),
           slot(uniform_load(p.slot_mapping)), et(t >> 4), en(t & 15) {}
     static __device__ __forceinline__ const StepInfo* info(Plan& p) {
         return reinterpret_cast<const StepInfo*>(p.region + p.at_step);
@@ -1238,7 +1243,8 @@ __global__ __launch_bounds__(64 * kStreamWaves) void decode_resident_init_kernel
         if (v == 0) {
             unsigned* const ctl = reinterpret_cast<unsigned*>(p.region);
             ctl[0] = ctl[1] = ctl[2] = 0;
-            reinterpret_cast<StepInfo*>(p.region + p.at_step)->pieces = pieces;
+            *reinterpret_cast<StepInfo*>(p.region + p.at_step) =
+                StepInfo{pieces, pieces && (p.hq * D > kDirectColumns || pieces * p.hq * (D + 2) > kDirectWords)};
         }
     }
     uint4_t* const list = reinterpret_cast<uint4_t*>(p.region + p.at_lists) + ((size_t)v * kStreamWaves + wave) * p.list;

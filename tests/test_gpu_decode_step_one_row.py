@@ -24,6 +24,8 @@ SHAPES = [  # hidden, query heads, KV heads, head width, MLP width, context, row
     (512, 8, 2, 64, 16384, 70, 64),        # the widest operand
     (512, 64, 8, 128, 512, 100, 16),       # one piece of a group's eight heads: 56 workgroups that merge a head have
                                            # q/k/v tiles and no piece of the context
+    (512, 8, 2, 64, 512, 1000, 16),        # eight pieces, read by the o projection itself in two rounds
+    (512, 24, 8, 64, 512, 500, 16),        # the most columns of heads that are read so
 ]
 
 
