@@ -1305,15 +1305,6 @@ bool resident_plan(const logismos_decode_config_t& c, ResidentPlan* p) {
     if (group > 16 || c.intermediate > 16384 || qd > 16384 || width > 32768) return false;
     const int cus = device_cu_count(), parts = cus < kMaxParts ? cus : kMaxParts;
     if (c.num_kv_heads > parts) return false;
-    // Long contexts: this kernel's attention reads K and V at 5.7 TB/s, the launches' at 7 (with one or two KV heads less),
-    // so that from some size on their stream outweighs the chain of launches.  us of eight layers with a full
-    // table, launches / here, at 256 | 384 | 512 MiB of K and V per layer: 32 KV heads of 128 762 / 740 | 916 / 926 |
-    // 1085 / 1117; 8 heads 795 / 737 | 963 / 935 | 1117 / 1133; 4 heads 711 / 661 | 887 / 860 | 1059 / 1058; 16 heads of
-    // 64 790 / 721 | 960 / 920 | 1112 / 1110; at 512 and 768 MiB 2 heads of 128 1184 / 1049 and 1520 / 1441, of 64
-    // 1017 / 997 and 1365 / 1383.  The host knows
-    // what the table can hold, not what it holds: the lines lie where a full one is still no slower.
-    const int64_t kv_bytes = 4 * (int64_t)c.num_kv_heads * d * c.block_size * c.max_blocks_per_seq;
-    if (kv_bytes > (c.num_kv_heads <= 2 ? (int64_t)512 : (int64_t)320) << 20) return false;
     *p = ResidentPlan{};
     p->layers = c.num_layers;
     p->hidden = c.hidden;
@@ -1434,6 +1425,24 @@ size_t decode_resident_bytes(const logismos_decode_config_t& c) {
     return resident_plan(c, &p) ? p.bytes + table_bytes(c) : 0;
 }
 
+// Few layers: the lists, the words' zeros and the start of the kernel are 10 to 15 us that the layers have to earn.  us at
+// 500 keys, launches / here, 2 | 4 | 8 layers: width 512 44 / 42 | 91 / 72 | 179 / 129; 896 51 / 52 | 103 / 92 | 206 / 167; 1536
+// (MLP of 8960) 59 / 63 | 117 / 112 | 229 / 213.  Wider, where a layer's weights take up more of it, 8 | 16 | 28 layers: 2048
+// (MLP of 11008, two KV heads) 254 / 276 | 523 / 540 | 940 / 927; 3072 (four KV heads) 329 / 339 | 681 / 667; 3584 (MLP of
+// 9472) 315 / 340 | 656 / 662 | 1148 / 1149; but 2048 (MLP of 6144) 257 / 190 and 4096 394 / 326 at 8.  Of 45 widths,
+// heads and MLP widths, each at 500 and 4000 keys, those past the lines below take 0.66 to 1.03 of the launches' time.
+//
+// Long contexts: this kernel's attention reads K and V at 5.7 TB/s, the launches' at 7 (with one or two KV heads less), so
+// that from some size on their stream outweighs the chain of launches.  us of eight layers with a full table, launches /
+// here, at 256 | 384 | 512 MiB of K and V per layer: 32 KV heads of 128 762 / 740 | 916 / 926 | 1085 / 1117; 8 heads
+// 795 / 737 | 963 / 935 | 1117 / 1133; 4 heads 711 / 661 | 887 / 860 | 1059 / 1058; 16 heads of 64 790 / 721 | 960 / 920 |
+// 1112 / 1110; at 512 and 768 MiB 2 heads of 128 1184 / 1049 and 1520 / 1441, of 64 1017 / 997 and 1365 / 1383.  The
+// host knows what the table can hold, not what it holds: the lines lie where a full one is still no slower.
+bool decode_resident_pays(const logismos_decode_config_t& c) {
+    const int64_t kv_bytes = 4 * (int64_t)c.num_kv_heads * c.head_dim * c.block_size * c.max_blocks_per_seq;
+    return c.num_layers >= (c.hidden <= 1536 ? 4 : 16) && kv_bytes <= (c.num_kv_heads <= 2 ? (int64_t)512 : 320) << 20;
+}
+
 bool decode_resident_applies(const logismos_decode_config_t& c, const logismos_decode_layer_t* layers,
                              const logismos_decode_batch_t& b, int t) {
     ResidentPlan p;
@@ -1474,7 +1483,8 @@ hipError_t decode_resident_launch(const logismos_decode_config_t& c, const logis
 
 }  // namespace lg
 
-// The launch by itself, for the tests (the header does not declare it).
+// The launch by itself and its rule, for the tests (the header does not declare them).
+extern "C" int lg_decode_resident_pays(const logismos_decode_config_t* cfg) { return lg::decode_resident_pays(*cfg); }
 extern "C" size_t lg_decode_resident_bytes(const logismos_decode_config_t* cfg) {
     return lg::decode_resident_bytes(*cfg);
 }

@@ -11,7 +11,10 @@ namespace lg {
 // Bytes of the step's workspace that the launch uses: 0 where the geometry is not one of its own.
 size_t decode_resident_bytes(const logismos_decode_config_t& c);
 
-// Whether a step of t rows over these operands runs there.
+// Whether a step of one row is better there than operator by operator.
+bool decode_resident_pays(const logismos_decode_config_t& c);
+
+// Whether a step of t rows over these operands can run there.
 bool decode_resident_applies(const logismos_decode_config_t& c, const logismos_decode_layer_t* layers,
                              const logismos_decode_batch_t& b, int t);
 

@@ -43,8 +43,8 @@ struct Workspace {
                       // steps; a many-row step has t_xn free by then)
     char* last_rows;  // bf16 [num_seqs][hidden]: the normed last rows, gathered
     char* last_xn;    // prepared activations of one chunk of them
-    char* resident;   // of the resident launch; in every step's workspace, so that one for many rows
-                      // is one for few
+    char* resident;   // of the resident launch, where one row would take it; in every step's workspace, so
+                      // that one for many rows is one for few
     bool tall;
     size_t xn_stride;
     int chunks;        // of 32 rows
@@ -91,7 +91,7 @@ Workspace carve(const logismos_decode_config_t& c, int num_seqs, int t, int num_
             w.head_ws =
                 take(logismos_qgemm_q4g128_greedy_workspace_bytes(kChunkRows, c.vocab, c.hidden));
         }
-        w.resident = take(lg::decode_resident_bytes(c));
+        w.resident = take(lg::decode_resident_pays(c) ? lg::decode_resident_bytes(c) : 0);
         w.total = off;
         return w;
     }
@@ -135,7 +135,7 @@ Workspace carve(const logismos_decode_config_t& c, int num_seqs, int t, int num_
         w.last_rows = take((size_t)num_seqs * c.hidden * 2);
         w.last_xn = take(logismos_q4_xprep_bytes(kChunkRows, c.hidden));
     }
-    w.resident = take(lg::decode_resident_bytes(c));
+    w.resident = take(lg::decode_resident_pays(c) ? lg::decode_resident_bytes(c) : 0);
     w.total = off;
     return w;
 }
@@ -334,8 +334,11 @@ int batch_max_q(const logismos_decode_batch_t* b) {
     return b->max_seqlen_q > 0 ? b->max_seqlen_q : 1;
 }
 
+// How the layers of a step of one row are launched.
+enum OneRow { kWhatIsFaster, kPerOperator, kOneLaunch };
+
 logismos_status_t launch_step(const logismos_decode_config_t* cfg, const logismos_decode_layer_t* layers,
-                              const logismos_decode_batch_t* batch, void* workspace, bool per_operator,
+                              const logismos_decode_batch_t* batch, void* workspace, OneRow one_row,
                               logismos_stream_t stream);
 
 }  // namespace
@@ -357,21 +360,28 @@ extern "C" logismos_status_t logismos_launch_decode_step(const logismos_decode_c
                                                          const logismos_decode_batch_t* batch,
                                                          void* workspace,
                                                          logismos_stream_t stream) {
-    return launch_step(cfg, layers, batch, workspace, false, stream);
+    return launch_step(cfg, layers, batch, workspace, kWhatIsFaster, stream);
 }
 extern "C" logismos_status_t logismos_launch_decode_step_per_operator(const logismos_decode_config_t* cfg,
                                                                       const logismos_decode_layer_t* layers,
                                                                       const logismos_decode_batch_t* batch,
                                                                       void* workspace,
                                                                       logismos_stream_t stream) {
-    return launch_step(cfg, layers, batch, workspace, true, stream);
+    return launch_step(cfg, layers, batch, workspace, kPerOperator, stream);
+}
+// For the tests (the header does not declare it): one launch where it is possible at all, otherwise refused.  The
+// workspace holds lg_decode_resident_bytes() more.
+extern "C" logismos_status_t lg_launch_decode_step_one_launch(const logismos_decode_config_t* cfg,
+                                                              const logismos_decode_layer_t* layers,
+                                                              const logismos_decode_batch_t* batch, void* workspace,
+                                                              logismos_stream_t stream) {
+    return launch_step(cfg, layers, batch, workspace, kOneLaunch, stream);
 }
 
 namespace {
 
-// per_operator: no launch takes several operators that depend on one another's whole results.
 logismos_status_t launch_step(const logismos_decode_config_t* cfg, const logismos_decode_layer_t* layers,
-                              const logismos_decode_batch_t* batch, void* workspace, bool per_operator,
+                              const logismos_decode_batch_t* batch, void* workspace, OneRow one_row,
                               logismos_stream_t stream) {
     if (!cfg || !layers || !batch || !workspace) return hipErrorInvalidValue;
     const int num_seqs = batch->num_seqs;
@@ -434,6 +444,9 @@ logismos_status_t launch_step(const logismos_decode_config_t* cfg, const logismo
                                                                 c.num_kv_heads, c.block_size,
                                                                 c.max_blocks_per_seq, max_q, batch->num_splits);
     float* const h = static_cast<float*>(batch->hidden_f32);
+    const bool one_launch = (one_row == kOneLaunch || (one_row == kWhatIsFaster && lg::decode_resident_pays(c))) &&
+                            lg::decode_resident_applies(c, layers, *batch, t);
+    if (one_row == kOneLaunch && !one_launch) return hipErrorInvalidValue;
 
     if (tokens_in)
         LG_TRY(logismos_launch_embed_lookup_bf16(batch->embed_table_bf16, batch->token_ids,
@@ -566,7 +579,7 @@ logismos_status_t launch_step(const logismos_decode_config_t* cfg, const logismo
         return last_only ? project_last_rows() : 0;
     }
     int res_parts = 0;  // split-K parts of the last down projection not yet folded into h
-    if (!per_operator && lg::decode_resident_applies(c, layers, *batch, t)) {
+    if (one_launch) {
         LG_TRY(lg::decode_resident_launch(c, layers, *batch, w.resident, static_cast<hipStream_t>(stream)));
     } else if (few_rows(c, layers, t)) {
         LG_TRY(few_rows_layers(c, layers, batch, w, t, max_q, direct, &res_parts, stream));

@@ -1,14 +1,17 @@
 """A step of one row, whose layers are one resident launch (decode_resident.hip): edges of its lists and
 pieces against the oracle, any number of workgroups bit for bit, and against the route of 2 to 16 rows."""
+import copy
 import ctypes as C
 
 import numpy as np
 import pytest
 
+import oracle as O
 from logismos_amd import hip, kernels
+from oracle import decode_step as OS
 from tests import workloads
 from tests.gpu_harness import DecodeStepRunner, PagedAttnRunner
-from tests.test_gpu_decode_step import _rel_l2, _run_both
+from tests.test_gpu_decode_step import _rel_l2
 
 pytestmark = pytest.mark.gpu
 
@@ -55,11 +58,32 @@ def _lib():
     return size, launch
 
 
+class OneLaunch(DecodeStepRunner):
+    """A step of one row whose layers are one launch whether that pays or not."""
+
+    def __init__(self, cfg, layers, batch, **kw):
+        super().__init__(cfg, layers, batch, **kw)
+        self.ws = hip.DeviceBuffer(self.ws.nbytes + _lib()[0](C.byref(self.cfg)))
+        self.ws.fill(0xFF)
+
+    def launch(self):
+        lib = C.CDLL(kernels.library()._name)
+        assert lib.lg_launch_decode_step_one_launch(C.byref(self.cfg), self.layers, C.byref(self.batch), self.ws.ptr,
+                                                    self.stream.raw if self.stream else None) == 0
+
+
+def _run_both(cfg, layers, batch):
+    r = OneLaunch(cfg, layers, batch)
+    r.launch()
+    got = O.bf16_bits_to_f32(r.result_bits())
+    lay, bat = copy.deepcopy(layers), dict(batch, h=batch["h"].copy())
+    return r, got, O.bf16_bits_to_f32(OS.decode_step(cfg, lay, bat)), lay, bat
+
+
 @pytest.mark.parametrize("shape", SHAPES)
 def test_against_the_oracle(shape):
     cfg, layers, batch = _problem(shape)
     r, got, want, lay, bat = _run_both(cfg, layers, batch)
-    assert _lib()[0](C.byref(r.cfg)) > 0  # the resident launch takes it
     # one layer: the decode batch's bounds (tests/test_gpu_decode_step.py)
     assert _rel_l2(got, want) < 6e-3
     assert np.all(np.abs(got - want) <= 1.5e-2 + 2e-2 * np.abs(want))
@@ -75,7 +99,7 @@ def test_against_the_oracle(shape):
 def test_any_number_of_workgroups(shape, workgroups):
     # the work is cut for all compute units; fewer workgroups take several parts each, phase by phase
     cfg, layers, batch = _problem(shape, layers=3)
-    whole = DecodeStepRunner(cfg, layers, batch)
+    whole = OneLaunch(cfg, layers, batch)
     size, launch = _lib()
     want = None
     for n in (0, workgroups, workgroups):
@@ -115,13 +139,13 @@ def test_closed_before_all_workgroups_are_there(shape):
 def test_beside_another_stream():
     # prompt attention on another stream holds compute units for longer than a step waits for them
     cfg, layers, batch = _problem(SHAPES[2], layers=3)
-    alone = DecodeStepRunner(cfg, layers, batch)
+    alone = OneLaunch(cfg, layers, batch)
     alone.launch()
     want = _state(alone, batch, layers)
     other = PagedAttnRunner(workloads.paged_case(np.random.default_rng(1), [64], [20000], hq=32, hkv=8,
                                                  pool_period_rows=4096), stream=hip.Stream())
     stream = hip.Stream()
-    steps = [DecodeStepRunner(cfg, layers, batch, stream=stream) for _ in range(6)]
+    steps = [OneLaunch(cfg, layers, batch, stream=stream) for _ in range(6)]
     hip.synchronize()
     for _ in range(10):
         other.launch()
@@ -144,7 +168,7 @@ def test_against_the_route_of_more_rows(shape, slot):
         batch["slots"] = np.array([-1 if slot == "none" else int(table[2]) * bs + 5], np.int64)
     states = []
     for off in (0, 4):
-        r = DecodeStepRunner(cfg, layers, batch)
+        r = (DecodeStepRunner if off else OneLaunch)(cfg, layers, batch)
         if off:
             for lay, L in zip(r.layers, layers):
                 s = np.ascontiguousarray(L["qkv"][1]).view(np.uint16).reshape(-1)
@@ -169,7 +193,7 @@ def test_against_the_route_of_more_rows(shape, slot):
 @pytest.mark.parametrize("hq,hkv,d,mib", [(8, 2, 128, 512), (8, 4, 64, 320), (4, 4, 128, 320)])
 def test_tables_too_long_for_one_launch(hq, hkv, d, mib):
     # past so many bytes of K and V that a layer's table can hold a step is launched operator by operator
-    cfg, layers, batch = _problem((512, hq, hkv, d, 512, 200, 16))
+    cfg, layers, batch = _problem((512, hq, hkv, d, 512, 200, 16), layers=4)
     blocks = (mib << 20) // (4 * hkv * d * 16)
     states = []
     for more in (0, 1):
@@ -179,7 +203,7 @@ def test_tables_too_long_for_one_launch(hq, hkv, d, mib):
         for name in ("cos", "sin"):
             b[name] = np.resize(batch[name], (b["block_tables"].shape[1] * 16, d // 2))
         r = DecodeStepRunner(cfg, layers, b)
-        assert (_lib()[0](C.byref(r.cfg)) > 0) == (more == 0)
+        assert C.CDLL(kernels.library()._name).lg_decode_resident_pays(C.byref(r.cfg)) == (more == 0)
         for call in (kernels.launch_decode_step, kernels.launch_decode_step_per_operator):
             r.h.copy_from_host(batch["h"].astype(np.float32))
             call(r.cfg, r.layers, r.batch, r.ws)
@@ -188,11 +212,30 @@ def test_tables_too_long_for_one_launch(hq, hkv, d, mib):
     assert np.array_equal(states[2][1], states[3][1]) and np.array_equal(states[2][0], states[3][0])
 
 
+@pytest.mark.parametrize("hidden,layers,pays", [(512, 3, 0), (512, 4, 1), (1536, 4, 1), (1664, 15, 0), (1664, 16, 1)])
+def test_few_layers_are_launched_operator_by_operator(hidden, layers, pays):
+    cfg, lay, batch = _problem((hidden, 4, 2, 64, 256, 40, 16), layers=layers)
+    r = DecodeStepRunner(cfg, lay, batch)
+    assert C.CDLL(kernels.library()._name).lg_decode_resident_pays(C.byref(r.cfg)) == pays
+    states = []
+    for call in (r.launch, lambda: kernels.launch_decode_step_per_operator(r.cfg, r.layers, r.batch, r.ws),
+                 OneLaunch.launch):
+        if call == OneLaunch.launch:
+            r = OneLaunch(cfg, lay, batch)
+            call = r.launch
+        r.h.copy_from_host(batch["h"].astype(np.float32))
+        call()
+        states.append(_state(r, batch, lay)[1])
+    # the route that it takes bit for bit; the other is last bits of bf16 values away, through the layers
+    assert np.array_equal(states[0], states[2 if pays else 1])
+    assert _rel_l2(states[1], states[2]) < 1e-2
+
+
 @pytest.mark.parametrize("rows", [1, 2, 16, 40])
 def test_a_launch_per_operator(rows):
     # at one row the route of 2 to 16 rows (what scales off 16 bytes take, bit for bit), otherwise the same step
     cfg, layers, batch = workloads.decode_step_problem(
-        np.random.default_rng(rows), num_layers=2, hidden=512, hq=8, hkv=2, inter=768, ctx=[300] * rows, qkv_bias=True)
+        np.random.default_rng(rows), num_layers=4, hidden=512, hq=8, hkv=2, inter=768, ctx=[300] * rows, qkv_bias=True)
     states = []
     for per_operator in (False, True):
         r = DecodeStepRunner(cfg, layers, batch)
@@ -266,7 +309,7 @@ def test_a_wait_that_runs_out_shows(shape):
             assert not np.isnan(got.view(np.float16)).any()
             assert set(np.nonzero((got != L[name].view(np.uint16)).any(axis=1))[0]) <= {slot}
     # the next step over the same region is a step like any other
-    want = DecodeStepRunner(cfg, layers, batch)
+    want = OneLaunch(cfg, layers, batch)
     want.launch()
     r.h.copy_from_host(batch["h"].astype(np.float32))
     assert launch(C.byref(r.cfg), r.layers, C.byref(r.batch), region.ptr) == 0
@@ -288,7 +331,6 @@ def test_pieces_of_keys_that_have_no_weight(shape):
         rows = batch["block_tables"][0][key // block].astype(np.int64) * block + key % block
         L["k_pool"][rows[:, None], np.arange(hkv) * d] = -np.inf
         r, got, want, _, bat = _run_both(cfg, layers, batch)
-        assert _lib()[0](C.byref(r.cfg)) > 0
         assert np.isfinite(want).all() and np.isfinite(got).all()
         assert _rel_l2(got, want) < 6e-3
         assert _rel_l2(r.h.to_numpy(np.float32, bat["h"].shape), bat["h"]) < 6e-3
