@@ -67,6 +67,9 @@ STEPS = {
     # 142 packed rows: the tiled GEMMs with their workspace and split tiles, the prefill kernel
     "many_rows": dict(num_layers=2, hidden=512, hq=4, hkv=2, inter=1024,
                       ctx=[700, 140, 3, 33, 37], new_tokens=[1, 100, 3, 1, 37], qkv_bias=True),
+    # one row: one launch for all layers, whose words every replay has to clear, and the operands of 26 layers handed over
+    # by two
+    "one_row": dict(num_layers=26, hidden=512, hq=8, hkv=2, inter=768, ctx=[700]),
     # TurboQuant-3 pools
     "turbo3": dict(num_layers=2, hidden=1024, hq=8, hkv=2, inter=2048,
                    ctx=[1, 17, 300, 64, 999, 5], kv_turbo3=True),
@@ -75,7 +78,7 @@ STEPS = {
 
 @pytest.mark.parametrize("kind", sorted(STEPS))
 def test_replays_of_a_captured_step_equal_the_eager_step(kind):
-    rng = np.random.default_rng({"decode": 11, "tokens": 12, "many_rows": 13, "turbo3": 14}[kind])
+    rng = np.random.default_rng({"decode": 11, "tokens": 12, "many_rows": 13, "turbo3": 14, "one_row": 15}[kind])
     cfg, layers, batch = workloads.decode_step_problem(rng, **STEPS[kind])
     stream = hip.Stream()
     eager = DecodeStepRunner(cfg, layers, batch, stream=stream)
