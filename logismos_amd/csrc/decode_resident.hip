@@ -20,12 +20,12 @@
 // the context for one KV head per workgroup | (merge of the pieces) | o projection + residual | row
 // normed -> gate/up, SwiGLU | down projection + residual.
 //
-// What bounds it, from clock stamps at widths 896 / 4096 (us per layer 20 / 40): six exchanges of 2-4 us,
-// of which the poll 1.3-2 and what follows it up to the barrier 1; products 0.6-2 / 1-8 (gate/up waits for memory:
-// 370 KiB per compute unit and layer at 23-27 B/ns); epilogues 0.6 each.  A compute unit's requests return in order, so
-// a poll also waits for what the streaming waves asked for before it.  Every instruction of a front wave is on the
-// chain: for two to four rows the same kernel was slower than the launches it replaces (0.81-1.01 of their speed),
-// hence one row.
+// What bounds it, from clock stamps at widths 896 / 4096 (us per layer 20 / 40): five exchanges of 2-4 us (six where the
+// pieces are merged), of which the poll 1.3-2 and what follows it up to the barrier 1; products 0.6-2 / 1-8 (at
+// 4096 they wait for memory: 370 KiB per compute unit and layer at 23-27 B/ns, 192 of them gate/up); epilogues 0.6 each.
+// A compute unit's requests return in order, so a poll also waits for what the streaming waves asked for before it.
+// Every instruction of a front wave is on the chain: for two to four rows the same kernel was slower than the launches it
+// replaces (0.81-1.01 of their speed), hence one row.
 //
 // Steps of one row, us (six launches a layer / here): 24 layers of 896 at 500 keys 674 / 502, 28 of 1536 at 4000 keys
 // 912 / 773, 36 of 4096 at 1500 keys 1885 / 1524.
@@ -37,7 +37,10 @@
 // Waits end: a launch does not assume that all of its workgroups run at once.  Each takes a ticket;
 // the last one, or one that has waited 100 us, closes the step to the n workgroups that hold tickets so
 // far, which are all running; later ones leave.  Workgroup r does the parts r, r + n, ... of the V, so
-// results do not depend on n.  A tag is written by whoever owns the value in every case, whatever the
+// results do not depend on n.  Times do (us with 256 | 255 | 128 | 64 | 32 | 10 workgroups: 24 layers of 896 473 | 635 | 580 |
+// 833 | 1470 | 4591, 36 of 4096 1425 | 2317 | 2398 | 4441 | 8427 | 26900): a wave with several parts requests no
+// weights ahead of its phase.  Waiting longer than 100 us was measured beside GEMMs, prompt attention and other steps on a
+// second stream and gained in none of them.  A tag is written by whoever owns the value in every case, whatever the
 // batch holds.  A budget of polls bounds the kernel even so.  A wave that has spent it says so in the region, and
 // all that its workgroup publishes from there on is NaN, which every product behind it hands on: the residual stream
 // ends as NaN, and K/V rows that are NaN on that account are left out of the pools.
@@ -64,6 +67,7 @@ constexpr int kFrontWaves = 4;
 constexpr int kFrontThreads = 64 * kFrontWaves;
 constexpr int kThreads = 64 * (kStreamWaves + kFrontWaves);
 constexpr int kSlot = 4096;         // bytes of a ring slot: four requests of a wave
+// (24 layers of 896 with 2 | 3 | 4 | 5 slots: 505 | 485 | 480 | 480 us; 28 of 1536 792 | 777 | 777 | 777)
 constexpr int kMaxSlots = 4;
 constexpr int kResLds = 160 * 1024;
 constexpr int kMaxParts = 256;      // V: parts the work is cut into, and pieces of its attention

@@ -572,7 +572,8 @@ hipError_t rows_prep_launch(const RowsArgs& a, hipStream_t st) {
 }
 template <int W, int DW>
 hipError_t rows_prep(const RowsArgs& a, hipStream_t st) {
-    if (a.e.out_f32 && qgemm_q4_rows_res_parts(a.tiles, a.k) == 2) return rows_prep_launch<W, DW, kPrepTwoParts>(a, st);
+    if constexpr (W == 16)  // (two parts are of more groups than eight waves ever take)
+        if (a.e.out_f32 && qgemm_q4_rows_res_parts(a.tiles, a.k) == 2) return rows_prep_launch<W, DW, kPrepTwoParts>(a, st);
     if (a.e.pending) return rows_prep_launch<W, DW, kPrepPending>(a, st);
     return rows_prep_launch<W, DW, kPrepPlain>(a, st);
 }
@@ -589,8 +590,11 @@ bool qgemm_q4_rows_applies(int b, int hidden, int widest, int qkv, const void* s
 // Two parts where a wave of one has more groups than it keeps in flight (16 waves of three groups), both
 // parts' workgroups, one to a compute unit, run at once, and the norm that takes the rest is one of the narrow ones
 // (up to 2048 columns): 1536 x 8960 is 96 workgroups of 70 groups.  28 layers of it, us per step, one part / two:
-// 2 rows 899 / 854, 8 rows 936 / 912, 12 rows 1055 / 1010, 16 rows 1157 / 1108.  (From 24 groups on, 896 x 4864
-// of 56 workgroups too: no difference.)
+// 2 rows 899 / 854, 8 rows 936 / 912, 12 rows 1055 / 1010, 16 rows 1157 / 1108.  Eight layers of widths 512 to 2048 with
+// 6400 to 16384, 2 to 16 rows: 0.935 to 0.99 of one part's time up to 1536, 0.96 to 1.006 at 2048 (2 rows of 512 x 6400
+// 207.7 / 201.2, 16 of 2048 x 16384 364.4 / 364.4).  The norm that reads the rest pays part of it back: q/k/v of 1536 at 16
+// rows takes 7.8 instead of 6.5, the down projection 6.9 instead of 10.1.  (From 24 groups on, 896 x 4864 of 56
+// workgroups too: no difference.)
 int qgemm_q4_rows_res_parts(int tiles, int k) {
     return (k >> 7) > 48 && tiles <= 128 && 2 * tiles <= device_cu_count() ? 2 : 1;
 }
