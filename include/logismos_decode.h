@@ -740,7 +740,7 @@ typedef struct {
      * rows and the largest number of new tokens of a sequence; 0 / 0 means one new token per
      * sequence.  Every per-row array above (hidden_f32, out_bf16, positions, slot_mapping) then
      * has total_tokens rows, in packed order.  A step of one row over fp16 pools (heads of 64 or 128, hidden up
-     * to 4096, block tables for up to 320 MiB of K and V per layer, 512 MiB with one or two KV heads; scales, gains,
+     * to 4096; four layers or more up to a hidden of 1536, 16 beyond; block tables for up to 320 MiB of K and V per layer, 512 MiB with one or two KV heads; scales, gains,
      * pools and hidden_f32 on 16 bytes) is one launch for all layers that takes every compute unit it can
      * get for the whole step (see logismos_launch_decode_step_per_operator); its workgroups wait for one another's
      * results, and should such a wait run out (after seconds), hidden_f32 ends as NaN and no K/V row that follows

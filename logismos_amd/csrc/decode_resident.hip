@@ -1432,9 +1432,11 @@ size_t decode_resident_bytes(const logismos_decode_config_t& c) {
 // Few layers: the lists, the words' zeros and the start of the kernel are 10 to 15 us that the layers have to earn.  us at
 // 500 keys, launches / here, 2 | 4 | 8 layers: width 512 44 / 42 | 91 / 72 | 179 / 129; 896 51 / 52 | 103 / 92 | 206 / 167; 1536
 // (MLP of 8960) 59 / 63 | 117 / 112 | 229 / 213.  Wider, where a layer's weights take up more of it, 8 | 16 | 28 layers: 2048
-// (MLP of 11008, two KV heads) 254 / 276 | 523 / 540 | 940 / 927; 3072 (four KV heads) 329 / 339 | 681 / 667; 3584 (MLP of
-// 9472) 315 / 340 | 656 / 662 | 1148 / 1149; but 2048 (MLP of 6144) 257 / 190 and 4096 394 / 326 at 8.  Of 45 widths,
-// heads and MLP widths, each at 500 and 4000 keys, those past the lines below take 0.66 to 1.03 of the launches' time.
+// (MLP of 11008, two KV heads) 254 / 276 | 520 / 543 | 934 / 940; 3072 (four KV heads) 329 / 339 | 681 / 667; 3584 (MLP of
+// 9472) 315 / 340 | 660 / 668 | 1155 / 1156; but 2048 (MLP of 6144) 257 / 190 and 4096 394 / 326 at 8.  40 geometries at 500 and
+// 4000 keys and 4, 8, 16 or 28 layers past the lines below take 0.60 to 1.05 of the launches' time, 0.83 on average.
+// More than 1 % longer: the first of these at 500 keys (at 4000 552 / 531 and 997 / 921), and 3584 with 28 KV heads at 4000
+// keys (803 / 826, at 500 714 / 687).
 //
 // Long contexts: this kernel's attention reads K and V at 5.7 TB/s, the launches' at 7 (with one or two KV heads less), so
 // that from some size on their stream outweighs the chain of launches.  us of eight layers with a full table, launches /
