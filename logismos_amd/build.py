@@ -56,8 +56,11 @@ EXTRA_FLAGS = {
 
 # Kernels that ask for operands in one assembly statement and wait for them in a later one, so that
 # work lies between the two.  A register that the compiler moved to memory (or copied) in between
-# would keep what it held before the read, with no error: a build in which one of them spills is refused.
-READS_IN_FLIGHT = ("qgemm_q4g128_tallp_kernel", "matmul_ring_fp16_kernel", "paged_attn_chunk64_kernel")
+# would keep what it held before the read, with no error: a build in which one of them spills is refused.  So is one of
+# decode_resident_kernel, whose requests go straight into LDS: there a reload from scratch waits for all of them
+# (24 layers of width 896 6 % slower).
+READS_IN_FLIGHT = ("qgemm_q4g128_tallp_kernel", "matmul_ring_fp16_kernel", "paged_attn_chunk64_kernel",
+                   "decode_resident_kernel")
 
 
 def spills(remarks: str) -> list[str]:

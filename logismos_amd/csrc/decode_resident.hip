@@ -25,7 +25,8 @@
 // 4096 they wait for memory: 370 KiB per compute unit and layer at 23-27 B/ns, 192 of them gate/up); epilogues 0.6 each.
 // A compute unit's requests return in order, so a poll also waits for what the streaming waves asked for before it.
 // Every instruction of a front wave is on the chain: for two to four rows the same kernel was slower than the launches it
-// replaces (0.81-1.01 of their speed), hence one row.
+// replaces (0.81-1.01 of their speed), hence one row.  (More uniform values are alive than there are scalar registers: 80-odd
+// of each instance lie in lanes of vector registers.  The build refuses one that spills a vector register.)
 //
 // Steps of one row, us (six launches a layer / here): 24 layers of 896 at 500 keys 674 / 502, 28 of 1536 at 4000 keys
 // 912 / 773, 36 of 4096 at 1500 keys 1885 / 1524.
